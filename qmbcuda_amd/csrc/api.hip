@@ -46,22 +46,13 @@ constexpr int kScanThreads = 256;
 constexpr int kScanItems = 8;
 constexpr int kScanTile = kScanThreads * kScanItems;
 
-template <class T>
-__device__ inline T block_exclusive_scan(T v, T *lds, T &total) {
-    // Hillis-Steele over 256 values in LDS; fine for tile-level use.
-    const int t = threadIdx.x;
-    lds[t] = v;
-    __syncthreads();
-    for (int off = 1; off < kScanThreads; off <<= 1) {
-        T add = (t >= off) ? lds[t - off] : T(0);
-        __syncthreads();
-        lds[t] += add;
-        __syncthreads();
+// Inclusive sums over the lanes of a wavefront.
+__device__ inline int64_t wave_inclusive(int64_t v) {
+    for (int off = 1; off < 64; off <<= 1) {
+        const int64_t o = __shfl_up(v, off, 64);
+        v += (int)(threadIdx.x & 63) >= off ? o : 0;
     }
-    total = lds[kScanThreads - 1];
-    T incl = lds[t];
-    __syncthreads();
-    return incl - v;
+    return v;
 }
 
 // bit words at stride 2 (the rank dictionary's records)
@@ -75,31 +66,47 @@ struct ArraySrc {
     __device__ int64_t operator()(int64_t i) const { return v[i]; }
 };
 
+// Sum of each tile (in any order: integers).
 template <class Src>
 __global__ __launch_bounds__(kScanThreads) void scan_tile_sums(Src src, int64_t n, int64_t *tile_sums) {
-    __shared__ int64_t lds[kScanThreads];
-    const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanItems;
+    __shared__ int64_t lds[kScanThreads / 64];
+    const int64_t base = (int64_t)blockIdx.x * kScanTile + threadIdx.x;
     int64_t s = 0;
+#pragma unroll
     for (int i = 0; i < kScanItems; ++i)
-        if (base + i < n) s += src(base + i);
-    int64_t total;
-    block_exclusive_scan<int64_t>(s, lds, total);
-    if (threadIdx.x == 0) tile_sums[blockIdx.x] = total;
+        if (base + i * kScanThreads < n) s += src(base + i * kScanThreads);
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int64_t t = 0;
+        for (int w = 0; w < kScanThreads / 64; ++w) t += lds[w];
+        tile_sums[blockIdx.x] = t;
+    }
 }
 
 // Single-block exclusive scan of the tile sums (in place); writes the grand total
 // at [n] and, when total_out is set, there too.
-__global__ __launch_bounds__(kScanThreads) void scan_tile_offsets(int64_t *tile_sums, int64_t n,
-                                                                  int64_t *total_out) {
-    __shared__ int64_t lds[kScanThreads];
+constexpr int kOffsetThreads = 1024;
+__global__ __launch_bounds__(kOffsetThreads) void scan_tile_offsets(int64_t *tile_sums, int64_t n,
+                                                                    int64_t *total_out) {
+    __shared__ int64_t lds[kOffsetThreads / 64];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     int64_t carry = 0;
-    for (int64_t base = 0; base < n; base += kScanThreads) {
+    for (int64_t base = 0; base < n; base += kOffsetThreads) {
         const int64_t i = base + threadIdx.x;
         const int64_t v = i < n ? tile_sums[i] : 0;
-        int64_t total;
-        const int64_t ex = block_exclusive_scan<int64_t>(v, lds, total);
-        if (i < n) tile_sums[i] = carry + ex;
+        const int64_t incl = wave_inclusive(v);
+        if (lane == 63) lds[wv] = incl;
+        __syncthreads();
+        int64_t below = carry, total = 0;
+        for (int w = 0; w < kOffsetThreads / 64; ++w) {
+            below += w < wv ? lds[w] : 0;
+            total += lds[w];
+        }
+        if (i < n) tile_sums[i] = below + incl - v;
         carry += total;
+        __syncthreads();
     }
     if (threadIdx.x == 0) {
         tile_sums[n] = carry;
@@ -107,23 +114,38 @@ __global__ __launch_bounds__(kScanThreads) void scan_tile_offsets(int64_t *tile_
     }
 }
 
-// out[i * stride + offset] = exclusive prefix of element i
+// out[i * stride + offset] = exclusive prefix of element i. A wavefront takes
+// kScanItems * 64 consecutive elements, 64 (one coalesced access) at a time.
+// tile_off NULL: the only tile; its sum goes to total (and total_out when set).
 template <class Src, class Out>
 __global__ __launch_bounds__(kScanThreads) void scan_write(Src src, int64_t n, const int64_t *tile_off,
-                                                           Out *out, int stride, int offset) {
-    __shared__ int64_t lds[kScanThreads];
-    const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanItems;
-    int64_t vals[kScanItems];
-    int64_t s = 0;
+                                                           Out *out, int stride, int offset, int64_t *total,
+                                                           int64_t *total_out) {
+    __shared__ int64_t lds[kScanThreads / 64];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)wv * kScanItems * 64 + lane;
+    int64_t before[kScanItems];
+    int64_t run = 0;
+#pragma unroll
     for (int i = 0; i < kScanItems; ++i) {
-        vals[i] = (base + i < n) ? src(base + i) : 0;
-        s += vals[i];
+        const int64_t v = (base + i * 64 < n) ? src(base + i * 64) : 0;
+        const int64_t incl = wave_inclusive(v);
+        before[i] = run + incl - v;
+        run += __shfl(incl, 63, 64);
     }
-    int64_t total;
-    int64_t run = block_exclusive_scan<int64_t>(s, lds, total) + tile_off[blockIdx.x];
-    for (int i = 0; i < kScanItems; ++i) {
-        if (base + i < n) out[(base + i) * stride + offset] = (Out)run;
-        run += vals[i];
+    if (lane == 0) lds[wv] = run;
+    __syncthreads();
+    int64_t below = tile_off ? tile_off[blockIdx.x] : 0, all = 0;
+    for (int w = 0; w < kScanThreads / 64; ++w) {
+        below += w < wv ? lds[w] : 0;
+        all += lds[w];
+    }
+#pragma unroll
+    for (int i = 0; i < kScanItems; ++i)
+        if (base + i * 64 < n) out[(base + i * 64) * stride + offset] = (Out)(below + before[i]);
+    if (!tile_off && threadIdx.x == 0) {
+        *total = all;
+        if (total_out) *total_out = all;
     }
 }
 
@@ -134,20 +156,27 @@ static const int64_t *launch_scan(qmb_ctx *ctx, Src src, int64_t n, Out *out, De
                                   int stride = 1, int offset = 0) {
     const int64_t tiles = (n + kScanTile - 1) / kScanTile;
     sums.alloc((size_t)(tiles + 1) * sizeof(int64_t));
+    int64_t *total = sums.as<int64_t>() + tiles;
+    if (tiles == 1) {  // no offsets to find: one launch instead of three
+        hipLaunchKernelGGL((scan_write<Src, Out>), dim3(1), dim3(kScanThreads), 0, ctx->stream, src, n, nullptr, out,
+                           stride, offset, total, total_out);
+        QMB_HIP(hipGetLastError());
+        return total;
+    }
     if (tiles > 0) {
         hipLaunchKernelGGL(scan_tile_sums<Src>, dim3((unsigned)tiles), dim3(kScanThreads), 0, ctx->stream, src, n,
                            sums.as<int64_t>());
         QMB_HIP(hipGetLastError());
     }
-    hipLaunchKernelGGL(scan_tile_offsets, dim3(1), dim3(kScanThreads), 0, ctx->stream, sums.as<int64_t>(), tiles,
+    hipLaunchKernelGGL(scan_tile_offsets, dim3(1), dim3(kOffsetThreads), 0, ctx->stream, sums.as<int64_t>(), tiles,
                        total_out);
     QMB_HIP(hipGetLastError());
     if (tiles > 0) {
         hipLaunchKernelGGL((scan_write<Src, Out>), dim3((unsigned)tiles), dim3(kScanThreads), 0, ctx->stream, src, n,
-                           sums.as<int64_t>(), out, stride, offset);
+                           sums.as<int64_t>(), out, stride, offset, nullptr, nullptr);
         QMB_HIP(hipGetLastError());
     }
-    return sums.as<int64_t>() + tiles;
+    return total;
 }
 
 template <class Src, class Out>
@@ -325,35 +354,27 @@ static bool build_ring_lut(qmb_group &g) {
     return true;
 }
 
-// A group that is not a ring itself but holds every rotation of the ring (with
-// or without the spin flip) as a subgroup H, e.g. translations x spin flip x a
-// reflection: G = H c_0 + H c_1 + ... (c_0 = identity, at most kMaxCosets
-// cosets). The orbit minimum is then the smallest of the ring minima of the
-// images c_i x (lut = 3); cos_tab names the element (rotation s, flip f) o c_i.
-static void build_coset_ring(qmb_group &g) {
+// Cosets of the subgroup H whose elements slot() names by an index below 64
+// (-1: not in H): G = H c_0 + H c_1 + ... (c_0 = identity, at most kMaxCosets).
+// H must hold size(hf) elements, each of a different index (hf: with the spin
+// flip, whose half has the indexes + 64). Sets n_cos, cos_rev, cos_tab and
+// lut_flip; false when the group has no such form.
+template <class Slot, class Size>
+static bool build_cosets(qmb_group &g, Slot slot, Size size) {
     const int N = g.n_sites, G = g.G;
-    if (g.torus || N < 8 || N > 56) return;
     std::vector<int> gid(128, -1), in_h(G, 0);
+    int nh = 0, hf = 0;
     for (int e = 0; e < G; ++e) {
-        const uint32_t *p = &g.perm[(size_t)e * N];
-        const int sh = (int)p[0];
-        bool rot = true;
-        for (int q = 0; q < N && rot; ++q) rot = (int)p[q] == (q + sh) % N;
-        if (!rot) continue;
-        const int i = (g.flip[e] ? 64 : 0) + sh;
-        if (gid[i] >= 0) return;  // repeated element
+        const int at = slot(&g.perm[(size_t)e * N]);
+        if (at < 0) continue;
+        const int i = (g.flip[e] ? 64 : 0) + at;
+        if (gid[i] >= 0) return false;  // repeated element
         gid[i] = e;
         in_h[e] = 1;
+        hf |= g.flip[e] ? 1 : 0;
+        ++nh;
     }
-    int hf = 0;
-    for (int e = 0; e < G; ++e) hf |= (in_h[e] && g.flip[e]) ? 1 : 0;
-    int nh = 0;
-    for (int f = 0; f <= hf; ++f)
-        for (int sh = 0; sh < N; ++sh) {
-            if (gid[f * 64 + sh] < 0) return;
-            ++nh;
-        }
-    if (nh == G || G % nh || G / nh > kMaxCosets || gid[0] != 0) return;
+    if (nh != size(hf) || nh == G || G % nh || G / nh > kMaxCosets || gid[0] != 0) return false;
     // cosets H c: c = the first element not yet covered
     std::vector<int> covered(G, 0), reps;
     for (int e = 0; e < G; ++e) {
@@ -362,7 +383,7 @@ static void build_coset_ring(qmb_group &g) {
         for (int h = 0; h < G; ++h)
             if (in_h[h]) covered[g.comp[(size_t)h * G + e]] = 1;
     }
-    if ((int)reps.size() * nh != G) return;
+    if ((int)reps.size() * nh != G) return false;
     // a coset holding the site reversal s -> N-1-s (no flip) is represented by
     // it: its image is one bit reversal on the device
     g.cos_rev = 0;
@@ -383,8 +404,72 @@ static void build_coset_ring(qmb_group &g) {
         for (int i = 0; i < 128; ++i)
             if (gid[i] >= 0) g.cos_tab[c * 128 + i] = g.comp[(size_t)gid[i] * G + reps[c]];
     g.n_cos = (int)reps.size();
-    g.lut = 3;
     g.lut_flip = hf;
+    return true;
+}
+
+// A group that is not a ring itself but holds every rotation of the ring (with
+// or without the spin flip) as a subgroup H, e.g. translations x spin flip x a
+// reflection: G = H c_0 + H c_1 + ... (c_0 = identity, at most kMaxCosets
+// cosets). The orbit minimum is then the smallest of the ring minima of the
+// images c_i x (lut = 3); cos_tab names the element (rotation s, flip f) o c_i.
+static void build_coset_ring(qmb_group &g) {
+    const int N = g.n_sites;
+    if (g.torus || N < 8 || N > 56) return;
+    auto slot = [&](const uint32_t *p) {
+        for (int q = 0; q < N; ++q)
+            if ((int)p[q] != (q + (int)p[0]) % N) return -1;
+        return (int)p[0];
+    };
+    if (build_cosets(g, slot, [&](int hf) { return (hf + 1) * N; })) g.lut = 3;
+}
+
+// tab[v], tab[256 + v] of a torus product with blocks of B sites.
+static void fill_rotation_minima(qmb_group &g, int B) {
+    g.lut_tab.assign(kLutBytes, 0);
+    const unsigned mB = (1u << B) - 1u;
+    for (unsigned v = 0; v <= mB; ++v) {
+        unsigned best = 0xFF, mask = 0;
+        for (int s = 0; s < B; ++s) {
+            const unsigned r = s ? (((v << s) | (v >> (B - s))) & mB) : v;
+            if (r < best) {
+                best = r;
+                mask = 1u << s;
+            } else if (r == best) {
+                mask |= 1u << s;
+            }
+        }
+        g.lut_tab[v] = (uint8_t)best;
+        g.lut_tab[256 + v] = (uint8_t)mask;
+    }
+}
+
+// A group that is no torus product itself but holds a full one (every block
+// shift and in-block shift of some block width B <= 8, nb <= 8, with or without
+// the spin flip) as a subgroup H, e.g. translations x the quarter turns of a
+// square lattice: G = H c_0 + H c_1 + ... as for the ring cosets (lut = 4);
+// cos_tab[i * 128 + (f * 8 + a) * 8 + s] names the element (flip f, block shift
+// a, in-block shift s) o c_i.
+static void build_coset_torus(qmb_group &g) {
+    const int N = g.n_sites;
+    if (g.torus) return;
+    for (int B = 2; B <= 8; ++B) {
+        if (N % B || N / B < 2 || N / B > 8) continue;
+        const int nb = N / B;
+        auto slot = [&](const uint32_t *p) {
+            const int a = (int)p[0] / B, s = (int)p[0] % B;
+            for (int q = 0; q < N; ++q)
+                if ((int)p[q] != ((q / B + a) % nb) * B + (q % B + s) % B) return -1;
+            return a * 8 + s;
+        };
+        auto size = [&](int hf) { return (hf + 1) * N; };
+        if (build_cosets(g, slot, size)) {
+            fill_rotation_minima(g, B);
+            g.block = B;
+            g.lut = 4;
+            return;
+        }
+    }
 }
 
 static void build_lut(qmb_group &g) {
@@ -408,22 +493,7 @@ static void build_lut(qmb_group &g) {
         for (int a = 0; a < nb; ++a)
             for (int s = 0; s < B; ++s)
                 if (gid[(f * 8 + a) * 8 + s] < 0) return;
-    g.lut_tab.assign(kLutBytes, 0);
-    const unsigned mB = (1u << B) - 1u;
-    for (unsigned v = 0; v <= mB; ++v) {
-        unsigned best = 0xFF, mask = 0;
-        for (int s = 0; s < B; ++s) {
-            const unsigned r = s ? (((v << s) | (v >> (B - s))) & mB) : v;
-            if (r < best) {
-                best = r;
-                mask = 1u << s;
-            } else if (r == best) {
-                mask |= 1u << s;
-            }
-        }
-        g.lut_tab[v] = (uint8_t)best;
-        g.lut_tab[256 + v] = (uint8_t)mask;
-    }
+    fill_rotation_minima(g, B);
     for (int i = 0; i < 2 * 8 * 8; ++i) g.lut_tab[512 + i] = (uint8_t)(gid[i] < 0 ? 0 : gid[i]);
     g.lut = 1;
     g.lut_flip = hf;
@@ -585,6 +655,7 @@ qmb_status qmb_group_create(int n_sites, int n_elems, const uint32_t *group_el, 
         detect_torus(*g);
         build_lut(*g);
         if (!g->lut) build_coset_ring(*g);
+        if (!g->lut) build_coset_torus(*g);
         *out = g.release();
     });
 }

@@ -6,10 +6,12 @@
 // Q/exact_diagonalization/HeisenbergGenericXXZ_AbelianSymms_CUDA.cu:277-400,
 // Q/exact_diagonalization/utils.cu:39-80,716-805). Nothing of size
 // C(N,k)*G is materialised:
-//   mark    : one thread per 64 consecutive sector ranks; unrank the first,
-//             step with the next-combination trick, keep a state when it is
-//             the minimum of its orbit (and, in the compact layout, when the
-//             irrep's character is 1 on its stabiliser) -> one bit word;
+//   mark    : a state is kept when it is the minimum of its orbit (and, in the
+//             compact layout, when the irrep's character is 1 on its stabiliser)
+//             -> one bit per state in ascending (colex) order. Cyclic groups
+//             first drop groups of 256 states by the bits all of them share,
+//             then test the rest one state per lane; other groups and small
+//             sectors test runs of consecutive states (next-combination trick);
 //   scan    : exclusive popcount scan of the words -> row offsets, stored
 //             beside each word (16-byte records);
 //   compact : rewrite the kept states in ascending order with their
@@ -31,7 +33,7 @@ qmb::GroupView qmb_basis::view() const {
     v.block = group->block;
     v.full = group->n_sites == 64 ? ~0ULL : ((1ULL << group->n_sites) - 1ULL);
     v.rep_unit = 0;
-    if (group->torus)
+    if (group->torus || group->lut == 4)
         for (int b0 = 0; b0 < group->n_sites; b0 += group->block) v.rep_unit |= 1ULL << b0;
     const uint8_t *t = g_tab.as<uint8_t>();
     v.keep = reinterpret_cast<const uint64_t *>(t);
@@ -42,10 +44,10 @@ qmb::GroupView qmb_basis::view() const {
     v.inv = t + o_inv;
     v.lut = group->lut;
     v.lut_flip = group->lut_flip;
-    v.lut_tab = (group->lut == 1 || group->lut == 2) ? t + o_lut : nullptr;
-    v.n_cos = group->lut == 3 ? group->n_cos : 0;
-    v.cos_rev = group->lut == 3 ? group->cos_rev : 0;
-    v.cos_tab = group->lut == 3 ? t + o_cos : nullptr;
+    v.lut_tab = (group->lut && group->lut != 3) ? t + o_lut : nullptr;
+    v.n_cos = group->lut >= 3 ? group->n_cos : 0;
+    v.cos_rev = group->lut >= 3 ? group->cos_rev : 0;
+    v.cos_tab = group->lut >= 3 ? t + o_cos : nullptr;
     return v;
 }
 
@@ -56,88 +58,70 @@ namespace qmb {
 // -> 35 ms)
 constexpr int kBasisThreads = 512;
 
+// basis_mark's run length: the longest that still gives this many runs (5x5
+// translations without a run test, 5.2 million states: 115 us a basis with 2^20
+// runs, 362 us with 2^17).
+constexpr int64_t kMinRuns = (int64_t)1 << 20;
+// Sectors of this many states and more are marked in two kernels (basis of a
+// 28-site ring with flip: 156 us, 421 us with one word per lane in one kernel;
+// 22 sites, 705,432 states: equal to basis_mark, 84-90 us; smaller ones lose the
+// extra launch and clear: 20 sites, 71 us against 105 us).
+constexpr int64_t kRejectDim = (int64_t)1 << 18;
+constexpr int64_t kMaxMarkBlocks = 4096;
+// basis_compact's words per wavefront: up to 8 with this many wavefronts, more
+// with eight times as many (the words at low ranks hold most rows: 28-site ring,
+// 627K words, 39 us at 8 a wavefront, 111 us at 64; 25 sites, 81K words, 17 us
+// at 8, 29 us at 1, where most wavefronts find no row).
+constexpr int64_t kMinCompactWaves = 8192;
+
 __device__ inline bool compatible(uint64_t slo, uint64_t shi, uint64_t tlo, uint64_t thi) {
     return ((slo & ~tlo) | (shi & ~thi)) == 0;
 }
 
+// True when no state of a run of consecutive sector states can be the minimum of
+// its orbit, from the bits that all of them share: those above the highest bit
+// in which the run's first and last state differ (the states lie between the
+// two as integers). Ring (lut 2, and the ring subgroup of lut 3): the rotation
+// that brings shared bit p to the top starts with the shared bits p .. d; when
+// these are below the state's own top p - d + 1 bits, the image is smaller.
+// Under the flip the complement of the rotation (the unrotated one included)
+// likewise. Torus product (lut 1, and the torus subgroup of lut 4): every block inside the shared bits must have
+// its smallest in-block rotation at or above the top block.
 template <class S>
-__global__ __launch_bounds__(kBasisThreads) void basis_mark(GroupView gv, const uint64_t *binom, int n_up,
-                                                            int64_t dim, int64_t n_words, int compact,
-                                                            uint64_t triv_lo, uint64_t triv_hi,
-                                                            uint64_t *dict) {
-    __shared__ uint8_t perm_lds[kMaxGroup * 64];
-    __shared__ uint64_t bin[64 * kBinJ];
-    __shared__ GroupLds gt;
-    stage_perm(perm_lds, gv);
-    stage_binom(bin, binom);
-    stage_group(gt, gv);
-    __syncthreads();
-    const int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (w >= n_words) return;
-    const int64_t r0 = w * 64;
-    const int cnt = (int)((dim - r0) < 64 ? (dim - r0) : 64);
-    S x = colex_unrank<S>(r0, n_up, gv.n_sites, bin);
-    uint64_t bits = 0;
-    if (gv.lut == 2) {
-        // Ring group, two passes. Pass 1 keeps the states that are not above
-        // their rotations by 1, 2 and 3 sites (nor, with the spin flip, above
-        // their complements or theirs): a necessary condition, branch-free.
-        // Pass 2 takes each lane's survivors in turn: the rotations by
-        // s = 1 .. N-1 one bit at a time (and their complements), exit at the
-        // first smaller image; element indices are looked up only for images
-        // equal to the state (stabiliser).
-        const int N = gv.n_sites;
-        const S full = (S)gv.full;
-        const bool hf = gv.lut_flip != 0;
-        auto rotl = [&](S v, int k) { return (S)(((v << k) | (v >> (N - k))) & full); };
-        uint64_t surv = 0;
-        S y = x;
-        for (int i = 0; i < cnt; ++i) {
-            const S a1 = rotl(y, 1), a2 = rotl(y, 2), a3 = rotl(y, 3);
-            bool ok = a1 >= y && a2 >= y && a3 >= y;
-            if (hf) ok = ok && (S)(y ^ full) >= y && (S)(a1 ^ full) >= y && (S)(a2 ^ full) >= y && (S)(a3 ^ full) >= y;
-            if (ok) surv |= 1ULL << i;
-            if (i + 1 < cnt) y = next_comb<S>(y);
+__device__ inline bool run_rejected(S first, S last, const GroupView &gv, const GroupLds &gt) {
+    const int N = gv.n_sites;
+    const S diff = first ^ last;
+    const int d = diff ? (int)(sizeof(S) * 8) - clz_s(diff) : 0;  // bits d .. N-1 are shared
+    const bool hf = gv.lut_flip != 0;
+    if (gv.lut == 1 || gv.lut == 4) {
+        const int B = gv.block, nb = N / B;
+        const unsigned mB = (1u << B) - 1u;
+        if (d > (nb - 1) * B) return false;
+        const unsigned t = (unsigned)(first >> ((nb - 1) * B)) & mB;
+        for (int j = nb - 1; j >= 0 && j * B >= d; --j) {
+            const unsigned v = (unsigned)(first >> (j * B)) & mB;
+            if (gt.lut[v] < t || (hf && gt.lut[v ^ mB] < t)) return true;
         }
-        y = x;
-        int at = 0;
-        while (surv) {
-            const int i = __builtin_ctzll(surv);
-            surv &= surv - 1;
-            for (; at < i; ++at) y = next_comb<S>(y);
-            uint64_t slo = 1, shi = 0;  // element 0 (identity) fixes y
-            auto mark = [&](int f, int sh) {
-                const int g = gt.lut[512 + f * 64 + sh];
-                if (g < 64)
-                    slo |= 1ULL << g;
-                else
-                    shi |= 1ULL << (g - 64);
-            };
-            bool rep = true;
-            S z = y;
-            for (int st = 0; st < N && rep; ++st) {
-                if (st > 0) {
-                    z = rotl(z, 1);
-                    if (z < y)
-                        rep = false;
-                    else if (z == y)
-                        mark(0, st);
-                }
-                if (rep && hf) {
-                    const S zf = (S)(z ^ full);
-                    if (zf < y)
-                        rep = false;
-                    else if (zf == y)
-                        mark(1, st);
-                }
-            }
-            if (rep && (!compact || compatible(slo, shi, triv_lo, triv_hi))) bits |= 1ULL << i;
-        }
-        dict[2 * w] = bits;
-        return;
+        return false;
     }
-    if (gv.lut == 1) {
-        // Full torus product, two passes. Pass 1 keeps the states whose top block
+    const int m = N - d;
+    if (m < 2) return false;
+    const S z = first >> d;  // the m shared bits
+    if (hf && ((z >> (m - 1)) & 1)) return true;
+    for (int len = m - 1; len >= 1; --len) {
+        const S top = z >> (m - len), mask = (S)(((S)1 << len) - 1);
+        if ((z & mask) < top || (hf && (S)(~z & mask) < top)) return true;
+    }
+    return false;
+}
+
+// Bit i of the result: state i of the run of cnt states from x is a row.
+template <class S>
+__device__ inline uint64_t mark_run(S x, int cnt, const GroupView &gv, const GroupLds &gt, const uint8_t *perm_lds,
+                                    int compact, uint64_t triv_lo, uint64_t triv_hi) {
+    uint64_t bits = 0;
+    if (gv.lut == 1 || gv.lut == 4) {
+        // Full torus product (times cosets for lut 4), two passes. Pass 1 keeps the states whose top block
         // equals the smallest in-block rotation of any block (complemented too
         // under flip): a necessary condition. The top block t is at most its own
         // rotation minimum only when it is one (lut[t] <= t), so the condition
@@ -172,18 +156,20 @@ __global__ __launch_bounds__(kBasisThreads) void basis_mark(GroupView gv, const 
             surv &= surv - 1;
             for (; at < i; ++at) y = next_comb<S>(y);
             uint64_t slo, shi;
-            if (rep_stab_lut<S>(y, gv, gt, slo, shi) && (!compact || compatible(slo, shi, triv_lo, triv_hi)))
+            if (rep_stab_lut<S>(y, gv, gt, perm_lds, slo, shi) && (!compact || compatible(slo, shi, triv_lo, triv_hi)))
                 bits |= 1ULL << i;
         }
-        dict[2 * w] = bits;
-        return;
+        return bits;
     }
-    if (gv.lut == 3) {
-        // Ring rotations times cosets, two passes as for the ring: the same
-        // branch-free filter (rotations by 1-3 sites and complements, images
-        // under the ring subgroup), then each lane's survivors: per coset c_i
-        // one image y = c_i x, then its rotations one bit at a time, exit at
-        // the first smaller image.
+    if (gv.lut == 2 || gv.lut == 3) {
+        // Ring rotations (times cosets for lut 3), two passes. Pass 1 keeps the
+        // states that are not above their rotations by 1, 2 and 3 sites (nor,
+        // with the spin flip, above their complements or theirs): a necessary
+        // condition, branch-free. Pass 2 takes each lane's survivors in turn:
+        // per coset c_i one image z = c_i y (the state itself for a plain ring) and
+        // the scan of its top bytes (ring_windows): a smaller byte rules the state
+        // out, and only the rotations that reach its own are formed; element
+        // indices are looked up only for images equal to the state (stabiliser).
         const int N = gv.n_sites;
         const S full = (S)gv.full;
         const bool hf = gv.lut_flip != 0;
@@ -211,28 +197,34 @@ __global__ __launch_bounds__(kBasisThreads) void basis_mark(GroupView gv, const 
                     shi |= 1ULL << (g - 64);
             };
             bool rep = true;
-            for (int ci = 0; ci < gv.n_cos && rep; ++ci) {
-                const uint8_t *ct = gt.cos + ci * 128;
-                S z = ci ? coset_image<S>(y, ci, gv, gt, perm_lds) : y;
-                for (int st = 0; st < N && rep; ++st) {
-                    if (st > 0) z = rotl(z, 1);
-                    if (z < y)
-                        rep = false;
-                    else if (z == y)
-                        mark(ct[st]);
-                    if (rep && hf) {
-                        const S zf = (S)(z ^ full);
-                        if (zf < y)
+            const unsigned top = (unsigned)(y >> (N - 8));
+            const int n_cos = gv.lut == 3 ? gv.n_cos : 1;
+            for (int ci = 0; ci < n_cos && rep; ++ci) {
+                const uint8_t *ct = gv.lut == 3 ? gt.cos + ci * 128 : gt.lut + 512;
+                const S z = ci ? coset_image<S>(y, ci, gv, gt, perm_lds) : y;
+                uint64_t c0, c1;
+                const unsigned tmin = ring_windows<S>(z, N, hf, c0, c1);
+                if (tmin > top) continue;
+                rep = tmin == top;
+                for (int f = 0; f < (hf ? 2 : 1); ++f) {
+                    uint64_t c = f ? c1 : c0;
+                    while (c && rep) {
+                        const int p = __builtin_ctzll(c);
+                        c &= c - 1;
+                        int st = N - 8 - p;
+                        if (st < 0) st += N;
+                        S v = rotl_ring<S>(z, st, N, full);
+                        if (f) v ^= full;
+                        if (v < y)
                             rep = false;
-                        else if (zf == y)
-                            mark(ct[64 + st]);
+                        else if (v == y)
+                            mark(ct[f * 64 + st]);
                     }
                 }
             }
             if (rep && (!compact || compatible(slo, shi, triv_lo, triv_hi))) bits |= 1ULL << i;
         }
-        dict[2 * w] = bits;
-        return;
+        return bits;
     }
     // One flat loop over (state, element) steps per lane: a lane moves to its
     // next state as soon as an image is smaller (most states exit after a few
@@ -267,48 +259,201 @@ __global__ __launch_bounds__(kBasisThreads) void basis_mark(GroupView gv, const 
             shi = 0;
         }
     }
-    dict[2 * w] = bits;
+    return bits;
 }
 
-// One thread per row: the row's bit word is the last word whose row offset
-// is <= row (binary search over the offsets), its bit the (row - offset)-th
-// set bit of that word. Every thread does the same work (one unrank, one
-// stabiliser count) and the writes are coalesced.
+// Every state of the sector, for groups without a run test (lut 0) and small
+// sectors. A lane takes the 2^ks consecutive states of one run; the 64 >> ks
+// lanes of a word join their bits by shuffles. A word per lane (ks = 6) unranks
+// once per 64 states but leaves a sector to few wavefronts, the ones at low
+// ranks (where most representatives are) running longest.
+template <class S>
+__global__ __launch_bounds__(kBasisThreads) void basis_mark(GroupView gv, const uint64_t *binom, int n_up,
+                                                            int64_t dim, int64_t n_words, int ks, int compact,
+                                                            uint64_t triv_lo, uint64_t triv_hi,
+                                                            uint64_t *dict) {
+    __shared__ alignas(8) uint8_t perm_lds[kMaxGroup * 64];
+    __shared__ typename RankOf<S>::T bin[sizeof(S) * 8 * kBinJ];
+    __shared__ GroupLds gt;
+    stage_images<S>(perm_lds, gv);
+    stage_binom_rows<S>(bin, binom, gv.n_sites);
+    stage_group(gt, gv);
+    __syncthreads();
+    const int per_word = 64 >> ks;
+    const int64_t runs = n_words << (6 - ks);
+    // whole wavefronts step together: the shuffles need every lane
+    for (int64_t t0 = (int64_t)blockIdx.x * blockDim.x; t0 < runs; t0 += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t t = t0 + threadIdx.x;
+        const int64_t r0 = t << ks;
+        const int64_t left = dim - r0;
+        const int cnt = (int)(left < 0 ? 0 : left < (1 << ks) ? left : (1 << ks));
+        uint64_t bits = 0;
+        if (cnt > 0)
+            bits = mark_run<S>(colex_unrank<S>((typename RankOf<S>::T)r0, n_up, gv.n_sites, bin), cnt, gv, gt, perm_lds, compact, triv_lo,
+                               triv_hi);
+        const int at = (int)(t & (per_word - 1));
+        bits <<= at << ks;
+        for (int off = 1; off < per_word; off <<= 1) bits |= __shfl_xor(bits, off, 64);
+        if (at == 0 && cnt > 0) dict[2 * (t >> (6 - ks))] = bits;
+    }
+}
+
+// Large sectors, first of two kernels: one group of kRunWords words per lane. A
+// group whose states are all ruled out by the bits they share gets its zeros
+// here; the others are listed (group indexes, any order) in the second halves
+// of the dict records, which the scan fills only later. *count = groups listed.
+// On a 26-site ring 6 % (with the flip; 13 % without) of the 64-state words are
+// not ruled out, and 1 % more in groups of four, at a quarter of the unranking.
+constexpr int kRunWords = 4;
+
+template <class S>
+__global__ __launch_bounds__(kBasisThreads) void basis_reject(GroupView gv, const uint64_t *binom, int n_up,
+                                                              int64_t dim, int64_t n_words, uint64_t *dict,
+                                                              unsigned long long *count) {
+    using R = typename RankOf<S>::T;
+    __shared__ R bin[sizeof(S) * 8 * kBinJ];
+    __shared__ GroupLds gt;
+    stage_binom_rows<S>(bin, binom, gv.n_sites);
+    stage_group(gt, gv);
+    __syncthreads();
+    const int lane = threadIdx.x & 63;
+    const int64_t n_runs = (n_words + kRunWords - 1) / kRunWords;
+    for (int64_t t0 = (int64_t)blockIdx.x * blockDim.x; t0 < n_runs; t0 += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t e = t0 + threadIdx.x;
+        bool keep = false;
+        if (e < n_runs) {
+            const int64_t r0 = e * kRunWords * 64, r1 = min(r0 + kRunWords * 64, dim) - 1;
+            keep = !run_rejected<S>(colex_unrank<S>((R)r0, n_up, gv.n_sites, bin),
+                                    colex_unrank<S>((R)r1, n_up, gv.n_sites, bin), gv, gt);
+            if (!keep)
+                for (int64_t w = e * kRunWords; w < min((e + 1) * kRunWords, n_words); ++w) dict[2 * w] = 0;
+        }
+        const uint64_t m = __ballot(keep);
+        if (!m) continue;
+        unsigned long long base = 0;
+        if (lane == 0) base = atomicAdd(count, (unsigned long long)__popcll(m));
+        base = __shfl(base, 0, 64);
+        if (keep) dict[2 * (base + __popcll(m & ((1ULL << lane) - 1ULL))) + 1] = (uint64_t)e;
+    }
+}
+
+// Second kernel: one wavefront per word of the listed groups, one state per lane.
+template <class S>
+__global__ __launch_bounds__(kBasisThreads) void basis_mark_words(GroupView gv, const uint64_t *binom, int n_up,
+                                                                  int64_t dim, int64_t n_words, int compact,
+                                                                  uint64_t triv_lo, uint64_t triv_hi,
+                                                                  uint64_t *dict,
+                                                                  const unsigned long long *count) {
+    __shared__ alignas(8) uint8_t perm_lds[kMaxGroup * 64];
+    __shared__ typename RankOf<S>::T bin[sizeof(S) * 8 * kBinJ];
+    __shared__ GroupLds gt;
+    stage_images<S>(perm_lds, gv);
+    stage_binom_rows<S>(bin, binom, gv.n_sites);
+    stage_group(gt, gv);
+    __syncthreads();
+    const int lane = threadIdx.x & 63;
+    const int64_t n = (int64_t)*count * kRunWords;
+    const int waves = kBasisThreads / 64;
+    for (int64_t i = (int64_t)blockIdx.x * waves + (threadIdx.x >> 6); i < n; i += (int64_t)gridDim.x * waves) {
+        const int64_t w = (int64_t)dict[2 * (i / kRunWords) + 1] * kRunWords + i % kRunWords;
+        if (w >= n_words) continue;
+        const int64_t r = w * 64 + lane;
+        uint64_t row = 0;
+        if (r < dim)
+            row = mark_run<S>(colex_unrank<S>((typename RankOf<S>::T)r, n_up, gv.n_sites, bin), 1, gv, gt, perm_lds, compact, triv_lo,
+                              triv_hi);
+        const uint64_t bits = __ballot(row != 0);
+        if (lane == 0) dict[2 * w] = bits;
+    }
+}
+
+// Position of the k-th set bit of w (k below its number of set bits).
+__device__ inline int select_bit(uint64_t w, int k) {
+    int pos = 0;
+#pragma unroll
+    for (int width = 32; width >= 1; width >>= 1) {
+        const int c = __popcll(w & ((1ULL << width) - 1ULL));
+        const bool up = k >= c;
+        k -= up ? c : 0;
+        w >>= up ? width : 0;
+        pos += up ? width : 0;
+    }
+    return pos;
+}
+
+// The rows in ascending order. A wavefront takes tile_words (a power of two, at
+// most 64) consecutive words: their records are one coalesced load, and 64 rows
+// at a time each lane finds its row's word among the tile's row offsets (a
+// search over the lanes by shuffles), its bit and its state. Lanes of a wave
+// hold consecutive rows, so the writes are coalesced; a word search in memory
+// per row took a chain of ~20 dependent reads. Ring: a state has a stabiliser
+// beyond the identity only if a rotation by N / q (q prime; bit N / q of
+// periods) fixes it or, with the flip, its complement equals it rotated by N / 2
+// (the anti-period's double is a period, and N is the only one left).
 template <class S>
 __global__ __launch_bounds__(kBasisThreads) void basis_compact(GroupView gv, const uint64_t *binom, int n_up,
-                                                               int64_t n_rows, int64_t n_words,
+                                                               int64_t n_words, int tile_words, uint64_t periods,
                                                                uint64_t triv_lo, uint64_t triv_hi,
                                                                const uint64_t *dict,
                                                                uint64_t *reps, uint8_t *stab, uint8_t *nullf) {
-    __shared__ uint8_t perm_lds[kMaxGroup * 64];
-    __shared__ uint64_t bin[64 * kBinJ];
+    using R = typename RankOf<S>::T;
+    __shared__ alignas(8) uint8_t perm_lds[kMaxGroup * 64];
+    __shared__ R bin[sizeof(S) * 8 * kBinJ];
     __shared__ GroupLds gt;
-    stage_perm(perm_lds, gv);
-    stage_binom(bin, binom);
+    stage_images<S>(perm_lds, gv);
+    stage_binom_rows<S>(bin, binom, gv.n_sites);
     stage_group(gt, gv);
     __syncthreads();
-    const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= n_rows) return;
-    int64_t lo = 0, hi = n_words - 1;  // the first word has 0 rows before it
-    while (lo < hi) {
-        const int64_t mid = (lo + hi + 1) >> 1;
-        if ((int64_t)dict[2 * mid + 1] <= r)
-            lo = mid;
-        else
-            hi = mid - 1;
+    const int lane = threadIdx.x & 63;
+    const int waves = kBasisThreads / 64;
+    const int64_t n_tiles = (n_words + tile_words - 1) / tile_words;
+    const bool narrow_group = gv.lut == 2;
+    for (int64_t t = (int64_t)blockIdx.x * waves + (threadIdx.x >> 6); t < n_tiles; t += (int64_t)gridDim.x * waves) {
+        const int64_t w = t * tile_words + lane;
+        ulonglong2 rec = make_ulonglong2(0, 0);
+        if (lane < tile_words && w < n_words) rec = reinterpret_cast<const ulonglong2 *>(dict)[w];
+        const int mine = __popcll(rec.x);
+        const int64_t row0 = (int64_t)__shfl(rec.y, 0, 64);  // the tile's first word exists
+        // rows of the tile before this lane's word; lanes past the tile hold its total
+        int before = mine;
+        for (int off = 1; off < 64; off <<= 1) {
+            const int o = __shfl_up(before, off, 64);
+            before += lane >= off ? o : 0;
+        }
+        const int total = __shfl(before, 63, 64);
+        before -= mine;
+        for (int q0 = 0; q0 < total; q0 += 64) {
+            const int q = min(q0 + lane, total - 1);
+            int at = 0;  // last word with at most q rows before it that holds row q
+            for (int step = 32; step >= 1; step >>= 1) {
+                const int o = __shfl(before, at + step, 64);
+                at += o <= q ? step : 0;
+            }
+            const uint64_t bits = __shfl(rec.x, at, 64);
+            const int i = select_bit(bits, q - __shfl(before, at, 64));
+            if (q0 + lane >= total) continue;
+            const S x = colex_unrank<S>((R)((t * tile_words + at) * 64 + i), n_up, gv.n_sites, bin);
+            uint64_t slo = 1, shi = 0;
+            if (gv.lut == 1 || gv.lut == 4) {
+                rep_stab_lut<S>(x, gv, gt, perm_lds, slo, shi);  // x is a representative: the candidates hold its stabiliser
+            } else {
+                bool trivial = narrow_group;
+                if (narrow_group) {
+                    const S full = (S)gv.full;
+                    for (uint64_t m = periods; m; m &= m - 1)
+                        if (rotl_ring<S>(x, __builtin_ctzll(m), gv.n_sites, full) == x) trivial = false;
+                    if (gv.lut_flip && !(gv.n_sites & 1) &&
+                        (S)(rotl_ring<S>(x, gv.n_sites / 2, gv.n_sites, full) ^ full) == x)
+                        trivial = false;
+                }
+                if (!trivial) stabiliser<S>(x, gv, gt, perm_lds, slo, shi);
+            }
+            const int64_t r = row0 + q;
+            reps[r] = (uint64_t)x;
+            stab[r] = (uint8_t)(__popcll(slo) + __popcll(shi));
+            nullf[r] = compatible(slo, shi, triv_lo, triv_hi) ? 0 : 1;
+        }
     }
-    uint64_t bits = dict[2 * lo];
-    for (int64_t k = r - (int64_t)dict[2 * lo + 1]; k > 0; --k) bits &= bits - 1;
-    const int i = __builtin_ctzll(bits);
-    const S x = colex_unrank<S>(lo * 64 + i, n_up, gv.n_sites, bin);
-    uint64_t slo, shi;
-    if (gv.lut == 1)
-        rep_stab_lut<S>(x, gv, gt, slo, shi);  // x is a representative: the candidates hold its stabiliser
-    else
-        is_representative<S>(x, gv, perm_lds, slo, shi);
-    reps[r] = (uint64_t)x;
-    stab[r] = (uint8_t)(__popcll(slo) + __popcll(shi));
-    nullf[r] = compatible(slo, shi, triv_lo, triv_hi) ? 0 : 1;
 }
 
 template <class S>
@@ -349,8 +494,8 @@ static void upload_group(qmb_basis *b, const qmb_group *g) {
         h[b->o_inv + e] = (uint8_t)g->inv[e];
     }
     for (size_t i = 0; i < G * n; ++i) h[b->o_perm + i] = (uint8_t)g->perm[i];
-    if (g->lut == 1 || g->lut == 2) std::memcpy(h.data() + b->o_lut, g->lut_tab.data(), kLutBytes);
-    if (g->lut == 3) std::memcpy(h.data() + b->o_cos, g->cos_tab.data(), kCosBytes);
+    if (g->lut && g->lut != 3) std::memcpy(h.data() + b->o_lut, g->lut_tab.data(), kLutBytes);
+    if (g->lut >= 3) std::memcpy(h.data() + b->o_cos, g->cos_tab.data(), kCosBytes);
     b->g_tab.alloc(total);
     QMB_HIP(hipMemcpy(b->g_tab.p, h.data(), total, hipMemcpyHostToDevice));
 }
@@ -414,11 +559,30 @@ qmb_status qmb_basis_build(qmb_ctx *ctx, const qmb_group *g, int n_up, int irrep
         upload_group(b.get(), g);
         const GroupView gv = b->view();
         b->dict.alloc((size_t)b->n_words * 2 * sizeof(uint64_t));
-        const unsigned blocks = (unsigned)((b->n_words + kBasisThreads - 1) / kBasisThreads);
         const bool narrow = g->n_sites <= 32;
-        hipLaunchKernelGGL(narrow ? basis_mark<uint32_t> : basis_mark<uint64_t>, dim3(blocks), dim3(kBasisThreads), 0, ctx->stream, gv,
-                           ctx->binom.as<uint64_t>(), n_up, b->sector_dim, b->n_words,
-                           layout == QMB_LAYOUT_COMPACT ? 1 : 0, b->triv_lo, b->triv_hi, b->dict.as<uint64_t>());
+        const int compact = layout == QMB_LAYOUT_COMPACT ? 1 : 0;
+        auto blocks_for = [](int64_t threads) {
+            return (unsigned)std::min<int64_t>((threads + kBasisThreads - 1) / kBasisThreads, kMaxMarkBlocks);
+        };
+        if (g->lut && b->sector_dim >= kRejectDim) {
+            DevBuf count(sizeof(unsigned long long));
+            QMB_HIP(hipMemsetAsync(count.p, 0, sizeof(unsigned long long), ctx->stream));
+            hipLaunchKernelGGL(narrow ? basis_reject<uint32_t> : basis_reject<uint64_t>, dim3(blocks_for((b->n_words + kRunWords - 1) / kRunWords)),
+                               dim3(kBasisThreads), 0, ctx->stream, gv, ctx->binom.as<uint64_t>(), n_up,
+                               b->sector_dim, b->n_words, b->dict.as<uint64_t>(), count.as<unsigned long long>());
+            QMB_HIP(hipGetLastError());
+            hipLaunchKernelGGL(narrow ? basis_mark_words<uint32_t> : basis_mark_words<uint64_t>,
+                               dim3(blocks_for(b->n_words * 64)), dim3(kBasisThreads), 0, ctx->stream, gv,
+                               ctx->binom.as<uint64_t>(), n_up, b->sector_dim, b->n_words, compact, b->triv_lo,
+                               b->triv_hi, b->dict.as<uint64_t>(), count.as<unsigned long long>());
+        } else {
+            int ks = 6;
+            while (ks > 0 && (b->sector_dim >> ks) < kMinRuns) --ks;
+            hipLaunchKernelGGL(narrow ? basis_mark<uint32_t> : basis_mark<uint64_t>,
+                               dim3(blocks_for(b->n_words << (6 - ks))), dim3(kBasisThreads), 0, ctx->stream, gv,
+                               ctx->binom.as<uint64_t>(), n_up, b->sector_dim, b->n_words, ks, compact, b->triv_lo,
+                               b->triv_hi, b->dict.as<uint64_t>());
+        }
         QMB_HIP(hipGetLastError());
         const int64_t rows = scan_popcount_dict(ctx, b->dict.as<uint64_t>(), b->n_words);
         QMB_REQUIRE(rows < (int64_t)INT32_MAX, "qmb_basis_build: more than 2^31 rows (int32 columns)");
@@ -427,9 +591,16 @@ qmb_status qmb_basis_build(qmb_ctx *ctx, const qmb_group *g, int n_up, int irrep
         b->stab.alloc((size_t)std::max<int64_t>(rows, 1));
         b->nullf.alloc((size_t)std::max<int64_t>(rows, 1));
         if (rows > 0) {
-            const unsigned rblocks = (unsigned)((rows + kBasisThreads - 1) / kBasisThreads);
-            hipLaunchKernelGGL(narrow ? basis_compact<uint32_t> : basis_compact<uint64_t>, dim3(rblocks), dim3(kBasisThreads), 0, ctx->stream, gv,
-                               ctx->binom.as<uint64_t>(), n_up, rows, b->n_words, b->triv_lo, b->triv_hi,
+            int tile_words = 64;
+            while (tile_words > 1 && b->n_words / tile_words < (tile_words > 8 ? 8 : 1) * kMinCompactWaves)
+                tile_words /= 2;
+            uint64_t periods = 0;
+            for (int q = 2, m = g->n_sites; m > 1; ++q)
+                for (; m % q == 0; m /= q) periods |= 1ULL << (g->n_sites / q);
+            hipLaunchKernelGGL(narrow ? basis_compact<uint32_t> : basis_compact<uint64_t>,
+                               dim3(blocks_for((b->n_words + tile_words - 1) / tile_words * 64)),
+                               dim3(kBasisThreads), 0, ctx->stream, gv, ctx->binom.as<uint64_t>(), n_up, b->n_words,
+                               tile_words, periods, b->triv_lo, b->triv_hi,
                                b->dict.as<uint64_t>(), b->reps.as<uint64_t>(),
                                b->stab.as<uint8_t>(), b->nullf.as<uint8_t>());
             QMB_HIP(hipGetLastError());

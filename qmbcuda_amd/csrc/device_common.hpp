@@ -22,12 +22,38 @@ constexpr int kBinJ = 33;
 
 __device__ inline int ctz_s(uint32_t x) { return __builtin_ctz(x); }
 __device__ inline int ctz_s(uint64_t x) { return __builtin_ctzll(x); }
+__device__ inline int clz_s(uint32_t x) { return __builtin_clz(x); }
+__device__ inline int clz_s(uint64_t x) { return __builtin_clzll(x); }
 __device__ inline int popc_s(uint32_t x) { return __popc(x); }
 __device__ inline int popc_s(uint64_t x) { return __popcll(x); }
 
 __device__ inline void stage_perm(uint8_t *perm_lds, const GroupView &g) {
     if (!g.torus)
         for (int i = threadIdx.x; i < g.G * g.n_sites; i += blockDim.x) perm_lds[i] = g.perm[i];
+}
+
+// Element tables of the lane-divergent image kernels. A group of cosets (lut 3
+// and 4) only takes the images of its coset representatives c_1, c_2, ...: per
+// representative one word per nibble value (entry (i - 1) * n_nib * 16 + k * 16 +
+// v = the sites that the set bits of v, at sites 4k .. 4k+3, move to), so an
+// image is ceil(N / 4) LDS reads instead of one per up spin (at most 128 / N
+// cosets: 4 KB). Other groups without a cyclic form stage their permutations.
+template <class S>
+__device__ inline void stage_images(uint8_t *lds, const GroupView &g) {
+    if (g.lut >= 3) {
+        S *tab = reinterpret_cast<S *>(lds);
+        const int N = g.n_sites, nn = (N + 3) / 4;
+        for (int i = threadIdx.x; i < (g.n_cos - 1) * nn * 16; i += blockDim.x) {
+            const uint8_t *p = g.perm + (size_t)g.cos_tab[(1 + i / (nn * 16)) * 128] * N;
+            const int k = i / 16 % nn, v = i & 15;
+            S w = 0;
+            for (int b = 0; b < 4; ++b)
+                if (((v >> b) & 1) && 4 * k + b < N) w |= (S)1 << p[4 * k + b];
+            tab[i] = w;
+        }
+        return;
+    }
+    stage_perm(lds, g);
 }
 
 __device__ inline void stage_binom(uint64_t *bin_lds, const uint64_t *bin) {
@@ -88,9 +114,9 @@ __device__ inline void stage_group(GroupLds &t, const GroupView &g) {
         t.flip[i] = g.flip[i];
         t.inv[i] = g.inv[i];
     }
-    if (g.lut == 1 || g.lut == 2)
+    if (g.lut == 1 || g.lut == 2 || g.lut == 4)
         for (int i = threadIdx.x; i < kLutBytes; i += blockDim.x) t.lut[i] = g.lut_tab[i];
-    if (g.lut == 3)
+    if (g.lut >= 3)
         for (int i = threadIdx.x; i < kCosBytes; i += blockDim.x) t.cos[i] = g.cos_tab[i];
 }
 
@@ -124,8 +150,9 @@ __device__ inline S apply_elem_div(S x, int g, const GroupView &gv, const GroupL
 
 // Colex rank: sum over set bits p_0 < p_1 < ... of C(p_j, j+1); equals the
 // reference's GetIndexInHilbertSubspace (utils.cu:9-36).
-template <class S>
-__device__ inline int64_t colex_rank(S x, const uint64_t *bin_lds) {
+// (the table's entries: uint64, or the narrow RankOf<S> of stage_binom_rows)
+template <class S, class T>
+__device__ inline int64_t colex_rank(S x, const T *bin_lds) {
     int64_t r = 0;
     int j = 1;
     while (x) {
@@ -137,18 +164,38 @@ __device__ inline int64_t colex_rank(S x, const uint64_t *bin_lds) {
     return r;
 }
 
-// Inverse of colex_rank for popcount k (k <= 32).
+// Ranks of narrow states (at most 32 sites) fit 32 bits, table entries too.
 template <class S>
-__device__ inline S colex_unrank(int64_t rank, int k, int n_sites, const uint64_t *bin_lds) {
+struct RankOf {
+    using T = uint64_t;
+};
+template <>
+struct RankOf<uint32_t> {
+    using T = uint32_t;
+};
+
+// The rows of the binomial table that unranking reads, as ranks of S.
+template <class S>
+__device__ inline void stage_binom_rows(typename RankOf<S>::T *lds, const uint64_t *bin, int n_sites) {
+    for (int i = threadIdx.x; i < n_sites * kBinJ; i += blockDim.x) lds[i] = (typename RankOf<S>::T)bin[i];
+}
+
+// Inverse of colex_rank for popcount k (k <= 32): from the top site down, site p
+// is up when at least C(p, j) states with the j remaining up spins lie below.
+// Branch-free (lanes of a wave differ in where their up spins are); C(p, j) = 0
+// for p < j places the last ones, and with j = 0 the rank left is 0 < C(p, 0).
+template <class S>
+__device__ inline S colex_unrank(typename RankOf<S>::T r, int k, int n_sites,
+                                 const typename RankOf<S>::T *bin_lds) {
     S x = 0;
-    uint64_t r = (uint64_t)rank;
-    int p = n_sites - 1;
-    for (int j = k; j >= 1; --j) {
-        while (p >= j && bin_lds[p * kBinJ + j] > r) --p;
-        if (p < j - 1) p = j - 1;
-        x |= (S)1 << p;
-        r -= bin_lds[p * kBinJ + j];
-        --p;
+    int at = (n_sites - 1) * kBinJ + k;
+#pragma unroll 4
+    for (int p = n_sites - 1; p >= 0; --p) {
+        const typename RankOf<S>::T c = bin_lds[at];
+        const bool up = r >= c;
+        x = (S)((x << 1) | (up ? 1 : 0));
+        r -= up ? c : 0;
+        at -= kBinJ + (up ? 1 : 0);
     }
     return x;
 }
@@ -161,8 +208,9 @@ __device__ inline S next_comb(S x) {
     return (S)((((r ^ x) >> 2) >> ctz_s(x)) | r);
 }
 
-// Image of x under coset representative c_i (i >= 1) of a lut-3 group: one bit
-// reversal when c_i is the site reversal, else the generic permutation.
+// Image of x under coset representative c_i (i >= 1) of a lut-3 or lut-4 group:
+// one bit reversal when c_i is the site reversal, else the nibble table of
+// stage_images.
 template <class S>
 __device__ inline S reverse_sites(S x, int n);
 template <>
@@ -176,7 +224,11 @@ __device__ inline uint64_t reverse_sites<uint64_t>(uint64_t x, int n) {
 template <class S>
 __device__ inline S coset_image(S x, int ci, const GroupView &gv, const GroupLds &t, const uint8_t *perm_lds) {
     if ((gv.cos_rev >> ci) & 1) return reverse_sites<S>(x, gv.n_sites);
-    return apply_elem_div<S>(x, t.cos[ci * 128], gv, t, perm_lds);
+    const int nn = (gv.n_sites + 3) / 4;
+    const S *tab = reinterpret_cast<const S *>(perm_lds) + (ci - 1) * nn * 16;
+    S y = 0;
+    for (int k = 0; k < nn; ++k) y |= tab[k * 16 + (int)((x >> (4 * k)) & 15)];
+    return t.flip[t.cos[ci * 128]] ? (S)(y ^ (S)gv.full) : y;
 }
 
 // Left rotation of an n-site ring state by s (0 <= s < n).
@@ -188,17 +240,15 @@ __device__ inline S rotl_ring(S y, int s, int n, S full) {
 // Stabiliser of x for a group of ring rotations times cosets (gv.lut == 3):
 // the images of (rotation s, flip f) o c_i are the rotations of c_i x.
 template <class S>
-__device__ inline void stabiliser_coset(S x, const GroupView &gv, const uint8_t *perm_lds, uint64_t &stab_lo,
-                                        uint64_t &stab_hi) {
+__device__ inline void stabiliser_coset(S x, const GroupView &gv, const GroupLds &t, const uint8_t *perm_lds,
+                                        uint64_t &stab_lo, uint64_t &stab_hi) {
     const int N = gv.n_sites;
     const S full = (S)gv.full;
     stab_lo = 0;
     stab_hi = 0;
     for (int ci = 0; ci < gv.n_cos; ++ci) {
-        const uint8_t *ct = gv.cos_tab + ci * 128;
-        S y = !ci                        ? x
-              : ((gv.cos_rev >> ci) & 1) ? reverse_sites<S>(x, N)
-                                         : apply_elem<S>(x, ct[0], gv, perm_lds);
+        const uint8_t *ct = t.cos + ci * 128;
+        S y = ci ? coset_image<S>(x, ci, gv, t, perm_lds) : x;
         for (int s = 0; s < N; ++s) {
             if (s) y = rotl_ring<S>(y, 1, N, full);
             for (int f = 0; f < (gv.lut_flip ? 2 : 1); ++f) {
@@ -213,49 +263,41 @@ __device__ inline void stabiliser_coset(S x, const GroupView &gv, const uint8_t 
     }
 }
 
-// Representative test. Returns true when x is the smallest integer of its
-// orbit; on success stab_lo/hi hold the stabiliser (elements with image x).
+// Stabiliser (elements with image x) of an orbit minimum x; ring groups read the
+// element table only for images equal to x.
 template <class S>
-__device__ inline bool is_representative(S x, const GroupView &gv, const uint8_t *perm_lds, uint64_t &stab_lo,
-                                         uint64_t &stab_hi) {
+__device__ inline void stabiliser(S x, const GroupView &gv, const GroupLds &t, const uint8_t *perm_lds,
+                                  uint64_t &stab_lo, uint64_t &stab_hi) {
     if (gv.lut == 3) {
-        stabiliser_coset<S>(x, gv, perm_lds, stab_lo, stab_hi);
-        return true;  // callers pass representatives only
+        stabiliser_coset<S>(x, gv, t, perm_lds, stab_lo, stab_hi);
+        return;
     }
+    stab_lo = 0;
+    stab_hi = 0;
     if (gv.lut == 2) {
-        // ring: the rotations one bit at a time (and their complements); the
-        // element table is read only for images equal to x
         const int N = gv.n_sites;
         const S full = (S)gv.full;
-        stab_lo = 0;
-        stab_hi = 0;
         S y = x;
         for (int st = 0; st < N; ++st) {
             if (st) y = rotl_ring<S>(y, 1, N, full);
             for (int f = 0; f < (gv.lut_flip ? 2 : 1); ++f) {
                 if ((f ? (S)(y ^ full) : y) != x) continue;
-                const int g = gv.lut_tab[512 + f * 64 + st];
+                const int g = t.lut[512 + f * 64 + st];
                 if (g < 64)
                     stab_lo |= 1ULL << g;
                 else
                     stab_hi |= 1ULL << (g - 64);
             }
         }
-        return true;  // callers pass representatives only
+        return;
     }
-    stab_lo = 0;
-    stab_hi = 0;
     for (int g = 0; g < gv.G; ++g) {
-        const S y = apply_elem<S>(x, g, gv, perm_lds);
-        if (y < x) return false;
-        if (y == x) {
-            if (g < 64)
-                stab_lo |= 1ULL << g;
-            else
-                stab_hi |= 1ULL << (g - 64);
-        }
+        if (apply_elem<S>(x, g, gv, perm_lds) != x) continue;
+        if (g < 64)
+            stab_lo |= 1ULL << g;
+        else
+            stab_hi |= 1ULL << (g - 64);
     }
-    return true;
 }
 
 // Orbit minimum of a state and the canonical element gm = the smallest g with
@@ -282,6 +324,19 @@ __device__ inline S orbit_min(S x, const GroupView &gv, const uint8_t *perm_lds,
     }
     gm = bi;
     return best;
+}
+
+// Image of x under the torus element (in-block shift sh, block shift by big
+// bits, flip f), formed directly (as apply_elem).
+template <class S>
+__device__ inline S torus_image(S x, int sh, int big, int f, int B, int N, S rep_unit, S full) {
+    S y = x;
+    if (sh) {
+        const S k = (S)(rep_unit * (S)((1u << (B - sh)) - 1u));
+        y = (S)(((y & k) << sh) | ((y & (S)~k & full) >> (B - sh)));
+    }
+    if (big) y = (S)(((y << big) | (y >> (N - big))) & full);
+    return f ? (S)(y ^ full) : y;
 }
 
 // orbit_min for a group that is the whole torus product (gv.lut): an image's
@@ -316,16 +371,8 @@ __device__ inline S orbit_min_lut(S x, const GroupView &gv, const GroupLds &t, i
             while (sm) {
                 const int sh = __builtin_ctz(sm);
                 sm &= sm - 1;
-                // the element (in-block shift sh, block shift a, flip f) applied
-                // directly (as apply_elem): its tables are read only for a new
-                // or tied minimum
-                S y = x;
-                if (sh) {
-                    const S k = (S)((S)gv.rep_unit * (S)((1u << (B - sh)) - 1u));
-                    y = (S)(((y & k) << sh) | ((y & (S)~k & full) >> (B - sh)));
-                }
-                if (big) y = (S)(((y << big) | (y >> (N - big))) & full);
-                if (f) y ^= full;
+                // the element's tables are read only for a new or tied minimum
+                const S y = torus_image<S>(x, sh, big, f, B, N, (S)gv.rep_unit, full);
                 if (bi < 0 || y < best) {
                     best = y;
                     bi = t.inv[t.lut[512 + (f * 8 + a) * 8 + sh]];
@@ -342,37 +389,99 @@ __device__ inline S orbit_min_lut(S x, const GroupView &gv, const GroupLds &t, i
     return best;
 }
 
-// Representative test for a full torus product (gv.lut == 1): x is the orbit
-// minimum iff no image is smaller. Only the images whose top block reaches the
-// smallest rotated block tmin can be <= x (the others have a larger top block),
-// so those candidates decide it, and the ones equal to x are the stabiliser.
-// The caller has checked that x's own top block is tmin.
+// orbit_min for a full torus product times cosets (gv.lut == 4): the orbit is
+// the union of the torus orbits of y_i = c_i x; only cosets whose smallest
+// rotated block reaches the smallest so far take full images of their
+// candidates. Same result and same gm as orbit_min.
 template <class S>
-__device__ inline bool rep_stab_lut(S x, const GroupView &gv, const GroupLds &t, uint64_t &stab_lo,
-                                    uint64_t &stab_hi) {
-    const int B = gv.block, nb = gv.n_sites / B;
+__device__ inline S orbit_min_torus_coset(S x, const GroupView &gv, const GroupLds &t, const uint8_t *perm_lds,
+                                          int &gm, int &mult) {
+    const int B = gv.block, N = gv.n_sites, nb = N / B;
+    const unsigned mB = (1u << B) - 1u;
+    const S full = (S)gv.full;
+    const int nf = gv.lut_flip ? 2 : 1;
+    S best = 0;
+    int bi = -1;
+    mult = 0;
+    unsigned tbest = 0xFFu;
+    for (int ci = 0; ci < gv.n_cos; ++ci) {
+        const uint8_t *ct = t.cos + ci * 128;
+        const S z = ci ? coset_image<S>(x, ci, gv, t, perm_lds) : x;
+        unsigned tmin = 0xFFu;
+        for (int j = 0; j < nb; ++j) {
+            const unsigned v = (unsigned)(z >> (j * B)) & mB;
+            tmin = min(tmin, (unsigned)t.lut[v]);
+            if (nf == 2) tmin = min(tmin, (unsigned)t.lut[v ^ mB]);
+        }
+        if (tmin > tbest) continue;
+        tbest = tmin;
+        for (int j = 0; j < nb; ++j) {
+            const unsigned v0 = (unsigned)(z >> (j * B)) & mB;
+            const int a = nb - 1 - j;
+            for (int f = 0; f < nf; ++f) {
+                const unsigned v = f ? (v0 ^ mB) : v0;
+                if (t.lut[v] != tmin) continue;
+                unsigned sm = t.lut[256 + v];
+                while (sm) {
+                    const int sh = __builtin_ctz(sm);
+                    sm &= sm - 1;
+                    const S y = torus_image<S>(z, sh, a * B, f, B, N, (S)gv.rep_unit, full);
+                    if (bi < 0 || y < best) {
+                        best = y;
+                        bi = t.inv[ct[(f * 8 + a) * 8 + sh]];
+                        mult = 1;
+                    } else if (y == best) {
+                        ++mult;
+                        const int ig = t.inv[ct[(f * 8 + a) * 8 + sh]];
+                        if (ig < bi) bi = ig;
+                    }
+                }
+            }
+        }
+    }
+    gm = bi;
+    return best;
+}
+
+// Representative test for a full torus product (gv.lut == 1), or one times cosets
+// (gv.lut == 4: the orbit is the union of the torus orbits of the images c_i x).
+// x is the orbit minimum iff no image is smaller. Only the images whose top
+// block reaches x's own, tmin, can be <= x (the others have a larger top block),
+// so those candidates decide it, and the ones equal to x are the stabiliser.
+// The caller has checked that no rotated block of x itself is below tmin.
+template <class S>
+__device__ inline bool rep_stab_lut(S x, const GroupView &gv, const GroupLds &t, const uint8_t *perm_lds,
+                                    uint64_t &stab_lo, uint64_t &stab_hi) {
+    const int B = gv.block, N = gv.n_sites, nb = N / B;
     const unsigned mB = (1u << B) - 1u;
     const unsigned tmin = (unsigned)(x >> ((nb - 1) * B)) & mB;
+    const S full = (S)gv.full;
+    const int n_cos = gv.lut == 4 ? gv.n_cos : 1;
     stab_lo = 0;
     stab_hi = 0;
-    for (int j = 0; j < nb; ++j) {
-        const unsigned v0 = (unsigned)(x >> (j * B)) & mB;
-        const int a = nb - 1 - j;
-        for (int f = 0; f < (gv.lut_flip ? 2 : 1); ++f) {
-            const unsigned v = f ? (v0 ^ mB) : v0;
-            if (t.lut[v] != tmin) continue;
-            unsigned sm = t.lut[256 + v];
-            while (sm) {
-                const int sh = __builtin_ctz(sm);
-                sm &= sm - 1;
-                const int g = t.lut[512 + (f * 8 + a) * 8 + sh];
-                const S y = apply_elem_div<S>(x, g, gv, t, nullptr);
-                if (y < x) return false;
-                if (y == x) {
-                    if (g < 64)
-                        stab_lo |= 1ULL << g;
-                    else
-                        stab_hi |= 1ULL << (g - 64);
+    for (int ci = 0; ci < n_cos; ++ci) {
+        const uint8_t *ct = gv.lut == 4 ? t.cos + ci * 128 : t.lut + 512;
+        const S z = ci ? coset_image<S>(x, ci, gv, t, perm_lds) : x;
+        for (int j = 0; j < nb; ++j) {
+            const unsigned v0 = (unsigned)(z >> (j * B)) & mB;
+            const int a = nb - 1 - j;
+            for (int f = 0; f < (gv.lut_flip ? 2 : 1); ++f) {
+                const unsigned v = f ? (v0 ^ mB) : v0;
+                if (t.lut[v] > tmin) continue;
+                if (t.lut[v] < tmin) return false;
+                unsigned sm = t.lut[256 + v];
+                while (sm) {
+                    const int sh = __builtin_ctz(sm);
+                    sm &= sm - 1;
+                    const S y = torus_image<S>(z, sh, a * B, f, B, N, (S)gv.rep_unit, full);
+                    if (y < x) return false;
+                    if (y == x) {
+                        const int g = ct[(f * 8 + a) * 8 + sh];
+                        if (g < 64)
+                            stab_lo |= 1ULL << g;
+                        else
+                            stab_hi |= 1ULL << (g - 64);
+                    }
                 }
             }
         }
@@ -498,6 +607,17 @@ __device__ inline S orbit_min_coset(S x, const GroupView &gv, const GroupLds &t,
     return best;
 }
 
+// The orbit minimum by the group's form (GroupView::lut).
+template <class S>
+__device__ inline S orbit_min_any(S x, const GroupView &gv, const GroupLds &t, const uint8_t *perm_lds, int &gm,
+                                  int &mult) {
+    return gv.lut == 1   ? orbit_min_lut<S>(x, gv, t, gm, mult)
+           : gv.lut == 2 ? orbit_min_ring<S>(x, gv, t, gm, mult)
+           : gv.lut == 3 ? orbit_min_coset<S>(x, gv, t, perm_lds, gm, mult)
+           : gv.lut == 4 ? orbit_min_torus_coset<S>(x, gv, t, perm_lds, gm, mult)
+                         : orbit_min<S>(x, gv, perm_lds, gm, mult);
+}
+
 // Colex rank by nibbles: T[(k * n_c + c) * 16 + v] is the rank contribution of
 // nibble k (sites 4k..4k+3) holding v when c set bits lie below it, i.e. the sum
 // over v's set bits i (ascending, j of v's bits below i) of C(4k + i, c + j + 1).
@@ -556,8 +676,8 @@ __device__ inline int64_t row_of_rank(int64_t rk, const uint64_t *dict) {
     return (int64_t)rec.y + __popcll(below);
 }
 
-template <class S>
-__device__ inline int64_t row_of_rep(S rep, const uint64_t *bin_lds, const uint64_t *dict) {
+template <class S, class T>
+__device__ inline int64_t row_of_rep(S rep, const T *bin_lds, const uint64_t *dict) {
     return row_of_rank(colex_rank<S>(rep, bin_lds), dict);
 }
 

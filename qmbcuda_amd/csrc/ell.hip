@@ -84,7 +84,7 @@ __global__ __launch_bounds__(kEllThreads) void ell_rows(GroupView gv, const uint
                                                         int all_rows, const int64_t *chunk_ptr, int32_t *col,
                                                         double *val, CodeView cv) {
     extern __shared__ uint64_t rank_lds[];
-    __shared__ uint8_t perm_lds[kMaxGroup * 64];
+    __shared__ alignas(8) uint8_t perm_lds[kMaxGroup * 64];
     __shared__ double2 s_chi[kMaxGroup];
     __shared__ double s_nrm[kMaxGroup + 1];
     __shared__ GroupLds gt;
@@ -94,7 +94,7 @@ __global__ __launch_bounds__(kEllThreads) void ell_rows(GroupView gv, const uint
     // (row length = 1 + the acting off-diagonal terms): no tables to stage
     const bool lookups = FILL || !all_rows;
     if (lookups) {
-        stage_perm(perm_lds, gv);
+        stage_images<S>(perm_lds, gv);
         stage_group(gt, gv);
         if (n_nib) {
             for (int i = threadIdx.x; i < n_nib * n_c * 16; i += blockDim.x) rank_lds[i] = rank_tab[i];
@@ -158,10 +158,7 @@ __global__ __launch_bounds__(kEllThreads) void ell_rows(GroupView gv, const uint
                 S tgt;
                 apply_term<S>(tv, h, src, tgt, cr, ci);
                 int gm, mult;
-                const S rep = gv.lut == 1   ? orbit_min_lut<S>(tgt, gv, gt, gm, mult)
-                              : gv.lut == 2 ? orbit_min_ring<S>(tgt, gv, gt, gm, mult)
-                              : gv.lut == 3 ? orbit_min_coset<S>(tgt, gv, gt, perm_lds, gm, mult)
-                                            : orbit_min<S>(tgt, gv, perm_lds, gm, mult);
+                const S rep = orbit_min_any<S>(tgt, gv, gt, perm_lds, gm, mult);
                 const int64_t r2 = row_of_rank(
                     n_nib ? colex_rank_nib<S>(rep, rank_lds, n_nib, n_c) : colex_rank<S>(rep, rank_lds), dict);
                 if (r2 < 0) continue;

@@ -44,15 +44,17 @@ __global__ __launch_bounds__(kExpThreads) void expect_rows(GroupView gv, const u
                                                            const uint8_t *nullf, const uint64_t *dict,
                                                            TermsView tv, const double2 *chi,
                                                            const double *nrm, const double *x, double *partials) {
-    __shared__ uint8_t perm_lds[kMaxGroup * 64];
-    __shared__ uint64_t bin[64 * kBinJ];
+    __shared__ alignas(8) uint8_t perm_lds[kMaxGroup * 64];
+    __shared__ typename RankOf<S>::T bin[sizeof(S) * 8 * kBinJ];
     __shared__ double2 s_chi[kMaxGroup];
     __shared__ double s_nrm[kMaxGroup + 1];
     __shared__ GroupLds gt;
     __shared__ double red[kWaves];
+    __shared__ alignas(8) uint8_t img_lds[4096];  // coset representatives' images (stage_images)
     stage_perm(perm_lds, gv);
+    if (gv.lut >= 3) stage_images<S>(img_lds, gv);
     stage_group(gt, gv);
-    stage_binom(bin, binom);
+    stage_binom_rows<S>(bin, binom, gv.n_sites);
     for (int i = threadIdx.x; i < gv.G; i += blockDim.x) s_chi[i] = chi[i];
     for (int i = threadIdx.x; i <= gv.G; i += blockDim.x) s_nrm[i] = nrm[i];
     __syncthreads();
@@ -99,10 +101,7 @@ __global__ __launch_bounds__(kExpThreads) void expect_rows(GroupView gv, const u
                     S tgt;
                     apply_term<S>(tv, h, u, tgt, cr, ci);
                     int gm, mult;
-                    const S rep2 = gv.lut == 1   ? orbit_min_lut<S>(tgt, gv, gt, gm, mult)
-                                   : gv.lut == 2 ? orbit_min_ring<S>(tgt, gv, gt, gm, mult)
-                                   : gv.lut == 3 ? orbit_min_coset<S>(tgt, gv, gt, perm_lds, gm, mult)
-                                                 : orbit_min<S>(tgt, gv, perm_lds, gm, mult);
+                    const S rep2 = orbit_min_any<S>(tgt, gv, gt, gv.lut >= 3 ? img_lds : perm_lds, gm, mult);
                     const int64_t r2 = row_of_rep<S>(rep2, bin, dict);
                     if (r2 < 0) continue;
                     if (layout == QMB_LAYOUT_REFERENCE && nullf[r2]) continue;

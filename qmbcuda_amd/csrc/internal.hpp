@@ -229,7 +229,7 @@ struct GroupView {
     int n_sites;
     int G;
     int torus;       // 1: cyclic-translation fast path, 0: generic permutation
-    int block;       // torus block width B
+    int block;       // torus block width B (lut 4: of the torus subgroup)
     uint64_t full;   // mask of n_sites bits
     uint64_t rep_unit;  // torus: bit 0 of every block (sum of 1 << (b * block))
     const uint64_t *keep;  // [G] torus in-block no-wrap mask
@@ -241,12 +241,14 @@ struct GroupView {
     int lut;               // 1: the group is every (block shift, in-block shift[, flip]) of a torus;
                            // 2: every rotation[, flip] of a ring
                            // 3: every rotation[, flip] of a ring times n_cos coset representatives
+                   // 4: every (block shift, in-block shift[, flip]) of a torus times n_cos of them
     int lut_flip;          //    with a spin-flip half
     const uint8_t *lut_tab;  // [kLutBytes] rotation minima and element index table (see device_common.hpp)
     int n_cos;
     int cos_rev;             // bit i: c_i is the site reversal s -> N-1-s
-    const uint8_t *cos_tab;  // lut 3: [kCosBytes] element index of (rotation s, flip f) o c_i at
-                             // i * 128 + f * 64 + s (c_i first; entry i * 128 is c_i itself)
+    const uint8_t *cos_tab;  // lut 3, 4: [kCosBytes] element index of (subgroup element s, flip f) o c_i
+                             // at i * 128 + f * 64 + s (c_i first; entry i * 128 is c_i itself); s = the
+                             // rotation (lut 3), or 8 * block shift + in-block shift (lut 4)
 };
 
 constexpr int kLutBytes = 256 + 256 + 2 * 8 * 8;
@@ -341,9 +343,10 @@ struct qmb_group : qmb::Counted {
     uint64_t hash = 0;              // FNV-1a of the element tables, flips and characters
     int lut = 0, lut_flip = 0;     // 1: full torus product with block width <= 8; 2: full ring;
                                    // 3: a full ring subgroup H times coset representatives
+                                   // 4: a full torus product times coset representatives
     std::vector<uint8_t> lut_tab;  // [kLutBytes]
     std::vector<uint8_t> comp;     // [G*G]: index of a o b (b applied first)
-    int n_cos = 0, cos_rev = 0;    // lut 3: cosets of the ring subgroup and their element table
+    int n_cos = 0, cos_rev = 0;    // lut 3, 4: cosets of the subgroup and their element table
     std::vector<uint8_t> cos_tab;  // [kCosBytes]
     std::vector<double> orbit_norms;  // [G + 1]: sqrt(G m)/G for stabiliser size m
 };
