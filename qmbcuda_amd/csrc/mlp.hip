@@ -54,210 +54,272 @@ __device__ inline bf16x8 load8(const uint16_t *p) {
 // B fragment: column l%32, k = 8*(l/32)..+7 (16 k per instruction).
 __device__ inline int mfma_row(int v, int lane) { return 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3); }
 
-// ---- forward: one wavefront per 32 rows --------------------------------------
-// Row r = c*256 + p: pattern p, coupling c. Writes out[r][2]; with store, also
-// H1 (FP32 and bf16) and H2 (FP32) for the backward pass.
+// ---- forward: four wavefronts per 32 rows --------------------------------------
+// Row r = c*256 + p: pattern p, coupling c (whole couplings). Writes
+// out[r][2]; with store, also H1 (FP32 and bf16) and H2 (FP32) for the backward
+// pass. The tile's work is a chain of short phases, so its four wavefronts share
+// the long ones: layer 1 by hidden unit and row half, layer 2 one 32-column MFMA
+// tile each (one wavefront per tile: 41 us for 192 couplings, 28 us for one; now
+// 26 and 11 us).
 constexpr int kTileLd = kH + 8;  // bf16 row stride of the LDS activation tile
+constexpr int kFwdThreads = 256;
 
-__global__ __launch_bounds__(64) void mlp_forward(const float *__restrict__ theta, const uint16_t *__restrict__ w2bf,
-                                                  const double *__restrict__ coup, int n_rows,
-                                                  float *__restrict__ out, float *__restrict__ H1,
-                                                  uint16_t *__restrict__ H1q, float *__restrict__ H2, int store) {
+__global__ __launch_bounds__(kFwdThreads) void mlp_forward(const float *__restrict__ theta,
+                                                           const uint16_t *__restrict__ w2bf,
+                                                           const double *__restrict__ coup, float *__restrict__ out, float *__restrict__ H1,
+                                                           uint16_t *__restrict__ H1q, float *__restrict__ H2,
+                                                           int store) {
     __shared__ float x[32][kIn];
-    __shared__ uint16_t a_tile[32 * kTileLd];
+    __shared__ alignas(16) uint16_t a_tile[32 * kTileLd];
     __shared__ float h2[32][kH + 1];
-    const int lane = threadIdx.x;
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
     const int r0 = blockIdx.x * 32;
-    if (lane < 32) {
-        const int r = r0 + lane;
-        const int p = r & 255;
-        const int c = r >> 8;
-        for (int i = 0; i < kWin; ++i) x[lane][i] = ((p >> i) & 1) ? 1.f : -1.f;
-        x[lane][8] = r < n_rows ? (float)coup[2 * c] : 0.f;
-        x[lane][9] = r < n_rows ? (float)coup[2 * c + 1] : 0.f;
+    if (t < 32) {
+        const int p = (r0 + t) & 255;
+        const int c = (r0 + t) >> 8;
+        for (int i = 0; i < kWin; ++i) x[t][i] = ((p >> i) & 1) ? 1.f : -1.f;
+        x[t][8] = (float)coup[2 * c];
+        x[t][9] = (float)coup[2 * c + 1];
     }
+    bf16x8 bw[kH / 16];
+#pragma unroll
+    for (int kb = 0; kb < kH / 16; ++kb)
+        bw[kb] = load8(w2bf + (size_t)(wv * 32 + (lane & 31)) * kH + kb * 16 + 8 * (lane >> 5));
+    const int k = t & (kH - 1), half = t >> 7;
+    float w[kIn];
+    for (int i = 0; i < kIn; ++i) w[i] = theta[oW1 + k * kIn + i];
+    const float b1 = theta[ob1 + k];
     __syncthreads();
-    // layer 1 (VALU): lane owns hidden units 2*lane, 2*lane+1
-    for (int u = 0; u < 2; ++u) {
-        const int k = 2 * lane + u;
-        float w[kIn];
-        for (int i = 0; i < kIn; ++i) w[i] = theta[oW1 + k * kIn + i];
-        const float b = theta[ob1 + k];
-        for (int row = 0; row < 32; ++row) {
-            float s = b;
-            for (int i = 0; i < kIn; ++i) s += w[i] * x[row][i];
-            const float h = tanhf(s);
-            const uint16_t q = to_bf16_bits(h);
-            a_tile[row * kTileLd + k] = q;
-            const int r = r0 + row;
-            if (store && r < n_rows) {
-                H1[(size_t)r * kH + k] = h;
-                H1q[(size_t)r * kH + k] = q;
-            }
+    // layer 1 (VALU): hidden unit k, 16 rows
+    for (int row = half * 16; row < half * 16 + 16; ++row) {
+        float s = b1;
+        for (int i = 0; i < kIn; ++i) s += w[i] * x[row][i];
+        const float h = tanhf(s);
+        const uint16_t q = to_bf16_bits(h);
+        a_tile[row * kTileLd + k] = q;
+        if (store) {
+            H1[(size_t)(r0 + row) * kH + k] = h;
+            H1q[(size_t)(r0 + row) * kH + k] = q;
         }
     }
     __syncthreads();
     // layer 2 (MFMA): H2 = tanh(H1q W2^T + b2)
-    for (int nt = 0; nt < 4; ++nt) {
+    {
         f32x16 acc = {};
+#pragma unroll
         for (int kb = 0; kb < kH / 16; ++kb) {
             const bf16x8 a = load8(a_tile + (lane & 31) * kTileLd + kb * 16 + 8 * (lane >> 5));
-            const bf16x8 b = load8(w2bf + (size_t)(nt * 32 + (lane & 31)) * kH + kb * 16 + 8 * (lane >> 5));
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bw[kb], acc, 0, 0, 0);
         }
-        const int col = nt * 32 + (lane & 31);
+        const int col = wv * 32 + (lane & 31);
         const float b2 = theta[ob2 + col];
-        for (int v = 0; v < 16; ++v) h2[mfma_row(v, lane)][col] = tanhf(acc[v] + b2);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            const float h = tanhf(acc[v] + b2);
+            h2[mfma_row(v, lane)][col] = h;
+            if (store) H2[(size_t)(r0 + mfma_row(v, lane)) * kH + col] = h;
+        }
     }
     __syncthreads();
-    // head (VALU): lane -> (row = lane%32, output = lane/32)
-    {
+    // head (VALU), in index order: lane -> (row = lane % 32, output = lane / 32)
+    if (wv == 0) {
         const int row = lane & 31, o = lane >> 5;
         float s = theta[ob3 + o];
-        for (int k = 0; k < kH; ++k) s += theta[oW3 + o * kH + k] * h2[row][k];
-        const int r = r0 + row;
-        if (r < n_rows) out[(size_t)r * 2 + o] = s;
-    }
-    if (store) {
-        for (int idx = lane; idx < 32 * kH; idx += 64) {
-            const int row = idx / kH, k = idx % kH;
-            const int r = r0 + row;
-            if (r < n_rows) H2[(size_t)r * kH + k] = h2[row][k];
-        }
+#pragma unroll 8
+        for (int j = 0; j < kH; ++j) s += theta[oW3 + o * kH + j] * h2[row][j];
+        out[(size_t)(r0 + row) * 2 + o] = s;
     }
 }
 
-// ---- backward, activations: dA2 = (dout W3) (1 - H2^2); dA1 = (dA2 W2) (1 - H1^2)
-// dA1 uses MFMA with B = W2 read column-wise through its transpose w2t[j][n].
-__global__ __launch_bounds__(64) void mlp_backward_act(const float *__restrict__ theta,
-                                                       const uint16_t *__restrict__ w2t, int n_rows,
-                                                       const float *__restrict__ dout, const float *__restrict__ H1,
-                                                       const float *__restrict__ H2, float *__restrict__ dA2,
-                                                       uint16_t *__restrict__ dA2q, float *__restrict__ dA1) {
-    __shared__ uint16_t a_tile[32 * kTileLd];
-    const int lane = threadIdx.x;
-    const int r0 = blockIdx.x * 32;
-    for (int idx = lane; idx < 32 * kH; idx += 64) {
-        const int row = idx / kH, k = idx % kH;
-        const int r = r0 + row;
-        float g = 0.f;
-        if (r < n_rows) {
-            const float h = H2[(size_t)r * kH + k];
-            g = (dout[(size_t)r * 2] * theta[oW3 + k] + dout[(size_t)r * 2 + 1] * theta[oW3 + kH + k]) * (1.f - h * h);
-            dA2[(size_t)r * kH + k] = g;
-        }
-        const uint16_t q = to_bf16_bits(g);
-        a_tile[row * kTileLd + k] = q;
-        if (r < n_rows) dA2q[(size_t)r * kH + k] = q;
-    }
+// ---- backward: one block per coupling (256 rows), every weight gradient ------
+// Tiles of 32 rows: dA2 = (dout W3) (1 - H2^2) goes to LDS in bf16, by rows and
+// transposed, with H1q transposed; dA1 = (dA2 W2) (1 - H1^2) on MFMA (wavefront w
+// owns columns 32 w .. 32 w + 31, its W2 fragments stay in registers), and
+// dW2 += dA2^T H1q on MFMA (wavefront w owns rows 32 w .. of dW2). dA2 and dA1
+// are used up where they are formed (the sums of b2, W3, b1, W1 too), so only
+// H1, H1q and H2 are read; the tiles are double buffered, one barrier each.
+// 192 couplings: 28 us, 38 us with the reduction; as four kernels that passed dA2 and dA1 through memory
+// (and split the rows of dW2 over 48 blocks only) 626 us.
+// dout comes from the pattern histograms: pattern p of the coupling has
+// hist[2 p], hist[2 p + 1] in units of 1 / kFix.
+constexpr int kBackThreads = 256;
+constexpr int kTr = 40;  // bf16 row stride of the transposed tiles (32 rows, 16-byte aligned)
+
+__global__ __launch_bounds__(kBackThreads) void mlp_backward(const float *__restrict__ theta,
+                                                             const uint16_t *__restrict__ w2t,
+                                                             const double *__restrict__ coup,
+                                                             const unsigned long long *__restrict__ hist, float scale,
+                                                             const float *__restrict__ H1,
+                                                             const uint16_t *__restrict__ H1q,
+                                                             const float *__restrict__ H2,
+                                                             float *__restrict__ part) {
+    __shared__ float dout[256][2];
+    __shared__ alignas(16) uint16_t a_tile[2][32 * kTileLd];  // dA2: [row][k]
+    __shared__ alignas(16) uint16_t at[2][kH * kTr];          // dA2^T: [k][row]
+    __shared__ alignas(16) uint16_t bt[2][kH * kTr];          // H1q^T: [k][row]
+    __shared__ float red[kH][3];
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    const int g = blockIdx.x;
+    const size_t r0 = (size_t)g * 256;
+    for (int i = t; i < 512; i += kBackThreads)
+        dout[i >> 1][i & 1] = (float)((double)(long long)hist[r0 * 2 + i] / kFix * scale);
+    bf16x8 bw[kH / 16];
+#pragma unroll
+    for (int kb = 0; kb < kH / 16; ++kb)
+        bw[kb] = load8(w2t + (size_t)(wv * 32 + (lane & 31)) * kH + kb * 16 + 8 * (lane >> 5));
+    // element-wise part: hidden unit k, rows 16 half .. of each tile
+    const int k = t & (kH - 1), half = t >> 7;
+    const float w3a = theta[oW3 + k], w3b = theta[oW3 + kH + k];
+    float gb2 = 0.f, gw3a = 0.f, gw3b = 0.f;
+    // dA1 part: column col of this lane
+    const int col = wv * 32 + (lane & 31), hi = lane >> 5;
+    float gw1[kWin] = {}, gb1 = 0.f;
+    f32x16 acc2[4] = {};
     __syncthreads();
-    for (int nt = 0; nt < 4; ++nt) {
-        f32x16 acc = {};
-        for (int kb = 0; kb < kH / 16; ++kb) {
-            const bf16x8 a = load8(a_tile + (lane & 31) * kTileLd + kb * 16 + 8 * (lane >> 5));
-            const bf16x8 b = load8(w2t + (size_t)(nt * 32 + (lane & 31)) * kH + kb * 16 + 8 * (lane >> 5));
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
+    for (int tl = 0; tl < 8; ++tl) {
+        const int bu = tl & 1;
+        uint16_t *ta = a_tile[bu], *tt = at[bu], *tb = bt[bu];
+        {
+            float h[16];
+            uint16_t q[16];
+            const size_t base = (r0 + tl * 32 + half * 16) * kH + k;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) h[i] = H2[base + (size_t)i * kH];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) q[i] = H1q[base + (size_t)i * kH];
+            __builtin_memcpy(__builtin_assume_aligned(tb + k * kTr + half * 16, 16), q, 32);
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int row = half * 16 + i;
+                const float da = dout[tl * 32 + row][0], db = dout[tl * 32 + row][1];
+                const float v = (da * w3a + db * w3b) * (1.f - h[i] * h[i]);
+                gb2 += v;
+                gw3a += da * h[i];
+                gw3b += db * h[i];
+                q[i] = to_bf16_bits(v);
+                ta[row * kTileLd + k] = q[i];
+            }
+            __builtin_memcpy(__builtin_assume_aligned(tt + k * kTr + half * 16, 16), q, 32);
         }
-        const int col = nt * 32 + (lane & 31);
-        for (int v = 0; v < 16; ++v) {
-            const int r = r0 + mfma_row(v, lane);
-            if (r < n_rows) {
-                const float h = H1[(size_t)r * kH + col];
-                dA1[(size_t)r * kH + col] = acc[v] * (1.f - h * h);
+        __syncthreads();
+        {
+            f32x16 acc = {};
+#pragma unroll
+            for (int kb = 0; kb < kH / 16; ++kb) {
+                const bf16x8 x = load8(ta + (lane & 31) * kTileLd + kb * 16 + 8 * hi);
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, bw[kb], acc, 0, 0, 0);
+            }
+            // row 8 (v / 4) + 4 hi + v % 4 of the tile: pattern bits 0, 1 = v % 4, bit 2 = hi,
+            // bits 3, 4 = v / 4, bits 5 .. 7 = the tile
+            float sum = 0.f, s0 = 0.f, s1 = 0.f, s3 = 0.f, s4 = 0.f;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const float h = H1[(r0 + tl * 32 + mfma_row(v, lane)) * kH + col];
+                const float d = acc[v] * (1.f - h * h);
+                sum += d;
+                s0 += (v & 1) ? d : -d;
+                s1 += (v & 2) ? d : -d;
+                s3 += (v & 4) ? d : -d;
+                s4 += (v & 8) ? d : -d;
+            }
+            gb1 += sum;
+            gw1[0] += s0;
+            gw1[1] += s1;
+            gw1[2] += hi ? sum : -sum;
+            gw1[3] += s3;
+            gw1[4] += s4;
+            gw1[5] += (tl & 1) ? sum : -sum;
+            gw1[6] += (tl & 2) ? sum : -sum;
+            gw1[7] += (tl & 4) ? sum : -sum;
+        }
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+            const bf16x8 x = load8(tt + (wv * 32 + (lane & 31)) * kTr + kb * 16 + 8 * hi);
+#pragma unroll
+            for (int nt = 0; nt < 4; ++nt) {
+                const bf16x8 y = load8(tb + (nt * 32 + (lane & 31)) * kTr + kb * 16 + 8 * hi);
+                acc2[nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, y, acc2[nt], 0, 0, 0);
             }
         }
     }
+    float *dst = part + (size_t)g * kParams;
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt)
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+            dst[oW2 + (wv * 32 + mfma_row(v, lane)) * kH + nt * 32 + (lane & 31)] = acc2[nt][v];
+    // lanes l and l + 32 hold the two row halves of one column
+    gb1 += __shfl_xor(gb1, 32, 64);
+#pragma unroll
+    for (int i = 0; i < kWin; ++i) gw1[i] += __shfl_xor(gw1[i], 32, 64);
+    if (hi == 0) {
+        for (int i = 0; i < kWin; ++i) dst[oW1 + col * kIn + i] = gw1[i];
+        dst[oW1 + col * kIn + 8] = gb1 * (float)coup[2 * g];
+        dst[oW1 + col * kIn + 9] = gb1 * (float)coup[2 * g + 1];
+        dst[ob1 + col] = gb1;
+    }
+    if (half) {
+        red[k][0] = gb2;
+        red[k][1] = gw3a;
+        red[k][2] = gw3b;
+    }
+    __syncthreads();
+    if (!half) {
+        dst[ob2 + k] = gb2 + red[k][0];
+        dst[oW3 + k] = gw3a + red[k][1];
+        dst[oW3 + kH + k] = gw3b + red[k][2];
+    }
+    if (wv == 3 && lane < 2) {
+        float s = 0.f;
+        for (int r = 0; r < 256; ++r) s += dout[r][lane];
+        dst[ob3 + lane] = s;
+    }
 }
 
-// ---- backward, dW2 = dA2^T H1q over a group of rows (MFMA, K = rows) ---------
-// grid (groups, 16): blockIdx.y = output tile (mt, nt); one partial tile per group.
-constexpr int kRowsPerGroup = 1024;
+// grad = sum over the couplings' partials: 64 parameters a block, four slices of
+// the couplings each, added in slice order. The last block: the mean loss.
+constexpr int kReduceParams = 64;
 
-__global__ __launch_bounds__(64) void mlp_wgrad2(int n_rows, const uint16_t *__restrict__ dA2q,
-                                                 const uint16_t *__restrict__ H1q, float *__restrict__ part) {
-    __shared__ uint16_t at[32][40];  // dA2^T tile: [m][row]
-    __shared__ uint16_t bt[32][40];  // H1q^T tile: [n][row]
-    const int lane = threadIdx.x;
-    const int mt = blockIdx.y >> 2, nt = blockIdx.y & 3;
-    const int g0 = blockIdx.x * kRowsPerGroup;
-    f32x16 acc = {};
-    for (int t0 = g0; t0 < g0 + kRowsPerGroup && t0 < n_rows; t0 += 32) {
-        for (int idx = lane; idx < 32 * 32; idx += 64) {
-            const int row = idx / 32, m = idx % 32;
-            const int r = t0 + row;
-            at[m][row] = r < n_rows ? dA2q[(size_t)r * kH + mt * 32 + m] : (uint16_t)0;
-            bt[m][row] = r < n_rows ? H1q[(size_t)r * kH + nt * 32 + m] : (uint16_t)0;
-        }
+__device__ inline void mean_loss(const double *__restrict__ stats, int ns, double *__restrict__ loss) {
+    // the samples' losses in sample order, 256 loaded at a time
+    __shared__ double v[256];
+    double mean = 0.0;
+    for (int k0 = 0; k0 < ns; k0 += 256) {
         __syncthreads();
-        for (int kb = 0; kb < 2; ++kb) {
-            const bf16x8 a = load8(&at[lane & 31][kb * 16 + 8 * (lane >> 5)]);
-            const bf16x8 b = load8(&bt[lane & 31][kb * 16 + 8 * (lane >> 5)]);
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
-        }
+        for (int k = threadIdx.x; k < 256 && k0 + k < ns; k += blockDim.x) v[k] = stats[(size_t)(k0 + k) * 8 + 4];
         __syncthreads();
+        if (threadIdx.x == 0)
+            for (int k = 0; k < 256 && k0 + k < ns; ++k) mean += v[k];
     }
-    float *dst = part + ((size_t)blockIdx.x * kH * kH);
-    for (int v = 0; v < 16; ++v) {
-        const int m = mt * 32 + mfma_row(v, lane), n = nt * 32 + (lane & 31);
-        dst[(size_t)m * kH + n] = acc[v];
-    }
+    if (threadIdx.x == 0) *loss = mean / ns;
 }
 
-// ---- backward, small parameters (VALU) over a group of rows ----------------
-// per group partial of W1, b1, b2, W3, b3 (W2 comes from mlp_wgrad2). Groups of
-// 256 rows (one coupling's patterns): four times as many blocks as the MFMA
-// weight gradient's groups, so the row loops are short.
-constexpr int kRowsPerSmallGroup = 256;
-
-__global__ __launch_bounds__(kH) void mlp_wgrad_small(const double *__restrict__ coup, int n_rows,
-                                                      const float *__restrict__ dout, const float *__restrict__ H2,
-                                                      const float *__restrict__ dA2, const float *__restrict__ dA1,
-                                                      float *__restrict__ part) {
-    const int k = threadIdx.x;  // hidden unit
-    const int g0 = blockIdx.x * kRowsPerSmallGroup;
-    float gw1[kIn] = {}, gb1 = 0.f, gb2 = 0.f, gw3a = 0.f, gw3b = 0.f, gb3a = 0.f, gb3b = 0.f;
-    for (int r = g0; r < g0 + kRowsPerSmallGroup && r < n_rows; ++r) {
-        const int p = r & 255, c = r >> 8;
-        const float d1 = dA1[(size_t)r * kH + k];
-        for (int i = 0; i < kWin; ++i) gw1[i] += d1 * (((p >> i) & 1) ? 1.f : -1.f);
-        gw1[8] += d1 * (float)coup[2 * c];
-        gw1[9] += d1 * (float)coup[2 * c + 1];
-        gb1 += d1;
-        gb2 += dA2[(size_t)r * kH + k];
-        const float h2 = H2[(size_t)r * kH + k];
-        gw3a += dout[(size_t)r * 2] * h2;
-        gw3b += dout[(size_t)r * 2 + 1] * h2;
-        if (k == 0) {
-            gb3a += dout[(size_t)r * 2];
-            gb3b += dout[(size_t)r * 2 + 1];
-        }
+__global__ __launch_bounds__(256) void mlp_reduce_grad(int n_groups, const float *__restrict__ part,
+                                                       float *__restrict__ grad, const double *__restrict__ stats,
+                                                       int ns, double *__restrict__ loss) {
+    if (blockIdx.x == gridDim.x - 1) {
+        mean_loss(stats, ns, loss);
+        return;
     }
-    float *dst = part + (size_t)blockIdx.x * kParams;
-    for (int i = 0; i < kIn; ++i) dst[oW1 + k * kIn + i] = gw1[i];
-    dst[ob1 + k] = gb1;
-    dst[ob2 + k] = gb2;
-    dst[oW3 + k] = gw3a;
-    dst[oW3 + kH + k] = gw3b;
-    if (k == 0) {
-        dst[ob3] = gb3a;
-        dst[ob3 + 1] = gb3b;
-    }
-}
-
-// grad = scale * sum over groups of the partials (W2 from part2 over n_groups2
-// MFMA groups, the rest from part over n_groups small groups).
-__global__ __launch_bounds__(256) void mlp_reduce_grad(int n_groups, int n_groups2, const float *__restrict__ part,
-                                                       const float *__restrict__ part2, float scale,
-                                                       float *__restrict__ grad) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= kParams) return;
+    __shared__ float red[3][kReduceParams];
+    const int sl = threadIdx.x / kReduceParams, at = threadIdx.x % kReduceParams;
+    const int i = blockIdx.x * kReduceParams + at;
     float s = 0.f;
-    if (i >= oW2 && i < ob2) {
-        for (int g = 0; g < n_groups2; ++g) s += part2[(size_t)g * kH * kH + (i - oW2)];
-    } else {
-        for (int g = 0; g < n_groups; ++g) s += part[(size_t)g * kParams + i];
+    if (i < kParams) {
+        const float *p = part + i;
+        int g = sl;
+        for (; g + 28 < n_groups; g += 32) {
+            float v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = p[(size_t)(g + 4 * u) * kParams];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) s += v[u];
+        }
+        for (; g < n_groups; g += 4) s += p[(size_t)g * kParams];
     }
-    grad[i] = s * scale;
+    if (sl) red[sl - 1][at] = s;
+    __syncthreads();
+    if (!sl && i < kParams) grad[i] = s + red[0][at] + red[1][at] + red[2][at];
 }
 
 // Adam (Kingma & Ba 2015) on the FP32 master weights; refresh the bf16 W2 and its transpose.
@@ -308,33 +370,92 @@ __device__ inline void stage_windows(uint8_t *lds, const uint8_t *win, int n_win
     for (int i = threadIdx.x; i < n_win * kWin; i += blockDim.x) lds[i] = win[i];
 }
 
+// Ring windows (sites q .. q + 7 mod N for every q, N >= 11) are taken four at a
+// time: windows q .. q + 3 together are 11 consecutive sites, so one read of a
+// table of 2048 sums replaces four reads of the 256 patterns' values, and one
+// addition into a histogram of 2048 bins four into the patterns' (the bins are
+// folded into the patterns once per block). The N % 4 windows left are taken one
+// at a time. The sums of four 32-bit values are held in 64 bits.
+constexpr int kGroupWin = 4, kGroupPat = 1 << (kWin + kGroupWin - 1);
+
+// sites q, q + 1, ... of an n-site ring from bit 0 up (at least 11 of them right)
+__device__ inline uint64_t ring_from(uint64_t s, int q, int n) { return q ? (s >> q) | (s << (n - q)) : s; }
+
+// t4[p] = sum of t over the four windows inside p
+__device__ inline void group_table(const float2 *t, double2 *t4) {
+    for (int p = threadIdx.x; p < kGroupPat; p += blockDim.x) {
+        double2 v = make_double2(0.0, 0.0);
+#pragma unroll
+        for (int i = 0; i < kGroupWin; ++i) {
+            const float2 w = t[(p >> i) & 255];
+            v.x += (double)w.x;
+            v.y += (double)w.y;
+        }
+        t4[p] = v;
+    }
+}
+
+// log-amplitude and phase sums over the windows of R states per thread
+template <int R>
+__device__ inline void window_sums(const uint64_t (&st)[R], int ring, int n_win, const float2 *t, const double2 *t4,
+                                   const uint8_t *wl, double (&a)[R], double (&b)[R]) {
+#pragma unroll
+    for (int i = 0; i < R; ++i) a[i] = b[i] = 0.0;
+    int q = 0;
+    if (ring) {
+        for (; q + kGroupWin <= n_win; q += kGroupWin) {
+#pragma unroll
+            for (int i = 0; i < R; ++i) {
+                const double2 v = t4[ring_from(st[i], q, n_win) & (kGroupPat - 1)];
+                a[i] += v.x;
+                b[i] += v.y;
+            }
+        }
+    }
+    for (; q < n_win; ++q) {
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            const float2 v = t[ring ? (int)(ring_from(st[i], q, n_win) & 255) : window_pattern(st[i], wl + q * kWin)];
+            a[i] += (double)v.x;
+            b[i] += (double)v.y;
+        }
+    }
+}
+
 // alpha_r, beta_r from the pattern table of this coupling; block max of alpha.
 // beta_r also carries the Marshall sign prior pi * (up spins on sublattice A):
 // the network learns the phase relative to the bipartite sign rule, whose
 // state (and not the uniform one, which is the fully polarised multiplet and
 // orthogonal to a singlet) is the natural starting point of training.
-__global__ __launch_bounds__(256) void mlp_state_logpsi(int64_t n, int n_win, const uint8_t *__restrict__ win,
+__global__ __launch_bounds__(256) void mlp_state_logpsi(int64_t n, int n_win, const uint8_t *__restrict__ win, int ring,
                                                         uint64_t sub_a, const uint64_t *__restrict__ reps,
                                                         const float *__restrict__ tab, double *__restrict__ alpha,
                                                         double *__restrict__ beta, double *__restrict__ part) {
-    __shared__ float t[512];
+    __shared__ float2 t[256];
+    __shared__ double2 t4[kGroupPat];
     __shared__ double lds[kWaves];
     __shared__ uint8_t wl[kMaxWin * kWin];
-    for (int i = threadIdx.x; i < 512; i += blockDim.x) t[i] = tab[i];
+    constexpr int R = 4;
+    for (int i = threadIdx.x; i < 256; i += blockDim.x) t[i] = reinterpret_cast<const float2 *>(tab)[i];
     stage_windows(wl, win, n_win);
     __syncthreads();
+    if (ring) group_table(t, t4);
+    __syncthreads();
     double mx = -1e300;
-    for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < n; r += (int64_t)gridDim.x * blockDim.x) {
-        const uint64_t s = reps[r];
-        double a = 0.0, b = 0.0;
-        for (int q = 0; q < n_win; ++q) {
-            const int p = window_pattern(s, wl + q * kWin);
-            a += (double)t[2 * p];
-            b += (double)t[2 * p + 1];
+    const int64_t step = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < n; r += R * step) {
+        uint64_t st[R];
+        double a[R], b[R];
+#pragma unroll
+        for (int i = 0; i < R; ++i) st[i] = r + i * step < n ? reps[r + i * step] : 0;
+        window_sums<R>(st, ring, n_win, t, t4, wl, a, b);
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            if (r + i * step >= n) continue;
+            alpha[r + i * step] = a[i];
+            beta[r + i * step] = b[i] + kMarshallPi * (double)__popcll(st[i] & sub_a);
+            mx = fmax(mx, a[i]);
         }
-        alpha[r] = a;
-        beta[r] = b + kMarshallPi * (double)__popcll(s & sub_a);
-        mx = fmax(mx, a);
     }
     for (int off = 32; off > 0; off >>= 1) mx = fmax(mx, __shfl_down(mx, off, 64));
     if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = mx;
@@ -451,213 +572,253 @@ __global__ __launch_bounds__(256) void mlp_finish_sum2(const double *__restrict_
 }
 
 // ---- the per-sample kernels batched over every sample of a training step ----
-// One launch per phase covers all samples: block b works on sample task[b],
-// with the row-to-thread assignment and the per-sample block count of the
-// single-sample kernel above, so every sample's sums are formed in a fixed order.
+// One launch per phase covers all samples: block b works on sample task[b]. A
+// wavefront task takes 64 * kBatchRows rows: kBatchRun * kBatchRows consecutive
+// ones from each of 64 / kBatchRun equal parts of the sample. Consecutive
+// representatives share their high sites, so with 64 consecutive rows a window
+// there has one pattern for all lanes and their histogram additions queue at one
+// bin; rows of one lane that share a pattern are summed before they are added.
+constexpr int kBatchThreads = 512, kBatchRows = 8, kBatchWaves = kBatchThreads / 64;
+constexpr int kBatchRun = 4;  // 192 samples, histogram / amplitude kernel: run 1 175 / 182 us, 2 131 / 120, 4 137 / 110, 8 151 / 112
+
 struct BSample {
-    int64_t n, off;  // rows; offset of the sample's rows in the concatenated alpha/beta
+    int64_t n, off;  // rows; offset of the sample's rows in the concatenated amplitudes
     const uint64_t *reps;
     const uint8_t *stab;
     const double *u;
     const uint8_t *win;
     uint64_t sub_a;
-    int n_win, G, blk0, nblk;  // blocks [blk0, blk0 + nblk) of every batched launch
+    int n_win, ring, G, blk0, nblk;  // blocks [blk0, blk0 + nblk) of every batched launch
 };
 
-__global__ __launch_bounds__(256) void mlp_batch_logpsi(const BSample *__restrict__ S, const int *__restrict__ task,
-                                                        const float *__restrict__ tabs, double *__restrict__ alpha,
-                                                        double *__restrict__ beta, double *__restrict__ part) {
-    __shared__ float t[512];
-    __shared__ double lds[kWaves];
+// wavefront tasks of a sample of n rows, and row i of a lane in task w (n or more: none)
+__host__ __device__ inline int64_t batch_tasks(int64_t n) {
+    return (n + 64 * kBatchRows - 1) / (64 * kBatchRows);
+}
+__device__ inline int64_t batch_row(int64_t n, int64_t w, int i, int lane) {
+    constexpr int span = kBatchRun * kBatchRows;
+    return w < batch_tasks(n) ? (lane / kBatchRun * batch_tasks(n) + w) * span + i * kBatchRun + lane % kBatchRun : n;
+}
+
+// Amplitudes c_r = exp(alpha_r - m) sqrt(G / m_r) (cos, sin)(beta_r), m = the
+// block's largest alpha, into c, and the block's m and sums of u c, |c|^2, u^2:
+// part[q * total + block], q = 0 .. 4. The sums of different blocks are brought
+// to one m when they are added, so the amplitudes need no second pass over the
+// windows. Bound by LDS reads and the 64-bit exp and sincos (192 samples, 9.9
+// million rows: 110 us; as two kernels, one window at a time, 380 us).
+__global__ __launch_bounds__(kBatchThreads) void mlp_batch_overlap(const BSample *__restrict__ S,
+                                                                   const int *__restrict__ task,
+                                                                   const float *__restrict__ tabs,
+                                                                   double2 *__restrict__ c, double *__restrict__ part,
+                                                                   int total) {
+    __shared__ float2 t[256];
+    __shared__ double2 t4[kGroupPat];
+    __shared__ double lds[4][kBatchWaves];
     __shared__ uint8_t wl[kMaxWin * kWin];
     const int si = task[blockIdx.x];
     const BSample s = S[si];
-    const float *tab = tabs + (size_t)si * 512;
-    for (int i = threadIdx.x; i < 512; i += blockDim.x) t[i] = tab[i];
-    stage_windows(wl, s.win, s.n_win);
+    for (int i = threadIdx.x; i < 256; i += blockDim.x)
+        t[i] = reinterpret_cast<const float2 *>(tabs)[(size_t)si * 256 + i];
+    if (!s.ring) stage_windows(wl, s.win, s.n_win);
     __syncthreads();
-    const int lb = blockIdx.x - s.blk0;
+    if (s.ring) group_table(t, t4);
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int64_t task_w = (int64_t)(blockIdx.x - s.blk0) * kBatchWaves + wv;
+    uint64_t st[kBatchRows];
+    double a[kBatchRows], b[kBatchRows];
+    bool act[kBatchRows];
+#pragma unroll
+    for (int i = 0; i < kBatchRows; ++i) {
+        const int64_t r = batch_row(s.n, task_w, i, lane);
+        act[i] = r < s.n;
+        st[i] = act[i] ? s.reps[r] : 0;
+    }
+    __syncthreads();
+    window_sums<kBatchRows>(st, s.ring, s.n_win, t, t4, wl, a, b);
     double mx = -1e300;
-    for (int64_t r = (int64_t)lb * blockDim.x + threadIdx.x; r < s.n; r += (int64_t)s.nblk * blockDim.x) {
-        const uint64_t st = s.reps[r];
-        double a = 0.0, b = 0.0;
-        for (int q = 0; q < s.n_win; ++q) {
-            const int p = window_pattern(st, wl + q * kWin);
-            a += (double)t[2 * p];
-            b += (double)t[2 * p + 1];
-        }
-        alpha[s.off + r] = a;
-        beta[s.off + r] = b + kMarshallPi * (double)__popcll(st & s.sub_a);
-        mx = fmax(mx, a);
-    }
-    for (int off = 32; off > 0; off >>= 1) mx = fmax(mx, __shfl_down(mx, off, 64));
-    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = mx;
+#pragma unroll
+    for (int i = 0; i < kBatchRows; ++i)
+        if (act[i]) mx = fmax(mx, a[i]);
+    for (int off = 32; off > 0; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off, 64));
+    if (lane == 0) lds[0][wv] = mx;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double m = lds[0];
-        for (int i = 1; i < kWaves; ++i) m = fmax(m, lds[i]);
-        part[blockIdx.x] = m;
-    }
-}
-
-// One block per sample: stats[8 si + 5] = max of the sample's block maxima.
-__global__ __launch_bounds__(256) void mlp_batch_finish_max(const BSample *__restrict__ S,
-                                                            const double *__restrict__ part,
-                                                            double *__restrict__ stats) {
-    __shared__ double lds[kWaves];
-    const BSample s = S[blockIdx.x];
-    double mx = -1e300;
-    for (int i = threadIdx.x; i < s.nblk; i += blockDim.x) mx = fmax(mx, part[s.blk0 + i]);
-    for (int off = 32; off > 0; off >>= 1) mx = fmax(mx, __shfl_down(mx, off, 64));
-    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = mx;
+    for (int w = 0; w < kBatchWaves; ++w) mx = fmax(mx, lds[0][w]);
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double m = lds[0];
-        for (int i = 1; i < kWaves; ++i) m = fmax(m, lds[i]);
-        stats[(size_t)blockIdx.x * 8 + 5] = m;
-    }
-}
-
-// Partials of Re/Im <u, c>, <c, c>, <u, u>: part[q * total + block].
-__global__ __launch_bounds__(256) void mlp_batch_overlap(const BSample *__restrict__ S, const int *__restrict__ task,
-                                                         const double *__restrict__ alpha,
-                                                         const double *__restrict__ beta,
-                                                         const double *__restrict__ stats, double *__restrict__ part,
-                                                         int total) {
-    __shared__ double lds[kWaves];
-    const int si = task[blockIdx.x];
-    const BSample s = S[si];
-    const double am = stats[(size_t)si * 8 + 5];
-    const int lb = blockIdx.x - s.blk0;
-    double o_re = 0, o_im = 0, nc = 0, nu = 0;
-    for (int64_t r = (int64_t)lb * blockDim.x + threadIdx.x; r < s.n; r += (int64_t)s.nblk * blockDim.x) {
-        const double mag = exp(alpha[s.off + r] - am) * sqrt((double)s.G / (double)s.stab[r]);
-        const double br = beta[s.off + r];
-        const double cr = mag * cos(br), ci = mag * sin(br);
+    double v[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int i = 0; i < kBatchRows; ++i) {
+        if (!act[i]) continue;
+        const int64_t r = batch_row(s.n, task_w, i, lane);
+        const double mag = exp(a[i] - mx) * sqrt((double)s.G / (double)s.stab[r]);
+        double sn, cs;
+        sincos(b[i] + kMarshallPi * (double)__popcll(st[i] & s.sub_a), &sn, &cs);
+        const double cr = mag * cs, ci = mag * sn;
         const double ur = s.u[r];
-        o_re += ur * cr;
-        o_im += ur * ci;
-        nc += mag * mag;
-        nu += ur * ur;
+        c[s.off + r] = make_double2(cr, ci);
+        v[0] += ur * cr;
+        v[1] += ur * ci;
+        v[2] += mag * mag;
+        v[3] += ur * ur;
     }
-    const double v[4] = {o_re, o_im, nc, nu};
+#pragma unroll
     for (int q = 0; q < 4; ++q) {
-        const double t = block_sum(v[q], lds);
-        if (threadIdx.x == 0) part[(size_t)q * total + blockIdx.x] = t;
+        v[q] = wave_sum(v[q]);
+        if (lane == 0) lds[q][wv] = v[q];
     }
+    __syncthreads();
+    if (threadIdx.x < 4) {
+        double tot = 0.0;
+        for (int w = 0; w < kBatchWaves; ++w) tot += lds[threadIdx.x][w];
+        part[(size_t)threadIdx.x * total + blockIdx.x] = tot;
+    }
+    if (threadIdx.x == 0) part[(size_t)4 * total + blockIdx.x] = mx;
 }
 
-// One block per sample: stats[8 si + 0..3] = Re O, Im O, Nc, Nu; stats[8 si + 4] = loss.
+// One block per sample: stats[8 si + 0..3] = Re O, Im O, Nc, Nu relative to the
+// sample's largest alpha, stats[8 si + 4] = loss, stats[8 si + 5] = that alpha;
+// hist (when set): the sample's bins are cleared.
 __global__ __launch_bounds__(256) void mlp_batch_finish_overlap(const BSample *__restrict__ S,
                                                                 const double *__restrict__ part, int total,
-                                                                double *__restrict__ stats) {
+                                                                double *__restrict__ stats,
+                                                                unsigned long long *__restrict__ hist) {
     __shared__ double lds[kWaves];
+    __shared__ double s_mx;
     const BSample s = S[blockIdx.x];
-    double v[4];
-    for (int q = 0; q < 4; ++q) v[q] = sum_partials(part + (size_t)q * total + s.blk0, s.nblk, lds);
+    if (hist)
+        for (int i = threadIdx.x; i < 512; i += blockDim.x) hist[(size_t)blockIdx.x * 512 + i] = 0ull;
+    const double *pm = part + (size_t)4 * total + s.blk0;
+    double mx = -1e300;
+    for (int i = threadIdx.x; i < s.nblk; i += blockDim.x) mx = fmax(mx, pm[i]);
+    for (int off = 32; off > 0; off >>= 1) mx = fmax(mx, __shfl_down(mx, off, 64));
+    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = mx;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double m = lds[0];
+        for (int i = 1; i < kWaves; ++i) m = fmax(m, lds[i]);
+        s_mx = m;
+    }
+    __syncthreads();
+    mx = s_mx;
+    double v[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int i = threadIdx.x; i < s.nblk; i += blockDim.x) {
+        const double f = exp(pm[i] - mx);
+        const double *pi = part + s.blk0 + i;
+        v[0] += f * pi[0];
+        v[1] += f * pi[(size_t)total];
+        v[2] += f * f * pi[(size_t)2 * total];
+        v[3] += pi[(size_t)3 * total];
+    }
+    for (int q = 0; q < 4; ++q) v[q] = block_sum(v[q], lds);
     if (threadIdx.x == 0) {
         double *st = stats + (size_t)blockIdx.x * 8;
         for (int q = 0; q < 4; ++q) st[q] = v[q];
         const double o2 = v[0] * v[0] + v[1] * v[1];
         st[4] = 1.0 - o2 / (v[2] * v[3]);
+        st[5] = mx;
     }
-}
-
-__global__ __launch_bounds__(256) void mlp_zero_u64(unsigned long long *__restrict__ p, int64_t n) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        p[i] = 0ull;
 }
 
 // Per-pattern gradient histograms (fixed point) of every sample: each block adds
-// its LDS histogram into its sample's hist[512] (integer sums, any order).
-__global__ __launch_bounds__(256) void mlp_batch_grad(const BSample *__restrict__ S, const int *__restrict__ task,
-                                                      const double *__restrict__ alpha,
-                                                      const double *__restrict__ beta,
-                                                      const double *__restrict__ stats,
-                                                      unsigned long long *__restrict__ hist) {
-    __shared__ unsigned long long h[512];
+// its LDS histogram into its sample's hist[512] (integer sums, any order). Bound
+// by the LDS additions and the reads of c (192 samples, 9.9 million rows: 137 us;
+// 859 us with an addition per window, consecutive rows in a wavefront and the
+// amplitudes formed again).
+__global__ __launch_bounds__(kBatchThreads) void mlp_batch_grad(const BSample *__restrict__ S,
+                                                                const int *__restrict__ task,
+                                                                const double2 *__restrict__ c,
+                                                                const double *__restrict__ part, int total,
+                                                                const double *__restrict__ stats,
+                                                                unsigned long long *__restrict__ hist) {
+    __shared__ unsigned long long ha[256], hb[256], ha4[kGroupPat], hb4[kGroupPat];
     __shared__ uint8_t wl[kMaxWin * kWin];
     const int si = task[blockIdx.x];
     const BSample s = S[si];
-    for (int i = threadIdx.x; i < 512; i += blockDim.x) h[i] = 0ull;
-    stage_windows(wl, s.win, s.n_win);
-    __syncthreads();
-    const double *st = stats + (size_t)si * 8;
-    const double am = st[5];
-    const double ore = st[0], oim = st[1], nc = st[2], nu = st[3];
+    for (int i = threadIdx.x; i < 256; i += blockDim.x) ha[i] = hb[i] = 0ull;
+    if (s.ring)
+        for (int i = threadIdx.x; i < kGroupPat; i += blockDim.x) ha4[i] = hb4[i] = 0ull;
+    else
+        stage_windows(wl, s.win, s.n_win);
+    const double *sv = stats + (size_t)si * 8;
+    const double f = exp(part[(size_t)4 * total + blockIdx.x] - sv[5]);
+    const double ore = sv[0], oim = sv[1], nc = sv[2], nu = sv[3];
     const double o2 = ore * ore + oim * oim;
-    const int lb = blockIdx.x - s.blk0;
-    const int lane = threadIdx.x & 63;
-    // wave-uniform loop (lane l of a wave handles row r0 + l, the same rows as a
-    // thread-strided loop): consecutive representatives share their high sites, so
-    // a window there often has one pattern across the wave; its 64 additions are
-    // then summed in registers and added once instead of contending for one bin
-    for (int64_t r0 = (int64_t)lb * blockDim.x + (threadIdx.x & ~63); r0 < s.n; r0 += (int64_t)s.nblk * blockDim.x) {
-        const int64_t r = r0 + lane;
-        const bool act = r < s.n;
-        long long qa = 0, qb = 0;
-        uint64_t stt = 0;
-        if (act) {
-            const double mag = exp(alpha[s.off + r] - am) * sqrt((double)s.G / (double)s.stab[r]);
-            const double br = beta[s.off + r];
-            const double cr = mag * cos(br), ci = mag * sin(br);
-            const double wr = s.u[r] * (ore * cr + oim * ci);
-            const double wi = s.u[r] * (ore * ci - oim * cr);
-            const double ga = -(2.0 * wr * nc - o2 * 2.0 * mag * mag) / (nc * nc * nu);
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int64_t task_w = (int64_t)(blockIdx.x - s.blk0) * kBatchWaves + wv;
+    uint64_t st[kBatchRows];
+    unsigned long long qa[kBatchRows], qb[kBatchRows];
+    bool act[kBatchRows];
+#pragma unroll
+    for (int i = 0; i < kBatchRows; ++i) {
+        const int64_t r = batch_row(s.n, task_w, i, lane);
+        act[i] = r < s.n;
+        st[i] = 0;
+        qa[i] = qb[i] = 0;
+        if (act[i]) {
+            double2 cv = c[s.off + r];
+            cv.x *= f;
+            cv.y *= f;
+            const double ur = s.u[r];
+            const double wr = ur * (ore * cv.x + oim * cv.y);
+            const double wi = ur * (ore * cv.y - oim * cv.x);
+            const double ga = -(2.0 * wr * nc - o2 * 2.0 * (cv.x * cv.x + cv.y * cv.y)) / (nc * nc * nu);
             const double gb = -(-2.0 * wi) / (nc * nu);
-            qa = (long long)llrint(ga * kFix);
-            qb = (long long)llrint(gb * kFix);
-            stt = s.reps[r];
-        }
-        const uint64_t st0 = __shfl(stt, 0, 64);  // lane 0's row exists (r0 < n)
-        if (!act) stt = st0;                     // rows past the end add 0 to lane 0's bins
-        for (int q = 0; q < s.n_win; ++q) {
-            const int p = window_pattern(stt, wl + q * kWin);
-            const int p0 = __shfl(p, 0, 64);
-            if (__all(p == p0)) {
-                long long sa = qa, sb = qb;
-                for (int off = 32; off > 0; off >>= 1) {
-                    sa += __shfl_xor(sa, off, 64);
-                    sb += __shfl_xor(sb, off, 64);
-                }
-                if (lane == 0) {
-                    atomicAdd(&h[2 * p0], (unsigned long long)sa);
-                    atomicAdd(&h[2 * p0 + 1], (unsigned long long)sb);
-                }
-            } else {
-                atomicAdd(&h[2 * p], (unsigned long long)qa);
-                atomicAdd(&h[2 * p + 1], (unsigned long long)qb);
-            }
+            qa[i] = (unsigned long long)(long long)llrint(ga * kFix);
+            qb[i] = (unsigned long long)(long long)llrint(gb * kFix);
+            st[i] = s.reps[r];
         }
     }
     __syncthreads();
+    // one window (group) of the lane's rows: sums over equal patterns, then adds
+    auto add = [&](unsigned long long *da, unsigned long long *db, auto pattern) {
+        int cur = pattern(0);
+        unsigned long long va = qa[0], vb = qb[0];
+#pragma unroll
+        for (int i = 1; i < kBatchRows; ++i) {
+            const int p = pattern(i);
+            if (p != cur) {
+                atomicAdd(&da[cur], va);
+                atomicAdd(&db[cur], vb);
+                cur = p;
+                va = vb = 0;
+            }
+            va += qa[i];
+            vb += qb[i];
+        }
+        atomicAdd(&da[cur], va);
+        atomicAdd(&db[cur], vb);
+    };
+    int q = 0;
+    if (s.ring)
+        for (; q + kGroupWin <= s.n_win; q += kGroupWin)
+            add(ha4, hb4, [&](int i) { return (int)(ring_from(st[i], q, s.n_win) & (kGroupPat - 1)); });
+    for (; q < s.n_win; ++q)
+        add(ha, hb, [&](int i) {
+            return s.ring ? (int)(ring_from(st[i], q, s.n_win) & 255) : window_pattern(st[i], wl + q * kWin);
+        });
+    __syncthreads();
+    if (s.ring) {
+        for (int p = threadIdx.x; p < kGroupPat; p += blockDim.x) {
+            const unsigned long long va = ha4[p], vb = hb4[p];
+            if (!va && !vb) continue;
+#pragma unroll
+            for (int i = 0; i < kGroupWin; ++i) {
+                atomicAdd(&ha[(p >> i) & 255], va);
+                atomicAdd(&hb[(p >> i) & 255], vb);
+            }
+        }
+        __syncthreads();
+    }
     unsigned long long *hs = hist + (size_t)si * 512;
-    for (int i = threadIdx.x; i < 512; i += blockDim.x)
-        if (h[i]) atomicAdd(&hs[i], h[i]);
-}
-
-// dout rows of every sample (512 per sample) from its histogram; loss = mean of
-// the samples' losses summed in sample order.
-__global__ __launch_bounds__(256) void mlp_batch_finish(const unsigned long long *__restrict__ hist, int ns,
-                                                        float *__restrict__ dout, float scale,
-                                                        const double *__restrict__ stats, double *__restrict__ loss) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < (int64_t)ns * 512;
-         i += (int64_t)gridDim.x * blockDim.x)
-        dout[i] = (float)((double)(long long)hist[i] / kFix * scale);
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        double mean = 0.0;
-        for (int k = 0; k < ns; ++k) mean += stats[(size_t)k * 8 + 4];
-        *loss = mean / ns;
+    for (int i = threadIdx.x; i < 256; i += blockDim.x) {
+        if (ha[i]) atomicAdd(&hs[2 * i], ha[i]);
+        if (hb[i]) atomicAdd(&hs[2 * i + 1], hb[i]);
     }
 }
 
 // Loss only: the mean of the samples' losses.
-__global__ __launch_bounds__(64) void mlp_batch_loss(const double *__restrict__ stats, int ns,
-                                                     double *__restrict__ loss) {
-    if (threadIdx.x != 0) return;
-    double mean = 0.0;
-    for (int k = 0; k < ns; ++k) mean += stats[(size_t)k * 8 + 4];
-    *loss = mean / ns;
+__global__ __launch_bounds__(256) void mlp_batch_loss(const double *__restrict__ stats, int ns,
+                                                      double *__restrict__ loss) {
+    mean_loss(stats, ns, loss);
 }
 
 }  // namespace qmb
@@ -669,9 +830,19 @@ using namespace qmb;
 struct MlpGeom {
     Ref<const qmb_basis> basis;
     int n_win = 0;
-    DevBuf win;  // uint8 [n_win * 8]
+    int ring = 0;  // the windows q .. q + 7 (mod n_win) of an n_win-site ring, n_win >= kGroupWin + 7
+    DevBuf win;    // uint8 [n_win * 8]
     uint64_t sub_a = 0;
 };
+
+// Whether the windows are a whole ring's in order (MlpGeom::ring).
+static int is_ring(const uint8_t *sites, int n_win, int n_sites) {
+    if (n_win != n_sites || n_win < kWin + kGroupWin - 1) return 0;
+    for (int q = 0; q < n_win; ++q)
+        for (int k = 0; k < kWin; ++k)
+            if (sites[q * kWin + k] != (q + k) % n_win) return 0;
+    return 1;
+}
 
 struct MlpSample {
     Ref<const qmb_basis> basis;
@@ -686,7 +857,7 @@ struct MlpBatch {
     bool valid = false;
     int ns = 0, total_blocks = 0;
     int64_t total_rows = 0;
-    DevBuf samples, task, alpha, beta, part, stats, hist, loss;
+    DevBuf samples, task, amp, part, stats, hist, loss;
 };
 
 struct qmb_mlp : Counted {
@@ -698,7 +869,7 @@ struct qmb_mlp : Counted {
     MlpBatch batch;
     // row buffers (sized for the current row count)
     int rows_cap = 0;
-    DevBuf coup, out, H1, H1q, H2, dout, dA2, dA2q, dA1, part, part2;
+    DevBuf coup, out, H1, H1q, H2, part;
     void ensure_rows(int rows);
 };
 
@@ -710,14 +881,7 @@ void qmb_mlp::ensure_rows(int rows) {
     H1.alloc((size_t)cap * kH * sizeof(float));
     H1q.alloc((size_t)cap * kH * sizeof(uint16_t));
     H2.alloc((size_t)cap * kH * sizeof(float));
-    dout.alloc((size_t)cap * 2 * sizeof(float));
-    dA2.alloc((size_t)cap * kH * sizeof(float));
-    dA2q.alloc((size_t)cap * kH * sizeof(uint16_t));
-    dA1.alloc((size_t)cap * kH * sizeof(float));
-    const int groups = (cap + kRowsPerGroup - 1) / kRowsPerGroup;
-    const int groups_s = (cap + kRowsPerSmallGroup - 1) / kRowsPerSmallGroup;
-    part.alloc((size_t)groups_s * kParams * sizeof(float));
-    part2.alloc((size_t)groups * kH * kH * sizeof(float));
+    part.alloc((size_t)(cap / 256) * kParams * sizeof(float));
     rows_cap = cap;
 }
 
@@ -748,6 +912,7 @@ int geom_for(qmb_mlp *m, const qmb_basis *b) {
     MlpGeom gm;
     gm.basis = b;
     gm.n_win = N;
+    gm.ring = is_ring(w.data(), N, N);
     gm.win.alloc(w.size());
     QMB_HIP(hipMemcpy(gm.win.p, w.data(), w.size(), hipMemcpyHostToDevice));
     for (int q = 0; q < N; q += 2) gm.sub_a |= 1ULL << q;
@@ -761,8 +926,8 @@ void forward_rows(qmb_mlp *m, const std::vector<double> &coup, bool store) {
     const int rows = (int)(coup.size() / 2) * 256;
     m->ensure_rows(rows);
     QMB_HIP(hipMemcpyAsync(m->coup.p, coup.data(), coup.size() * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-    hipLaunchKernelGGL(mlp_forward, dim3((rows + 31) / 32), dim3(64), 0, ctx->stream, m->theta.as<float>(),
-                       m->w2bf.as<uint16_t>(), m->coup.as<double>(), rows, m->out.as<float>(), m->H1.as<float>(),
+    hipLaunchKernelGGL(mlp_forward, dim3(rows / 32), dim3(kFwdThreads), 0, ctx->stream, m->theta.as<float>(),
+                       m->w2bf.as<uint16_t>(), m->coup.as<double>(), m->out.as<float>(), m->H1.as<float>(),
                        m->H1q.as<uint16_t>(), m->H2.as<float>(), store ? 1 : 0);
     QMB_HIP(hipGetLastError());
 }
@@ -787,7 +952,7 @@ struct StateWork {
 void state_logpsi(qmb_ctx *ctx, const qmb_basis *b, const MlpGeom &gm, const float *tab, StateWork &w) {
     w.ensure(b->n_rows);
     hipLaunchKernelGGL(mlp_state_logpsi, dim3(w.nb), dim3(256), 0, ctx->stream, b->n_rows, gm.n_win,
-                       gm.win.as<uint8_t>(), gm.sub_a, b->reps.as<uint64_t>(), tab, w.alpha.as<double>(),
+                       gm.win.as<uint8_t>(), gm.ring, gm.sub_a, b->reps.as<uint64_t>(), tab, w.alpha.as<double>(),
                        w.beta.as<double>(), w.part.as<double>());
     QMB_HIP(hipGetLastError());
     hipLaunchKernelGGL(mlp_finish_max, dim3(1), dim3(256), 0, ctx->stream, w.part.as<double>(), w.nb,
@@ -795,8 +960,7 @@ void state_logpsi(qmb_ctx *ctx, const qmb_basis *b, const MlpGeom &gm, const flo
     QMB_HIP(hipGetLastError());
 }
 
-// Sample table and work arrays of the batched kernels: each sample keeps the
-// block count of the single-sample kernels (min(1024, ceil(n/256))).
+// Sample table and work arrays of the batched kernels.
 void ensure_batch(qmb_mlp *m) {
     MlpBatch &B = m->batch;
     if (B.valid) return;
@@ -817,9 +981,10 @@ void ensure_batch(qmb_mlp *m) {
         d.win = gm.win.as<uint8_t>();
         d.sub_a = gm.sub_a;
         d.n_win = gm.n_win;
+        d.ring = gm.ring;
         d.G = b->group->G;
         d.blk0 = (int)task.size();
-        d.nblk = (int)std::min<int64_t>(1024, (b->n_rows + 255) / 256);
+        d.nblk = (int)((batch_tasks(b->n_rows) + kBatchWaves - 1) / kBatchWaves);
         for (int k = 0; k < d.nblk; ++k) task.push_back(i);
         off += b->n_rows;
     }
@@ -828,9 +993,8 @@ void ensure_batch(qmb_mlp *m) {
     B.total_rows = off;
     B.samples.alloc((size_t)ns * sizeof(BSample));
     B.task.alloc(task.size() * sizeof(int));
-    B.alpha.alloc((size_t)off * sizeof(double));
-    B.beta.alloc((size_t)off * sizeof(double));
-    B.part.alloc((size_t)B.total_blocks * 4 * sizeof(double));
+    B.amp.alloc((size_t)off * sizeof(double2));
+    B.part.alloc((size_t)B.total_blocks * 5 * sizeof(double));
     B.stats.alloc((size_t)ns * 8 * sizeof(double));
     B.hist.alloc((size_t)ns * 512 * sizeof(unsigned long long));
     B.loss.alloc(sizeof(double));
@@ -839,8 +1003,8 @@ void ensure_batch(qmb_mlp *m) {
     B.valid = true;
 }
 
-// Loss (and the dout rows of every sample when want_grad) of all samples, one
-// launch per phase; the mean loss is left in batch.loss.
+// Loss statistics (and the pattern histograms when want_grad) of all samples,
+// one launch per phase.
 void batch_loss(qmb_mlp *m, bool want_grad) {
     qmb_ctx *ctx = m->ctx;
     ensure_batch(m);
@@ -848,34 +1012,21 @@ void batch_loss(qmb_mlp *m, bool want_grad) {
     const BSample *S = B.samples.as<BSample>();
     const int *task = B.task.as<int>();
     const unsigned nb = (unsigned)B.total_blocks, ns = (unsigned)B.ns;
-    hipLaunchKernelGGL(mlp_batch_logpsi, dim3(nb), dim3(256), 0, ctx->stream, S, task, m->out.as<float>(),
-                       B.alpha.as<double>(), B.beta.as<double>(), B.part.as<double>());
-    QMB_HIP(hipGetLastError());
-    hipLaunchKernelGGL(mlp_batch_finish_max, dim3(ns), dim3(256), 0, ctx->stream, S, B.part.as<double>(),
-                       B.stats.as<double>());
-    QMB_HIP(hipGetLastError());
-    hipLaunchKernelGGL(mlp_batch_overlap, dim3(nb), dim3(256), 0, ctx->stream, S, task, B.alpha.as<double>(),
-                       B.beta.as<double>(), B.stats.as<double>(), B.part.as<double>(), B.total_blocks);
+    hipLaunchKernelGGL(mlp_batch_overlap, dim3(nb), dim3(kBatchThreads), 0, ctx->stream, S, task, m->out.as<float>(),
+                       B.amp.as<double2>(), B.part.as<double>(), B.total_blocks);
     QMB_HIP(hipGetLastError());
     hipLaunchKernelGGL(mlp_batch_finish_overlap, dim3(ns), dim3(256), 0, ctx->stream, S, B.part.as<double>(),
-                       B.total_blocks, B.stats.as<double>());
+                       B.total_blocks, B.stats.as<double>(),
+                       want_grad ? B.hist.as<unsigned long long>() : nullptr);
     QMB_HIP(hipGetLastError());
     if (!want_grad) {
-        hipLaunchKernelGGL(mlp_batch_loss, dim3(1), dim3(64), 0, ctx->stream, B.stats.as<double>(), B.ns,
+        hipLaunchKernelGGL(mlp_batch_loss, dim3(1), dim3(256), 0, ctx->stream, B.stats.as<double>(), B.ns,
                            B.loss.as<double>());
         QMB_HIP(hipGetLastError());
         return;
     }
-    const int64_t nh = (int64_t)B.ns * 512;
-    hipLaunchKernelGGL(mlp_zero_u64, dim3((unsigned)std::min<int64_t>(1024, (nh + 255) / 256)), dim3(256), 0,
-                       ctx->stream, B.hist.as<unsigned long long>(), nh);
-    QMB_HIP(hipGetLastError());
-    hipLaunchKernelGGL(mlp_batch_grad, dim3(nb), dim3(256), 0, ctx->stream, S, task, B.alpha.as<double>(),
-                       B.beta.as<double>(), B.stats.as<double>(), B.hist.as<unsigned long long>());
-    QMB_HIP(hipGetLastError());
-    hipLaunchKernelGGL(mlp_batch_finish, dim3((unsigned)std::min<int64_t>(1024, (nh + 255) / 256)), dim3(256), 0,
-                       ctx->stream, B.hist.as<unsigned long long>(), B.ns, m->dout.as<float>(), 1.0f / B.ns,
-                       B.stats.as<double>(), B.loss.as<double>());
+    hipLaunchKernelGGL(mlp_batch_grad, dim3(nb), dim3(kBatchThreads), 0, ctx->stream, S, task, B.amp.as<double2>(),
+                       B.part.as<double>(), B.total_blocks, B.stats.as<double>(), B.hist.as<unsigned long long>());
     QMB_HIP(hipGetLastError());
 }
 
@@ -923,24 +1074,16 @@ double loss_and_grad(qmb_mlp *m, bool want_grad) {
         coup[2 * i + 1] = m->samples[i].j2;
     }
     forward_rows(m, coup, want_grad);
-    const int rows = ns * 256;
     batch_loss(m, want_grad);
     if (want_grad) {
-        hipLaunchKernelGGL(mlp_backward_act, dim3((rows + 31) / 32), dim3(64), 0, ctx->stream, m->theta.as<float>(),
-                           m->w2t.as<uint16_t>(), rows, m->dout.as<float>(), m->H1.as<float>(), m->H2.as<float>(),
-                           m->dA2.as<float>(), m->dA2q.as<uint16_t>(), m->dA1.as<float>());
-        QMB_HIP(hipGetLastError());
-        const int groups = (rows + kRowsPerGroup - 1) / kRowsPerGroup;
-        hipLaunchKernelGGL(mlp_wgrad2, dim3(groups, 16), dim3(64), 0, ctx->stream, rows, m->dA2q.as<uint16_t>(),
-                           m->H1q.as<uint16_t>(), m->part2.as<float>());
-        QMB_HIP(hipGetLastError());
-        const int groups_s = (rows + kRowsPerSmallGroup - 1) / kRowsPerSmallGroup;
-        hipLaunchKernelGGL(mlp_wgrad_small, dim3(groups_s), dim3(kH), 0, ctx->stream, m->coup.as<double>(), rows,
-                           m->dout.as<float>(), m->H2.as<float>(), m->dA2.as<float>(), m->dA1.as<float>(),
+        hipLaunchKernelGGL(mlp_backward, dim3(ns), dim3(kBackThreads), 0, ctx->stream, m->theta.as<float>(),
+                           m->w2t.as<uint16_t>(), m->coup.as<double>(), m->batch.hist.as<unsigned long long>(),
+                           1.0f / ns, m->H1.as<float>(), m->H1q.as<uint16_t>(), m->H2.as<float>(),
                            m->part.as<float>());
         QMB_HIP(hipGetLastError());
-        hipLaunchKernelGGL(mlp_reduce_grad, dim3((kParams + 255) / 256), dim3(256), 0, ctx->stream, groups_s, groups,
-                           m->part.as<float>(), m->part2.as<float>(), 1.0f, m->grad.as<float>());
+        hipLaunchKernelGGL(mlp_reduce_grad, dim3((kParams + kReduceParams - 1) / kReduceParams + 1), dim3(256), 0,
+                           ctx->stream, ns, m->part.as<float>(), m->grad.as<float>(), m->batch.stats.as<double>(), ns,
+                           m->batch.loss.as<double>());
         QMB_HIP(hipGetLastError());
     }
     double *hl = ctx->host_stage<double>(sizeof(double));
@@ -1071,6 +1214,7 @@ qmb_status qmb_mlp_set_windows(qmb_mlp *m, const qmb_basis *b, int n_win, const 
         MlpGeom gm;
         gm.basis = b;
         gm.n_win = n_win;
+        gm.ring = is_ring(sites, n_win, b->n_sites);
         gm.win.alloc((size_t)n_win * kWin);
         QMB_HIP(hipMemcpy(gm.win.p, sites, (size_t)n_win * kWin, hipMemcpyHostToDevice));
         gm.sub_a = sublattice_a;
