@@ -11,10 +11,10 @@
 //      the gathers), phi_n = w/b written out, the block partials of a[n] in
 //      the same pass;
 //   K2 lz_update: w = (-a) phi_n + (y - b phi_{n-1}) and the partials of ||w||^2.
-// In the plain recurrence every block of K2 sums K1's partials into a[n] and
-// every block of the next K1 sums K2's into b[n+1] (same fixed order as a
-// separate one-block finish_sum, which runs only before a convergence check and
-// with reorthogonalisation). The host reads a[], b[] every check_every steps and solves the
+// Every block of K2 sums K1's partials into a[n]; in the plain recurrence every
+// block of the next K1 sums K2's into b[n+1] (same fixed order as a separate
+// one-block finish_sum, which runs only before a convergence check and with
+// reorthogonalisation). The host reads a[], b[] every check_every steps and solves the
 // tridiagonal problem in FP64 (lanczos_host.cpp). Reductions are deterministic:
 // fixed block partial slots summed in a fixed order.
 #include <algorithm>
@@ -204,22 +204,25 @@ __device__ inline bool gated_off(const double *gate) { return gate && *gate == 0
 // Fixed-order sum of the block partials of the previous kernel (one block):
 // mode 0 -> out = s; mode 1 -> out = sqrt(s), out_inv = 1/sqrt(s) (0 if s = 0),
 // skipped when the gate is 0; mode 2 (after a first Gram-Schmidt pass) -> as
-// mode 1, and *gate = 1 if sqrt(s) < kDgks * (the previous *out), else 0.
+// mode 1, and *gate = 1 if sqrt(s) < kDgks * (the norm before), else 0; that norm
+// is sqrt of the sum of the n_old partials at old, or the previous *out (old NULL).
 // A separate launch instead of a "last block" finish: on this chip a
 // device-scope fence in every block writes back and invalidates the L2 and
 // costs more than the SpMV's own traffic.
 __global__ __launch_bounds__(kThreads) void finish_sum(const double *__restrict__ partials, int n,
                                                        double *__restrict__ out, double *__restrict__ out_inv,
-                                                       int mode, double *__restrict__ gate) {
+                                                       int mode, double *__restrict__ gate,
+                                                       const double *__restrict__ old, int n_old) {
     __shared__ double lds[kWaves];
     if (mode == 1 && gated_off(gate)) return;
     const double s = sum_partials(partials, n, lds);
+    const double s_old = old ? sum_partials(old, n_old, lds) : 0.0;
     if (threadIdx.x == 0) {
         if (mode == 0) {
             *out = s;
         } else {
             const double nb = sqrt(s);
-            if (mode == 2) *gate = nb < kDgks * *out ? 1.0 : 0.0;
+            if (mode == 2) *gate = nb < kDgks * (old ? sqrt(s_old) : *out) ? 1.0 : 0.0;
             if (out) *out = nb;
             if (out_inv) *out_inv = nb > 0.0 ? 1.0 / nb : 0.0;
         }
@@ -315,7 +318,9 @@ __global__ __launch_bounds__(kThreads) void vec_axpy(int64_t cnt, double c, cons
 // dots: coef[j] = <V_j, w> for j < nv; grid (blocks, ceil(nv / kDotGroup)). A
 // block takes kDotGroup vectors at once, so w is read once per group instead of
 // once per vector; every dot keeps its own accumulator in the same index order,
-// so the partials are those of one vector per block.
+// so the partials are those of one vector per block. One combined reduction at
+// the end (208,012 complex rows, 1 to 95 vectors: 34 us on average; 38 us with
+// two block sums per vector; two or eight vectors a block 31 and 36 us).
 constexpr int kDotGroup = 4;
 
 template <bool CPLX>
@@ -323,10 +328,13 @@ __global__ __launch_bounds__(kThreads) void reorth_dots(int64_t n, int64_t strid
                                                         const double *__restrict__ V,
                                                         const double *__restrict__ w, double *__restrict__ part,
                                                         int nb, const double *__restrict__ gate) {
-    __shared__ double lds[kWaves];
+    __shared__ double lds[kWaves][2 * kDotGroup];
     if (gated_off(gate)) return;
     const int j0 = blockIdx.y * kDotGroup;
     const int nj = min(kDotGroup, nv - j0);
+    const double *vj[kDotGroup];  // past the last vector: the last one again, not used
+#pragma unroll
+    for (int q = 0; q < kDotGroup; ++q) vj[q] = V + (size_t)(j0 + min(q, nj - 1)) * stride;
     double sr[kDotGroup], si[kDotGroup];
 #pragma unroll
     for (int q = 0; q < kDotGroup; ++q) {
@@ -335,33 +343,40 @@ __global__ __launch_bounds__(kThreads) void reorth_dots(int64_t n, int64_t strid
     }
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
         if (CPLX) {
-            const double wr = w[2 * i], wi = w[2 * i + 1];
+            const double2 x = reinterpret_cast<const double2 *>(w)[i];
+            double2 v[kDotGroup];
+#pragma unroll
+            for (int q = 0; q < kDotGroup; ++q) v[q] = reinterpret_cast<const double2 *>(vj[q])[i];
 #pragma unroll
             for (int q = 0; q < kDotGroup; ++q) {
-                if (q < nj) {
-                    const double *vj = V + (size_t)(j0 + q) * stride;
-                    const double vr = vj[2 * i], vi = vj[2 * i + 1];
-                    sr[q] += vr * wr + vi * wi;
-                    si[q] += vr * wi - vi * wr;
-                }
+                sr[q] += v[q].x * x.x + v[q].y * x.y;
+                si[q] += v[q].x * x.y - v[q].y * x.x;
             }
         } else {
-            const double wr = w[i];
+            const double x = w[i];
+            double v[kDotGroup];
 #pragma unroll
-            for (int q = 0; q < kDotGroup; ++q)
-                if (q < nj) sr[q] += V[(size_t)(j0 + q) * stride + i] * wr;
+            for (int q = 0; q < kDotGroup; ++q) v[q] = vj[q][i];
+#pragma unroll
+            for (int q = 0; q < kDotGroup; ++q) sr[q] += v[q] * x;
         }
     }
+    // every sum over the wavefront, then one combination of the wavefronts in order
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
 #pragma unroll
     for (int q = 0; q < kDotGroup; ++q) {
-        if (q < nj) {  // nj is uniform over the block: every thread takes part in each sum
-            const double tr = block_sum(sr[q], lds);
-            const double ti = CPLX ? block_sum(si[q], lds) : 0.0;
-            if (threadIdx.x == 0) {
-                part[((size_t)(j0 + q) * nb + blockIdx.x) * 2] = tr;
-                part[((size_t)(j0 + q) * nb + blockIdx.x) * 2 + 1] = ti;
-            }
+        const double tr = wave_sum(sr[q]);
+        const double ti = CPLX ? wave_sum(si[q]) : 0.0;
+        if (lane == 0) {
+            lds[wv][2 * q] = tr;
+            lds[wv][2 * q + 1] = ti;
         }
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < 2 * nj) {
+        double t = 0.0;
+        for (int i = 0; i < kWaves; ++i) t += lds[i][threadIdx.x];
+        part[((size_t)(j0 + threadIdx.x / 2) * nb + blockIdx.x) * 2 + threadIdx.x % 2] = t;
     }
 }
 
@@ -383,7 +398,13 @@ __global__ __launch_bounds__(kThreads) void reorth_reduce(const double *__restri
     }
 }
 
-// w -= sum_j coef_j V_j; block partials of ||w||^2.
+// w -= sum_j coef_j V_j; block partials of ||w||^2. Bound by the read of the
+// vectors: eight of them are loaded before they are subtracted (in order), and
+// each thread takes one element where the grid allows (208,012 complex rows,
+// 1 to 95 vectors: 30 us on average, 69 us with four elements per thread and one
+// load in flight).
+constexpr int kApplyGroup = 8;
+
 template <bool CPLX>
 __global__ __launch_bounds__(kThreads) void reorth_apply(int64_t n, int64_t stride, int nv,
                                                          const double *__restrict__ V,
@@ -396,18 +417,39 @@ __global__ __launch_bounds__(kThreads) void reorth_apply(int64_t n, int64_t stri
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
         if (CPLX) {
             double wr = w[2 * i], wi = w[2 * i + 1];
-            for (int j = 0; j < nv; ++j) {
+            int j = 0;
+            for (; j + kApplyGroup <= nv; j += kApplyGroup) {
+                double2 v[kApplyGroup];
+#pragma unroll
+                for (int u = 0; u < kApplyGroup; ++u)
+                    v[u] = reinterpret_cast<const double2 *>(V + (size_t)(j + u) * stride)[i];
+#pragma unroll
+                for (int u = 0; u < kApplyGroup; ++u) {
+                    const double cr = coef[2 * (j + u)], ci = coef[2 * (j + u) + 1];
+                    wr -= cr * v[u].x - ci * v[u].y;
+                    wi -= cr * v[u].y + ci * v[u].x;
+                }
+            }
+            for (; j < nv; ++j) {
                 const double cr = coef[2 * j], ci = coef[2 * j + 1];
-                const double vr = V[(size_t)j * stride + 2 * i], vi = V[(size_t)j * stride + 2 * i + 1];
-                wr -= cr * vr - ci * vi;
-                wi -= cr * vi + ci * vr;
+                const double2 v = reinterpret_cast<const double2 *>(V + (size_t)j * stride)[i];
+                wr -= cr * v.x - ci * v.y;
+                wi -= cr * v.y + ci * v.x;
             }
             w[2 * i] = wr;
             w[2 * i + 1] = wi;
             acc += wr * wr + wi * wi;
         } else {
             double wr = w[i];
-            for (int j = 0; j < nv; ++j) wr -= coef[2 * j] * V[(size_t)j * stride + i];
+            int j = 0;
+            for (; j + kApplyGroup <= nv; j += kApplyGroup) {
+                double v[kApplyGroup];
+#pragma unroll
+                for (int u = 0; u < kApplyGroup; ++u) v[u] = V[(size_t)(j + u) * stride + i];
+#pragma unroll
+                for (int u = 0; u < kApplyGroup; ++u) wr -= coef[2 * (j + u)] * v[u];
+            }
+            for (; j < nv; ++j) wr -= coef[2 * j] * V[(size_t)j * stride + i];
             w[i] = wr;
             acc += wr * wr;
         }
@@ -416,13 +458,21 @@ __global__ __launch_bounds__(kThreads) void reorth_apply(int64_t n, int64_t stri
     if (threadIdx.x == 0) partials[blockIdx.x] = t;
 }
 
-// x = sum_j z_j V_j (eigenvector from a stored basis).
+// x = sum_j z_j V_j (eigenvector from a stored basis), eight loads in flight.
 __global__ __launch_bounds__(kThreads) void basis_combine(int64_t cnt, int64_t stride, int nv,
                                                           const double *__restrict__ V, const double *__restrict__ z,
                                                           double *__restrict__ x) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < cnt; i += (int64_t)gridDim.x * blockDim.x) {
         double s = 0.0;
-        for (int j = 0; j < nv; ++j) s = s + z[j] * V[(size_t)j * stride + i];
+        int j = 0;
+        for (; j + kApplyGroup <= nv; j += kApplyGroup) {
+            double v[kApplyGroup];
+#pragma unroll
+            for (int u = 0; u < kApplyGroup; ++u) v[u] = V[(size_t)(j + u) * stride + i];
+#pragma unroll
+            for (int u = 0; u < kApplyGroup; ++u) s = s + z[j + u] * v[u];
+        }
+        for (; j < nv; ++j) s = s + z[j] * V[(size_t)j * stride + i];
         x[i] = s;
     }
 }
@@ -449,9 +499,9 @@ struct LzWork {
 };
 
 static void launch_finish(qmb_ctx *ctx, const double *partials, unsigned n, double *out, double *out_inv, int mode,
-                          double *gate = nullptr) {
+                          double *gate = nullptr, const double *old = nullptr, unsigned n_old = 0) {
     hipLaunchKernelGGL(finish_sum, dim3(1), dim3(kThreads), 0, ctx->stream, partials, (int)n, out, out_inv, mode,
-                       gate);
+                       gate, old, (int)n_old);
     QMB_HIP(hipGetLastError());
 }
 
@@ -640,21 +690,17 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
     std::vector<char> b_ready(M + 1, 0);
     b_ready[0] = 1;
     auto k1 = [&](int it, hipEvent_t after) {
-        if (fuse) {
-            FusedBeta fb;
-            fb.partials = part1;
-            if (!b_ready[it]) {
-                fb.bpart = part2;
-                fb.n_bpart = (int)ublocks;
-                fb.beta_out = wk.beta() + it;
-                fb.invb_out = wk.invb() + it;
-            }
-            launch_spmv(ctx, e, P.as<double>(), Y.as<double>(), true, wk.invb() + it, vcur(it), &wk,
-                        wk.alpha() + it, after, &fb);
-            return;
+        // a[n] is left to K2, which sums K1's partials, in every scheme
+        FusedBeta fb;
+        fb.partials = part1;
+        if (fuse && !b_ready[it]) {
+            fb.bpart = part2;
+            fb.n_bpart = (int)ublocks;
+            fb.beta_out = wk.beta() + it;
+            fb.invb_out = wk.invb() + it;
         }
         launch_spmv(ctx, e, P.as<double>(), Y.as<double>(), true, wk.invb() + it, vcur(it), &wk, wk.alpha() + it,
-                    after);
+                    after, &fb);
     };
     // Partial reorthogonalisation (H. D. Simon, Math. Comp. 42 (1984) 115-142):
     // om_cur[k] estimates <phi_j, phi_k> through the recurrence the Lanczos
@@ -708,8 +754,9 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
     // w (in P) -= sum_j <V_j, w> V_j over nv vectors of stride cnt, classical
     // Gram-Schmidt; pass 1 only where pass 0 cancelled most of the norm (the flag
     // in misc[3] is set by pass 0's finish on the device); the new norm goes to
-    // b[bslot], 1/b[bslot]
-    auto gram_schmidt = [&](const double *V, int nv, int bslot) {
+    // b[bslot], 1/b[bslot] (before: the partials of the norm it had, or b[bslot] holds that norm)
+    const unsigned ablocks = grid_for(n, kThreads);
+    auto gram_schmidt = [&](const double *V, int nv, int bslot, const double *before = nullptr) {
         double *gate = wk.misc() + 3;
         for (int pass = 0; pass < 2; ++pass) {
             const double *g = pass ? gate : nullptr;
@@ -721,11 +768,11 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
                                (int)rblocks, rcoef.as<double>(), g);
             QMB_HIP(hipGetLastError());
             auto ka = cplx ? reorth_apply<true> : reorth_apply<false>;
-            hipLaunchKernelGGL(ka, dim3(rblocks), dim3(kThreads), 0, ctx->stream, n, (int64_t)cnt, nv, V,
-                               rcoef.as<double>(), P.as<double>(), wk.partials.as<double>(), g);
+            hipLaunchKernelGGL(ka, dim3(ablocks), dim3(kThreads), 0, ctx->stream, n, (int64_t)cnt, nv, V,
+                               rcoef.as<double>(), P.as<double>(), part1, g);
             QMB_HIP(hipGetLastError());
-            launch_finish(ctx, wk.partials.as<double>(), rblocks, wk.beta() + bslot, wk.invb() + bslot, pass ? 1 : 2,
-                          gate);
+            launch_finish(ctx, part1, ablocks, wk.beta() + bslot, wk.invb() + bslot, pass ? 1 : 2, gate,
+                          pass ? nullptr : before, ublocks);
         }
     };
     // Selective orthogonalisation (B. N. Parlett and D. S. Scott, Math. Comp. 33
@@ -742,24 +789,23 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
     bool so_full = false;
     // finish: write b[it+1], 1/b[it+1] now (needed by a convergence check)
     auto k2 = [&](int it, bool finish) {
+        hipLaunchKernelGGL(lz_update, dim3(ublocks), dim3(kThreads), 0, ctx->stream, cnt, Y.as<double>(), vcur(it),
+                           vprev(it), P.as<double>(), wk.alpha() + it, wk.beta() + it, part2, part1, (int)sblocks);
+        QMB_HIP(hipGetLastError());
         if (fuse) {
-            hipLaunchKernelGGL(lz_update, dim3(ublocks), dim3(kThreads), 0, ctx->stream, cnt, Y.as<double>(),
-                               vcur(it), vprev(it), P.as<double>(), wk.alpha() + it, wk.beta() + it, part2, part1,
-                               (int)sblocks);
-            QMB_HIP(hipGetLastError());
             if (finish) {
                 launch_finish(ctx, part2, ublocks, wk.beta() + it + 1, wk.invb() + it + 1, 1);
                 b_ready[it + 1] = 1;
             }
             return;
         }
-        hipLaunchKernelGGL(lz_update, dim3(ublocks), dim3(kThreads), 0, ctx->stream, cnt, Y.as<double>(), vcur(it),
-                           vprev(it), P.as<double>(), wk.alpha() + it, wk.beta() + it, wk.partials.as<double>(),
-                           nullptr, 0);
-        QMB_HIP(hipGetLastError());
-        launch_finish(ctx, wk.partials.as<double>(), ublocks, wk.beta() + it + 1, wk.invb() + it + 1, 1);
-        const bool run = rmode == 1 || (rmode == 2 && pro_decide(it)) ||
-                         (selective && (so_full || !good_theta.empty()));
+        if (rmode == 1) {  // the norm before the orthogonalisation serves its gate only
+            ++n_reorth;
+            gram_schmidt(VB.as<double>(), it + 1, it + 1, part2);
+            return;
+        }
+        launch_finish(ctx, part2, ublocks, wk.beta() + it + 1, wk.invb() + it + 1, 1);
+        const bool run = (rmode == 2 && pro_decide(it)) || (selective && (so_full || !good_theta.empty()));
         if (run) {
             ++n_reorth;
             if (selective && !so_full)
