@@ -287,6 +287,196 @@ __global__ __launch_bounds__(kThreads) void lz_update(int64_t cnt, const double 
     if (threadIdx.x == 0) partials[blockIdx.x] = tb;
 }
 
+// ---- small sectors: a window of steps in one workgroup -------------------------
+// The words of a small sector's matrix fit one CU's LDS beside the vector, so one
+// workgroup runs a whole window of the plain recurrence: the words, the value
+// tables and w stay in LDS (the values of an FP64 matrix are read from memory: it
+// takes the same route, so its results are the packed form's), phi_n, phi_{n-1} and y in registers, and a step has
+// two block sums instead of two launches (a 16-site ring with flip, 415 rows:
+// 3.2 us a step; launched kernel by kernel ~13 us, most of it the host's). Row
+// sums run in slot order as in spmv_sell; the sums of a[n] and b[n] run over the
+// wavefronts in order. P, the last phi, a[], b[] and 1/b[] are left in memory as
+// the kernels of larger sectors leave them, so windows, checks and checkpoints
+// are the same. init: the start vector (seeded when `random`, else P) is
+// normalised first. z: the replay that adds up x = sum_n z[n] phi_n into X and
+// ||H x - e x|| into *res.
+constexpr int kSmallThreads = 1024, kSmallWaves = kSmallThreads / 64;
+constexpr size_t kSmallLds = 140 * 1024;  // vector and words; value tables of up to 16 KB beside them
+
+struct SmallMatrix {
+    int n, n_chunks, stored, n_values, n_values_im, cb, rb;
+    const int64_t *chunk_ptr;
+    const uint16_t *row_len;
+    const uint32_t *words;
+    const double *diag, *vtab, *val;
+};
+
+// LDS of a matrix: vector and words, and the value tables (each a multiple of 16 bytes)
+inline size_t up16(size_t b) { return (b + 15) & ~(size_t)15; }
+inline size_t small_lds_bytes(int64_t n, int64_t stored, int vs) {
+    return up16((size_t)n * vs * 8) + up16((size_t)stored * 4);
+}
+inline size_t small_table_bytes(int n_values, int n_values_im) { return up16((size_t)(n_values + n_values_im) * 8); }
+
+template <bool CPLX, bool PACK, int KR>
+__global__ __launch_bounds__(kSmallThreads) void lz_small(SmallMatrix m, int it0, int steps, int init, int random,
+                                                          uint64_t seed, double *P, double *V0, double *V1,
+                                                          double *alpha, double *beta, double *invb,
+                                                          const double *z, double e, double *X, double *res) {
+    constexpr int VS = CPLX ? 2 : 1;
+    extern __shared__ __align__(16) double small_lds[];
+    __shared__ double red[2][kSmallWaves];
+    double *x = small_lds;
+    double *vt = x + (m.n * VS + 1) / 2 * 2;
+    uint32_t *words = reinterpret_cast<uint32_t *>(vt + (m.n_values + m.n_values_im + 1) / 2 * 2);
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    for (int i = threadIdx.x; i < m.stored; i += kSmallThreads) words[i] = m.words[i];
+    for (int i = threadIdx.x; i < m.n_values; i += kSmallThreads) vt[i] = m.vtab[i];
+    for (int i = threadIdx.x; i < m.n_values_im; i += kSmallThreads) vt[m.n_values + i] = m.vtab[kMaxValues + i];
+    int base[KR], L[KR], len[KR];
+    double d[KR][VS], w[KR][VS], prev[KR][VS], y[KR][VS], sum[KR][VS];
+#pragma unroll
+    for (int k = 0; k < KR; ++k) {
+        const int c = wv + k * kSmallWaves, r = c * 64 + lane;
+        base[k] = L[k] = len[k] = 0;
+        if (c < m.n_chunks) {
+            base[k] = (int)m.chunk_ptr[c];
+            L[k] = ((int)m.chunk_ptr[c + 1] - base[k]) >> 6;
+        }
+        if (r < m.n) len[k] = (int)m.row_len[r];
+#pragma unroll
+        for (int q = 0; q < VS; ++q) {
+            const int i = r * VS + q;
+            d[k][q] = PACK && r < m.n ? m.diag[i] : 0.0;
+            w[k][q] = r < m.n ? (init && random ? splitmix_uniform(seed, (uint64_t)i) : P[i]) : 0.0;
+            prev[k][q] = r < m.n && it0 > 0 ? ((it0 - 1) & 1 ? V1 : V0)[i] : 0.0;
+            sum[k][q] = 0.0;
+            if (r < m.n) x[i] = w[k][q];
+        }
+    }
+    // sum over the block, wavefronts in order, to every thread; alternate buffers
+    // leave one barrier between a buffer's readers and its next writers
+    auto block_total = [&](double v, int buf) {
+        v = wave_sum(v);
+        if (lane == 0) red[buf][wv] = v;
+        __syncthreads();
+        double t = 0.0;
+#pragma unroll
+        for (int i = 0; i < kSmallWaves; ++i) t += red[buf][i];
+        return t;
+    };
+    // H x of the thread's rows into y (x complete in LDS)
+    auto product = [&](const double (&own)[KR][VS]) {
+#pragma unroll
+        for (int k = 0; k < KR; ++k) {
+            if (L[k] == 0) {
+#pragma unroll
+                for (int q = 0; q < VS; ++q) y[k][q] = 0.0;
+                continue;
+            }
+            const int p0 = base[k] + lane;
+            if constexpr (CPLX) {
+                const double2 a =
+                    PACK ? sell_row_cplx_packed<false, 4>(words, vt, vt + m.n_values, x, p0, L[k], len[k], m.cb, m.rb,
+                                                          make_double2(d[k][0], d[k][1]),
+                                                          make_double2(own[k][0], own[k][1]))
+                         : sell_row_cplx<false>(reinterpret_cast<const int32_t *>(words), m.val, x, p0, L[k], len[k]);
+                y[k][0] = a.x;
+                y[k][1] = a.y;
+            } else {
+                y[k][0] = PACK ? sell_row_packed<false, 4>(words, vt, x, p0, L[k], len[k], m.cb, d[k][0], own[k][0])
+                               : sell_row_real<false>(reinterpret_cast<const int32_t *>(words), m.val, x, p0, L[k],
+                                                      len[k]);
+            }
+        }
+    };
+    double s, b = 0.0;
+    if (init) {
+        double t = 0.0;
+#pragma unroll
+        for (int k = 0; k < KR; ++k)
+#pragma unroll
+            for (int q = 0; q < VS; ++q) t += w[k][q] * w[k][q];
+        const double nr = sqrt(block_total(t, 1));
+        s = nr > 0.0 ? 1.0 / nr : 0.0;
+        if (threadIdx.x == 0) {
+            invb[0] = s;
+            beta[0] = 0.0;
+        }
+    } else {
+        s = invb[it0];
+        b = beta[it0];
+        __syncthreads();
+    }
+    for (int it = it0; it < it0 + steps; ++it) {
+        product(w);
+        double dot = 0.0;
+#pragma unroll
+        for (int k = 0; k < KR; ++k)
+#pragma unroll
+            for (int q = 0; q < VS; ++q) {
+                y[k][q] *= s;
+                w[k][q] = w[k][q] * s;  // phi
+                dot += w[k][q] * y[k][q];
+            }
+        const double a = block_total(dot, 0);
+        const double zc = z ? z[it] : 0.0;
+        double nn = 0.0;
+#pragma unroll
+        for (int k = 0; k < KR; ++k) {
+            const int r = (wv + k * kSmallWaves) * 64 + lane;
+#pragma unroll
+            for (int q = 0; q < VS; ++q) {
+                const double phi = w[k][q];
+                const double t = y[k][q] + (-b) * prev[k][q];
+                const double wi = (-a) * phi + t;
+                sum[k][q] = sum[k][q] + zc * phi;
+                prev[k][q] = phi;
+                w[k][q] = wi;
+                nn += wi * wi;
+                if (r < m.n) x[r * VS + q] = wi;
+            }
+        }
+        b = sqrt(block_total(nn, 1));
+        s = b > 0.0 ? 1.0 / b : 0.0;
+        if (threadIdx.x == 0) {
+            alpha[it] = a;
+            beta[it + 1] = b;
+            invb[it + 1] = s;
+        }
+    }
+    double *vlast = (it0 + steps - 1) & 1 ? V1 : V0;
+#pragma unroll
+    for (int k = 0; k < KR; ++k) {
+        const int r = (wv + k * kSmallWaves) * 64 + lane;
+#pragma unroll
+        for (int q = 0; q < VS; ++q) {
+            if (r >= m.n) continue;
+            const int i = r * VS + q;
+            if (z) {
+                X[i] = sum[k][q];
+                x[i] = sum[k][q];  // every gather of w lies before the last barrier
+            } else {
+                P[i] = w[k][q];
+                vlast[i] = prev[k][q];
+            }
+        }
+    }
+    if (!z) return;
+    __syncthreads();
+    product(sum);
+    double t = 0.0;
+#pragma unroll
+    for (int k = 0; k < KR; ++k)
+#pragma unroll
+        for (int q = 0; q < VS; ++q) {
+            const double v = y[k][q] - e * sum[k][q];
+            t += v * v;
+        }
+    t = block_total(t, 0);
+    if (threadIdx.x == 0) *res = sqrt(t);
+}
+
 // ---- start vector, norms, eigenvector helpers -------------------------------
 __global__ __launch_bounds__(kThreads) void lz_random(int64_t cnt, uint64_t seed, double *w) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < cnt; i += (int64_t)gridDim.x * blockDim.x)
@@ -490,10 +680,11 @@ struct LzWork {
     double *beta() const { return scal.as<double>() + M; }
     double *invb() const { return scal.as<double>() + 2 * M + 1; }
     double *misc() const { return scal.as<double>() + 3 * M + 2; }
-    void init(qmb_ctx *ctx, int max_iter) {
+    void init(qmb_ctx *ctx, int max_iter, bool clear) {
         M = max_iter;
         partials.alloc(kMaxBlocks * sizeof(double) * 2);
         scal.alloc((size_t)(3 * M + 2 + 8) * sizeof(double));
+        if (!clear) return;
         QMB_HIP(hipMemsetAsync(scal.p, 0, (size_t)(3 * M + 2 + 8) * sizeof(double), ctx->stream));
     }
 };
@@ -550,6 +741,50 @@ void launch_spmv(qmb_ctx *ctx, const qmb_ell *e, const double *x, double *y, boo
     QMB_HIP(hipGetLastError());
     if (after) QMB_HIP(hipEventRecord(after, ctx->stream));
     if (lz && !fb) launch_finish(ctx, wk->partials.as<double>(), blocks, alpha_out, nullptr, 0);
+}
+
+// Whether a window of the plain recurrence runs in one workgroup (lz_small): the
+// words and a vector within kSmallLds, at most 4 rows a thread (2 complex).
+static bool fits_small(const qmb_ell *e) {
+    const bool cplx = e->value_type == QMB_COMPLEX;
+    return e->n_chunks <= (cplx ? 2 : 4) * kSmallWaves &&
+           small_lds_bytes(e->n_rows, e->stored, cplx ? 2 : 1) <= kSmallLds;
+}
+
+static void launch_small(qmb_ctx *ctx, const qmb_ell *e, LzWork &wk, int it0, int steps, bool init, bool random,
+                         uint64_t seed, double *P, double *V0, double *V1, const double *z = nullptr, double eig = 0.0,
+                         double *X = nullptr, double *res = nullptr) {
+    const bool cplx = e->value_type == QMB_COMPLEX;
+    SmallMatrix m{};
+    m.n = (int)e->n_rows;
+    m.n_chunks = (int)e->n_chunks;
+    m.stored = (int)e->stored;
+    m.chunk_ptr = e->chunk_ptr.as<int64_t>();
+    m.row_len = e->row_len.as<uint16_t>();
+    m.words = e->col.as<uint32_t>();
+    if (e->packed) {
+        m.n_values = e->n_values;
+        m.n_values_im = e->n_values_im;
+        m.cb = e->col_bits;
+        m.rb = e->re_bits;
+        m.diag = e->diag.as<double>();
+        m.vtab = e->vtab.as<double>();
+    } else {
+        m.val = e->val.as<double>();
+    }
+    using K = decltype(&lz_small<false, false, 1>);
+    // [complex][packed][rows a thread: 1, 2, 4]
+    static const K table[2][2][3] = {{{lz_small<false, false, 1>, lz_small<false, false, 2>, lz_small<false, false, 4>},
+                                      {lz_small<false, true, 1>, lz_small<false, true, 2>, lz_small<false, true, 4>}},
+                                     {{lz_small<true, false, 1>, lz_small<true, false, 2>, nullptr},
+                                      {lz_small<true, true, 1>, lz_small<true, true, 2>, nullptr}}};
+    const int kr = (int)((e->n_chunks + kSmallWaves - 1) / kSmallWaves);
+    const K k = table[cplx ? 1 : 0][e->packed ? 1 : 0][kr <= 1 ? 0 : kr <= 2 ? 1 : 2];
+    const size_t lds = small_lds_bytes(e->n_rows, e->stored, cplx ? 2 : 1) +
+                       small_table_bytes(m.n_values, m.n_values_im);
+    hipLaunchKernelGGL(k, dim3(1), dim3(kSmallThreads), lds, ctx->stream, m, it0, steps, init ? 1 : 0, random ? 1 : 0,
+                       seed, P, V0, V1, wk.alpha(), wk.beta(), wk.invb(), z, eig, X, res);
+    QMB_HIP(hipGetLastError());
 }
 
 unsigned spmv_blocks(const qmb_ell *e) { return grid_for(e->n_chunks, kWaves); }
@@ -615,6 +850,7 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
     const int rmode = o.reorth;
     const bool reorth = rmode != 0;
     const bool selective = rmode == 3;
+    const bool small = rmode == 0 && !o.profile && fits_small(e);
     // the selective scheme looks for converged Ritz pairs after every step
     const int check = o.fixed_iter ? M : selective ? 1 : (o.check_every > 0 ? o.check_every : 10);
     constexpr int kMaxGood = 8;  // Ritz vectors kept by the selective scheme (full reorthogonalisation beyond)
@@ -640,7 +876,7 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
         }
     }
     LzWork wk;
-    wk.init(ctx, M);
+    wk.init(ctx, M, !small);
     DevBuf P(cnt * sizeof(double)), Y(cnt * sizeof(double)), Z(cnt * sizeof(double));
     DevBuf V0, V1, VB;
     if (reorth) {
@@ -649,7 +885,7 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
         V0.alloc(cnt * sizeof(double));
         V1.alloc(cnt * sizeof(double));
     }
-    QMB_HIP(hipMemsetAsync(Z.p, 0, cnt * sizeof(double), ctx->stream));
+    if (!small) QMB_HIP(hipMemsetAsync(Z.p, 0, cnt * sizeof(double), ctx->stream));
     DevBuf rpart, rcoef;
     if (reorth) {
         rpart.alloc((size_t)M * rblocks * 2 * sizeof(double));
@@ -671,13 +907,15 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
         } else if (o.start == QMB_START_DEVICE) {
             QMB_REQUIRE(o.start_vec != nullptr, "qmb_lanczos: start == DEVICE needs start_vec");
             QMB_HIP(hipMemcpyAsync(P.p, o.start_vec, cnt * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
-        } else {
+        } else if (!small) {
             hipLaunchKernelGGL(lz_random, dim3(grid_for(cnt, kThreads * 4)), dim3(kThreads), 0, ctx->stream, cnt,
                                o.seed, P.as<double>());
             QMB_HIP(hipGetLastError());
         }
-        launch_norm(ctx, cnt, P.as<double>(), nullptr, 0.0, wk, wk.misc(), wk.invb());
+        // lz_small draws the seeded vector and takes the norm itself
+        if (!small) launch_norm(ctx, cnt, P.as<double>(), nullptr, 0.0, wk, wk.misc(), wk.invb());
     };
+    const bool random_start = o.start == QMB_START_RANDOM;
     const unsigned ublocks = grid_for(cnt, kThreads * 4);
     // Plain recurrence: the a[n] and b[n+1] one-block finishes are folded into
     // the next kernel (every block re-sums the fixed partial slots in the same
@@ -954,7 +1192,7 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
     // explicit b finish, which gives the same values as the fused one), so the
     // device does not idle. Not after a check the decay prediction scheduled:
     // that one usually ends the run, and its queued step would be wasted.
-    const bool can_queue_ahead = fuse && !o.fixed_iter && !(ck && ck->path);
+    const bool can_queue_ahead = fuse && !small && !o.fixed_iter && !(ck && ck->path);
     bool predicted = false;
     int it_q = it;  // steps queued so far
     int wpar = 0;   // event half of the current window
@@ -973,6 +1211,12 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
     while (it < M) {
         const int win0 = it;
         const int win1 = std::min(M, it + next);
+        if (small) {
+            launch_small(ctx, e, wk, win0, win1 - win0, win0 == 0, random_start, o.seed, P.as<double>(),
+                         V0.as<double>(), V1.as<double>());
+            it = it_q = win1;
+            b_ready[it] = 1;
+        }
         for (; it < win1; ++it)
             if (it >= it_q) queue_step(it, it - win0, wpar, it + 1 == win1);
         n_spmv += win1 - win0;
@@ -1128,6 +1372,14 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
             hipLaunchKernelGGL(basis_combine, dim3(grid_for(cnt, kThreads * 4)), dim3(kThreads), 0, ctx->stream, cnt,
                                (int64_t)cnt, m, VB.as<double>(), dz.as<double>(), X.as<double>());
             QMB_HIP(hipGetLastError());
+        } else if (small) {
+            DevBuf dz(m * sizeof(double));
+            double *hz = ctx->host_stage<double>(m * sizeof(double));
+            std::copy(z0.begin(), z0.begin() + m, hz);
+            QMB_HIP(hipMemcpyAsync(dz.p, hz, m * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
+            init_start();
+            launch_small(ctx, e, wk, 0, m, true, random_start, o.seed, P.as<double>(), V0.as<double>(),
+                         V1.as<double>(), dz.as<double>(), evals[0], X.as<double>(), wk.misc() + 1);
         } else {
             QMB_HIP(hipMemsetAsync(X.p, 0, cnt * sizeof(double), ctx->stream));
             QMB_HIP(hipMemsetAsync(Z.p, 0, cnt * sizeof(double), ctx->stream));
@@ -1142,8 +1394,10 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
                 k2(j, false);
             }
         }
-        launch_spmv(ctx, e, X.as<double>(), Y.as<double>(), false, nullptr, nullptr, nullptr, nullptr);
-        launch_norm(ctx, cnt, Y.as<double>(), X.as<double>(), evals[0], wk, wk.misc() + 1, wk.misc() + 2);
+        if (!small) {
+            launch_spmv(ctx, e, X.as<double>(), Y.as<double>(), false, nullptr, nullptr, nullptr, nullptr);
+            launch_norm(ctx, cnt, Y.as<double>(), X.as<double>(), evals[0], wk, wk.misc() + 1, wk.misc() + 2);
+        }
         QMB_HIP(hipMemcpyAsync(&eig_res, wk.misc() + 1, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
         if (eigvec)
             QMB_HIP(hipMemcpyAsync(eigvec, X.p, cnt * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
