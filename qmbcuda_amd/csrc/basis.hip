@@ -367,20 +367,6 @@ __global__ __launch_bounds__(kBasisThreads) void basis_mark_words(GroupView gv, 
     }
 }
 
-// Position of the k-th set bit of w (k below its number of set bits).
-__device__ inline int select_bit(uint64_t w, int k) {
-    int pos = 0;
-#pragma unroll
-    for (int width = 32; width >= 1; width >>= 1) {
-        const int c = __popcll(w & ((1ULL << width) - 1ULL));
-        const bool up = k >= c;
-        k -= up ? c : 0;
-        w >>= up ? width : 0;
-        pos += up ? width : 0;
-    }
-    return pos;
-}
-
 // The rows in ascending order. A wavefront takes tile_words (a power of two, at
 // most 64) consecutive words: their records are one coalesced load, and 64 rows
 // at a time each lane finds its row's word among the tile's row offsets (a

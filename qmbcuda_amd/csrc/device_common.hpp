@@ -208,6 +208,20 @@ __device__ inline S next_comb(S x) {
     return (S)((((r ^ x) >> 2) >> ctz_s(x)) | r);
 }
 
+// Position of the k-th set bit of w (k below its number of set bits).
+__device__ inline int select_bit(uint64_t w, int k) {
+    int pos = 0;
+#pragma unroll
+    for (int width = 32; width >= 1; width >>= 1) {
+        const int c = __popcll(w & ((1ULL << width) - 1ULL));
+        const bool up = k >= c;
+        k -= up ? c : 0;
+        w >>= up ? width : 0;
+        pos += up ? width : 0;
+    }
+    return pos;
+}
+
 // Image of x under coset representative c_i (i >= 1) of a lut-3 or lut-4 group:
 // one bit reversal when c_i is the site reversal, else the nibble table of
 // stage_images.

@@ -28,6 +28,12 @@ namespace qmb {
 // nibble rank table)
 constexpr int kEllThreads = 512;
 
+// Lanes per row (2^ts, at most 2^kMaxSplit) while rows x lanes stay within this
+// (ELL build: 5x5 with quarter turns, 52,244 rows, 681 us with 2^16, 386 with 2^18,
+// 418 with 2^20; 24-site ring, 56,450 rows, 242, 219 and 250 us; one lane 251 us).
+constexpr int kMaxSplit = 4;
+constexpr int64_t kSplitLanes = (int64_t)1 << 18;
+
 constexpr int kSetSlots = 4096;  // global set of distinct values
 constexpr int kLdsSet = 256;     // per-block set
 constexpr unsigned long long kEmptyKey = ~0ull;
@@ -73,8 +79,11 @@ struct CodeView {
 
 // Rank tables in dynamic LDS: the nibble table (rank_tab, n_nib > 0) when it
 // fits, else the binomial table (binom). CODED (fill only): codes instead of
-// values (CodeView).
-template <class S, bool FILL, bool CPLX, bool CODED = false>
+// values (CodeView). SPLIT: 2^ts neighbouring lanes share a row. Each applies all
+// terms (pass A), then takes every 2^ts-th candidate; a round's surviving
+// candidates find their slots in term order from a ballot. A row is a chain of
+// one lookup per acting term, which only many rows hide.
+template <class S, bool FILL, bool CPLX, bool CODED = false, bool SPLIT = false>
 __global__ __launch_bounds__(kEllThreads) void ell_rows(GroupView gv, const uint64_t *binom,
                                                         const uint64_t *rank_tab, int n_nib, int n_c, int layout,
                                                         int64_t n_rows, const uint64_t *reps, const uint8_t *stab,
@@ -82,7 +91,7 @@ __global__ __launch_bounds__(kEllThreads) void ell_rows(GroupView gv, const uint
                                                         TermsView tv, const double2 *chi,
                                                         const double *nrm, int W, uint16_t *row_len, int *err,
                                                         int all_rows, const int64_t *chunk_ptr, int32_t *col,
-                                                        double *val, CodeView cv) {
+                                                        double *val, CodeView cv, int ts) {
     extern __shared__ uint64_t rank_lds[];
     __shared__ alignas(8) uint8_t perm_lds[kMaxGroup * 64];
     __shared__ double2 s_chi[kMaxGroup];
@@ -109,8 +118,10 @@ __global__ __launch_bounds__(kEllThreads) void ell_rows(GroupView gv, const uint
         }
         __syncthreads();
     }
-    const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t r = SPLIT ? t >> ts : t;
     if (r >= n_rows) return;
+    const int split = SPLIT ? 1 << ts : 1, sub = SPLIT ? (int)t & (split - 1) : 0;
     const int64_t c = r / kChunk;
     const int lane = (int)(r % kChunk);
     int64_t base = 0;
@@ -151,74 +162,96 @@ __global__ __launch_bounds__(kEllThreads) void ell_rows(GroupView gv, const uint
                 slot += __popcll(cand);
                 continue;
             }
-            while (cand) {
-                const int h = h0 + __builtin_ctzll(cand);
-                cand &= cand - 1;
-                double cr, ci;
+            // one candidate: its row (-1: none) and, when it has one, its entry at slot `at`
+            auto lookup = [&](int h, int &gm, int &mult, double &cr, double &ci) -> int64_t {
                 S tgt;
                 apply_term<S>(tv, h, src, tgt, cr, ci);
-                int gm, mult;
                 const S rep = orbit_min_any<S>(tgt, gv, gt, perm_lds, gm, mult);
                 const int64_t r2 = row_of_rank(
                     n_nib ? colex_rank_nib<S>(rep, rank_lds, n_nib, n_c) : colex_rank<S>(rep, rank_lds), dict);
-                if (r2 < 0) continue;
-                if (layout == QMB_LAYOUT_REFERENCE && nullf[r2]) continue;
-                if (FILL && CODED) {
-                    if (slot < L) {
-                        const TermC &tm = tv.t[h];
-                        const int neg = popc_s((S)(~src & (S)tm.sz)) & 1;
-                        const int cs = s_mcls[m_src], ct = s_mcls[mult];
-                        const bool ok = cs != 0xFF && ct != 0xFF;
-                        if (!ok) *cv.bad = 1;
-                        const int code =
-                            ok ? ((((int)tm.vclass * 2 + neg) * cv.n_chi + s_xcls[gm]) * cv.n_m + cs) * cv.n_m + ct
-                               : 0;
-                        const int64_t pos = base + (int64_t)slot * kChunk + lane;
-                        col[pos] = (int32_t)r2;
-                        cv.code[pos] = (uint16_t)code;
-                    }
-                } else if (FILL) {
-                    if (slot < L) {
-                        // mult = the target row's stabiliser size (no read of stab[r2]);
-                        // equal sizes give the ratio 1 exactly
-                        const double ratio = mult == m_src ? 1.0 : s_nrm[mult] / n_src;
-                        const double2 x = s_chi[gm];
-                        const double pr = cr * x.x - ci * x.y;
-                        const double pi = cr * x.y + ci * x.x;
-                        const int64_t pos = base + (int64_t)slot * kChunk + lane;
-                        col[pos] = (int32_t)r2;
-                        if (CPLX) {
-                            val[2 * pos] = pr * ratio;
-                            val[2 * pos + 1] = pi * ratio;
-                        } else {
-                            val[pos] = pr * ratio;
-                        }
+                if (r2 >= 0 && layout == QMB_LAYOUT_REFERENCE && nullf[r2]) return -1;
+                return r2;
+            };
+            auto write = [&](int at, int h, int64_t r2, int gm, int mult, double cr, double ci) {
+                if (!FILL || at >= L) return;
+                const int64_t pos = base + (int64_t)at * kChunk + lane;
+                col[pos] = (int32_t)r2;
+                if (CODED) {
+                    const TermC &tm = tv.t[h];
+                    const int neg = popc_s((S)(~src & (S)tm.sz)) & 1;
+                    const int cs = s_mcls[m_src], ct = s_mcls[mult];
+                    const bool ok = cs != 0xFF && ct != 0xFF;
+                    if (!ok) *cv.bad = 1;
+                    const int code =
+                        ok ? ((((int)tm.vclass * 2 + neg) * cv.n_chi + s_xcls[gm]) * cv.n_m + cs) * cv.n_m + ct : 0;
+                    cv.code[pos] = (uint16_t)code;
+                } else {
+                    // mult = the target row's stabiliser size (no read of stab[r2]);
+                    // equal sizes give the ratio 1 exactly
+                    const double ratio = mult == m_src ? 1.0 : s_nrm[mult] / n_src;
+                    const double2 x = s_chi[gm];
+                    const double pr = cr * x.x - ci * x.y;
+                    const double pi = cr * x.y + ci * x.x;
+                    if (CPLX) {
+                        val[2 * pos] = pr * ratio;
+                        val[2 * pos + 1] = pi * ratio;
+                    } else {
+                        val[pos] = pr * ratio;
                     }
                 }
+            };
+            if (SPLIT) {
+                const int nc = __popcll(cand);
+                for (int k0 = 0; k0 < nc; k0 += split) {  // the same rounds for the lanes of a row
+                    int64_t r2 = -1;
+                    int h = 0, gm = 0, mult = 0;
+                    double cr = 0.0, ci = 0.0;
+                    if (k0 + sub < nc) {
+                        h = h0 + select_bit(cand, k0 + sub);
+                        r2 = lookup(h, gm, mult, cr, ci);
+                    }
+                    const uint64_t found =
+                        (__ballot(r2 >= 0) >> ((threadIdx.x & 63) - sub)) & ((1ULL << split) - 1ULL);
+                    if (r2 >= 0) write(slot + __popcll(found & ((1ULL << sub) - 1ULL)), h, r2, gm, mult, cr, ci);
+                    slot += __popcll(found);
+                }
+                continue;
+            }
+            while (cand) {
+                const int h = h0 + __builtin_ctzll(cand);
+                cand &= cand - 1;
+                int gm, mult;
+                double cr, ci;
+                const int64_t r2 = lookup(h, gm, mult, cr, ci);
+                if (r2 < 0) continue;
+                write(slot, h, r2, gm, mult, cr, ci);
                 ++slot;
             }
         }
     }
     const int len = null_row ? 0 : slot;
     if (!FILL) {
+        if (sub) return;
         if (len > W) atomicMax(err, 1);
         row_len[r] = (uint16_t)(len < 65535 ? len : 65535);
         return;
     }
     if (CODED) {
         // the diagonal into its own array; slot 0 and the padding slots hold the row
-        if (CPLX) {
-            cv.diag[2 * r] = null_row ? 0.0 : dr;
-            cv.diag[2 * r + 1] = null_row ? 0.0 : di;
-        } else {
-            cv.diag[r] = null_row ? 0.0 : dr;
+        if (sub == 0) {
+            if (CPLX) {
+                cv.diag[2 * r] = null_row ? 0.0 : dr;
+                cv.diag[2 * r + 1] = null_row ? 0.0 : di;
+            } else {
+                cv.diag[r] = null_row ? 0.0 : dr;
+            }
+            if (L > 0) col[base + lane] = (int32_t)r;
         }
-        if (L > 0) col[base + lane] = (int32_t)r;
-        for (int s = (len > 1 ? len : 1); s < L; ++s) col[base + (int64_t)s * kChunk + lane] = (int32_t)r;
+        for (int s = (len > 1 ? len : 1) + sub; s < L; s += split) col[base + (int64_t)s * kChunk + lane] = (int32_t)r;
         return;
     }
     // diagonal slot (also written for empty rows, like the reference's ind[id*W] = id)
-    if (L > 0) {
+    if (L > 0 && sub == 0) {
         const int64_t pos0 = base + lane;
         col[pos0] = (int32_t)r;
         if (CPLX) {
@@ -228,7 +261,7 @@ __global__ __launch_bounds__(kEllThreads) void ell_rows(GroupView gv, const uint
             val[pos0] = null_row ? 0.0 : dr;
         }
     }
-    for (int s = (len > 1 ? len : 1); s < L; ++s) {
+    for (int s = (len > 1 ? len : 1) + sub; s < L; s += split) {
         const int64_t pos = base + (int64_t)s * kChunk + lane;
         col[pos] = (int32_t)r;
         if (CPLX) {
@@ -898,20 +931,29 @@ qmb_status qmb_ell_build(qmb_ctx *ctx, const qmb_basis *b, const qmb_terms *t, i
         e->row_len.alloc((size_t)std::max<int64_t>(n, 1) * sizeof(uint16_t));
         e->chunk_ptr.alloc((size_t)(e->n_chunks + 1) * sizeof(int64_t));
         const RankTables rank(*b);
-        const unsigned blocks = (unsigned)std::max<int64_t>(1, (n + kEllThreads - 1) / kEllThreads);
+        // lanes per row of the passes that make lookups: as many as keep the chip busy
+        int ts = 0;
+        while (ts < kMaxSplit && (n << (ts + 1)) <= kSplitLanes) ++ts;
+        auto blocks_for = [&](int shift) {
+            return (unsigned)std::max<int64_t>(1, ((n << shift) + kEllThreads - 1) / kEllThreads);
+        };
         const bool cplx = value_type == QMB_COMPLEX;
+        const bool narrow = b->n_sites <= 32;
+        using K = decltype(&ell_rows<uint32_t, false, false>);
         if (n > 0) {
-            const bool narrow = b->n_sites <= 32;
-            auto kcount = narrow ? (cplx ? ell_rows<uint32_t, false, true> : ell_rows<uint32_t, false, false>)
-                                 : (cplx ? ell_rows<uint64_t, false, true> : ell_rows<uint64_t, false, false>);
+            const int cts = b->all_rows ? 0 : ts;
+            // [64-bit states][complex][split]; the count does not depend on the values
+            static const K counts[2][2] = {{ell_rows<uint32_t, false, false>, ell_rows<uint32_t, false, false, false, true>},
+                                           {ell_rows<uint64_t, false, false>, ell_rows<uint64_t, false, false, false, true>}};
+            const K kcount = counts[narrow ? 0 : 1][cts ? 1 : 0];
             // the count pass of a sector without null orbits makes no orbit lookups
-            hipLaunchKernelGGL(kcount, dim3(blocks), dim3(kEllThreads), b->all_rows ? 0 : rank.lds_bytes,
+            hipLaunchKernelGGL(kcount, dim3(blocks_for(cts)), dim3(kEllThreads), b->all_rows ? 0 : rank.lds_bytes,
                                ctx->stream, gv, ctx->binom.as<uint64_t>(), rank.tab(), rank.n_nib, rank.n_c,
                                b->layout, n, b->reps.as<uint64_t>(),
                                b->stab.as<uint8_t>(), b->nullf.as<uint8_t>(), b->dict.as<uint64_t>(),
                                tv, dt.chi, dt.nrm, W,
                                e->row_len.as<uint16_t>(), d_err.as<int>(), b->all_rows ? 1 : 0, nullptr, nullptr,
-                               nullptr, CodeView{});
+                               nullptr, CodeView{}, cts);
             QMB_HIP(hipGetLastError());
         }
         // the offsets are scanned before the overflow flag is read (one synchronisation)
@@ -929,20 +971,25 @@ qmb_status qmb_ell_build(qmb_ctx *ctx, const qmb_basis *b, const qmb_terms *t, i
         const bool coded = vp.on && vp.plan_codes(ctx, *e, *b, dt, ch, g->G);
         // the fill (coded, or with FP64 values) and the padding of the last chunk
         auto fill = [&](bool with_codes) {
-            const bool narrow = b->n_sites <= 32;
-            auto kfill = with_codes
-                             ? (narrow ? (cplx ? ell_rows<uint32_t, true, true, true> : ell_rows<uint32_t, true, false, true>)
-                                       : (cplx ? ell_rows<uint64_t, true, true, true> : ell_rows<uint64_t, true, false, true>))
-                             : (narrow ? (cplx ? ell_rows<uint32_t, true, true> : ell_rows<uint32_t, true, false>)
-                                       : (cplx ? ell_rows<uint64_t, true, true> : ell_rows<uint64_t, true, false>));
+            // [64-bit states][complex][coded][split]
+            static const K fills[2][2][2][2] = {
+                {{{ell_rows<uint32_t, true, false>, ell_rows<uint32_t, true, false, false, true>},
+                  {ell_rows<uint32_t, true, false, true>, ell_rows<uint32_t, true, false, true, true>}},
+                 {{ell_rows<uint32_t, true, true>, ell_rows<uint32_t, true, true, false, true>},
+                  {ell_rows<uint32_t, true, true, true>, ell_rows<uint32_t, true, true, true, true>}}},
+                {{{ell_rows<uint64_t, true, false>, ell_rows<uint64_t, true, false, false, true>},
+                  {ell_rows<uint64_t, true, false, true>, ell_rows<uint64_t, true, false, true, true>}},
+                 {{ell_rows<uint64_t, true, true>, ell_rows<uint64_t, true, true, false, true>},
+                  {ell_rows<uint64_t, true, true, true>, ell_rows<uint64_t, true, true, true, true>}}}};
+            const K kfill = fills[narrow ? 0 : 1][cplx ? 1 : 0][with_codes ? 1 : 0][ts ? 1 : 0];
             double *val = with_codes ? nullptr : e->val.as<double>();
-            hipLaunchKernelGGL(kfill, dim3(blocks), dim3(kEllThreads), rank.lds_bytes, ctx->stream, gv,
+            hipLaunchKernelGGL(kfill, dim3(blocks_for(ts)), dim3(kEllThreads), rank.lds_bytes, ctx->stream, gv,
                                ctx->binom.as<uint64_t>(), rank.tab(), rank.n_nib, rank.n_c, b->layout, n,
                                b->reps.as<uint64_t>(),
                                b->stab.as<uint8_t>(), b->nullf.as<uint8_t>(), b->dict.as<uint64_t>(),
                                tv, dt.chi, dt.nrm, W,
                                e->row_len.as<uint16_t>(), d_err.as<int>(), 0, e->chunk_ptr.as<int64_t>(),
-                               e->col.as<int32_t>(), val, with_codes ? vp.cv : CodeView{});
+                               e->col.as<int32_t>(), val, with_codes ? vp.cv : CodeView{}, ts);
             QMB_HIP(hipGetLastError());
             if (n % kChunk) {
                 hipLaunchKernelGGL(ell_pad_tail, dim3(1), dim3(kChunk), 0, ctx->stream, n, e->n_chunks,
