@@ -167,7 +167,7 @@ __device__ inline uint64_t mark_run(S x, int cnt, const GroupView &gv, const Gro
         // with the spin flip, above their complements or theirs): a necessary
         // condition, branch-free. Pass 2 takes each lane's survivors in turn:
         // per coset c_i one image z = c_i y (the state itself for a plain ring) and
-        // the scan of its top bytes (ring_windows): a smaller byte rules the state
+        // the scan of its top bytes (ring_candidates): a smaller byte rules the state
         // out, and only the rotations that reach its own are formed; element
         // indices are looked up only for images equal to the state (stabiliser).
         const int N = gv.n_sites;
@@ -201,15 +201,15 @@ __device__ inline uint64_t mark_run(S x, int cnt, const GroupView &gv, const Gro
             const int n_cos = gv.lut == 3 ? gv.n_cos : 1;
             for (int ci = 0; ci < n_cos && rep; ++ci) {
                 const uint8_t *ct = gv.lut == 3 ? gt.cos + ci * 128 : gt.lut + 512;
-                const S z = ci ? coset_image<S>(y, ci, gv, gt, perm_lds) : y;
-                uint64_t c0, c1;
-                const unsigned tmin = ring_windows<S>(z, N, hf, c0, c1);
+                const S z = ci ? coset_image<S>(y, ci, gv, perm_lds) : y;
+                S c0, c1;
+                const unsigned tmin = ring_candidates<S>(z, N, hf, c0, c1);
                 if (tmin > top) continue;
                 rep = tmin == top;
                 for (int f = 0; f < (hf ? 2 : 1); ++f) {
-                    uint64_t c = f ? c1 : c0;
+                    S c = f ? c1 : c0;
                     while (c && rep) {
-                        const int p = __builtin_ctzll(c);
+                        const int p = ctz_s(c);
                         c &= c - 1;
                         int st = N - 8 - p;
                         if (st < 0) st += N;

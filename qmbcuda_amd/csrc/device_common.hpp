@@ -68,7 +68,7 @@ __device__ inline S full_mask(const GroupView &gv) {
 // Image of state x under element g: the reference's bit move s -> group_el[g][s]
 // (Q/exact_diagonalization/utils.cu:52-59), plus the spin flip of this build.
 template <class S>
-__device__ inline S apply_elem(S x, int g, const GroupView &gv, const uint8_t *perm_lds) {
+__device__ __forceinline__ S apply_elem(S x, int g, const GroupView &gv, const uint8_t *perm_lds) {
     const S full = (S)gv.full;
     S y;
     if (gv.torus) {
@@ -119,6 +119,55 @@ __device__ inline void stage_group(GroupLds &t, const GroupView &g) {
     if (g.lut >= 3)
         for (int i = threadIdx.x; i < kCosBytes; i += blockDim.x) t.cos[i] = g.cos_tab[i];
 }
+
+// LDS tables of the orbit minimum (orbit_min_any). blk (torus products): for a
+// block value v the smallest in-block rotation of v and, under flip, of its
+// complement (bits 0-7), and the shifts that reach it, plain (bits 8-15) and
+// complemented (bits 16-23). einv: inverse element of (flip, shift) o c_i at the
+// index of GroupView's element tables, 128 per coset.
+struct OrbitLds {
+    uint32_t blk[256];
+    uint8_t einv[kCosBytes];
+};
+
+__device__ inline void stage_orbit(OrbitLds &t, const GroupView &g) {
+    if (g.lut == 1 || g.lut == 4) {
+        const unsigned mB = (1u << g.block) - 1u;
+        for (unsigned v = threadIdx.x; v <= mB; v += blockDim.x) {
+            const unsigned a = g.lut_tab[v], b = g.lut_flip ? g.lut_tab[v ^ mB] : 0xFFu, m = a < b ? a : b;
+            t.blk[v] = m | (a == m ? (unsigned)g.lut_tab[256 + v] << 8 : 0u) |
+                       (b == m && g.lut_flip ? (unsigned)g.lut_tab[256 + (v ^ mB)] << 16 : 0u);
+        }
+    }
+    if (g.lut == 1 || g.lut == 2)
+        for (int i = threadIdx.x; i < 128; i += blockDim.x) t.einv[i] = g.inv[g.lut_tab[512 + i]];
+    if (g.lut >= 3)
+        for (int i = threadIdx.x; i < g.n_cos * 128; i += blockDim.x) t.einv[i] = g.inv[g.cos_tab[i]];
+}
+
+// The smallest image found so far. Elements are named by their index in einv:
+// the inverse is looked up once at the end, and at ties (which only states with a
+// stabiliser have) for the smallest.
+template <class S>
+struct OrbitBest {
+    S best = 0;
+    int at = -1;    // index of the only element so far, or -1
+    int elem = -1;  // smallest inverse element of several
+    int mult = 0;
+    __device__ __forceinline__ void take(S y, int i, const OrbitLds &t) {
+        if (mult == 0 || y < best) {
+            best = y;
+            at = i;
+            mult = 1;
+        } else if (y == best) {
+            ++mult;
+            const int a = at >= 0 ? (int)t.einv[at] : elem, b = t.einv[i];
+            elem = a < b ? a : b;
+            at = -1;
+        }
+    }
+    __device__ __forceinline__ int element(const OrbitLds &t) const { return at >= 0 ? (int)t.einv[at] : elem; }
+};
 
 // apply_elem with the element index varying across lanes (tables from LDS).
 template <class S>
@@ -185,7 +234,7 @@ __device__ inline void stage_binom_rows(typename RankOf<S>::T *lds, const uint64
 // Branch-free (lanes of a wave differ in where their up spins are); C(p, j) = 0
 // for p < j places the last ones, and with j = 0 the rank left is 0 < C(p, 0).
 template <class S>
-__device__ inline S colex_unrank(typename RankOf<S>::T r, int k, int n_sites,
+__device__ __forceinline__ S colex_unrank(typename RankOf<S>::T r, int k, int n_sites,
                                  const typename RankOf<S>::T *bin_lds) {
     S x = 0;
     int at = (n_sites - 1) * kBinJ + k;
@@ -236,13 +285,13 @@ __device__ inline uint64_t reverse_sites<uint64_t>(uint64_t x, int n) {
     return __builtin_bitreverse64(x) >> (64 - n);
 }
 template <class S>
-__device__ inline S coset_image(S x, int ci, const GroupView &gv, const GroupLds &t, const uint8_t *perm_lds) {
+__device__ __forceinline__ S coset_image(S x, int ci, const GroupView &gv, const uint8_t *perm_lds) {
     if ((gv.cos_rev >> ci) & 1) return reverse_sites<S>(x, gv.n_sites);
     const int nn = (gv.n_sites + 3) / 4;
     const S *tab = reinterpret_cast<const S *>(perm_lds) + (ci - 1) * nn * 16;
     S y = 0;
     for (int k = 0; k < nn; ++k) y |= tab[k * 16 + (int)((x >> (4 * k)) & 15)];
-    return t.flip[t.cos[ci * 128]] ? (S)(y ^ (S)gv.full) : y;
+    return gv.flip[gv.cos_tab[ci * 128]] ? (S)(y ^ (S)gv.full) : y;
 }
 
 // Left rotation of an n-site ring state by s (0 <= s < n).
@@ -262,7 +311,7 @@ __device__ inline void stabiliser_coset(S x, const GroupView &gv, const GroupLds
     stab_hi = 0;
     for (int ci = 0; ci < gv.n_cos; ++ci) {
         const uint8_t *ct = t.cos + ci * 128;
-        S y = ci ? coset_image<S>(x, ci, gv, t, perm_lds) : x;
+        S y = ci ? coset_image<S>(x, ci, gv, perm_lds) : x;
         for (int s = 0; s < N; ++s) {
             if (s) y = rotl_ring<S>(y, 1, N, full);
             for (int f = 0; f < (gv.lut_flip ? 2 : 1); ++f) {
@@ -320,7 +369,7 @@ __device__ inline void stabiliser(S x, const GroupView &gv, const GroupLds &t, c
 // the stabiliser size of the minimum (those elements form a coset of x's
 // stabiliser, which has the same size as the minimum's).
 template <class S>
-__device__ inline S orbit_min(S x, const GroupView &gv, const uint8_t *perm_lds, int &gm, int &mult) {
+__device__ __forceinline__ S orbit_min(S x, const GroupView &gv, const uint8_t *perm_lds, int &gm, int &mult) {
     S best = x;
     int bi = gv.inv[0];
     mult = 1;
@@ -343,7 +392,7 @@ __device__ inline S orbit_min(S x, const GroupView &gv, const uint8_t *perm_lds,
 // Image of x under the torus element (in-block shift sh, block shift by big
 // bits, flip f), formed directly (as apply_elem).
 template <class S>
-__device__ inline S torus_image(S x, int sh, int big, int f, int B, int N, S rep_unit, S full) {
+__device__ __forceinline__ S torus_image(S x, int sh, int big, int f, int B, int N, S rep_unit, S full) {
     S y = x;
     if (sh) {
         const S k = (S)(rep_unit * (S)((1u << (B - sh)) - 1u));
@@ -353,108 +402,55 @@ __device__ inline S torus_image(S x, int sh, int big, int f, int B, int N, S rep
     return f ? (S)(y ^ full) : y;
 }
 
-// orbit_min for a group that is the whole torus product (gv.lut): an image's
-// top block is source block j rotated by the in-block shift s (complemented
-// under flip), placed on top by the block shift a = nb-1-j. Integer order is
-// decided by the top block first, so the minimum image has the smallest top
-// block tmin over all (j, s, f), and only the elements reaching tmin need full
-// images. Same result and same gm as orbit_min.
+// orbit_min for a group that is the whole torus product (gv.lut == 1), or one
+// times cosets (gv.lut == 4: the orbit is the union of the torus orbits of the
+// images c_i x). An image's top block is source block j rotated by the in-block
+// shift s (complemented under flip), placed on top by the block shift nb-1-j.
+// Integer order is decided by the top block first, so the minimum image has the
+// smallest top block over all (j, s, f), and only the elements reaching it need
+// full images: one table read per block gives its smallest rotation and the
+// shifts, and the candidates of all blocks form one list (bit 8 j + s), so a
+// wavefront goes round as often as its longest list, not once per block and
+// flip. Same result and same gm as orbit_min.
 template <class S>
-__device__ inline S orbit_min_lut(S x, const GroupView &gv, const GroupLds &t, int &gm, int &mult) {
+__device__ __forceinline__ S orbit_min_torus(S x, const GroupView &gv, const OrbitLds &t, const uint8_t *perm_lds, bool cosets,
+                                    int &gm, int &mult) {
     const int B = gv.block, N = gv.n_sites, nb = N / B;
     const unsigned mB = (1u << B) - 1u;
     const S full = (S)gv.full;
-    const int nf = gv.lut_flip ? 2 : 1;
-    unsigned tmin = 0xFFu;
-    for (int j = 0; j < nb; ++j) {
-        const unsigned v = (unsigned)(x >> (j * B)) & mB;
-        tmin = min(tmin, (unsigned)t.lut[v]);
-        if (nf == 2) tmin = min(tmin, (unsigned)t.lut[v ^ mB]);
-    }
-    S best = 0;
-    int bi = -1;
-    mult = 0;
-    for (int j = 0; j < nb; ++j) {
-        const unsigned v0 = (unsigned)(x >> (j * B)) & mB;
-        const int a = nb - 1 - j;
-        for (int f = 0; f < nf; ++f) {
-            const unsigned v = f ? (v0 ^ mB) : v0;
-            if (t.lut[v] != tmin) continue;
-            unsigned sm = t.lut[256 + v];
-            const int big = a * B;
-            while (sm) {
-                const int sh = __builtin_ctz(sm);
-                sm &= sm - 1;
-                // the element's tables are read only for a new or tied minimum
-                const S y = torus_image<S>(x, sh, big, f, B, N, (S)gv.rep_unit, full);
-                if (bi < 0 || y < best) {
-                    best = y;
-                    bi = t.inv[t.lut[512 + (f * 8 + a) * 8 + sh]];
-                    mult = 1;
-                } else if (y == best) {
-                    ++mult;
-                    const int ig = t.inv[t.lut[512 + (f * 8 + a) * 8 + sh]];
-                    if (ig < bi) bi = ig;
-                }
-            }
-        }
-    }
-    gm = bi;
-    return best;
-}
-
-// orbit_min for a full torus product times cosets (gv.lut == 4): the orbit is
-// the union of the torus orbits of y_i = c_i x; only cosets whose smallest
-// rotated block reaches the smallest so far take full images of their
-// candidates. Same result and same gm as orbit_min.
-template <class S>
-__device__ inline S orbit_min_torus_coset(S x, const GroupView &gv, const GroupLds &t, const uint8_t *perm_lds,
-                                          int &gm, int &mult) {
-    const int B = gv.block, N = gv.n_sites, nb = N / B;
-    const unsigned mB = (1u << B) - 1u;
-    const S full = (S)gv.full;
-    const int nf = gv.lut_flip ? 2 : 1;
-    S best = 0;
-    int bi = -1;
-    mult = 0;
+    OrbitBest<S> o;
     unsigned tbest = 0xFFu;
-    for (int ci = 0; ci < gv.n_cos; ++ci) {
-        const uint8_t *ct = t.cos + ci * 128;
-        const S z = ci ? coset_image<S>(x, ci, gv, t, perm_lds) : x;
-        unsigned tmin = 0xFFu;
+    for (int ci = 0; ci < (cosets ? gv.n_cos : 1); ++ci) {
+        const S z = ci ? coset_image<S>(x, ci, gv, perm_lds) : x;
+        uint64_t c0 = 0, c1 = 0;
+        S v = z;
         for (int j = 0; j < nb; ++j) {
-            const unsigned v = (unsigned)(z >> (j * B)) & mB;
-            tmin = min(tmin, (unsigned)t.lut[v]);
-            if (nf == 2) tmin = min(tmin, (unsigned)t.lut[v ^ mB]);
+            const unsigned e = t.blk[(unsigned)v & mB];
+            v = (S)(v >> B);
+            const unsigned m = e & 0xFFu;
+            if (m > tbest) continue;
+            const uint64_t k0 = (uint64_t)((e >> 8) & 0xFFu) << (8 * j), k1 = (uint64_t)(e >> 16) << (8 * j);
+            c0 = m < tbest ? k0 : c0 | k0;
+            c1 = m < tbest ? k1 : c1 | k1;
+            if (m < tbest) o.mult = 0;  // images of earlier cosets have a larger top block
+            tbest = m;
         }
-        if (tmin > tbest) continue;
-        tbest = tmin;
-        for (int j = 0; j < nb; ++j) {
-            const unsigned v0 = (unsigned)(z >> (j * B)) & mB;
-            const int a = nb - 1 - j;
-            for (int f = 0; f < nf; ++f) {
-                const unsigned v = f ? (v0 ^ mB) : v0;
-                if (t.lut[v] != tmin) continue;
-                unsigned sm = t.lut[256 + v];
-                while (sm) {
-                    const int sh = __builtin_ctz(sm);
-                    sm &= sm - 1;
-                    const S y = torus_image<S>(z, sh, a * B, f, B, N, (S)gv.rep_unit, full);
-                    if (bi < 0 || y < best) {
-                        best = y;
-                        bi = t.inv[ct[(f * 8 + a) * 8 + sh]];
-                        mult = 1;
-                    } else if (y == best) {
-                        ++mult;
-                        const int ig = t.inv[ct[(f * 8 + a) * 8 + sh]];
-                        if (ig < bi) bi = ig;
-                    }
-                }
-            }
+        while (c0 | c1) {
+            const bool f = c0 == 0;
+            const uint64_t c = f ? c1 : c0;
+            const int p = __builtin_ctzll(c);
+            if (f)
+                c1 = c & (c - 1);
+            else
+                c0 = c & (c - 1);
+            const int sh = p & 7, a = nb - 1 - (p >> 3);
+            o.take(torus_image<S>(z, sh, a * B, f, B, N, (S)gv.rep_unit, full), ci * 128 + (f ? 64 : 0) + a * 8 + sh,
+                   t);
         }
     }
-    gm = bi;
-    return best;
+    gm = o.element(t);
+    mult = o.mult;
+    return o.best;
 }
 
 // Representative test for a full torus product (gv.lut == 1), or one times cosets
@@ -475,7 +471,7 @@ __device__ inline bool rep_stab_lut(S x, const GroupView &gv, const GroupLds &t,
     stab_hi = 0;
     for (int ci = 0; ci < n_cos; ++ci) {
         const uint8_t *ct = gv.lut == 4 ? t.cos + ci * 128 : t.lut + 512;
-        const S z = ci ? coset_image<S>(x, ci, gv, t, perm_lds) : x;
+        const S z = ci ? coset_image<S>(x, ci, gv, perm_lds) : x;
         for (int j = 0; j < nb; ++j) {
             const unsigned v0 = (unsigned)(z >> (j * B)) & mB;
             const int a = nb - 1 - j;
@@ -503,49 +499,6 @@ __device__ inline bool rep_stab_lut(S x, const GroupView &gv, const GroupLds &t,
     return true;
 }
 
-// orbit_min for a ring group (gv.lut == 2): ring_windows finds the smallest
-// top byte over the rotations (and complements) and the lane's candidate
-// positions; full images are taken of the candidates only. Same result and
-// same gm as orbit_min.
-template <class S>
-__host__ __device__ inline unsigned ring_windows(S y, int N, bool hf, uint64_t &c0, uint64_t &c1);
-
-template <class S>
-__device__ inline S orbit_min_ring(S x, const GroupView &gv, const GroupLds &t, int &gm, int &mult) {
-    const int N = gv.n_sites;
-    const S full = (S)gv.full;
-    const bool hf = gv.lut_flip != 0;
-    uint64_t c0, c1;
-    ring_windows<S>(x, N, hf, c0, c1);
-    S best = 0;
-    int bi = -1;
-    mult = 0;
-    for (int f = 0; f < (hf ? 2 : 1); ++f) {
-        uint64_t c = f ? c1 : c0;
-        while (c) {
-            const int p = __builtin_ctzll(c);
-            c &= c - 1;
-            int s = N - 8 - p;
-            if (s < 0) s += N;
-            // rotation by s (complemented under f) in registers; the element
-            // tables are read only for a new or tied minimum
-            S y = rotl_ring<S>(x, s, N, full);
-            if (f) y ^= full;
-            if (bi < 0 || y < best) {
-                best = y;
-                bi = t.inv[t.lut[512 + f * 64 + s]];
-                mult = 1;
-            } else if (y == best) {
-                ++mult;
-                const int ig = t.inv[t.lut[512 + f * 64 + s]];
-                if (ig < bi) bi = ig;
-            }
-        }
-    }
-    gm = bi;
-    return best;
-}
-
 // Window scan of the ring orbit minimum: the smallest top byte over the
 // rotations of y (and their complements when hf) and the window positions p
 // that reach it (c0: plain, c1: complemented). The top 8 bits of rotation s
@@ -554,17 +507,20 @@ __device__ inline S orbit_min_ring(S x, const GroupView &gv, const GroupLds &t, 
 // bit-sliced from the top bit down: at bit i the candidates whose window bit
 // is 0 (complemented: 1) survive if there are any, else bit i of the minimum
 // is 1 and every candidate stays.
+// Narrow states rotate within N <= 32 bits instead, in 32-bit words.
 template <class S>
-__host__ __device__ inline unsigned ring_windows(S y, int N, bool hf, uint64_t &c0, uint64_t &c1) {
-    const uint64_t yy = (uint64_t)y | ((uint64_t)y << N);  // 8 <= N <= 56: bits p + i < 64
-    const uint64_t all = (1ull << N) - 1ull;
-    uint64_t a = all, b = hf ? all : 0ull;
+__host__ __device__ __forceinline__ unsigned ring_candidates(S y, int N, bool hf, S &c0, S &c1) {
+    constexpr bool narrow = sizeof(S) == 4;
+    const uint64_t yy = narrow ? 0 : (uint64_t)y | ((uint64_t)y << N);  // 8 <= N <= 56: bits p + i < 64
+    const S all = (S)((N == 32 && narrow) ? ~(S)0 : (((S)1 << N) - 1));
+    S a = all, b = hf ? all : (S)0;
     unsigned tmin = 0;
 #pragma unroll
     for (int i = 7; i >= 0; --i) {
-        const uint64_t bi = yy >> i;
-        const uint64_t z0 = a & ~bi, z1 = b & bi;
-        const bool any = (z0 | z1) != 0ull;
+        // bit p: site p + i (mod N)
+        const S bi = narrow ? (i ? (S)((y >> i) | (y << (N - i))) : y) : (S)(yy >> i);
+        const S z0 = a & ~bi, z1 = b & bi;
+        const bool any = (z0 | z1) != 0;
         a = any ? z0 : a;
         b = any ? z1 : b;
         tmin |= any ? 0u : (1u << i);
@@ -574,62 +530,64 @@ __host__ __device__ inline unsigned ring_windows(S y, int N, bool hf, uint64_t &
     return tmin;
 }
 
-// orbit_min for ring rotations times cosets (gv.lut == 3): the orbit is the
-// union of the ring orbits of y_i = c_i x. Each coset's window scan gives its
-// smallest top byte; only cosets reaching the smallest so far take full images
-// of their candidate rotations. Same result and same gm as orbit_min.
+// ring_candidates with 64-bit masks.
 template <class S>
-__device__ inline S orbit_min_coset(S x, const GroupView &gv, const GroupLds &t, const uint8_t *perm_lds,
-                                    int &gm, int &mult) {
+__host__ __device__ inline unsigned ring_windows(S y, int N, bool hf, uint64_t &c0, uint64_t &c1) {
+    S a, b;
+    const unsigned t = ring_candidates<S>(y, N, hf, a, b);
+    c0 = a;
+    c1 = b;
+    return t;
+}
+
+// orbit_min for a ring group (gv.lut == 2), or ring rotations times cosets (gv.lut
+// == 3: the orbit is the union of the ring orbits of the images c_i x):
+// ring_candidates finds the smallest top byte over the rotations (and
+// complements) and its positions; only cosets reaching the smallest so far take
+// full images of their candidates. Same result and same gm as orbit_min.
+template <class S>
+__device__ __forceinline__ S orbit_min_ring(S x, const GroupView &gv, const OrbitLds &t, const uint8_t *perm_lds, bool cosets,
+                                   int &gm, int &mult) {
     const int N = gv.n_sites;
     const S full = (S)gv.full;
     const bool hf = gv.lut_flip != 0;
-    S best = 0;
-    int bi = -1;
-    mult = 0;
+    OrbitBest<S> o;
     unsigned tbest = 0x1FFu;
-    for (int ci = 0; ci < gv.n_cos; ++ci) {
-        const uint8_t *ct = t.cos + ci * 128;
-        const S y = ci ? coset_image<S>(x, ci, gv, t, perm_lds) : x;
-        uint64_t c0, c1;
-        const unsigned tmin = ring_windows<S>(y, N, hf, c0, c1);
+    for (int ci = 0; ci < (cosets ? gv.n_cos : 1); ++ci) {
+        const S z = ci ? coset_image<S>(x, ci, gv, perm_lds) : x;
+        S c0, c1;
+        const unsigned tmin = ring_candidates<S>(z, N, hf, c0, c1);
         if (tmin > tbest) continue;
         tbest = tmin;
-        for (int f = 0; f < (hf ? 2 : 1); ++f) {
-            uint64_t c = f ? c1 : c0;
-            while (c) {
-                const int p = __builtin_ctzll(c);
-                c &= c - 1;
-                int s = N - 8 - p;
-                if (s < 0) s += N;
-                const int g = ct[f * 64 + s];
-                S z = rotl_ring<S>(y, s, N, full);
-                if (f) z ^= full;
-                const int ig = t.inv[g];
-                if (bi < 0 || z < best) {
-                    best = z;
-                    bi = ig;
-                    mult = 1;
-                } else if (z == best) {
-                    ++mult;
-                    if (ig < bi) bi = ig;
-                }
-            }
+        while (c0 | c1) {
+            const bool f = c0 == 0;
+            const S c = f ? c1 : c0;
+            const int p = ctz_s(c);
+            if (f)
+                c1 = c & (c - 1);
+            else
+                c0 = c & (c - 1);
+            int s = N - 8 - p;
+            s += s < 0 ? N : 0;
+            const S y = rotl_ring<S>(z, s, N, full);
+            o.take(f ? (S)(y ^ full) : y, ci * 128 + (f ? 64 : 0) + s, t);
         }
     }
-    gm = bi;
-    return best;
+    gm = o.element(t);
+    mult = o.mult;
+    return o.best;
 }
 
-// The orbit minimum by the group's form (GroupView::lut).
-template <class S>
-__device__ inline S orbit_min_any(S x, const GroupView &gv, const GroupLds &t, const uint8_t *perm_lds, int &gm,
+// The orbit minimum by the group's form: LUT = GroupView::lut where the kernel
+// is built for it (its registers and LDS then serve that form alone), -1 for
+// the form that the view names.
+template <class S, int LUT = -1>
+__device__ __forceinline__ S orbit_min_any(S x, const GroupView &gv, const OrbitLds &t, const uint8_t *perm_lds, int &gm,
                                   int &mult) {
-    return gv.lut == 1   ? orbit_min_lut<S>(x, gv, t, gm, mult)
-           : gv.lut == 2 ? orbit_min_ring<S>(x, gv, t, gm, mult)
-           : gv.lut == 3 ? orbit_min_coset<S>(x, gv, t, perm_lds, gm, mult)
-           : gv.lut == 4 ? orbit_min_torus_coset<S>(x, gv, t, perm_lds, gm, mult)
-                         : orbit_min<S>(x, gv, perm_lds, gm, mult);
+    const int lut = LUT < 0 ? gv.lut : LUT;
+    if (lut == 1 || lut == 4) return orbit_min_torus<S>(x, gv, t, perm_lds, lut == 4, gm, mult);
+    if (lut == 2 || lut == 3) return orbit_min_ring<S>(x, gv, t, perm_lds, lut == 3, gm, mult);
+    return orbit_min<S>(x, gv, perm_lds, gm, mult);
 }
 
 // Colex rank by nibbles: T[(k * n_c + c) * 16 + v] is the rank contribution of
@@ -637,8 +595,8 @@ __device__ inline S orbit_min_any(S x, const GroupView &gv, const GroupLds &t, c
 // over v's set bits i (ascending, j of v's bits below i) of C(4k + i, c + j + 1).
 // ceil(n_sites / 4) table reads instead of one per set bit; same value as
 // colex_rank for every state with at most n_c - 1 set bits.
-template <class S>
-__host__ __device__ inline int64_t colex_rank_nib(S x, const uint64_t *tab, int n_nib, int n_c) {
+template <class S, class T>
+__host__ __device__ __forceinline__ int64_t colex_rank_nib(S x, const T *tab, int n_nib, int n_c) {
     int64_t r = 0;
     int c = 0;
     for (int k = 0; k < n_nib; ++k) {
@@ -681,7 +639,7 @@ inline std::vector<uint64_t> rank_nibble_table(int n_sites, int n_up, int &n_nib
 // Row of a representative through the rank dictionary (rank -> record -> rows
 // before the word + popcount of the lower bits). Returns -1 when the
 // representative is not a row.
-__device__ inline int64_t row_of_rank(int64_t rk, const uint64_t *dict) {
+__device__ __forceinline__ int64_t row_of_rank(int64_t rk, const uint64_t *dict) {
     const ulonglong2 rec = reinterpret_cast<const ulonglong2 *>(dict)[rk >> 6];
     const uint64_t w = rec.x;
     const int b = (int)(rk & 63);

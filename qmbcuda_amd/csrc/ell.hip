@@ -22,10 +22,8 @@
 
 namespace qmb {
 
-// 8 waves per block share the staged tables (rank, group, characters), so more
-// waves fit a CU's LDS than with 4-wave blocks (6x6 ELL build: 145 ms with
-// 4-wave blocks and the binomial rank loop, 131 ms with 8-wave blocks and the
-// nibble rank table)
+// 8 waves per block share the staged tables (rank, group, terms), so more waves
+// fit a CU's LDS than with 4-wave blocks (6x6 ELL build: 80 ms, 4 waves 88 ms).
 constexpr int kEllThreads = 512;
 
 // Lanes per row (2^ts, at most 2^kMaxSplit) while rows x lanes stay within this
@@ -77,41 +75,74 @@ struct CodeView {
     int *bad = nullptr;              // set when a stabiliser size has no class
 };
 
-// Rank tables in dynamic LDS: the nibble table (rank_tab, n_nib > 0) when it
-// fits, else the binomial table (binom). CODED (fill only): codes instead of
-// values (CodeView). SPLIT: 2^ts neighbouring lanes share a row. Each applies all
-// terms (pass A), then takes every 2^ts-th candidate; a round's surviving
-// candidates find their slots in term order from a ballot. A row is a chain of
-// one lookup per acting term, which only many rows hide.
-template <class S, bool FILL, bool CPLX, bool CODED = false, bool SPLIT = false>
-__global__ __launch_bounds__(kEllThreads) void ell_rows(GroupView gv, const uint64_t *binom,
+// An off-diagonal term as the fill's lookups read it, from LDS: a lane's next
+// candidate is any term. vcode = the term's part of the value code.
+template <class S>
+struct OffTerm {
+    S set, set_val, sz;
+    S vcode;
+};
+constexpr size_t kMaxOffBytes = 8 * 1024;  // beyond: the compiled terms in memory
+
+// Rows of the matrix: their lengths (count), then their entries (FILL). Terms that
+// change the state come first in the table: pass A tests 64 of them (uniform
+// loads, four instructions each) and marks the lane's candidates, pass B takes
+// each lane's candidates in term order, so every round of the orbit lookup, the
+// expensive part, keeps almost all lanes busy. The diagonal terms are added in
+// table order. Rank tables in dynamic LDS: the nibble table (rank_tab, n_nib >
+// 0) when it fits, else the binomial table (binom), in 32 bits for narrow states;
+// then the off-diagonal terms (n_lds of them). CODED (fill only): codes instead
+// of values (CodeView). LUT: the group's form, or -1 (orbit_min_any). SPLIT: 2^ts
+// neighbouring lanes share a row: each takes every 2^ts-th candidate, and a
+// round's surviving candidates find their slots in term order from a ballot. A
+// row is a chain of one lookup per acting term, which only many rows hide.
+// Bound by VALU and LDS work (28-site J1-J2 ring, 716,728 rows: fill 226 us, count
+// 18 us; 6x6: 63 and 2.1 ms; when the passes applied every term through its full
+// record, read candidates' terms from memory and looked images up per block, flip
+// and element: 300 and 95 us, 94 and 11.5 ms). One lane a row is held to the
+// registers of 8 wavefronts a SIMD (6x6 build 80 ms; 86 ms with 7).
+template <class S, bool FILL, bool CPLX, bool CODED, bool SPLIT, int LUT>
+__global__ __launch_bounds__(kEllThreads, SPLIT ? 1 : 8) void ell_rows(GroupView gv, const uint64_t *binom,
                                                         const uint64_t *rank_tab, int n_nib, int n_c, int layout,
                                                         int64_t n_rows, const uint64_t *reps, const uint8_t *stab,
                                                         const uint8_t *nullf, const uint64_t *dict,
-                                                        TermsView tv, const double2 *chi,
+                                                        TermsView tv, int n_lds, const double2 *chi,
                                                         const double *nrm, int W, uint16_t *row_len, int *err,
                                                         int all_rows, const int64_t *chunk_ptr, int32_t *col,
                                                         double *val, CodeView cv, int ts) {
-    extern __shared__ uint64_t rank_lds[];
-    __shared__ alignas(8) uint8_t perm_lds[kMaxGroup * 64];
-    __shared__ double2 s_chi[kMaxGroup];
-    __shared__ double s_nrm[kMaxGroup + 1];
-    __shared__ GroupLds gt;
+    using R = typename RankOf<S>::T;
+    constexpr bool kPerm = LUT != 1 && LUT != 2;  // images by tables
+    constexpr bool kValues = FILL && !CODED;
+    extern __shared__ __align__(16) uint64_t rank_dyn[];
+    __shared__ alignas(8) uint8_t perm_lds[kPerm ? kMaxGroup * 64 : 8];
+    __shared__ double2 s_chi[kValues ? kMaxGroup : 1];
+    __shared__ double s_nrm[kValues ? kMaxGroup + 1 : 1];
+    __shared__ OrbitLds gt;
     __shared__ uint16_t s_xcls[CODED ? kMaxGroup : 1];
     __shared__ uint8_t s_mcls[CODED ? kMaxGroup + 1 : 1];
+    R *rank_lds = reinterpret_cast<R *>(rank_dyn);
+    const int n_rank = n_nib ? n_nib * n_c * 16 : (int)sizeof(S) * 8 * kBinJ;
+    OffTerm<S> *off = reinterpret_cast<OffTerm<S> *>(rank_lds + (n_rank + 3) / 4 * 4);
     // the count pass over a sector without null orbits needs no orbit lookups
     // (row length = 1 + the acting off-diagonal terms): no tables to stage
     const bool lookups = FILL || !all_rows;
     if (lookups) {
-        stage_images<S>(perm_lds, gv);
-        stage_group(gt, gv);
+        if (kPerm) stage_images<S>(perm_lds, gv);
+        stage_orbit(gt, gv);
         if (n_nib) {
-            for (int i = threadIdx.x; i < n_nib * n_c * 16; i += blockDim.x) rank_lds[i] = rank_tab[i];
+            for (int i = threadIdx.x; i < n_rank; i += blockDim.x) rank_lds[i] = (R)rank_tab[i];
         } else {
-            stage_binom(rank_lds, binom);
+            stage_binom_rows<S>(rank_lds, binom, gv.n_sites);
         }
-        for (int i = threadIdx.x; i < gv.G; i += blockDim.x) s_chi[i] = chi[i];
-        for (int i = threadIdx.x; i <= gv.G; i += blockDim.x) s_nrm[i] = nrm[i];
+        for (int i = threadIdx.x; i < n_lds; i += blockDim.x) {
+            const TermC &tm = tv.t[i];
+            off[i] = OffTerm<S>{(S)tm.set, (S)tm.set_val, (S)tm.sz,
+                                (S)((int)tm.vclass * 2 * cv.n_chi * cv.n_m * cv.n_m)};
+        }
+        if (kValues) {
+            for (int i = threadIdx.x; i < gv.G; i += blockDim.x) s_chi[i] = chi[i];
+            for (int i = threadIdx.x; i <= gv.G; i += blockDim.x) s_nrm[i] = nrm[i];
+        }
         if (CODED) {
             for (int i = threadIdx.x; i < gv.G; i += blockDim.x) s_xcls[i] = cv.xcls[i];
             for (int i = threadIdx.x; i <= kMaxGroup; i += blockDim.x) s_mcls[i] = cv.mcls[i];
@@ -136,58 +167,68 @@ __global__ __launch_bounds__(kEllThreads) void ell_rows(GroupView gv, const uint
     if (!null_row) {
         const S src = (S)reps[r];
         const int m_src = FILL ? (int)stab[r] : 0;
-        const double n_src = FILL ? s_nrm[m_src] : 0.0;
-        // Terms are taken 64 at a time. Pass A applies the operators (cheap bit
-        // tests, wave-uniform term index), adds diagonal terms in term order and
-        // marks the lane's off-diagonal candidates; pass B pops each lane's
-        // candidates in term order, so every iteration of the expensive orbit
-        // lookup keeps almost all lanes busy.
-        for (int h0 = 0; h0 < tv.n_terms; h0 += 64) {
-            const int h1 = min(h0 + 64, tv.n_terms);
-            uint64_t cand = 0;
-            for (int h = h0; h < h1; ++h) {
-                double cr, ci;
-                S tgt;
-                if (!apply_term<S>(tv, h, src, tgt, cr, ci)) continue;
-                if (tgt == src) {
-                    dr += cr;
-                    di += ci;
-                    continue;
-                }
-                cand |= 1ULL << (h - h0);
+        const double n_src = kValues ? s_nrm[m_src] : 0.0;
+        const int cs = CODED ? (int)s_mcls[m_src] : 0;
+        if (FILL) {
+            for (int h = tv.n_off; h < tv.n_terms; ++h) {
+                const TermC &tm = tv.t[h];
+                if ((src & (S)tm.req) != (S)tm.req_val) continue;
+                const bool neg = (popc_s((S)(~src & (S)tm.sz)) & 1) != 0;
+                dr += neg ? -tm.coef.x : tm.coef.x;
+                if (CPLX) di += neg ? -tm.coef.y : tm.coef.y;
             }
+        }
+        for (int h0 = 0; h0 < tv.n_off; h0 += 64) {
+            const int nh = min(64, tv.n_off - h0);
+            const ulonglong2 *ts_ = tv.tests + h0;
             if (!FILL && all_rows) {
                 // every orbit is a row (no null orbits for this irrep): the row
                 // length needs no orbit lookup
-                slot += __popcll(cand);
+#pragma unroll 8
+                for (int h = 0; h < nh; ++h) slot += (src & (S)ts_[h].x) == (S)ts_[h].y ? 1 : 0;
                 continue;
             }
-            // one candidate: its row (-1: none) and, when it has one, its entry at slot `at`
-            auto lookup = [&](int h, int &gm, int &mult, double &cr, double &ci) -> int64_t {
+            uint32_t lo = 0, hi = 0;
+#pragma unroll 8
+            for (int h = 0; h < min(32, nh); ++h) lo |= (src & (S)ts_[h].x) == (S)ts_[h].y ? 1u << h : 0u;
+#pragma unroll 8
+            for (int h = 32; h < nh; ++h) hi |= (src & (S)ts_[h].x) == (S)ts_[h].y ? 1u << (h - 32) : 0u;
+            uint64_t cand = (uint64_t)hi << 32 | lo;
+            // one candidate: its row (-1: none)
+            auto lookup = [&](int h, int &gm, int &mult, int &vcode) __attribute__((always_inline)) -> int64_t {
                 S tgt;
-                apply_term<S>(tv, h, src, tgt, cr, ci);
-                const S rep = orbit_min_any<S>(tgt, gv, gt, perm_lds, gm, mult);
+                if (h < n_lds) {
+                    const OffTerm<S> o = off[h];
+                    tgt = (S)((src & (S)~o.set) | o.set_val);
+                    if (CODED) vcode = (int)o.vcode + (popc_s((S)(~src & o.sz)) & 1) * cv.n_chi * cv.n_m * cv.n_m;
+                } else {
+                    const TermC &tm = tv.t[h];
+                    tgt = (S)((src & (S)~(S)tm.set) | (S)tm.set_val);
+                    if (CODED)
+                        vcode = ((int)tm.vclass * 2 + (popc_s((S)(~src & (S)tm.sz)) & 1)) * cv.n_chi * cv.n_m * cv.n_m;
+                }
+                const S rep = orbit_min_any<S, LUT>(tgt, gv, gt, perm_lds, gm, mult);
                 const int64_t r2 = row_of_rank(
                     n_nib ? colex_rank_nib<S>(rep, rank_lds, n_nib, n_c) : colex_rank<S>(rep, rank_lds), dict);
                 if (r2 >= 0 && layout == QMB_LAYOUT_REFERENCE && nullf[r2]) return -1;
                 return r2;
             };
-            auto write = [&](int at, int h, int64_t r2, int gm, int mult, double cr, double ci) {
+            // its entry at slot `at`
+            auto write = [&](int at, int h, int64_t r2, int gm, int mult, int vcode) __attribute__((always_inline)) {
                 if (!FILL || at >= L) return;
                 const int64_t pos = base + (int64_t)at * kChunk + lane;
                 col[pos] = (int32_t)r2;
                 if (CODED) {
-                    const TermC &tm = tv.t[h];
-                    const int neg = popc_s((S)(~src & (S)tm.sz)) & 1;
-                    const int cs = s_mcls[m_src], ct = s_mcls[mult];
+                    const int ct = s_mcls[mult];
                     const bool ok = cs != 0xFF && ct != 0xFF;
                     if (!ok) *cv.bad = 1;
-                    const int code =
-                        ok ? ((((int)tm.vclass * 2 + neg) * cv.n_chi + s_xcls[gm]) * cv.n_m + cs) * cv.n_m + ct : 0;
-                    cv.code[pos] = (uint16_t)code;
+                    cv.code[pos] = (uint16_t)(ok ? vcode + ((int)s_xcls[gm] * cv.n_m + cs) * cv.n_m + ct : 0);
                 } else {
                     // mult = the target row's stabiliser size (no read of stab[r2]);
                     // equal sizes give the ratio 1 exactly
+                    const TermC &tm = tv.t[h];
+                    const bool neg = (popc_s((S)(~src & (S)tm.sz)) & 1) != 0;
+                    const double cr = neg ? -tm.coef.x : tm.coef.x, ci = neg ? -tm.coef.y : tm.coef.y;
                     const double ratio = mult == m_src ? 1.0 : s_nrm[mult] / n_src;
                     const double2 x = s_chi[gm];
                     const double pr = cr * x.x - ci * x.y;
@@ -204,15 +245,14 @@ __global__ __launch_bounds__(kEllThreads) void ell_rows(GroupView gv, const uint
                 const int nc = __popcll(cand);
                 for (int k0 = 0; k0 < nc; k0 += split) {  // the same rounds for the lanes of a row
                     int64_t r2 = -1;
-                    int h = 0, gm = 0, mult = 0;
-                    double cr = 0.0, ci = 0.0;
+                    int h = 0, gm = 0, mult = 0, vcode = 0;
                     if (k0 + sub < nc) {
                         h = h0 + select_bit(cand, k0 + sub);
-                        r2 = lookup(h, gm, mult, cr, ci);
+                        r2 = lookup(h, gm, mult, vcode);
                     }
                     const uint64_t found =
                         (__ballot(r2 >= 0) >> ((threadIdx.x & 63) - sub)) & ((1ULL << split) - 1ULL);
-                    if (r2 >= 0) write(slot + __popcll(found & ((1ULL << sub) - 1ULL)), h, r2, gm, mult, cr, ci);
+                    if (r2 >= 0) write(slot + __popcll(found & ((1ULL << sub) - 1ULL)), h, r2, gm, mult, vcode);
                     slot += __popcll(found);
                 }
                 continue;
@@ -220,11 +260,10 @@ __global__ __launch_bounds__(kEllThreads) void ell_rows(GroupView gv, const uint
             while (cand) {
                 const int h = h0 + __builtin_ctzll(cand);
                 cand &= cand - 1;
-                int gm, mult;
-                double cr, ci;
-                const int64_t r2 = lookup(h, gm, mult, cr, ci);
+                int gm, mult, vcode = 0;
+                const int64_t r2 = lookup(h, gm, mult, vcode);
                 if (r2 < 0) continue;
-                write(slot, h, r2, gm, mult, cr, ci);
+                write(slot, h, r2, gm, mult, vcode);
                 ++slot;
             }
         }
@@ -271,6 +310,42 @@ __global__ __launch_bounds__(kEllThreads) void ell_rows(GroupView gv, const uint
             val[pos] = 0.0;
         }
     }
+}
+
+using EllRows = decltype(&ell_rows<uint32_t, false, false, false, false, -1>);
+
+// The count does not depend on the values. One lane a row (the large sectors) is
+// built for the torus product and the ring, everything else for any group.
+static EllRows ell_count_kernel(bool narrow, bool split, int lut) {
+    static const EllRows any[2][2] = {
+        {ell_rows<uint64_t, false, false, false, false, -1>, ell_rows<uint64_t, false, false, false, true, -1>},
+        {ell_rows<uint32_t, false, false, false, false, -1>, ell_rows<uint32_t, false, false, false, true, -1>}};
+    static const EllRows one[2][2] = {
+        {ell_rows<uint64_t, false, false, false, false, 1>, ell_rows<uint64_t, false, false, false, false, 2>},
+        {ell_rows<uint32_t, false, false, false, false, 1>, ell_rows<uint32_t, false, false, false, false, 2>}};
+    if (!split && (lut == 1 || lut == 2)) return one[narrow][lut - 1];
+    return any[narrow][split];
+}
+
+static EllRows ell_fill_kernel(bool narrow, bool cplx, bool coded, bool split, int lut) {
+    // [narrow][complex][coded][split]
+    static const EllRows any[2][2][2][2] = {
+        {{{ell_rows<uint64_t, true, false, false, false, -1>, ell_rows<uint64_t, true, false, false, true, -1>},
+          {ell_rows<uint64_t, true, false, true, false, -1>, ell_rows<uint64_t, true, false, true, true, -1>}},
+         {{ell_rows<uint64_t, true, true, false, false, -1>, ell_rows<uint64_t, true, true, false, true, -1>},
+          {ell_rows<uint64_t, true, true, true, false, -1>, ell_rows<uint64_t, true, true, true, true, -1>}}},
+        {{{ell_rows<uint32_t, true, false, false, false, -1>, ell_rows<uint32_t, true, false, false, true, -1>},
+          {ell_rows<uint32_t, true, false, true, false, -1>, ell_rows<uint32_t, true, false, true, true, -1>}},
+         {{ell_rows<uint32_t, true, true, false, false, -1>, ell_rows<uint32_t, true, true, false, true, -1>},
+          {ell_rows<uint32_t, true, true, true, false, -1>, ell_rows<uint32_t, true, true, true, true, -1>}}}};
+    // [narrow][complex][torus product, ring], coded, one lane a row
+    static const EllRows one[2][2][2] = {
+        {{ell_rows<uint64_t, true, false, true, false, 1>, ell_rows<uint64_t, true, false, true, false, 2>},
+         {ell_rows<uint64_t, true, true, true, false, 1>, ell_rows<uint64_t, true, true, true, false, 2>}},
+        {{ell_rows<uint32_t, true, false, true, false, 1>, ell_rows<uint32_t, true, false, true, false, 2>},
+         {ell_rows<uint32_t, true, true, true, false, 1>, ell_rows<uint32_t, true, true, true, false, 2>}}};
+    if (coded && !split && (lut == 1 || lut == 2)) return one[narrow][cplx][lut - 1];
+    return any[narrow][cplx][coded][split];
 }
 
 // Padding entries of the rows past n_rows in the last chunk.
@@ -870,8 +945,10 @@ struct RankTables {
     static constexpr size_t kMaxBytes = 48 * 1024;
     DevBuf buf;
     int n_nib = 0, n_c = 0;
-    size_t lds_bytes = 64 * kBinJ * sizeof(uint64_t);
+    size_t lds_bytes = 0;
     explicit RankTables(const qmb_basis &b) {
+        const bool narrow = b.n_sites <= 32;
+        lds_bytes = narrow ? 32 * kBinJ * sizeof(uint32_t) : 64 * kBinJ * sizeof(uint64_t);
         int nn = 0, nc = 0;
         const std::vector<uint64_t> t = rank_nibble_table(b.n_sites, b.n_up, nn, nc);
         const size_t bytes = t.size() * sizeof(uint64_t);
@@ -880,7 +957,7 @@ struct RankTables {
         QMB_HIP(hipMemcpy(buf.p, t.data(), bytes, hipMemcpyHostToDevice));
         n_nib = nn;
         n_c = nc;
-        lds_bytes = bytes;
+        lds_bytes = narrow ? bytes / 2 : bytes;
     }
     const uint64_t *tab() const { return n_nib ? buf.as<uint64_t>() : nullptr; }
 };
@@ -922,7 +999,7 @@ qmb_status qmb_ell_build(qmb_ctx *ctx, const qmb_basis *b, const qmb_terms *t, i
         e->n_chunks = (b->n_rows + kChunk - 1) / kChunk;
         // term table and irrep data on device
         const std::vector<int> order = locality ? locality_order(*t) : std::vector<int>();
-        const DeviceTerms dt(*t, ch, g->G, locality ? &order : nullptr);
+        const DeviceTerms dt(*t, ch, g->G, locality ? &order : nullptr, true);
         const TermsView tv = dt.view;
         DevBuf d_err(sizeof(int));
         QMB_HIP(hipMemsetAsync(d_err.p, 0, sizeof(int), ctx->stream));
@@ -939,19 +1016,18 @@ qmb_status qmb_ell_build(qmb_ctx *ctx, const qmb_basis *b, const qmb_terms *t, i
         };
         const bool cplx = value_type == QMB_COMPLEX;
         const bool narrow = b->n_sites <= 32;
-        using K = decltype(&ell_rows<uint32_t, false, false>);
+        const size_t off_bytes = (size_t)tv.n_off * (narrow ? sizeof(OffTerm<uint32_t>) : sizeof(OffTerm<uint64_t>));
+        const int n_lds = off_bytes <= kMaxOffBytes ? tv.n_off : 0;
+        const size_t lds_bytes = (rank.lds_bytes + 15) / 16 * 16 + (n_lds ? off_bytes : 0);
         if (n > 0) {
             const int cts = b->all_rows ? 0 : ts;
-            // [64-bit states][complex][split]; the count does not depend on the values
-            static const K counts[2][2] = {{ell_rows<uint32_t, false, false>, ell_rows<uint32_t, false, false, false, true>},
-                                           {ell_rows<uint64_t, false, false>, ell_rows<uint64_t, false, false, false, true>}};
-            const K kcount = counts[narrow ? 0 : 1][cts ? 1 : 0];
+            const EllRows kcount = ell_count_kernel(narrow, cts != 0, gv.lut);
             // the count pass of a sector without null orbits makes no orbit lookups
-            hipLaunchKernelGGL(kcount, dim3(blocks_for(cts)), dim3(kEllThreads), b->all_rows ? 0 : rank.lds_bytes,
+            hipLaunchKernelGGL(kcount, dim3(blocks_for(cts)), dim3(kEllThreads), b->all_rows ? 0 : lds_bytes,
                                ctx->stream, gv, ctx->binom.as<uint64_t>(), rank.tab(), rank.n_nib, rank.n_c,
                                b->layout, n, b->reps.as<uint64_t>(),
                                b->stab.as<uint8_t>(), b->nullf.as<uint8_t>(), b->dict.as<uint64_t>(),
-                               tv, dt.chi, dt.nrm, W,
+                               tv, n_lds, dt.chi, dt.nrm, W,
                                e->row_len.as<uint16_t>(), d_err.as<int>(), b->all_rows ? 1 : 0, nullptr, nullptr,
                                nullptr, CodeView{}, cts);
             QMB_HIP(hipGetLastError());
@@ -971,23 +1047,13 @@ qmb_status qmb_ell_build(qmb_ctx *ctx, const qmb_basis *b, const qmb_terms *t, i
         const bool coded = vp.on && vp.plan_codes(ctx, *e, *b, dt, ch, g->G);
         // the fill (coded, or with FP64 values) and the padding of the last chunk
         auto fill = [&](bool with_codes) {
-            // [64-bit states][complex][coded][split]
-            static const K fills[2][2][2][2] = {
-                {{{ell_rows<uint32_t, true, false>, ell_rows<uint32_t, true, false, false, true>},
-                  {ell_rows<uint32_t, true, false, true>, ell_rows<uint32_t, true, false, true, true>}},
-                 {{ell_rows<uint32_t, true, true>, ell_rows<uint32_t, true, true, false, true>},
-                  {ell_rows<uint32_t, true, true, true>, ell_rows<uint32_t, true, true, true, true>}}},
-                {{{ell_rows<uint64_t, true, false>, ell_rows<uint64_t, true, false, false, true>},
-                  {ell_rows<uint64_t, true, false, true>, ell_rows<uint64_t, true, false, true, true>}},
-                 {{ell_rows<uint64_t, true, true>, ell_rows<uint64_t, true, true, false, true>},
-                  {ell_rows<uint64_t, true, true, true>, ell_rows<uint64_t, true, true, true, true>}}}};
-            const K kfill = fills[narrow ? 0 : 1][cplx ? 1 : 0][with_codes ? 1 : 0][ts ? 1 : 0];
+            const EllRows kfill = ell_fill_kernel(narrow, cplx, with_codes, ts != 0, gv.lut);
             double *val = with_codes ? nullptr : e->val.as<double>();
-            hipLaunchKernelGGL(kfill, dim3(blocks_for(ts)), dim3(kEllThreads), rank.lds_bytes, ctx->stream, gv,
+            hipLaunchKernelGGL(kfill, dim3(blocks_for(ts)), dim3(kEllThreads), lds_bytes, ctx->stream, gv,
                                ctx->binom.as<uint64_t>(), rank.tab(), rank.n_nib, rank.n_c, b->layout, n,
                                b->reps.as<uint64_t>(),
                                b->stab.as<uint8_t>(), b->nullf.as<uint8_t>(), b->dict.as<uint64_t>(),
-                               tv, dt.chi, dt.nrm, W,
+                               tv, n_lds, dt.chi, dt.nrm, W,
                                e->row_len.as<uint16_t>(), d_err.as<int>(), 0, e->chunk_ptr.as<int64_t>(),
                                e->col.as<int32_t>(), val, with_codes ? vp.cv : CodeView{}, ts);
             QMB_HIP(hipGetLastError());

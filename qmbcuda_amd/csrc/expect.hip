@@ -48,12 +48,12 @@ __global__ __launch_bounds__(kExpThreads) void expect_rows(GroupView gv, const u
     __shared__ typename RankOf<S>::T bin[sizeof(S) * 8 * kBinJ];
     __shared__ double2 s_chi[kMaxGroup];
     __shared__ double s_nrm[kMaxGroup + 1];
-    __shared__ GroupLds gt;
+    __shared__ OrbitLds gt;
     __shared__ double red[kWaves];
     __shared__ alignas(8) uint8_t img_lds[4096];  // coset representatives' images (stage_images)
     stage_perm(perm_lds, gv);
     if (gv.lut >= 3) stage_images<S>(img_lds, gv);
-    stage_group(gt, gv);
+    stage_orbit(gt, gv);
     stage_binom_rows<S>(bin, binom, gv.n_sites);
     for (int i = threadIdx.x; i < gv.G; i += blockDim.x) s_chi[i] = chi[i];
     for (int i = threadIdx.x; i <= gv.G; i += blockDim.x) s_nrm[i] = nrm[i];

@@ -31,7 +31,17 @@ struct TermC {
 struct TermsView {
     int n_terms;
     const TermC *t;  // [n_terms]
+    // of a table sorted for the ELL passes (DeviceTerms): terms [0, n_off) change
+    // the state, the others are diagonal; tests[h] = {req, req_val} of term h < n_off
+    int n_off = 0;
+    const ulonglong2 *tests = nullptr;
 };
+
+// Whether a term that acts leaves the state as it is: every site it sets lies in
+// req (an S+ or S- reaches an unknown site once and requires its value), so
+// this does not depend on the state.
+inline bool is_diagonal(const TermC &c) { return c.set_val == (c.req_val & c.set); }
+inline bool never_acts(const TermC &c) { return (c.req_val & ~c.req) != 0; }
 
 // The term h on src. Returns false when the term annihilates src.
 template <class S>
@@ -136,20 +146,34 @@ struct DeviceTerms {
     const double *nrm = nullptr;   // [G + 1]
     static constexpr size_t kMaxClasses = 1 << 14;
     std::vector<double2> classes;  // distinct term coefficients, in order of first use (TermC::vclass)
-    DeviceTerms(const qmb_terms &t, const double *chi_row, int G, const std::vector<int> *order = nullptr) {
-        const int nt = t.n_terms;
+    // sorted: for the ELL passes, the terms that change the state first, then the
+    // diagonal ones, each in the given order, without those that never act
+    DeviceTerms(const qmb_terms &t, const double *chi_row, int G, const std::vector<int> *order = nullptr,
+                bool sorted = false) {
+        std::vector<TermC> terms(t.n_terms);
+        for (int k = 0; k < t.n_terms; ++k) terms[k] = compile_term(t, order ? (*order)[k] : k);
+        int n_off = 0;
+        if (sorted) {
+            terms.erase(std::remove_if(terms.begin(), terms.end(), never_acts), terms.end());
+            const auto mid = std::stable_partition(terms.begin(), terms.end(),
+                                                   [](const TermC &c) { return !is_diagonal(c); });
+            n_off = (int)(mid - terms.begin());
+        }
+        const int nt = (int)terms.size();
         auto up16 = [](size_t x) { return (x + 15) & ~(size_t)15; };
         const size_t o_terms = 0, o_chi = up16((size_t)std::max(1, nt) * sizeof(TermC)),
-                     o_nrm = up16(o_chi + (size_t)G * 16), total = up16(o_nrm + (size_t)(G + 1) * 8);
+                     o_nrm = up16(o_chi + (size_t)G * 16), o_tests = up16(o_nrm + (size_t)(G + 1) * 8),
+                     total = up16(o_tests + (size_t)n_off * sizeof(ulonglong2));
         std::vector<unsigned char> h(total, 0);
         TermC *tc = reinterpret_cast<TermC *>(h.data() + o_terms);
-        for (int k = 0; k < nt; ++k) tc[k] = compile_term(t, order ? (*order)[k] : k);
-        // classes of the terms that can leave the diagonal (the others never give
-        // an off-diagonal entry: no operator changes a spin, or none acts); beyond
-        // kMaxClasses the classes are not used and no longer counted
+        std::copy(terms.begin(), terms.end(), tc);
+        ulonglong2 *tests = reinterpret_cast<ulonglong2 *>(h.data() + o_tests);
+        for (int k = 0; k < n_off; ++k) tests[k] = make_ulonglong2(tc[k].req, tc[k].req_val);
+        // classes of the terms that can leave the diagonal; beyond kMaxClasses the
+        // classes are not used and no longer counted
         for (int k = 0; k < nt; ++k) {
             tc[k].vclass = 0;
-            if (tc[k].set == 0 || tc[k].req_val > tc[k].req || classes.size() > kMaxClasses) continue;
+            if (k >= n_off || classes.size() > kMaxClasses) continue;
             for (const double2 &c : classes) {
                 if (std::memcmp(&c, &tc[k].coef, sizeof(double2)) == 0) break;
                 ++tc[k].vclass;
@@ -164,7 +188,8 @@ struct DeviceTerms {
         char *d = static_cast<char *>(blob.p);
         chi = reinterpret_cast<const double2 *>(d + o_chi);
         nrm = reinterpret_cast<const double *>(d + o_nrm);
-        view = TermsView{nt, reinterpret_cast<const TermC *>(d + o_terms)};
+        view = TermsView{nt, reinterpret_cast<const TermC *>(d + o_terms), n_off,
+                         reinterpret_cast<const ulonglong2 *>(d + o_tests)};
     }
 };
 
