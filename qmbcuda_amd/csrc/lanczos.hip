@@ -33,6 +33,8 @@
 namespace qmb {
 
 constexpr int kMaxBlocks = 4096;
+constexpr int kWideWaves = 16;   // a block of the streamed SpMV
+constexpr int kWideBlocks = 256;  // one a CU
 
 // ---- K1: SELL-64 SpMV --------------------------------------------------------
 // One wavefront per 64-row chunk (row products in sell.hpp); the x gathers are
@@ -40,21 +42,29 @@ constexpr int kMaxBlocks = 4096;
 // dot: y = s (H x), phi = s x, partial sums of phi . y. PACK: the packed value
 // format (4 B per off-diagonal entry, value tables staged in LDS; complex: real
 // parts at [0, n_values), imaginary parts at kMaxValues + [0, n_values_im)).
-template <bool CPLX, bool LZ, bool PACK, bool NT>
-__global__ __launch_bounds__(kThreads) void spmv_sell(int64_t n_rows, int64_t n_chunks,
-                                                      const int64_t *__restrict__ chunk_ptr,
-                                                      const uint16_t *__restrict__ row_len,
-                                                      const int32_t *__restrict__ col,
-                                                      const double *__restrict__ val,
-                                                      const double *__restrict__ diag,
-                                                      const double *__restrict__ vtab, int n_values, int cb,
-                                                      int n_values_im, int rb,
-                                                      const double *__restrict__ x, double *__restrict__ y,
-                                                      const double *__restrict__ invb, double *__restrict__ vout,
-                                                      double *__restrict__ partials, const double *__restrict__ bpart,
-                                                      int n_bpart, double *__restrict__ beta_out,
-                                                      double *__restrict__ invb_out) {
-    __shared__ double lds[kWaves];
+//
+// WIDE: the form for a matrix larger than the memory-side cache. What bounds it is
+// the gathers: of the 128 B lines of x that a chunk's slot touches, few lie in L1
+// and many of those that miss are in no L2 either. So the words bypass the caches
+// (nontemporal), and one block of 16 wavefronts a CU takes 16 neighbouring chunks,
+// kept in step by a barrier after each group of slots: neighbouring rows gather
+// from the same lines, and the lines of the group are still in L1 when the next
+// wavefront asks. Two blocks a CU (all 32 wavefronts) are up to 7 % slower, blocks
+// of 8 between 7 % faster (complex, 23 MB vector) and 4 % slower (6x6), the same
+// blocks without the barrier 20 - 35 % slower. In a Lanczos run, with four
+// wavefronts a block and no barrier / so: 4x8 lattice (9.4 million rows, 1.5 GB of
+// words) 1456 / 1230 us, complex 5233 / 4600, 6x6 24.1 / 20.0 ms, 30 sites with J2
+// 391 / 353 us.
+template <bool CPLX, bool LZ, bool PACK, bool WIDE>
+__global__ __launch_bounds__(WIDE ? kWideWaves * 64 : kThreads, WIDE ? 4 : 1) void spmv_sell(
+    int64_t n_rows, int64_t n_chunks, const int64_t *__restrict__ chunk_ptr, const uint16_t *__restrict__ row_len,
+    const int32_t *__restrict__ col, const double *__restrict__ val, const double *__restrict__ diag,
+    const double *__restrict__ vtab, int n_values, int cb, int n_values_im, int rb, const double *__restrict__ x,
+    double *__restrict__ y, const double *__restrict__ invb, double *__restrict__ vout,
+    double *__restrict__ partials, const double *__restrict__ bpart, int n_bpart, double *__restrict__ beta_out,
+    double *__restrict__ invb_out, int xcd) {
+    constexpr int NW = WIDE ? kWideWaves : kWaves;
+    __shared__ double lds[NW];
     __shared__ double s_vt[PACK ? (CPLX ? 2 : 1) * kMaxValues : 1];
     __shared__ double s_scale;
     if (PACK) {
@@ -71,13 +81,13 @@ __global__ __launch_bounds__(kThreads) void spmv_sell(int64_t n_rows, int64_t n_
     // first kPre partials of each thread are loaded at once, and s is formed
     // after the block's first chunk product (which does not need it), so the
     // sum's latency overlaps the SpMV.
-    constexpr int kPre = 4;
+    constexpr int kPre = WIDE ? 0 : 4;
     const bool fused = LZ && bpart != nullptr;
-    double pv[kPre];
+    double pv[kPre ? kPre : 1];
     if (fused) {
 #pragma unroll
         for (int u = 0; u < kPre; ++u) {
-            const int i = (int)threadIdx.x + u * (int)blockDim.x;
+            const int i = (int)threadIdx.x + u * kThreads;
             pv[u] = i < n_bpart ? bpart[i] : 0.0;
         }
     }
@@ -86,10 +96,10 @@ __global__ __launch_bounds__(kThreads) void spmv_sell(int64_t n_rows, int64_t n_
         double t = 0.0;
 #pragma unroll
         for (int u = 0; u < kPre; ++u)
-            if ((int)threadIdx.x + u * (int)blockDim.x < n_bpart) t += pv[u];
-        for (int i = (int)threadIdx.x + kPre * (int)blockDim.x; i < n_bpart; i += blockDim.x)
-            t += bpart[i];
-        t = block_sum(t, lds);
+            if ((int)threadIdx.x + u * kThreads < n_bpart) t += pv[u];
+        if (threadIdx.x < kThreads)
+            for (int i = (int)threadIdx.x + kPre * kThreads; i < n_bpart; i += kThreads) t += bpart[i];
+        t = block_sum<NW>(t, lds);
         if (threadIdx.x == 0) {
             const double nb = sqrt(t);
             const double inv = nb > 0.0 ? 1.0 / nb : 0.0;
@@ -103,31 +113,43 @@ __global__ __launch_bounds__(kThreads) void spmv_sell(int64_t n_rows, int64_t n_
         s = s_scale;
     };
     double dot = 0.0;
-    // row product of chunk c (unscaled) and its output with the scale s
-    auto product = [&](int64_t c, double2 &acc, double2 &xr) {
-        const int64_t r = c * 64 + lane;
-        const int64_t base = chunk_ptr[c];
-        const int L = (int)((chunk_ptr[c + 1] - base) >> 6);
-        const int len = r < n_rows ? (int)row_len[r] : 0;
+    // row product of chunk c = c0 + wv (unscaled; none past the last chunk) and its
+    // output with the scale s
+    struct Barrier {
+        __device__ inline void operator()() const {
+            if (WIDE) __syncthreads();
+        }
+    };
+    auto product = [&](int64_t c0, double2 &acc, double2 &xr) {
+        const int64_t c = c0 + wv, r = c * 64 + lane;
+        const bool have = c < n_chunks;
+        const int64_t base = have ? chunk_ptr[c] : 0;
+        int L = have ? (int)((chunk_ptr[c + 1] - base) >> 6) : 0;
+        if (WIDE) {  // the longest chunk of the block, found by every wavefront
+            const int64_t q = c0 + (lane & (NW - 1));
+            L = q < n_chunks ? (int)((chunk_ptr[q + 1] - chunk_ptr[q]) >> 6) : 0;
+            for (int off = NW / 2; off > 0; off >>= 1) L = max(L, __shfl_xor(L, off, 64));
+        }
+        const int len = have && r < n_rows ? (int)row_len[r] : 0;
         const int64_t p0 = base + lane;
+        const uint32_t *wd = reinterpret_cast<const uint32_t *>(col);
         if (!CPLX) {
+            xr.x = have && r < n_rows ? x[r] : 0.0;
             if (PACK) {
-                xr.x = r < n_rows ? x[r] : 0.0;
-                const double d = r < n_rows ? diag[r] : 0.0;
-                const uint32_t *wd = reinterpret_cast<const uint32_t *>(col);
-                acc.x = sell_row_packed<NT>(wd, s_vt, x, p0, L, len, cb, d, xr.x);
+                const double d = have && r < n_rows ? diag[r] : 0.0;
+                acc.x = sell_row_packed<WIDE, WIDE ? 8 : 4>(wd, s_vt, x, p0, L, len, cb, d, xr.x, Barrier());
             } else {
-                acc.x = sell_row_real<NT>(col, val, x, p0, L, len);
-                if (LZ) xr.x = r < n_rows ? x[r] : 0.0;
+                acc.x = sell_row_real<WIDE>(col, val, x, p0, L, len, Barrier());
             }
         } else {
-            xr = r < n_rows ? reinterpret_cast<const double2 *>(x)[r] : make_double2(0.0, 0.0);
+            xr = have && r < n_rows ? reinterpret_cast<const double2 *>(x)[r] : make_double2(0.0, 0.0);
             if (PACK) {
-                const double2 d = r < n_rows ? reinterpret_cast<const double2 *>(diag)[r] : make_double2(0.0, 0.0);
-                const uint32_t *wd = reinterpret_cast<const uint32_t *>(col);
-                acc = sell_row_cplx_packed<NT>(wd, s_vt, s_vt + kMaxValues, x, p0, L, len, cb, rb, d, xr);
+                const double2 d =
+                    have && r < n_rows ? reinterpret_cast<const double2 *>(diag)[r] : make_double2(0.0, 0.0);
+                acc = sell_row_cplx_packed<WIDE>(wd, s_vt, s_vt + kMaxValues, x, p0, L, len, cb, rb, d, xr,
+                                                  Barrier());
             } else {
-                acc = sell_row_cplx<NT>(col, val, x, p0, L, len);
+                acc = sell_row_cplx<WIDE>(col, val, x, p0, L, len, Barrier());
             }
         }
     };
@@ -162,32 +184,27 @@ __global__ __launch_bounds__(kThreads) void spmv_sell(int64_t n_rows, int64_t n_
             }
         }
     };
-    // Streamed (large) matrices: XCD-contiguous chunk assignment. The hardware
-    // places block b on XCD b % 8; logical block lb gives each XCD one contiguous
-    // eighth of every pass over the chunks, so x lines that nearby rows gather stay
-    // in that XCD's L2 (on the 6x6 sector 37 % of the targets lie within 16K rows
-    // of their row: K1 27.6 -> 26.1 ms). A cached matrix keeps the interleaved
-    // assignment (the N=28 chain's K1 went from 51 to 60 us with it).
+    // XCD-contiguous chunk assignment (xcd): the hardware places block b on XCD
+    // b % 8; logical block lb gives each XCD one contiguous eighth of every pass
+    // over the chunks (on the 6x6 sector 37 % of the targets lie within 16K rows of
+    // their row).
     const unsigned nb = gridDim.x;
-    const unsigned lb = (NT && nb % 8u == 0u) ? (blockIdx.x % 8u) * (nb / 8u) + blockIdx.x / 8u : blockIdx.x;
-    const int64_t cstride = (int64_t)gridDim.x * kWaves;
-    int64_t c = (int64_t)lb * kWaves + wv;
-    if (fused) {
-        // every thread joins the block sum, with or without a chunk
-        double2 acc0 = make_double2(0.0, 0.0), xr0 = make_double2(0.0, 0.0);
-        const bool have = c < n_chunks;
-        if (have) product(c, acc0, xr0);
+    const unsigned lb = xcd ? (blockIdx.x % 8u) * (nb / 8u) + blockIdx.x / 8u : blockIdx.x;
+    bool scale = fused;  // form s after the first product; wide blocks first (fewer registers)
+    if (WIDE && scale) {
         form_scale();
-        if (have) emit(c, acc0, xr0);
-        c += cstride;
+        scale = false;
     }
-    for (; c < n_chunks; c += cstride) {
+    for (int64_t c0 = (int64_t)lb * NW; c0 < n_chunks; c0 += (int64_t)nb * NW) {
         double2 acc = make_double2(0.0, 0.0), xr = make_double2(0.0, 0.0);
-        product(c, acc, xr);
-        emit(c, acc, xr);
+        product(c0, acc, xr);
+        if (scale) form_scale();
+        scale = false;
+        if (c0 + wv < n_chunks) emit(c0 + wv, acc, xr);
     }
+    if (scale) form_scale();  // a block past the last chunk
     if (LZ) {
-        const double t = block_sum(dot, lds);
+        const double t = block_sum<NW>(dot, lds);
         if (threadIdx.x == 0) partials[blockIdx.x] = t;
     }
 }
@@ -708,36 +725,66 @@ struct FusedBeta {
     double *partials = nullptr;  // where this SpMV's a[n] partials go
 };
 
-// MI355X's memory-side cache (MALL) holds 256 MB: a packed matrix that fits it
-// beside the Lanczos vectors is read with plain loads, so its lines stay cached
-// from one SpMV to the next; a larger one is streamed (nontemporal loads).
-constexpr double kMallBytes = 256.0 * 1024 * 1024;
+// MI355X's memory-side cache (MALL), and the L2 of one of its eight XCDs
+constexpr double kMallBytes = 256.0 * 1024 * 1024, kL2Bytes = 4.0 * 1024 * 1024;
+
+// The shape of an SpMV's launch.
+// wide: the matrix is past the memory-side cache, read once a product. Below the
+// line plain loads find it there again and four wavefronts a block, up to eight
+// blocks a CU, hide the shorter waits better: narrow / wide, in a Lanczos run,
+// 28 sites complex (155 MB) 67.5 / 82.3 us, 27 with J2 (120 MB) 63.5 / 73.0; above
+// it, 28 sites complex by table (238 MB on a 4x7 lattice) 180 / 177, 30 sites
+// (228 MB) 110 / 104.
+// xcd: each XCD takes a contiguous eighth of every pass over the chunks, so that
+// the lines its rows gather come into one 4 MB L2 and not into all eight. A vector
+// of up to two L2s is found in each anyway, and there interleaved blocks share the
+// lines of the moment: interleaved / contiguous, 28 sites complex (23 MB vector)
+// 78.1 / 67.5 us, 4x7 lattice (23 MB) 198 / 180, 27 sites with J2 (12 MB) 58.8 / 55.1
+// for a product alone; 28 with J2 (5.7 MB) 45.9 / 50.2, 24 (0.5 MB) 9.2 / 9.6.
+// blocks: passes of equal size; a last pass with few blocks left most of the chip
+// idle (30 sites, 5061 blocks in two passes of at most 4096: 112 us, 100 in equal ones).
+struct SpmvShape {
+    bool wide, xcd;
+    unsigned blocks;
+};
+
+static SpmvShape spmv_shape(const qmb_ell *e) {
+    const double vec_bytes = (e->value_type == QMB_COMPLEX ? 16.0 : 8.0) * (double)e->n_rows;
+    SpmvShape s;
+    s.wide = e->format_bytes() > 0.75 * kMallBytes;
+    s.xcd = s.wide || vec_bytes > 2.0 * kL2Bytes;
+    const int64_t per = s.wide ? kWideWaves : kWaves, total = (e->n_chunks + per - 1) / per;
+    const int64_t most = s.wide ? kWideBlocks : s.xcd ? kMaxBlocks / 2 : kMaxBlocks;
+    const int64_t passes = std::max<int64_t>(1, (total + most - 1) / most);
+    s.blocks = (unsigned)std::max<int64_t>(1, (total + passes - 1) / passes);
+    if (s.xcd) s.blocks = (s.blocks + 7) / 8 * 8;
+    return s;
+}
+
+unsigned spmv_blocks(const qmb_ell *e) { return spmv_shape(e).blocks; }
 
 void launch_spmv(qmb_ctx *ctx, const qmb_ell *e, const double *x, double *y, bool lz, const double *invb,
                  double *vout, LzWork *wk, double *alpha_out, hipEvent_t after = nullptr,
                  const FusedBeta *fb = nullptr) {
-    const unsigned blocks = grid_for(e->n_chunks, kWaves);
-    const double vec_bytes = (e->value_type == QMB_COMPLEX ? 16.0 : 8.0) * (double)e->n_rows;
-    const bool stream = e->format_bytes() + 8.0 * vec_bytes > 0.75 * kMallBytes;
+    const SpmvShape shape = spmv_shape(e);
+    const unsigned blocks = shape.blocks;
     const bool cplx = e->value_type == QMB_COMPLEX;
     using K = decltype(&spmv_sell<false, false, false, false>);
-    // [complex][packed][lz][stream]
+#define QMB_SPMV(C, P, L) {spmv_sell<C, L, P, false>, spmv_sell<C, L, P, true>}
+    // [complex][packed][lz][wide]
     static const K table[2][2][2][2] = {
-        {{{spmv_sell<false, false, false, false>, spmv_sell<false, false, false, true>},
-          {spmv_sell<false, true, false, false>, spmv_sell<false, true, false, true>}},
-         {{spmv_sell<false, false, true, false>, spmv_sell<false, false, true, true>},
-          {spmv_sell<false, true, true, false>, spmv_sell<false, true, true, true>}}},
-        {{{spmv_sell<true, false, false, false>, spmv_sell<true, false, false, true>},
-          {spmv_sell<true, true, false, false>, spmv_sell<true, true, false, true>}},
-         {{spmv_sell<true, false, true, false>, spmv_sell<true, false, true, true>},
-          {spmv_sell<true, true, true, false>, spmv_sell<true, true, true, true>}}}};
-    const K k = table[cplx ? 1 : 0][e->packed ? 1 : 0][lz ? 1 : 0][stream ? 1 : 0];
-    hipLaunchKernelGGL(k, dim3(blocks), dim3(kThreads), 0, ctx->stream, e->n_rows, e->n_chunks,
+        {{QMB_SPMV(false, false, false), QMB_SPMV(false, false, true)},
+         {QMB_SPMV(false, true, false), QMB_SPMV(false, true, true)}},
+        {{QMB_SPMV(true, false, false), QMB_SPMV(true, false, true)},
+         {QMB_SPMV(true, true, false), QMB_SPMV(true, true, true)}}};
+#undef QMB_SPMV
+    const K k = table[cplx][e->packed ? 1 : 0][lz][shape.wide];
+    hipLaunchKernelGGL(k, dim3(blocks), dim3(shape.wide ? 64 * kWideWaves : kThreads), 0, ctx->stream, e->n_rows, e->n_chunks,
                        e->chunk_ptr.as<int64_t>(), e->row_len.as<uint16_t>(), e->col.as<int32_t>(),
                        e->val.as<double>(), e->diag.as<double>(), e->vtab.as<double>(), e->n_values, e->col_bits,
                        e->n_values_im, e->re_bits, x, y, invb, vout, fb ? fb->partials : wk ? wk->partials.as<double>() : nullptr,
                        fb ? fb->bpart : nullptr, fb ? fb->n_bpart : 0, fb ? fb->beta_out : nullptr,
-                       fb ? fb->invb_out : nullptr);
+                       fb ? fb->invb_out : nullptr, shape.xcd ? 1 : 0);
     QMB_HIP(hipGetLastError());
     if (after) QMB_HIP(hipEventRecord(after, ctx->stream));
     if (lz && !fb) launch_finish(ctx, wk->partials.as<double>(), blocks, alpha_out, nullptr, 0);
@@ -786,8 +833,6 @@ static void launch_small(qmb_ctx *ctx, const qmb_ell *e, LzWork &wk, int it0, in
                        seed, P, V0, V1, wk.alpha(), wk.beta(), wk.invb(), z, eig, X, res);
     QMB_HIP(hipGetLastError());
 }
-
-unsigned spmv_blocks(const qmb_ell *e) { return grid_for(e->n_chunks, kWaves); }
 
 static void launch_norm(qmb_ctx *ctx, int64_t cnt, const double *a, const double *b, double e, LzWork &wk,
                         double *out_norm, double *out_inv) {

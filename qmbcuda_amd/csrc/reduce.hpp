@@ -17,7 +17,8 @@ __device__ inline double wave_sum(double v) {
     return v;
 }
 
-// Sum over the block, valid in thread 0.
+// Sum over the block (NW wavefronts), valid in thread 0.
+template <int NW = kWaves>
 __device__ inline double block_sum(double v, double *lds) {
     v = wave_sum(v);
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -25,7 +26,7 @@ __device__ inline double block_sum(double v, double *lds) {
     __syncthreads();
     double t = 0.0;
     if (threadIdx.x == 0)
-        for (int i = 0; i < kWaves; ++i) t += lds[i];
+        for (int i = 0; i < NW; ++i) t += lds[i];
     __syncthreads();
     return t;
 }
