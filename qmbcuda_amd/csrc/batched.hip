@@ -990,9 +990,7 @@ static void run_batched(qmb_ctx *ctx, int n, const qmb_ell *const *ells, const q
                 } else {
                     QMB_HIP(hipMemsetAsync(X.p, 0, (size_t)cnt * sizeof(double), ctx->stream));
                 }
-                QMB_HIP(hipMemcpyAsync(vecs[gi], X.p, (size_t)cnt * sizeof(double), hipMemcpyDeviceToHost,
-                                       ctx->stream));
-                QMB_HIP(hipStreamSynchronize(ctx->stream));  // dz and X are reused or freed next
+                download(ctx, vecs[gi], X.p, (size_t)cnt * sizeof(double));  // waits: dz and X are reused or freed next
             }
         }
         if (!all_conv) throw Error{QMB_ERR_NOT_CONVERGED, "qmb_lanczos_batched: some instances did not converge"};

@@ -317,6 +317,7 @@ struct qmb_ctx : qmb::Counted {
         }
         return stage->as<T>();
     }
+    std::unique_ptr<qmb::PinnedBuf> bulk;  // slots of download_bulk (16 MB, made by the first large read-back)
     ~qmb_ctx() {
         if (stream) {
             (void)hipSetDevice(device);
@@ -324,6 +325,7 @@ struct qmb_ctx : qmb::Counted {
         }
         binom.release();
         stage.reset();
+        bulk.reset();
         pool.trim();
         pool.stream = nullptr;
         if (stream) (void)hipStreamDestroy(stream);
@@ -427,6 +429,10 @@ inline void require_device_range(const qmb_ctx *ctx, const void *p, size_t bytes
     QMB_REQUIRE(r == hipSuccess && static_cast<const char *>(p) + bytes <= static_cast<const char *>(base) + size,
                 what + " is smaller than the data it must hold");
 }
+
+// Device to host memory of the caller, after the work on the context's stream; the
+// data is there when it returns.
+void download(qmb_ctx *ctx, void *dst, const void *src, size_t bytes);
 
 // Exclusive scans on device (3-phase). Values come from a functor.
 int64_t scan_popcount_dict(qmb_ctx *ctx, uint64_t *dict, int64_t n_words);

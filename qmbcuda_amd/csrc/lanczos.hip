@@ -1445,8 +1445,9 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
         }
         QMB_HIP(hipMemcpyAsync(&eig_res, wk.misc() + 1, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
         if (eigvec)
-            QMB_HIP(hipMemcpyAsync(eigvec, X.p, cnt * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-        QMB_HIP(hipStreamSynchronize(ctx->stream));
+            download(ctx, eigvec, X.p, cnt * sizeof(double));
+        else
+            QMB_HIP(hipStreamSynchronize(ctx->stream));
         n_spmv += m + 1;
     }
     if (rep) {
@@ -1674,8 +1675,7 @@ qmb_status qmb_spmv_host(qmb_ctx *ctx, const qmb_ell *e, const double *x, double
         DevBuf dx(cnt * sizeof(double)), dy(cnt * sizeof(double));
         QMB_HIP(hipMemcpyAsync(dx.p, x, cnt * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
         launch_spmv(ctx, e, dx.as<double>(), dy.as<double>(), false, nullptr, nullptr, nullptr, nullptr);
-        QMB_HIP(hipMemcpyAsync(y, dy.p, cnt * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-        QMB_HIP(hipStreamSynchronize(ctx->stream));
+        download(ctx, y, dy.p, cnt * sizeof(double));
     });
 }
 

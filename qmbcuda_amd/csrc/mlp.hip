@@ -1273,8 +1273,7 @@ qmb_status qmb_mlp_start_vector(qmb_mlp *m, const qmb_basis *b, double delta, do
         DevBuf dx((size_t)b->n_rows * sizeof(double));
         StateWork w;
         const bool ok = build_start(m, b, delta, j2, 0, dx.as<double>(), w);
-        QMB_HIP(hipMemcpyAsync(x, dx.p, b->n_rows * sizeof(double), hipMemcpyDeviceToHost, m->ctx->stream));
-        QMB_HIP(hipStreamSynchronize(m->ctx->stream));
+        download(m->ctx, x, dx.p, b->n_rows * sizeof(double));
         if (fallback) *fallback = ok ? 0 : 1;
     });
 }

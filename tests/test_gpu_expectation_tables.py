@@ -71,3 +71,46 @@ def test_no_terms_left(ctx):
     never = [[(0, SP, 1.0 + 0j), (0, SP, 1.0 + 0j), (1, SM, 1.0 + 0j), (1, SM, 1.0 + 0j)]]
     for op in (gone, never):
         assert b.expectation(q.Terms(10, OM.conjugated_term_table(op)), x)[0] == 0.0
+
+
+def invariant(case, terms):
+    """Whether every image of the terms (equal products summed, the order kept on one site) is the same sum."""
+    def summed(perm, flip):
+        out = {}
+        for t in terms:
+            c, ops = 1.0 + 0j, []
+            for s, o, f in t:
+                c *= f
+                if flip:
+                    c, o = (-c, o) if o == SZ else (c, SM if o == SP else SP)
+                ops.append((int(perm[s]), o))
+            key = tuple(sorted(ops, key=lambda p: p[0]))
+            out[key] = out.get(key, 0) + c
+        return {k: v for k, v in out.items() if abs(v) > 1e-9}
+    n = case["n_sites"]
+    flip = case["flip"] if case["flip"] is not None else np.zeros(len(case["group_el"]))
+    base = summed(np.arange(n), False)
+    return all(b.keys() == base.keys() and all(abs(b[k] - base[k]) < 1e-9 for k in b)
+               for b in (summed(p, f) for p, f in zip(np.asarray(case["group_el"]), flip)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("flip", [False, True])
+def test_commutation(ctx, flip):
+    """`averaged` for sums over the ring of products of 0 to 10 operators, several on one site,
+    even and odd numbers of Sz, with one term missing and with a cancelling pair."""
+    n = 10
+    case = chain_case(n, 1.0, 1.0, 0.0, flip=flip)
+    b = q.Basis(ctx, q.Group(case["group_el"], case["chars"], case["flip"]), 5, 0)
+    x = np.random.default_rng(1).normal(size=b.n_rows)
+    shapes = [[], [(0, SZ)], [(0, SZ), (1, SZ)], [(0, SZ), (0, SZ)], [(0, SP), (0, SM)], [(0, SM), (0, SP), (3, SZ)],
+              [(2, SP), (0, SM)], [(3, SZ), (0, SP), (1, SM)], [(i, SZ) for i in range(8)],
+              [(i // 2, SZ) for i in range(9)], [(i, (SP, SM)[i % 2]) for i in range(8)] + [(8, SZ), (4, SZ)]]
+    for shape in shapes:
+        both = [shape, [(s, {SP: SM, SM: SP, SZ: SZ}[o]) for s, o in shape]]
+        ring = [[((s + r) % n, o, 1.0 + 0j) for s, o in t] for t in both for r in range(n)]
+        extra = [[(0, SP, 0.4 + 0j), (5, SM, 1.0 + 0j)], [(0, SP, -0.4 + 0j), (5, SM, 1.0 + 0j)]]
+        for terms in (ring, ring[1:], ring + extra, ring + extra[:1]):
+            print(f"[gpu-case] commutation flip={flip} {shape} {len(terms)} terms", flush=True)
+            _, averaged = b.expectation(q.Terms(n, OM.conjugated_term_table(terms)), x)
+            assert averaged != invariant(case, terms)
