@@ -483,7 +483,7 @@ static void upload_group(qmb_basis *b, const qmb_group *g) {
     if (g->lut && g->lut != 3) std::memcpy(h.data() + b->o_lut, g->lut_tab.data(), kLutBytes);
     if (g->lut >= 3) std::memcpy(h.data() + b->o_cos, g->cos_tab.data(), kCosBytes);
     b->g_tab.alloc(total);
-    QMB_HIP(hipMemcpy(b->g_tab.p, h.data(), total, hipMemcpyHostToDevice));
+    upload(b->ctx, b->g_tab.p, h.data(), total);
 }
 
 static uint64_t binom_host(int n, int k) {

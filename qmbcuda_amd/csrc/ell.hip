@@ -151,7 +151,18 @@ __global__ __launch_bounds__(kEllThreads, SPLIT ? 1 : 8) void ell_rows(GroupView
     }
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t r = SPLIT ? t >> ts : t;
-    if (r >= n_rows) return;
+    if (r >= n_rows) {
+        // padding entries of the rows past n_rows in the last chunk
+        const int64_t c = (n_rows - 1) / kChunk;
+        if (!FILL || r >= (c + 1) * kChunk || (SPLIT && ((int)t & ((1 << ts) - 1)) != 0)) return;
+        for (int64_t pos = chunk_ptr[c] + r % kChunk; pos < chunk_ptr[c + 1]; pos += kChunk) {
+            col[pos] = 0;
+            if (CODED) continue;
+            val[CPLX ? 2 * pos : pos] = 0.0;
+            if (CPLX) val[2 * pos + 1] = 0.0;
+        }
+        return;
+    }
     const int split = SPLIT ? 1 << ts : 1, sub = SPLIT ? (int)t & (split - 1) : 0;
     const int64_t c = r / kChunk;
     const int lane = (int)(r % kChunk);
@@ -348,28 +359,6 @@ static EllRows ell_fill_kernel(bool narrow, bool cplx, bool coded, bool split, i
     return any[narrow][cplx][coded][split];
 }
 
-// Padding entries of the rows past n_rows in the last chunk.
-__global__ void ell_pad_tail(int64_t n_rows, int64_t n_chunks, const int64_t *chunk_ptr, int32_t *col, double *val,
-                             int cplx) {
-    const int lane = threadIdx.x;
-    const int64_t c = n_chunks - 1;
-    const int64_t r = c * kChunk + lane;
-    if (r < n_rows) return;
-    const int64_t base = chunk_ptr[c];
-    const int L = (int)((chunk_ptr[c + 1] - base) / kChunk);
-    for (int s = 0; s < L; ++s) {
-        const int64_t pos = base + (int64_t)s * kChunk + lane;
-        col[pos] = 0;
-        if (!val) continue;  // coded build: no FP64 values
-        if (cplx) {
-            val[2 * pos] = 0.0;
-            val[2 * pos + 1] = 0.0;
-        } else {
-            val[pos] = 0.0;
-        }
-    }
-}
-
 // ---- packed values -----------------------------------------------------------
 // The sector matrices of these models hold a few dozen distinct values (term
 // scalars times characters times ratios of orbit norms), so a real ELL is
@@ -562,6 +551,8 @@ __global__ __launch_bounds__(kEllThreads) void ell_pack_values_cplx(int64_t n_ro
     }
 }
 
+__global__ void ell_clear(unsigned *words) { words[threadIdx.x] = 0u; }
+
 // ---- coded values -------------------------------------------------------------
 // Stabiliser sizes present among the rows: bit m of mask[0..4] (m <= kMaxGroup).
 __global__ __launch_bounds__(kEllThreads) void ell_stab_sizes(int64_t n_rows, const uint8_t *stab, unsigned *mask) {
@@ -629,50 +620,91 @@ struct CodeTables {
     int n_chi = 0, n_m = 0;
 };
 
-// One block: the value of every code in use, formed as the fill forms it
-// (same operands, same operations, no contraction), into cval and the sets of
-// distinct values (real parts in vset, imaginary parts in vset + kSetSlots).
-__global__ __launch_bounds__(1024) void ell_code_values(const unsigned *used, int n_codes, CodeTables ct, int cplx,
-                                                        double2 *cval, unsigned long long *vset, int *vflag) {
-    for (int c = threadIdx.x; c < n_codes; c += blockDim.x) {
-        if (!((used[c >> 5] >> (c & 31)) & 1u)) continue;
-        int t = c;
-        const int mt = t % ct.n_m;
-        t /= ct.n_m;
-        const int ms = t % ct.n_m;
-        t /= ct.n_m;
-        const int xc = t % ct.n_chi;
-        t /= ct.n_chi;
-        const double2 co = ct.coef[t >> 1];
-        const bool neg = (t & 1) != 0;
-        const double cr = neg ? -co.x : co.x;
-        const double ci = neg ? -co.y : co.y;
-        const int m_src = ct.m[ms], mult = ct.m[mt];
-        const double n_src = ct.nrm[m_src];
-        const double ratio = mult == m_src ? 1.0 : ct.nrm[mult] / n_src;
-        const double2 x = ct.chi[xc];
-        const double pr = cr * x.x - ci * x.y;
-        const double pi = cr * x.y + ci * x.x;
-        const double vr = pr * ratio, vi = pi * ratio;
-        cval[c] = make_double2(vr, cplx ? vi : 0.0);
-        if (!set_insert(vset, kSetSlots, (unsigned long long)__double_as_longlong(vr))) vflag[0] = 1;
-        if (cplx && !set_insert(vset + kSetSlots, kSetSlots, (unsigned long long)__double_as_longlong(vi)))
-            vflag[0] = 1;
-    }
+__device__ inline uint32_t key_index(const unsigned long long *keys, int n, unsigned long long key, int *missing);
+
+// The value of a code, formed as the fill forms it (same operands, same operations,
+// no contraction).
+__device__ inline double2 code_value(int c, const CodeTables &ct, int cplx) {
+    int t = c;
+    const int mt = t % ct.n_m;
+    t /= ct.n_m;
+    const int ms = t % ct.n_m;
+    t /= ct.n_m;
+    const int xc = t % ct.n_chi;
+    t /= ct.n_chi;
+    const double2 co = ct.coef[t >> 1];
+    const bool neg = (t & 1) != 0;
+    const double cr = neg ? -co.x : co.x;
+    const double ci = neg ? -co.y : co.y;
+    const int m_src = ct.m[ms], mult = ct.m[mt];
+    const double n_src = ct.nrm[m_src];
+    const double ratio = mult == m_src ? 1.0 : ct.nrm[mult] / n_src;
+    const double2 x = ct.chi[xc];
+    const double pr = cr * x.x - ci * x.y;
+    const double pi = cr * x.y + ci * x.x;
+    const double vr = pr * ratio, vi = pi * ratio;
+    return make_double2(vr, cplx ? vi : 0.0);
 }
 
-// One block, when the tables are complete (f: the packing flags): map[c] = the
-// value index of code c (complex: re index | im index << 16).
-__global__ __launch_bounds__(1024) void ell_code_map(const unsigned *used, int n_codes, const double2 *cval,
-                                                     const unsigned long long *keys, int *f, int cplx,
-                                                     uint32_t *map) {
-    if (!f[2] || (cplx && !f[5])) return;
-    for (int c = threadIdx.x; c < n_codes; c += blockDim.x) {
-        if (!((used[c >> 5] >> (c & 31)) & 1u)) continue;
-        const double2 v = cval[c];
-        uint32_t m = key_index(keys, f[1], (unsigned long long)__double_as_longlong(v.x), f + 3);
-        if (cplx) m |= key_index(keys + kMaxValues, f[4], (unsigned long long)__double_as_longlong(v.y), f + 3) << 16;
-        map[c] = m;
+// One block, after a coded fill: the values of the codes in use (cval), their
+// distinct parts in ascending bit order, +0.0 first (keys, meta f as of
+// ell_sort_values), and when the tables are complete map[c] = the value index of code
+// c (complex: re index | im index << 16). One launch; the steps by a kernel each were
+// five launches around a set in memory.
+__global__ __launch_bounds__(1024) void ell_code_tables(const unsigned *used, int n_codes, CodeTables ct, int cplx,
+                                                        int cap, double2 *cval, unsigned long long *keys, int *f,
+                                                        uint32_t *map) {
+    __shared__ unsigned long long set[kSetSlots];
+    __shared__ unsigned long long a[kMaxValues], sorted[2][kMaxValues];
+    __shared__ int m, full;
+    const int t = threadIdx.x;
+    bool all_ok = true;
+    for (int part = 0; part < (cplx ? 2 : 1); ++part) {
+        for (int i = t; i < kSetSlots; i += blockDim.x) set[i] = kEmptyKey;
+        if (t == 0) m = full = 0;
+        __syncthreads();
+        for (int c = t; c < n_codes; c += blockDim.x) {
+            if (!((used[c >> 5] >> (c & 31)) & 1u)) continue;
+            const double2 v = part ? cval[c] : code_value(c, ct, cplx);
+            if (!part) cval[c] = v;
+            if (!set_insert(set, kSetSlots, (unsigned long long)__double_as_longlong(part ? v.y : v.x))) full = 1;
+        }
+        __syncthreads();
+        for (int i = t; i < kSetSlots; i += blockDim.x) {
+            const unsigned long long k = set[i];
+            if (k == kEmptyKey || k == 0ull) continue;
+            const int at = atomicAdd(&m, 1);
+            if (at < kMaxValues) a[at] = k;
+        }
+        __syncthreads();
+        const int n = m + 1;
+        const bool ok = !full && n <= cap;
+        if (ok)
+            for (int i = t; i < m; i += blockDim.x) {
+                const unsigned long long k = a[i];
+                int rank = 0;
+                for (int j = 0; j < m; ++j) rank += a[j] < k ? 1 : 0;
+                keys[part * kMaxValues + 1 + rank] = sorted[part][1 + rank] = k;
+            }
+        if (t == 0) {
+            keys[part * kMaxValues] = sorted[part][0] = 0ull;
+            if (full) f[0] = 1;
+            f[part ? 4 : 1] = n;
+            f[part ? 5 : 2] = ok ? 1 : 0;
+        }
+        all_ok = all_ok && ok;
+        __syncthreads();
+        if (part == 0) {
+            if (ok)
+                for (int c = t; c < n_codes; c += blockDim.x)
+                    if ((used[c >> 5] >> (c & 31)) & 1u)
+                        map[c] = key_index(sorted[0], n, (unsigned long long)__double_as_longlong(cval[c].x), f + 3);
+        } else if (all_ok) {
+            for (int c = t; c < n_codes; c += blockDim.x)
+                if ((used[c >> 5] >> (c & 31)) & 1u)
+                    map[c] |= key_index(sorted[1], n, (unsigned long long)__double_as_longlong(cval[c].y), f + 3) << 16;
+        }
+        __syncthreads();
     }
 }
 
@@ -721,49 +753,40 @@ __global__ __launch_bounds__(kEllThreads) void ell_pack_codes(int64_t n_rows, co
 struct ValuePacking {
     bool on = false, cplx = false;
     int cb = 0, cap = 0;
-    DevBuf vset, flags;
+    DevBuf vset;
+    int *f = nullptr;  // the flags (device, cleared)
     // coded build (plan_codes, before the fill): flags[6] = a stabiliser size without a class
     bool coded = false;
     int n_codes = 0;
-    DevBuf codes, used, cval, map, ctab;
+    DevBuf codes, cval, map, ctab;
+    unsigned *used = nullptr;
     CodeView cv;
     CodeTables ct;
-    bool prepare(qmb_ctx *ctx, const qmb_ell &e) {
+    void prepare(const qmb_ell &e, int *flags) {
         const int64_t n = e.n_rows;
-        if (n < 2) return false;
+        if (n < 2) return;
         cplx = e.value_type == QMB_COMPLEX;
         cb = 1;
         while (((int64_t)1 << cb) < n) ++cb;
-        if (cb > 31) return false;
+        if (cb > 31) return;
         cap = cplx ? kMaxValues : (int)std::min<int64_t>(kMaxValues, (int64_t)1 << (32 - cb));
-        const int parts = cplx ? 2 : 1;
-        vset.alloc((size_t)parts * kSetSlots * 8);
-        flags.alloc(8 * sizeof(int));
-        QMB_HIP(hipMemsetAsync(vset.p, 0xFF, vset.bytes, ctx->stream));
-        QMB_HIP(hipMemsetAsync(flags.p, 0, flags.bytes, ctx->stream));
+        f = flags;
         on = true;
-        return true;
+    }
+    static bool codes_wanted() {
+        const char *env = std::getenv("QMB_VALUE_CODES");
+        return !(env && env[0] == '0');
     }
     // Whether the fill writes codes: the coefficient classes of the terms, the
-    // character classes of the irrep row and the stabiliser sizes present (one
-    // small kernel and a read-back) must give at most kMaxCodes codes. Sets up
-    // the code tables, the code array and the diagonal.
+    // character classes of the irrep row and the stabiliser sizes present (hm, the mask
+    // of ell_stab_sizes) must give at most kMaxCodes codes. Sets up the code tables,
+    // the code array and the diagonal; used: kMaxCodes cleared bits.
     // QMB_VALUE_CODES=0 in the environment selects the FP64 fill and the value
     // collection pass instead (the route of tables with too many codes), so
     // tests can compare the two routes.
-    bool plan_codes(qmb_ctx *ctx, qmb_ell &e, const qmb_basis &b, const DeviceTerms &dt, const double *ch, int G) {
-        const char *env = std::getenv("QMB_VALUE_CODES");
-        if (env && env[0] == '0') return false;
+    bool plan_codes(qmb_ctx *ctx, qmb_ell &e, const unsigned *hm, unsigned *used_bits, const DeviceTerms &dt,
+                    const double *ch, int G) {
         if (!on || dt.classes.size() > DeviceTerms::kMaxClasses || G > kMaxGroup) return false;
-        DevBuf dmask(5 * sizeof(unsigned));
-        QMB_HIP(hipMemsetAsync(dmask.p, 0, dmask.bytes, ctx->stream));
-        const unsigned blocks = (unsigned)std::min<int64_t>(1024, (e.n_rows + kEllThreads - 1) / kEllThreads);
-        hipLaunchKernelGGL(ell_stab_sizes, dim3(blocks), dim3(kEllThreads), 0, ctx->stream, e.n_rows,
-                           b.stab.as<uint8_t>(), dmask.as<unsigned>());
-        QMB_HIP(hipGetLastError());
-        unsigned *hm = ctx->host_stage<unsigned>(5 * sizeof(unsigned));
-        QMB_HIP(hipMemcpyAsync(hm, dmask.p, 5 * sizeof(unsigned), hipMemcpyDeviceToHost, ctx->stream));
-        QMB_HIP(hipStreamSynchronize(ctx->stream));
         std::vector<int> m_of;
         std::vector<uint8_t> mcls(kMaxGroup + 1, 0xFF);
         for (int m = 0; m <= kMaxGroup; ++m)
@@ -797,11 +820,10 @@ struct ValuePacking {
         std::memcpy(h.data() + o_xc, xc.data(), xc.size() * 16);
         std::memcpy(h.data() + o_mo, m_of.data(), m_of.size() * sizeof(int));
         ctab.alloc(total);
-        QMB_HIP(hipMemcpy(ctab.p, h.data(), total, hipMemcpyHostToDevice));
+        upload(ctx, ctab.p, h.data(), total);
         const char *d = static_cast<const char *>(ctab.p);
         codes.alloc((size_t)std::max<int64_t>(e.stored, 1) * sizeof(uint16_t));
-        used.alloc(kMaxCodes / 8);
-        QMB_HIP(hipMemsetAsync(used.p, 0, used.bytes, ctx->stream));
+        used = used_bits;
         cval.alloc((size_t)n_codes * sizeof(double2));
         map.alloc((size_t)n_codes * sizeof(uint32_t));
         e.diag.alloc((size_t)e.n_rows * (cplx ? 2 : 1) * sizeof(double));
@@ -811,7 +833,7 @@ struct ValuePacking {
         cv.n_m = (int)m_of.size();
         cv.code = codes.as<uint16_t>();
         cv.diag = e.diag.as<double>();
-        cv.bad = flags.as<int>() + 6;
+        cv.bad = f + 6;
         ct.coef = reinterpret_cast<const double2 *>(d + o_tc);
         ct.chi = reinterpret_cast<const double2 *>(d + o_xc);
         ct.m = reinterpret_cast<const int *>(d + o_mo);
@@ -826,39 +848,28 @@ struct ValuePacking {
     void launch_coded(qmb_ctx *ctx, qmb_ell &e) {
         const int parts = cplx ? 2 : 1;
         e.vtab.alloc((size_t)parts * kMaxValues * 8);
-        int *f = flags.as<int>();
         unsigned long long *keys = e.vtab.as<unsigned long long>();
         const unsigned blocks = (unsigned)std::min<int64_t>(4096, (e.n_rows + kEllThreads - 1) / kEllThreads);
         hipLaunchKernelGGL(ell_collect_codes, dim3(blocks), dim3(kEllThreads), 0, ctx->stream, e.n_rows,
                            e.chunk_ptr.as<int64_t>(), e.row_len.as<uint16_t>(), codes.as<uint16_t>(), n_codes,
-                           used.as<unsigned>());
+                           used);
         QMB_HIP(hipGetLastError());
-        hipLaunchKernelGGL(ell_code_values, dim3(1), dim3(1024), 0, ctx->stream, used.as<unsigned>(), n_codes, ct,
-                           cplx ? 1 : 0, cval.as<double2>(), vset.as<unsigned long long>(), f);
-        QMB_HIP(hipGetLastError());
-        hipLaunchKernelGGL(ell_sort_values, dim3(1), dim3(1024), 0, ctx->stream, vset.as<unsigned long long>(), f,
-                           keys, f + 1, cap);
-        QMB_HIP(hipGetLastError());
-        if (cplx) {
-            hipLaunchKernelGGL(ell_sort_values, dim3(1), dim3(1024), 0, ctx->stream,
-                               vset.as<unsigned long long>() + kSetSlots, f, keys + kMaxValues, f + 4, cap);
-            QMB_HIP(hipGetLastError());
-        }
-        hipLaunchKernelGGL(ell_code_map, dim3(1), dim3(1024), 0, ctx->stream, used.as<unsigned>(), n_codes,
-                           cval.as<double2>(), keys, f, cplx ? 1 : 0, map.as<uint32_t>());
+        hipLaunchKernelGGL(ell_code_tables, dim3(1), dim3(1024), 0, ctx->stream, used, n_codes, ct, cplx ? 1 : 0, cap,
+                           cval.as<double2>(), keys, f, map.as<uint32_t>());
         QMB_HIP(hipGetLastError());
         hipLaunchKernelGGL(ell_pack_codes, dim3(blocks), dim3(kEllThreads), 0, ctx->stream, e.n_rows,
                            e.chunk_ptr.as<int64_t>(), e.row_len.as<uint16_t>(), e.col.as<uint32_t>(),
                            codes.as<uint16_t>(), map.as<uint32_t>(), f, cplx ? 1 : 0, cb);
         QMB_HIP(hipGetLastError());
-        QMB_HIP(hipMemcpyAsync(ctx->host_stage<int>(8 * sizeof(int)), flags.p, 8 * sizeof(int),
+        QMB_HIP(hipMemcpyAsync(ctx->host_stage<int>(8 * sizeof(int)), f, 8 * sizeof(int),
                                hipMemcpyDeviceToHost, ctx->stream));
     }
     void launch(qmb_ctx *ctx, qmb_ell &e) {
         const int parts = cplx ? 2 : 1;
+        vset.alloc((size_t)parts * kSetSlots * 8);
+        QMB_HIP(hipMemsetAsync(vset.p, 0xFF, vset.bytes, ctx->stream));
         e.vtab.alloc((size_t)parts * kMaxValues * 8);
         e.diag.alloc((size_t)e.n_rows * parts * sizeof(double));
-        int *f = flags.as<int>();
         unsigned long long *keys = e.vtab.as<unsigned long long>();
         const unsigned cblocks = (unsigned)std::min<int64_t>(4096, (e.n_rows + kEllThreads - 1) / kEllThreads);
         hipLaunchKernelGGL(cplx ? ell_collect_values<true> : ell_collect_values<false>, dim3(cblocks),
@@ -884,7 +895,7 @@ struct ValuePacking {
                                e.chunk_ptr.as<int64_t>(), e.row_len.as<uint16_t>(), e.col.as<uint32_t>(),
                                e.val.as<double>(), keys, f + 1, cb, e.diag.as<double>(), f + 3);
         QMB_HIP(hipGetLastError());
-        QMB_HIP(hipMemcpyAsync(ctx->host_stage<int>(8 * sizeof(int)), flags.p, 8 * sizeof(int),
+        QMB_HIP(hipMemcpyAsync(ctx->host_stage<int>(8 * sizeof(int)), f, 8 * sizeof(int),
                                hipMemcpyDeviceToHost, ctx->stream));
     }
     // after the stream has drained (the flags were copied into the context's
@@ -946,7 +957,7 @@ struct RankTables {
     DevBuf buf;
     int n_nib = 0, n_c = 0;
     size_t lds_bytes = 0;
-    explicit RankTables(const qmb_basis &b) {
+    RankTables(qmb_ctx *ctx, const qmb_basis &b) {
         const bool narrow = b.n_sites <= 32;
         lds_bytes = narrow ? 32 * kBinJ * sizeof(uint32_t) : 64 * kBinJ * sizeof(uint64_t);
         int nn = 0, nc = 0;
@@ -954,7 +965,7 @@ struct RankTables {
         const size_t bytes = t.size() * sizeof(uint64_t);
         if (bytes > kMaxBytes) return;
         buf.alloc(bytes);
-        QMB_HIP(hipMemcpy(buf.p, t.data(), bytes, hipMemcpyHostToDevice));
+        upload(ctx, buf.p, t.data(), bytes);
         n_nib = nn;
         n_c = nc;
         lds_bytes = narrow ? bytes / 2 : bytes;
@@ -999,20 +1010,27 @@ qmb_status qmb_ell_build(qmb_ctx *ctx, const qmb_basis *b, const qmb_terms *t, i
         e->n_chunks = (b->n_rows + kChunk - 1) / kChunk;
         // term table and irrep data on device
         const std::vector<int> order = locality ? locality_order(*t) : std::vector<int>();
-        const DeviceTerms dt(*t, ch, g->G, locality ? &order : nullptr, true);
+        const DeviceTerms dt(ctx, *t, ch, g->G, locality ? &order : nullptr);
         const TermsView tv = dt.view;
-        DevBuf d_err(sizeof(int));
-        QMB_HIP(hipMemsetAsync(d_err.p, 0, sizeof(int), ctx->stream));
+        // small words of the build, cleared at once: the overflow flag, the statistics
+        // with the stabiliser sizes' mask in their last half, the packing flags and the
+        // bits of the codes in use
+        constexpr size_t o_stats = 64, o_flags = 128, o_used = 256, n_words = (o_used + kMaxCodes / 8) / 4;
+        DevBuf words(n_words * 4);
+        hipLaunchKernelGGL(ell_clear, dim3(1), dim3(n_words), 0, ctx->stream, words.as<unsigned>());
+        QMB_HIP(hipGetLastError());
+        int *d_err = words.as<int>();
+        int64_t *d_stats = reinterpret_cast<int64_t *>(words.as<char>() + o_stats);
         const GroupView gv = b->view();
         const int64_t n = b->n_rows;
         e->row_len.alloc((size_t)std::max<int64_t>(n, 1) * sizeof(uint16_t));
         e->chunk_ptr.alloc((size_t)(e->n_chunks + 1) * sizeof(int64_t));
-        const RankTables rank(*b);
+        const RankTables rank(ctx, *b);
         // lanes per row of the passes that make lookups: as many as keep the chip busy
         int ts = 0;
         while (ts < kMaxSplit && (n << (ts + 1)) <= kSplitLanes) ++ts;
-        auto blocks_for = [&](int shift) {
-            return (unsigned)std::max<int64_t>(1, ((n << shift) + kEllThreads - 1) / kEllThreads);
+        auto blocks_for = [](int64_t rows, int shift) {
+            return (unsigned)std::max<int64_t>(1, ((rows << shift) + kEllThreads - 1) / kEllThreads);
         };
         const bool cplx = value_type == QMB_COMPLEX;
         const bool narrow = b->n_sites <= 32;
@@ -1023,45 +1041,53 @@ qmb_status qmb_ell_build(qmb_ctx *ctx, const qmb_basis *b, const qmb_terms *t, i
             const int cts = b->all_rows ? 0 : ts;
             const EllRows kcount = ell_count_kernel(narrow, cts != 0, gv.lut);
             // the count pass of a sector without null orbits makes no orbit lookups
-            hipLaunchKernelGGL(kcount, dim3(blocks_for(cts)), dim3(kEllThreads), b->all_rows ? 0 : lds_bytes,
+            hipLaunchKernelGGL(kcount, dim3(blocks_for(n, cts)), dim3(kEllThreads), b->all_rows ? 0 : lds_bytes,
                                ctx->stream, gv, ctx->binom.as<uint64_t>(), rank.tab(), rank.n_nib, rank.n_c,
                                b->layout, n, b->reps.as<uint64_t>(),
                                b->stab.as<uint8_t>(), b->nullf.as<uint8_t>(), b->dict.as<uint64_t>(),
                                tv, n_lds, dt.chi, dt.nrm, W,
-                               e->row_len.as<uint16_t>(), d_err.as<int>(), b->all_rows ? 1 : 0, nullptr, nullptr,
+                               e->row_len.as<uint16_t>(), d_err, b->all_rows ? 1 : 0, nullptr, nullptr,
                                nullptr, CodeView{}, cts);
             QMB_HIP(hipGetLastError());
         }
-        // the offsets are scanned before the overflow flag is read (one synchronisation)
-        int herr = 0, max_len = 0;
-        e->stored = n > 0 ? scan_chunks_i64(ctx, e->row_len.as<uint16_t>(), n, e->chunk_ptr.as<int64_t>(),
-                                            e->n_chunks, &e->nnz, &max_len, d_err.as<int>(), &herr)
-                          : 0;
-        QMB_REQUIRE(herr == 0, "qmb_ell_build: a row needs more than max_terms = " + std::to_string(W) + " slots");
-        e->max_row_len = max_len;
-        e->col.alloc((size_t)std::max<int64_t>(e->stored, 1) * sizeof(int32_t));
+        // the offsets are scanned and the stabiliser sizes collected before the overflow
+        // flag is read (one synchronisation)
         ValuePacking vp;
-        if (n > 0 && !keep_fp64) vp.prepare(ctx, *e);
+        if (n > 0 && !keep_fp64) vp.prepare(*e, reinterpret_cast<int *>(words.as<char>() + o_flags));
+        const bool try_codes = vp.on && ValuePacking::codes_wanted();
+        if (try_codes) {
+            const unsigned blocks = (unsigned)std::min<int64_t>(1024, (n + kEllThreads - 1) / kEllThreads);
+            hipLaunchKernelGGL(ell_stab_sizes, dim3(blocks), dim3(kEllThreads), 0, ctx->stream, n,
+                               b->stab.as<uint8_t>(), reinterpret_cast<unsigned *>(d_stats + 4));
+            QMB_HIP(hipGetLastError());
+        }
+        int64_t stats[kScanStats] = {};
+        if (n > 0)
+            scan_chunks_i64(ctx, e->row_len.as<uint16_t>(), n, e->chunk_ptr.as<int64_t>(), e->n_chunks, d_err, d_stats,
+                            stats);
+        QMB_REQUIRE(stats[3] == 0, "qmb_ell_build: a row needs more than max_terms = " + std::to_string(W) + " slots");
+        e->stored = stats[0];
+        e->nnz = stats[1];
+        e->max_row_len = (int)stats[2];
+        e->col.alloc((size_t)std::max<int64_t>(e->stored, 1) * sizeof(int32_t));
         // a packed build writes value codes (2 B per entry) instead of FP64 values
         // when the factors of the values give few enough codes
-        const bool coded = vp.on && vp.plan_codes(ctx, *e, *b, dt, ch, g->G);
-        // the fill (coded, or with FP64 values) and the padding of the last chunk
+        unsigned mask[5];
+        std::memcpy(mask, stats + 4, sizeof mask);
+        const bool coded = try_codes && vp.plan_codes(ctx, *e, mask, reinterpret_cast<unsigned *>(words.as<char>() + o_used),
+                                                      dt, ch, g->G);
+        // the fill (coded, or with FP64 values), with the padding of the last chunk
         auto fill = [&](bool with_codes) {
             const EllRows kfill = ell_fill_kernel(narrow, cplx, with_codes, ts != 0, gv.lut);
             double *val = with_codes ? nullptr : e->val.as<double>();
-            hipLaunchKernelGGL(kfill, dim3(blocks_for(ts)), dim3(kEllThreads), lds_bytes, ctx->stream, gv,
+            hipLaunchKernelGGL(kfill, dim3(blocks_for(e->n_chunks * kChunk, ts)), dim3(kEllThreads), lds_bytes, ctx->stream, gv,
                                ctx->binom.as<uint64_t>(), rank.tab(), rank.n_nib, rank.n_c, b->layout, n,
                                b->reps.as<uint64_t>(),
                                b->stab.as<uint8_t>(), b->nullf.as<uint8_t>(), b->dict.as<uint64_t>(),
                                tv, n_lds, dt.chi, dt.nrm, W,
-                               e->row_len.as<uint16_t>(), d_err.as<int>(), 0, e->chunk_ptr.as<int64_t>(),
+                               e->row_len.as<uint16_t>(), d_err, 0, e->chunk_ptr.as<int64_t>(),
                                e->col.as<int32_t>(), val, with_codes ? vp.cv : CodeView{}, ts);
             QMB_HIP(hipGetLastError());
-            if (n % kChunk) {
-                hipLaunchKernelGGL(ell_pad_tail, dim3(1), dim3(kChunk), 0, ctx->stream, n, e->n_chunks,
-                                   e->chunk_ptr.as<int64_t>(), e->col.as<int32_t>(), val, cplx ? 1 : 0);
-                QMB_HIP(hipGetLastError());
-            }
         };
         if (!coded) e->val.alloc((size_t)std::max<int64_t>(e->stored, 1) * (cplx ? 16 : 8));
         if (n > 0) {

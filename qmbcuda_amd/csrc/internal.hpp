@@ -317,6 +317,9 @@ struct qmb_ctx : qmb::Counted {
         }
         return stage->as<T>();
     }
+    std::unique_ptr<qmb::PinnedBuf> up;  // slots of upload(), used in turn
+    size_t up_at = 0;
+    hipEvent_t up_done = nullptr;  // after the last upload
     std::unique_ptr<qmb::PinnedBuf> bulk;  // slots of download_bulk (16 MB, made by the first large read-back)
     ~qmb_ctx() {
         if (stream) {
@@ -326,6 +329,8 @@ struct qmb_ctx : qmb::Counted {
         binom.release();
         stage.reset();
         bulk.reset();
+        up.reset();
+        if (up_done) (void)hipEventDestroy(up_done);
         pool.trim();
         pool.stream = nullptr;
         if (stream) (void)hipStreamDestroy(stream);
@@ -434,14 +439,20 @@ inline void require_device_range(const qmb_ctx *ctx, const void *p, size_t bytes
 // data is there when it returns.
 void download(qmb_ctx *ctx, void *dst, const void *src, size_t bytes);
 
+// A host table to the device on the context's stream, through pinned slots: the call
+// returns at once (a copy from ordinary memory waits for the stream: some 15 us each
+// in the build of a small matrix).
+void upload(qmb_ctx *ctx, void *dst, const void *src, size_t bytes);
+
 // Exclusive scans on device (3-phase). Values come from a functor.
 int64_t scan_popcount_dict(qmb_ctx *ctx, uint64_t *dict, int64_t n_words);
-// Chunk offsets of a SELL-64 layout from its row lengths (chunk_ptr[n_chunks] =
-// stored total, returned), with the entry count and longest row; d_err (if set)
-// is read back in the same synchronisation into err_out.
-int64_t scan_chunks_i64(qmb_ctx *ctx, const uint16_t *row_len, int64_t n_rows, int64_t *chunk_ptr,
-                        int64_t n_chunks, int64_t *nnz_out, int *max_len_out, const int *d_err = nullptr,
-                        int *err_out = nullptr);
+// Chunk offsets of a SELL-64 layout from its row lengths. h = {stored total (also
+// chunk_ptr[n_chunks]), entries, longest row, *d_err, then the words the caller has in
+// d_stats[4..8)}, read back in one synchronisation; d_stats: kScanStats words of device
+// memory, or NULL.
+constexpr int kScanStats = 8;
+void scan_chunks_i64(qmb_ctx *ctx, const uint16_t *row_len, int64_t n_rows, int64_t *chunk_ptr, int64_t n_chunks,
+                     const int *d_err, int64_t *d_stats, int64_t (&h)[kScanStats]);
 
 void ensure_binom(qmb_ctx *ctx);
 

@@ -1581,13 +1581,14 @@ qmb_ell *ell_from_reference_device(qmb_ctx *ctx, int64_t n, int W, const uint32_
     hipLaunchKernelGGL(ref_row_len, dim3(blocks), dim3(256), 0, ctx->stream, track, n, W, e->row_len.as<uint16_t>(),
                        err.as<int>());
     QMB_HIP(hipGetLastError());
-    int herr = 0, mx = 0;
-    int64_t nnz = 0;
-    e->stored = scan_chunks_i64(ctx, e->row_len.as<uint16_t>(), n, e->chunk_ptr.as<int64_t>(), e->n_chunks, &nnz,
-                                &mx, err.as<int>(), &herr);
+    int64_t h[kScanStats];
+    scan_chunks_i64(ctx, e->row_len.as<uint16_t>(), n, e->chunk_ptr.as<int64_t>(), e->n_chunks, err.as<int>(),
+                    nullptr, h);
+    int herr = (int)h[3];
     QMB_REQUIRE(herr == 0, "reference ELL: track out of range [0, max_terms]");
-    e->nnz = nnz;
-    e->max_row_len = mx;
+    e->stored = h[0];
+    e->nnz = h[1];
+    e->max_row_len = (int)h[2];
     e->col.alloc((size_t)std::max<int64_t>(e->stored, 1) * sizeof(int32_t));
     e->val.alloc((size_t)std::max<int64_t>(e->stored, 1) * vs * sizeof(double));
     hipLaunchKernelGGL(ref_fill, dim3(blocks), dim3(256), 0, ctx->stream, ind, val, n, W, vs,

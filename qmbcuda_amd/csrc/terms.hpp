@@ -146,19 +146,15 @@ struct DeviceTerms {
     const double *nrm = nullptr;   // [G + 1]
     static constexpr size_t kMaxClasses = 1 << 14;
     std::vector<double2> classes;  // distinct term coefficients, in order of first use (TermC::vclass)
-    // sorted: for the ELL passes, the terms that change the state first, then the
-    // diagonal ones, each in the given order, without those that never act
-    DeviceTerms(const qmb_terms &t, const double *chi_row, int G, const std::vector<int> *order = nullptr,
-                bool sorted = false) {
+    // the terms that change the state first, then the diagonal ones, each in the given
+    // order, without those that never act
+    DeviceTerms(qmb_ctx *ctx, const qmb_terms &t, const double *chi_row, int G, const std::vector<int> *order) {
         std::vector<TermC> terms(t.n_terms);
         for (int k = 0; k < t.n_terms; ++k) terms[k] = compile_term(t, order ? (*order)[k] : k);
-        int n_off = 0;
-        if (sorted) {
-            terms.erase(std::remove_if(terms.begin(), terms.end(), never_acts), terms.end());
-            const auto mid = std::stable_partition(terms.begin(), terms.end(),
-                                                   [](const TermC &c) { return !is_diagonal(c); });
-            n_off = (int)(mid - terms.begin());
-        }
+        terms.erase(std::remove_if(terms.begin(), terms.end(), never_acts), terms.end());
+        const auto mid = std::stable_partition(terms.begin(), terms.end(),
+                                               [](const TermC &c) { return !is_diagonal(c); });
+        const int n_off = (int)(mid - terms.begin());
         const int nt = (int)terms.size();
         auto up16 = [](size_t x) { return (x + 15) & ~(size_t)15; };
         const size_t o_terms = 0, o_chi = up16((size_t)std::max(1, nt) * sizeof(TermC)),
@@ -180,11 +176,11 @@ struct DeviceTerms {
             }
             if (tc[k].vclass == classes.size()) classes.push_back(tc[k].coef);
         }
-        if (chi_row) std::memcpy(h.data() + o_chi, chi_row, (size_t)G * 16);
+        std::memcpy(h.data() + o_chi, chi_row, (size_t)G * 16);
         const std::vector<double> nt_tab = orbit_norm_table(G);
         std::memcpy(h.data() + o_nrm, nt_tab.data(), nt_tab.size() * 8);
         blob.alloc(total);
-        QMB_HIP(hipMemcpy(blob.p, h.data(), total, hipMemcpyHostToDevice));
+        upload(ctx, blob.p, h.data(), total);
         char *d = static_cast<char *>(blob.p);
         chi = reinterpret_cast<const double2 *>(d + o_chi);
         nrm = reinterpret_cast<const double *>(d + o_nrm);
