@@ -308,17 +308,42 @@ __global__ __launch_bounds__(kThreads) void lz_update(int64_t cnt, const double 
 // The words of a small sector's matrix fit one CU's LDS beside the vector, so one
 // workgroup runs a whole window of the plain recurrence: the words, the value
 // tables and w stay in LDS (the values of an FP64 matrix are read from memory: it
-// takes the same route, so its results are the packed form's), phi_n, phi_{n-1} and y in registers, and a step has
-// two block sums instead of two launches (a 16-site ring with flip, 415 rows:
-// 3.2 us a step; launched kernel by kernel ~13 us, most of it the host's). Row
-// sums run in slot order as in spmv_sell; the sums of a[n] and b[n] run over the
-// wavefronts in order. P, the last phi, a[], b[] and 1/b[] are left in memory as
-// the kernels of larger sectors leave them, so windows, checks and checkpoints
-// are the same. init: the start vector (seeded when `random`, else P) is
-// normalised first. z: the replay that adds up x = sum_n z[n] phi_n into X and
-// ||H x - e x|| into *res.
+// takes the same route, so its results are the packed form's), phi_n, phi_{n-1} and y
+// in registers, and a step has two block sums instead of two launches. A step is a
+// chain of LDS reads and sums: with DPP sums, eight slots at a time and a wavefront a
+// chunk it takes 2.2 us (16-site ring with flip, 415 rows; 2.9 us with shuffles, four
+// slots and always 16 wavefronts; launched kernel by kernel ~13 us, most of it the
+// host's). Row sums run in slot order as in spmv_sell. P, the last phi, a[], b[] and
+// 1/b[] are left in memory as the kernels of larger sectors leave them, so windows,
+// checks and checkpoints are the same. init: the start vector (seeded when `random`,
+// else P) is normalised first. keep: phi_n goes to keep + n cnt. z: x = sum_n z[n]
+// phi_n into X and ||H x - e x|| into *res, from the kept vectors or (keep NULL) by
+// replaying the steps. host: pinned memory that takes a[n] at [n] and b[n] at [host_b +
+// n] too; it, X and res in pinned memory save a copy each.
 constexpr int kSmallThreads = 1024, kSmallWaves = kSmallThreads / 64;
 constexpr size_t kSmallLds = 140 * 1024;  // vector and words; value tables of up to 16 KB beside them
+constexpr size_t kSmallKeep = (size_t)64 << 20;  // the kept vectors of a small sector
+
+// v plus its neighbour's by a DPP move (lanes without one add 0)
+template <int CTRL, int ROWS = 0xf>
+__device__ __forceinline__ double dpp_add(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, true);
+    return v + __hiloint2double(hi, lo);
+}
+
+// Sum over the 16 lanes of a row, valid in its last lane.
+__device__ __forceinline__ double row_total(double v) {
+    v = dpp_add<0x111>(v);  // row_shr:1, 2, 4, 8
+    v = dpp_add<0x112>(v);
+    v = dpp_add<0x114>(v);
+    return dpp_add<0x118>(v);
+}
+
+__device__ __forceinline__ double read_lane(double v, int lane) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
 
 struct SmallMatrix {
     int n, n_chunks, stored, n_values, n_values_im, cb, rb;
@@ -339,17 +364,18 @@ template <bool CPLX, bool PACK, int KR>
 __global__ __launch_bounds__(kSmallThreads) void lz_small(SmallMatrix m, int it0, int steps, int init, int random,
                                                           uint64_t seed, double *P, double *V0, double *V1,
                                                           double *alpha, double *beta, double *invb,
-                                                          const double *z, double e, double *X, double *res) {
+                                                          const double *z, double e, double *X, double *res,
+                                                          double *keep, double *host, int host_b) {
     constexpr int VS = CPLX ? 2 : 1;
     extern __shared__ __align__(16) double small_lds[];
     __shared__ double red[2][kSmallWaves];
     double *x = small_lds;
     double *vt = x + (m.n * VS + 1) / 2 * 2;
     uint32_t *words = reinterpret_cast<uint32_t *>(vt + (m.n_values + m.n_values_im + 1) / 2 * 2);
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    for (int i = threadIdx.x; i < m.stored; i += kSmallThreads) words[i] = m.words[i];
-    for (int i = threadIdx.x; i < m.n_values; i += kSmallThreads) vt[i] = m.vtab[i];
-    for (int i = threadIdx.x; i < m.n_values_im; i += kSmallThreads) vt[m.n_values + i] = m.vtab[kMaxValues + i];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, n_waves = blockDim.x >> 6;
+    for (int i = threadIdx.x; i < m.stored; i += blockDim.x) words[i] = m.words[i];
+    for (int i = threadIdx.x; i < m.n_values; i += blockDim.x) vt[i] = m.vtab[i];
+    for (int i = threadIdx.x; i < m.n_values_im; i += blockDim.x) vt[m.n_values + i] = m.vtab[kMaxValues + i];
     int base[KR], L[KR], len[KR];
     double d[KR][VS], w[KR][VS], prev[KR][VS], y[KR][VS], sum[KR][VS];
 #pragma unroll
@@ -371,16 +397,14 @@ __global__ __launch_bounds__(kSmallThreads) void lz_small(SmallMatrix m, int it0
             if (r < m.n) x[i] = w[k][q];
         }
     }
-    // sum over the block, wavefronts in order, to every thread; alternate buffers
-    // leave one barrier between a buffer's readers and its next writers
+    // sum over the block, to every thread; alternate buffers leave one barrier between
+    // a buffer's readers and its next writers
     auto block_total = [&](double v, int buf) {
-        v = wave_sum(v);
-        if (lane == 0) red[buf][wv] = v;
+        v = dpp_add<0x143, 0xc>(dpp_add<0x142, 0xa>(row_total(v)));  // row_bcast:15, 31: lane 63 has all
+        if (lane == 63) red[buf][wv] = v;
         __syncthreads();
-        double t = 0.0;
-#pragma unroll
-        for (int i = 0; i < kSmallWaves; ++i) t += red[buf][i];
-        return t;
+        const int w = lane & (kSmallWaves - 1);
+        return read_lane(row_total(w < n_waves ? red[buf][w] : 0.0), 15);
     };
     // H x of the thread's rows into y (x complete in LDS)
     auto product = [&](const double (&own)[KR][VS]) {
@@ -401,14 +425,31 @@ __global__ __launch_bounds__(kSmallThreads) void lz_small(SmallMatrix m, int it0
                 y[k][0] = a.x;
                 y[k][1] = a.y;
             } else {
-                y[k][0] = PACK ? sell_row_packed<false, 4>(words, vt, x, p0, L[k], len[k], m.cb, d[k][0], own[k][0])
+                y[k][0] = PACK ? sell_row_packed<false, KR == 4 ? 4 : 8>(words, vt, x, p0, L[k], len[k], m.cb, d[k][0], own[k][0])
                                : sell_row_real<false>(reinterpret_cast<const int32_t *>(words), m.val, x, p0, L[k],
                                                       len[k]);
             }
         }
     };
+    const bool replay = !(z && keep);
     double s, b = 0.0;
-    if (init) {
+    if (!replay) {
+#pragma unroll
+        for (int k = 0; k < KR; ++k) {
+            const int r = (wv + k * kSmallWaves) * 64 + lane;
+            if (r >= m.n) continue;
+#pragma unroll
+            for (int q = 0; q < VS; ++q) {
+                const double *v = keep + r * VS + q;
+                const int64_t step = (int64_t)m.n * VS;
+                double t = 0.0;
+#pragma unroll 8
+                for (int it = 0; it < steps; ++it) t = t + z[it] * v[it * step];
+                sum[k][q] = t;
+            }
+        }
+        __syncthreads();
+    } else if (init) {
         double t = 0.0;
 #pragma unroll
         for (int k = 0; k < KR; ++k)
@@ -419,13 +460,14 @@ __global__ __launch_bounds__(kSmallThreads) void lz_small(SmallMatrix m, int it0
         if (threadIdx.x == 0) {
             invb[0] = s;
             beta[0] = 0.0;
+            if (host) host[host_b] = 0.0;
         }
     } else {
         s = invb[it0];
         b = beta[it0];
         __syncthreads();
     }
-    for (int it = it0; it < it0 + steps; ++it) {
+    for (int it = it0; replay && it < it0 + steps; ++it) {
         product(w);
         double dot = 0.0;
 #pragma unroll
@@ -451,7 +493,10 @@ __global__ __launch_bounds__(kSmallThreads) void lz_small(SmallMatrix m, int it0
                 prev[k][q] = phi;
                 w[k][q] = wi;
                 nn += wi * wi;
-                if (r < m.n) x[r * VS + q] = wi;
+                if (r < m.n) {
+                    x[r * VS + q] = wi;
+                    if (keep) keep[((int64_t)it * m.n + r) * VS + q] = phi;
+                }
             }
         }
         b = sqrt(block_total(nn, 1));
@@ -460,6 +505,10 @@ __global__ __launch_bounds__(kSmallThreads) void lz_small(SmallMatrix m, int it0
             alpha[it] = a;
             beta[it + 1] = b;
             invb[it + 1] = s;
+            if (host) {
+                host[it] = a;
+                host[host_b + it + 1] = b;
+            }
         }
     }
     double *vlast = (it0 + steps - 1) & 1 ? V1 : V0;
@@ -665,12 +714,12 @@ __global__ __launch_bounds__(kThreads) void reorth_apply(int64_t n, int64_t stri
     if (threadIdx.x == 0) partials[blockIdx.x] = t;
 }
 
-// x = sum_j z_j V_j (eigenvector from a stored basis), eight loads in flight.
+// x (+)= sum_j z_j V_j (eigenvector from a stored basis), eight loads in flight.
 __global__ __launch_bounds__(kThreads) void basis_combine(int64_t cnt, int64_t stride, int nv,
                                                           const double *__restrict__ V, const double *__restrict__ z,
-                                                          double *__restrict__ x) {
+                                                          double *__restrict__ x, int add) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < cnt; i += (int64_t)gridDim.x * blockDim.x) {
-        double s = 0.0;
+        double s = add ? x[i] : 0.0;
         int j = 0;
         for (; j + kApplyGroup <= nv; j += kApplyGroup) {
             double v[kApplyGroup];
@@ -800,7 +849,8 @@ static bool fits_small(const qmb_ell *e) {
 
 static void launch_small(qmb_ctx *ctx, const qmb_ell *e, LzWork &wk, int it0, int steps, bool init, bool random,
                          uint64_t seed, double *P, double *V0, double *V1, const double *z = nullptr, double eig = 0.0,
-                         double *X = nullptr, double *res = nullptr) {
+                         double *X = nullptr, double *res = nullptr, double *keep = nullptr,
+                         double *host = nullptr) {
     const bool cplx = e->value_type == QMB_COMPLEX;
     SmallMatrix m{};
     m.n = (int)e->n_rows;
@@ -829,8 +879,10 @@ static void launch_small(qmb_ctx *ctx, const qmb_ell *e, LzWork &wk, int it0, in
     const K k = table[cplx ? 1 : 0][e->packed ? 1 : 0][kr <= 1 ? 0 : kr <= 2 ? 1 : 2];
     const size_t lds = small_lds_bytes(e->n_rows, e->stored, cplx ? 2 : 1) +
                        small_table_bytes(m.n_values, m.n_values_im);
-    hipLaunchKernelGGL(k, dim3(1), dim3(kSmallThreads), lds, ctx->stream, m, it0, steps, init ? 1 : 0, random ? 1 : 0,
-                       seed, P, V0, V1, wk.alpha(), wk.beta(), wk.invb(), z, eig, X, res);
+    const int threads = 64 * (int)std::min<int64_t>(kSmallWaves, e->n_chunks);
+    hipLaunchKernelGGL(k, dim3(1), dim3(threads), lds, ctx->stream, m, it0, steps, init ? 1 : 0, random ? 1 : 0,
+                       seed, P, V0, V1, wk.alpha(), wk.beta(), wk.invb(), z, eig, X, res,
+                       keep, host, wk.M);
     QMB_HIP(hipGetLastError());
 }
 
@@ -902,6 +954,14 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
     const double tol = o.tol > 0 ? o.tol : 1e-13;
     QMB_HIP(hipSetDevice(ctx->device));
     const unsigned rblocks = grid_for(n, kThreads * 4);
+    // An eigenvector of the plain recurrence: phi_n is kept instead of overwritten for
+    // as many steps as a quarter of the free memory holds, in blocks made as the run
+    // reaches them, and the vector is combined from them at the end. A run that goes
+    // beyond repeats all its steps for it, as one with a checkpoint file does (28 sites with
+    // J2, 717K rows, energy and vector: 6357 us by repeating, 3347 by keeping).
+    constexpr int kKeepBlock = 16;
+    std::vector<DevBuf> kept;
+    int64_t keep_most = 0;  // phi_n with n below it are kept
     {
         // the plan's vectors, refused up front when they cannot fit in device memory:
         // w, H phi, zero, then phi_{n-1}, phi_n or every kept phi_n with its coefficients
@@ -919,7 +979,12 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
                           need / 1e9, reorth ? M : 2, (double)cnt * sizeof(double) / 1e9, avail / 1e9);
             throw Error{QMB_ERR_OOM, msg};
         }
+        if (o.want_eigvec && !reorth && !small && !ck)
+            keep_most = (int64_t)std::min((double)M, (avail - need) / 4 / ((double)cnt * sizeof(double)));
     }
+    DevBuf small_keep;
+    if (o.want_eigvec && small && !ck && (size_t)M * cnt * sizeof(double) <= kSmallKeep)
+        small_keep.alloc((size_t)M * cnt * sizeof(double));
     LzWork wk;
     wk.init(ctx, M, !small);
     DevBuf P(cnt * sizeof(double)), Y(cnt * sizeof(double)), Z(cnt * sizeof(double));
@@ -938,6 +1003,16 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
     }
     auto vcur = [&](int it) -> double * {
         if (reorth) return VB.as<double>() + (size_t)it * cnt;
+        if (it < keep_most) {
+            if ((size_t)(it / kKeepBlock) < kept.size())
+                return kept[it / kKeepBlock].as<double>() + (size_t)(it % kKeepBlock) * cnt;
+            try {
+                kept.emplace_back((size_t)kKeepBlock * cnt * sizeof(double));
+                return kept.back().as<double>();
+            } catch (const Error &) {  // taken by another program meanwhile
+                keep_most = it;
+            }
+        }
         return (it & 1) ? V1.as<double>() : V0.as<double>();
     };
     auto vprev = [&](int it) -> const double * {
@@ -1258,7 +1333,8 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
         const int win1 = std::min(M, it + next);
         if (small) {
             launch_small(ctx, e, wk, win0, win1 - win0, win0 == 0, random_start, o.seed, P.as<double>(),
-                         V0.as<double>(), V1.as<double>());
+                         V0.as<double>(), V1.as<double>(), nullptr, 0.0, nullptr, nullptr,
+                         small_keep.as<double>(), ctx->host_stage<double>((size_t)(2 * M + 1) * sizeof(double)));
             it = it_q = win1;
             b_ready[it] = 1;
         }
@@ -1269,12 +1345,18 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
         // into pinned memory
         const size_t span = (size_t)M + it + 1;
         double *st = ctx->host_stage<double>(span * sizeof(double));
-        QMB_HIP(hipMemcpyAsync(st, wk.alpha(), span * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-        QMB_HIP(hipEventRecord(ev_copy, ctx->stream));
-        if (can_queue_ahead && !predicted && it < M) queue_step(it, 0, wpar ^ 1, true);
-        QMB_HIP(hipEventSynchronize(ev_copy));
-        std::copy(st, st + it, ha.begin());
-        std::copy(st + M, st + M + it + 1, hb.begin());
+        const bool direct = small && !ck;  // the window's kernel has written its part there
+        if (direct) {
+            QMB_HIP(hipStreamSynchronize(ctx->stream));
+        } else {
+            QMB_HIP(hipMemcpyAsync(st, wk.alpha(), span * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+            QMB_HIP(hipEventRecord(ev_copy, ctx->stream));
+            if (can_queue_ahead && !predicted && it < M) queue_step(it, 0, wpar ^ 1, true);
+            QMB_HIP(hipEventSynchronize(ev_copy));
+        }
+        const int from = direct ? win0 : 0;
+        std::copy(st + from, st + it, ha.begin() + from);
+        std::copy(st + M + from + (from > 0), st + M + it + 1, hb.begin() + from + (from > 0));
         if (o.profile) {
             for (int q = 0; q < it - win0; ++q) {
                 if (!timed(win0 + q)) continue;
@@ -1365,7 +1447,7 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
                 QMB_HIP(hipMemcpyAsync(dz, zs.data() + (size_t)slot * M, (size_t)m * sizeof(double),
                                        hipMemcpyHostToDevice, ctx->stream));
                 hipLaunchKernelGGL(basis_combine, dim3(grid_for(cnt, kThreads * 4)), dim3(kThreads), 0, ctx->stream,
-                                   cnt, (int64_t)cnt, m, VB.as<double>(), dz, GV.as<double>() + (size_t)slot * cnt);
+                                   cnt, (int64_t)cnt, m, VB.as<double>(), dz, GV.as<double>() + (size_t)slot * cnt, 0);
                 QMB_HIP(hipGetLastError());
                 good_theta.push_back(theta);
                 ++added;
@@ -1415,16 +1497,36 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
             DevBuf dz(m * sizeof(double));
             QMB_HIP(hipMemcpyAsync(dz.p, z0.data(), m * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
             hipLaunchKernelGGL(basis_combine, dim3(grid_for(cnt, kThreads * 4)), dim3(kThreads), 0, ctx->stream, cnt,
-                               (int64_t)cnt, m, VB.as<double>(), dz.as<double>(), X.as<double>());
+                               (int64_t)cnt, m, VB.as<double>(), dz.as<double>(), X.as<double>(), 0);
             QMB_HIP(hipGetLastError());
         } else if (small) {
+            // z, x and the residual in pinned memory; a replay reads z every step
+            double *hz = ctx->host_stage<double>((size_t)(m + cnt + 1) * sizeof(double));
+            std::copy(z0.begin(), z0.begin() + m, hz);
+            const double *z = hz;
+            DevBuf dz;
+            if (!small_keep.p) {
+                dz.alloc(m * sizeof(double));
+                QMB_HIP(hipMemcpyAsync(dz.p, hz, m * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
+                z = dz.as<double>();
+                init_start();
+            }
+            launch_small(ctx, e, wk, 0, m, true, random_start, o.seed, P.as<double>(), V0.as<double>(),
+                         V1.as<double>(), z, evals[0], hz + m, hz + m + cnt, small_keep.as<double>());
+            QMB_HIP(hipStreamSynchronize(ctx->stream));
+            eig_res = hz[m + cnt];
+            if (eigvec) std::copy(hz + m, hz + m + cnt, eigvec);
+        } else if (m <= keep_most) {
             DevBuf dz(m * sizeof(double));
             double *hz = ctx->host_stage<double>(m * sizeof(double));
             std::copy(z0.begin(), z0.begin() + m, hz);
             QMB_HIP(hipMemcpyAsync(dz.p, hz, m * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-            init_start();
-            launch_small(ctx, e, wk, 0, m, true, random_start, o.seed, P.as<double>(), V0.as<double>(),
-                         V1.as<double>(), dz.as<double>(), evals[0], X.as<double>(), wk.misc() + 1);
+            for (int j = 0; j < m; j += kKeepBlock) {
+                hipLaunchKernelGGL(basis_combine, dim3(grid_for(cnt, kThreads * 4)), dim3(kThreads), 0, ctx->stream,
+                                   cnt, (int64_t)cnt, std::min(kKeepBlock, m - j), kept[j / kKeepBlock].as<double>(),
+                                   dz.as<double>() + j, X.as<double>(), j > 0 ? 1 : 0);
+                QMB_HIP(hipGetLastError());
+            }
         } else {
             QMB_HIP(hipMemsetAsync(X.p, 0, cnt * sizeof(double), ctx->stream));
             QMB_HIP(hipMemsetAsync(Z.p, 0, cnt * sizeof(double), ctx->stream));
@@ -1443,11 +1545,13 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
             launch_spmv(ctx, e, X.as<double>(), Y.as<double>(), false, nullptr, nullptr, nullptr, nullptr);
             launch_norm(ctx, cnt, Y.as<double>(), X.as<double>(), evals[0], wk, wk.misc() + 1, wk.misc() + 2);
         }
-        QMB_HIP(hipMemcpyAsync(&eig_res, wk.misc() + 1, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-        if (eigvec)
-            download(ctx, eigvec, X.p, cnt * sizeof(double));
-        else
-            QMB_HIP(hipStreamSynchronize(ctx->stream));
+        if (!small) {
+            QMB_HIP(hipMemcpyAsync(&eig_res, wk.misc() + 1, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+            if (eigvec)
+                download(ctx, eigvec, X.p, cnt * sizeof(double));
+            else
+                QMB_HIP(hipStreamSynchronize(ctx->stream));
+        }
         n_spmv += m + 1;
     }
     if (rep) {
