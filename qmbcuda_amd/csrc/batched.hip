@@ -3,19 +3,18 @@
 // Q/exact_diagonalization/HeisenbergGenericXXZ_AbelianSymms_CUDA.cu:127-229).
 //
 // All instances advance in lockstep with one iteration counter on the device.
-// Every phase is ONE launch covering every instance: a block task table maps
-// each block to (instance, chunk or element range); each instance owns a
-// contiguous block range, so its dot products are reduced deterministically by
-// a finishing kernel with one block per instance. Instances with real and complex matrices form two
-// families with their own kernel instantiations. A chunk of iterations is
+// Every phase is ONE launch covering every instance, real and complex: a block task
+// table maps each block to (instance, chunk or element range); each instance owns a
+// contiguous block range, so its dot products are reduced deterministically, by the
+// blocks of the next kernel or one block per instance. A chunk of iterations is
 // captured once as a HIP graph and replayed; between replays the host solves
 // the tridiagonal problems and clears the active flag of converged instances
 // (their blocks return at once). With reorthogonalisation the Krylov vectors are
 // kept and every new vector is orthogonalised against them by classical
 // Gram-Schmidt, a second time only for the instances whose first pass removed
 // most of the norm (decided on the device, so the graph stays fixed).
-// SpMV tile shape (chunks per block) is picked per family by timing the
-// candidates on the actual batch (autotuner with a per-process cache).
+// SpMV tile shape (chunks per block) is picked by timing the candidates on the
+// actual batch (autotuner with a per-process cache).
 #include <algorithm>
 #include <chrono>
 #include <cmath>
@@ -25,6 +24,7 @@
 #include <mutex>
 #include <thread>
 #include <tuple>
+#include <type_traits>
 
 #include "internal.hpp"
 #include "reduce.hpp"
@@ -38,12 +38,12 @@ struct BInst {
     const int32_t *col;
     const double *val;
     const double *diag, *vtab;   // packed values (packed = 1): diagonal, value table(s)
-    int packed, col_bits, re_bits;
+    int packed, col_bits, re_bits, cplx;
     int64_t n_rows, n_chunks;
     double *P, *Y, *VB;          // w, H phi, Krylov basis [M][n*vs] (two slots, it & 1, without reorthogonalisation)
     double *alpha, *beta, *invb;  // [M], [M+1], [M+1]
     double *coef;                 // [M*2] reorthogonalisation coefficients
-    double *gate;                 // [1] second Gram-Schmidt pass wanted (1) or not (0)
+    double *gate;                 // [2] second Gram-Schmidt pass wanted (1) or not (0); ||w|| after the first
     double *pro;                  // [3] this step orthogonalises (1/0), second-step flag, steps that did
     double *omega;                // [3][M+2] orthogonality estimates (partial reorthogonalisation)
     int spmv_first, spmv_nblk;
@@ -56,7 +56,7 @@ __device__ inline size_t vb_slot(const BInst &I, int it) { return (size_t)(I.vb_
 
 struct BTask {
     int inst;
-    int pad;
+    int cplx;
     int64_t lo, hi;
 };
 
@@ -64,17 +64,13 @@ struct BTask {
 // 8 per thread 3 % slower, 16 per thread 17 % slower, 2 per thread equal)
 constexpr int kVecPerBlock = kThreads * 4;
 
+// The iteration of a launch: a graph holds a chunk of iterations, launch q of each
+// phase belongs to iteration *it_p + q, and the counter advances once a chunk.
+//
 // NT: matrix stream past the caches (nontemporal) or plain loads; U: slots per
 // group of the packed row products. Both are picked by the autotuner.
 template <bool CPLX, bool NT, int U>
-__global__ __launch_bounds__(kThreads) void bk_spmv(const BInst *__restrict__ insts, const BTask *__restrict__ tasks,
-                                                    const int *__restrict__ active, const int *__restrict__ it_p,
-                                                    double *__restrict__ part) {
-    __shared__ double lds[kWaves];
-    const BTask t = tasks[blockIdx.x];
-    if (!active[t.inst]) return;
-    const BInst I = insts[t.inst];
-    const int it = *it_p;
+__device__ __forceinline__ double spmv_rows(const BTask &t, const BInst &I, int it) {
     const double s = I.invb[it];
     const int vs = CPLX ? 2 : 1;
     double *vout = I.VB + vb_slot(I, it) * I.n_rows * vs;
@@ -112,14 +108,25 @@ __global__ __launch_bounds__(kThreads) void bk_spmv(const BInst *__restrict__ in
             a.y *= s;
             if (r < I.n_rows) {
                 reinterpret_cast<double2 *>(I.Y)[r] = a;
-                double2 vr = reinterpret_cast<const double2 *>(I.P)[r];
-                vr.x = vr.x * s;
-                vr.y = vr.y * s;
+                const double2 vr = make_double2(xr.x * s, xr.y * s);
                 reinterpret_cast<double2 *>(vout)[r] = vr;
                 dot += vr.x * a.x + vr.y * a.y;
             }
         }
     }
+    return dot;
+}
+
+template <bool NT, int U>
+__global__ __launch_bounds__(kThreads) void bk_spmv(const BInst *__restrict__ insts, const BTask *__restrict__ tasks,
+                                                    const int *__restrict__ active, const int *__restrict__ it_p,
+                                                    int q, double *__restrict__ part) {
+    __shared__ double lds[kWaves];
+    const BTask t = tasks[blockIdx.x];
+    if (!active[t.inst]) return;
+    const int it = *it_p + q;
+    const BInst I = insts[t.inst];
+    const double dot = t.cplx ? spmv_rows<true, NT, U>(t, I, it) : spmv_rows<false, NT, U>(t, I, it);
     const double tb = block_sum(dot, lds);
     if (threadIdx.x == 0) part[blockIdx.x] = tb;
 }
@@ -128,109 +135,124 @@ __global__ __launch_bounds__(kThreads) void bk_spmv(const BInst *__restrict__ in
 // of the norm (Daniel, Gragg, Kaufman, Stewart 1976).
 constexpr double kDgks = 0.7071067811865476;
 
-// One block per instance of the family: fixed-order sum of the instance's block
-// partials. mode 0: alpha[it] = s; 1: beta[it+1] = sqrt(s), invb[it+1];
-// 2 (start vector): invb[0] = 1/sqrt(s), beta[0] = 0; 3 (after the first
-// Gram-Schmidt pass): as 1, and gate = 1 if sqrt(s) < kDgks * the old
-// beta[it+1]; 4 (after the second pass): as 1 where the gate is 1.
-__global__ __launch_bounds__(kThreads) void bk_finish(const BInst *__restrict__ insts, const int *__restrict__ active,
-                                                      const int *__restrict__ it_p, const double *__restrict__ part,
-                                                      int first_inst, int mode) {
-    __shared__ double lds[kWaves];
-    const int inst = first_inst + blockIdx.x;
-    if (active && !active[inst]) return;
-    const BInst I = insts[inst];
-    if ((mode == 3 || mode == 4) && I.pro[0] == 0.0) return;
-    if (mode == 4 && *I.gate == 0.0) return;
-    const int it = it_p ? *it_p : 0;
-    const int first = mode == 0 ? I.spmv_first : I.vec_first;
-    const int nblk = mode == 0 ? I.spmv_nblk : I.vec_nblk;
+// The fixed-order sum of an instance's block partials, to every thread.
+__device__ inline double instance_sum(const double *part, int first, int nblk, double *lds, double *all) {
     const double s = sum_partials(part + first, nblk, lds);
-    if (threadIdx.x == 0) {
-        if (mode == 0) {
-            I.alpha[it] = s;
-        } else if (mode == 1 || mode == 3 || mode == 4) {
-            const double nb = sqrt(s);
-            if (mode == 3) *I.gate = nb < kDgks * I.beta[it + 1] ? 1.0 : 0.0;
-            I.beta[it + 1] = nb;
-            I.invb[it + 1] = nb > 0.0 ? 1.0 / nb : 0.0;
-        } else {
-            const double nr = sqrt(s);
-            I.invb[0] = nr > 0.0 ? 1.0 / nr : 0.0;
-            I.beta[0] = 0.0;
-        }
-    }
+    if (threadIdx.x == 0) *all = s;
+    __syncthreads();
+    return *all;
 }
 
-// w = (-a) phi_it + (y + (-b) phi_{it-1}); ||w|| -> beta[it+1]. Ranges are in doubles.
+// One block per instance, after the start vector (start: invb[0] = 1/||w||, beta[0] =
+// 0) or after a second Gram-Schmidt pass (beta[it+1] and invb[it+1], where the gate is 1).
+__global__ __launch_bounds__(kThreads) void bk_finish(const BInst *__restrict__ insts, const int *__restrict__ active,
+                                                      const int *__restrict__ it_p, int q,
+                                                      const double *__restrict__ part, int start) {
+    __shared__ double lds[kWaves];
+    const int inst = blockIdx.x;
+    if (!start && !active[inst]) return;
+    const BInst I = insts[inst];
+    if (!start && (I.pro[0] == 0.0 || I.gate[0] == 0.0)) return;
+    const double nb = sqrt(sum_partials(part + I.vec_first, I.vec_nblk, lds));
+    if (threadIdx.x != 0) return;
+    const int at = start ? 0 : *it_p + q + 1;
+    I.beta[at] = start ? 0.0 : nb;
+    I.invb[at] = nb > 0.0 ? 1.0 / nb : 0.0;
+}
+
+// w = (-a) phi_it + (y + (-b) phi_{it-1}) and the partials of ||w||^2. a is summed by
+// every block from its instance's SpMV partials (spart; the first block stores it).
+// Ranges are in doubles.
 __global__ __launch_bounds__(kThreads) void bk_update(const BInst *__restrict__ insts, const BTask *__restrict__ tasks,
                                                       const int *__restrict__ active, const int *__restrict__ it_p,
-                                                      double *__restrict__ part, int vs) {
-    __shared__ double lds[kWaves];
+                                                      int q, const double *__restrict__ spart,
+                                                      double *__restrict__ part) {
+    __shared__ double lds[kWaves], all;
     const BTask t = tasks[blockIdx.x];
     if (!active[t.inst]) return;
     const BInst I = insts[t.inst];
-    const int it = *it_p;
-    const int64_t cnt = I.n_rows * vs;
-    const double a = I.alpha[it], b = I.beta[it];
-    const double *v = I.VB + vb_slot(I, it) * cnt;
-    const double *vp = it > 0 ? I.VB + vb_slot(I, it - 1) * cnt : nullptr;
+    const int it = *it_p + q;
+    const int64_t cnt = I.n_rows * (t.cplx ? 2 : 1);
+    const double b = I.beta[it];
+    const double *__restrict__ v = I.VB + vb_slot(I, it) * cnt;
+    const double *__restrict__ vp = it > 0 ? I.VB + vb_slot(I, it - 1) * cnt : nullptr;
+    const double *__restrict__ y = I.Y;
+    // the first four elements a thread are loaded while a is summed
+    double rv[4], rp[4], ry[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int64_t i = t.lo + threadIdx.x + u * kThreads;
+        const bool in = i < t.hi;
+        rv[u] = in ? v[i] : 0.0;
+        rp[u] = in && vp ? vp[i] : 0.0;
+        ry[u] = in ? y[i] : 0.0;
+    }
+    const double a = instance_sum(spart, I.spmv_first, I.spmv_nblk, lds, &all);
+    if ((int)blockIdx.x == I.vec_first && threadIdx.x == 0) I.alpha[it] = a;
     double acc = 0.0;
-    for (int64_t i = t.lo + threadIdx.x; i < t.hi; i += blockDim.x) {
-        const double tt = vp ? I.Y[i] + (-b) * vp[i] : I.Y[i] + (-b) * 0.0;
-        const double wi = (-a) * v[i] + tt;
+    auto step = [&](int64_t i, double vi, double pi, double yi) {
+        const double wi = (-a) * vi + (yi + (-b) * pi);
         I.P[i] = wi;
         acc += wi * wi;
+    };
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int64_t i = t.lo + threadIdx.x + u * kThreads;
+        if (i < t.hi) step(i, rv[u], rp[u], ry[u]);
     }
+    for (int64_t i = t.lo + threadIdx.x + 4 * kThreads; i < t.hi; i += kThreads)
+        step(i, v[i], vp ? vp[i] : 0.0, y[i]);
     const double tb = block_sum(acc, lds);
     if (threadIdx.x == 0) part[blockIdx.x] = tb;
 }
 
-// Reorthogonalisation launch shape: blockIdx.y = 0..kJY-1 splits the Krylov
-// index, and a block takes kJB vectors per pass over its range (w read once,
-// one combined reduction for the kJB dots).
+// Reorthogonalisation launch shape: blockIdx.y = 0..kJY-1 splits the Krylov index
+// (1, 2, 4, 8: 62.6, 59.6, 58.4, 58.7 ms for 72 sectors of 24 sites, 6.7, 6.1, 5.7,
+// 5.7 for 40 of 20), and a block takes kJB vectors per pass over its range (w read
+// once, one combined reduction for the kJB dots).
 constexpr int kJY = 8;
 constexpr int kJB = 4;
 
-// part2[(j*nbv + block)*2 + {0,1}] = <V_j, w> over the block's range, j <= it.
-// Per dot: thread-strided sums, wave shuffles, then the waves in order.
 template <bool CPLX>
-__global__ __launch_bounds__(kThreads) void bk_rdots(const BInst *__restrict__ insts, const BTask *__restrict__ tasks,
-                                                     const int *__restrict__ active, const int *__restrict__ it_p,
-                                                     double *__restrict__ part2, int nbv, int gated) {
-    __shared__ double lds[kWaves * kJB * 2];
-    const BTask t = tasks[blockIdx.x];
-    if (!active[t.inst]) return;
-    const BInst I = insts[t.inst];
-    if (I.pro[0] == 0.0 || (gated && *I.gate == 0.0)) return;
-    const int it = *it_p;
-    const int vs = CPLX ? 2 : 1;
-    const int64_t cnt = I.n_rows * vs;
+__device__ __forceinline__ void dots_of(const BTask &t, const BInst &I, int it, double *__restrict__ part2, int nbv,
+                                        double *lds) {
+    using T = std::conditional_t<CPLX, double2, double>;
+    const int64_t n = I.n_rows;
+    const int64_t lo = CPLX ? t.lo / 2 : t.lo, hi = CPLX ? t.hi / 2 : t.hi;
+    const T *__restrict__ w = reinterpret_cast<const T *>(I.P);
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    for (int j0 = (int)blockIdx.y * kJB; j0 <= it; j0 += kJY * kJB) {
+    for (int j0 = (int)blockIdx.y * kJB; j0 <= it; j0 += (int)gridDim.y * kJB) {
         const int nj = min(kJB, it + 1 - j0);
+        const T *vj[kJB];  // past the last vector: the last one again, not used
+#pragma unroll
+        for (int u = 0; u < kJB; ++u) vj[u] = reinterpret_cast<const T *>(I.VB) + (size_t)(j0 + min(u, nj - 1)) * n;
         double sr[kJB], si[kJB];
 #pragma unroll
         for (int u = 0; u < kJB; ++u) sr[u] = si[u] = 0.0;
-        if (CPLX) {
-            for (int64_t i = t.lo / 2 + threadIdx.x; i < t.hi / 2; i += blockDim.x) {
-                const double wr = I.P[2 * i], wi = I.P[2 * i + 1];
+        // two elements of each of the kJB vectors in flight
+        for (int64_t i0 = lo + threadIdx.x; i0 < hi; i0 += 2 * kThreads) {
+            const bool two = i0 + kThreads < hi;
+            const int64_t i1 = two ? i0 + kThreads : i0;
+            const T w0 = w[i0], w1 = w[i1];
+            T v0[kJB], v1[kJB];
 #pragma unroll
-                for (int u = 0; u < kJB; ++u) {
-                    if (u < nj) {
-                        const double *vj = I.VB + (size_t)(j0 + u) * cnt;
-                        const double vr = vj[2 * i], vi = vj[2 * i + 1];
-                        sr[u] += vr * wr + vi * wi;
-                        si[u] += vr * wi - vi * wr;
-                    }
-                }
+            for (int u = 0; u < kJB; ++u) {
+                v0[u] = vj[u][i0];
+                v1[u] = vj[u][i1];
             }
-        } else {
-            for (int64_t i = t.lo + threadIdx.x; i < t.hi; i += blockDim.x) {
-                const double w = I.P[i];
 #pragma unroll
-                for (int u = 0; u < kJB; ++u)
-                    if (u < nj) sr[u] += I.VB[(size_t)(j0 + u) * cnt + i] * w;
+            for (int u = 0; u < kJB; ++u) {
+                if constexpr (CPLX) {
+                    sr[u] += v0[u].x * w0.x + v0[u].y * w0.y;
+                    si[u] += v0[u].x * w0.y - v0[u].y * w0.x;
+                    if (two) {
+                        sr[u] += v1[u].x * w1.x + v1[u].y * w1.y;
+                        si[u] += v1[u].x * w1.y - v1[u].y * w1.x;
+                    }
+                } else {
+                    sr[u] += v0[u] * w0;
+                    if (two) sr[u] += v1[u] * w1;
+                }
             }
         }
 #pragma unroll
@@ -248,24 +270,62 @@ __global__ __launch_bounds__(kThreads) void bk_rdots(const BInst *__restrict__ i
         if ((int)threadIdx.x < 2 * nj) {
             const int u = (int)threadIdx.x >> 1, c = (int)threadIdx.x & 1;
             double tot = 0.0;
-            for (int w = 0; w < kWaves; ++w) tot += lds[(w * kJB + u) * 2 + c];
+            for (int x = 0; x < kWaves; ++x) tot += lds[(x * kJB + u) * 2 + c];
             part2[((size_t)(j0 + u) * nbv + blockIdx.x) * 2 + c] = tot;
         }
         __syncthreads();
     }
 }
 
+// part2[(j*nbv + block)*2 + {0,1}] = <V_j, w> over the block's range, j <= it.
+// Per dot: thread-strided sums, wave shuffles, then the waves in order. second: every
+// block sums ||w|| after the first pass and decides whether its instance has a second
+// one (the first block of the instance stores both).
+__global__ __launch_bounds__(kThreads) void bk_rdots(const BInst *__restrict__ insts, const BTask *__restrict__ tasks,
+                                                     const int *__restrict__ active, const int *__restrict__ it_p,
+                                                     int q, const double *__restrict__ part,
+                                                     double *__restrict__ part2, int nbv, int second) {
+    __shared__ double lds[kWaves * kJB * 2], all;
+    const BTask t = tasks[blockIdx.x];
+    if (!active[t.inst]) return;
+    const BInst I = insts[t.inst];
+    if (I.pro[0] == 0.0) return;
+    const int it = *it_p + q;
+    if (second) {
+        const double nb = sqrt(instance_sum(part, I.vec_first, I.vec_nblk, lds, &all));
+        const bool again = nb < kDgks * I.beta[it + 1];
+        if ((int)blockIdx.x == I.vec_first && blockIdx.y == 0 && threadIdx.x == 0) {
+            I.gate[0] = again ? 1.0 : 0.0;
+            I.gate[1] = nb;
+        }
+        if (!again) return;
+    }
+    if (t.cplx)
+        dots_of<true>(t, I, it, part2, nbv, lds);
+    else
+        dots_of<false>(t, I, it, part2, nbv, lds);
+}
+
 // coef_j = sum of the instance's block partials in a fixed order (lane-strided
 // sums, then wave shuffles): one wavefront per Krylov index j, gridDim.y blocks
-// of kWaves wavefronts per instance.
+// of kWaves wavefronts per instance. second: also beta[it+1] and invb[it+1] of the
+// first pass.
 __global__ __launch_bounds__(kThreads) void bk_rreduce(const BInst *__restrict__ insts, const int *__restrict__ active,
-                                                       const int *__restrict__ it_p, const double *__restrict__ part2,
-                                                       int nbv, int first_inst, int gated) {
-    const int inst = first_inst + blockIdx.x;
+                                                       const int *__restrict__ it_p, int q,
+                                                       const double *__restrict__ part2, int nbv, int second) {
+    const int inst = blockIdx.x;
     if (!active[inst]) return;
     const BInst I = insts[inst];
-    if (I.pro[0] == 0.0 || (gated && *I.gate == 0.0)) return;
-    const int it = *it_p;
+    if (I.pro[0] == 0.0) return;
+    const int it = *it_p + q;
+    if (second) {
+        if (blockIdx.y == 0 && threadIdx.x == 0) {
+            const double nb = I.gate[1];
+            I.beta[it + 1] = nb;
+            I.invb[it + 1] = nb > 0.0 ? 1.0 / nb : 0.0;
+        }
+        if (I.gate[0] == 0.0) return;
+    }
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     for (int j = (int)blockIdx.y * kWaves + wv; j <= it; j += (int)gridDim.y * kWaves) {
         const double *pj = part2 + ((size_t)j * nbv + I.vec_first) * 2;
@@ -283,87 +343,74 @@ __global__ __launch_bounds__(kThreads) void bk_rreduce(const BInst *__restrict__
     }
 }
 
-// w -= sum_j coef_j V_j (j in order; four vectors loaded per step), ||w||^2 partials.
+constexpr int kRapplyAhead = 8;
+
 template <bool CPLX>
+__device__ __forceinline__ double apply_of(const BTask &t, const BInst &I, int it) {
+    using T = std::conditional_t<CPLX, double2, double>;
+    const int64_t n = I.n_rows;
+    const int64_t lo = CPLX ? t.lo / 2 : t.lo, hi = CPLX ? t.hi / 2 : t.hi;
+    T *w = reinterpret_cast<T *>(I.P);
+    const T *__restrict__ V = reinterpret_cast<const T *>(I.VB);
+    const double *__restrict__ coef = I.coef;
+    double acc = 0.0;
+    for (int64_t i = lo + threadIdx.x; i < hi; i += kThreads) {
+        T x = w[i];
+        auto take = [&](int j, T v) {
+            if constexpr (CPLX) {
+                const double cr = coef[2 * j], ci = coef[2 * j + 1];
+                x.x -= cr * v.x - ci * v.y;
+                x.y -= cr * v.y + ci * v.x;
+            } else {
+                x -= coef[2 * j] * v;
+            }
+        };
+        int j = 0;
+        for (; j + kRapplyAhead <= it + 1; j += kRapplyAhead) {
+            T v[kRapplyAhead];
+#pragma unroll
+            for (int u = 0; u < kRapplyAhead; ++u) v[u] = V[(size_t)(j + u) * n + i];
+#pragma unroll
+            for (int u = 0; u < kRapplyAhead; ++u) take(j + u, v[u]);
+        }
+        for (; j <= it; ++j) take(j, V[(size_t)j * n + i]);
+        w[i] = x;
+        if constexpr (CPLX)
+            acc += x.x * x.x + x.y * x.y;
+        else
+            acc += x * x;
+    }
+    return acc;
+}
+
+// w -= sum_j coef_j V_j (j in order; eight vectors loaded ahead), ||w||^2 partials.
 __global__ __launch_bounds__(kThreads) void bk_rapply(const BInst *__restrict__ insts, const BTask *__restrict__ tasks,
                                                       const int *__restrict__ active, const int *__restrict__ it_p,
-                                                      double *__restrict__ part, int gated) {
+                                                      int q, double *__restrict__ part, int second) {
     __shared__ double lds[kWaves];
     const BTask t = tasks[blockIdx.x];
     if (!active[t.inst]) return;
     const BInst I = insts[t.inst];
-    if (I.pro[0] == 0.0 || (gated && *I.gate == 0.0)) return;
-    const int it = *it_p;
-    const int vs = CPLX ? 2 : 1;
-    const int64_t cnt = I.n_rows * vs;
-    double acc = 0.0;
-    if (CPLX) {
-        for (int64_t i = t.lo / 2 + threadIdx.x; i < t.hi / 2; i += blockDim.x) {
-            double wr = I.P[2 * i], wi = I.P[2 * i + 1];
-            int j = 0;
-            for (; j + 4 <= it + 1; j += 4) {
-                double vr[4], vi[4];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    vr[u] = I.VB[(size_t)(j + u) * cnt + 2 * i];
-                    vi[u] = I.VB[(size_t)(j + u) * cnt + 2 * i + 1];
-                }
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const double cr = I.coef[2 * (j + u)], ci = I.coef[2 * (j + u) + 1];
-                    wr -= cr * vr[u] - ci * vi[u];
-                    wi -= cr * vi[u] + ci * vr[u];
-                }
-            }
-            for (; j <= it; ++j) {
-                const double cr = I.coef[2 * j], ci = I.coef[2 * j + 1];
-                const double vr = I.VB[(size_t)j * cnt + 2 * i], vi = I.VB[(size_t)j * cnt + 2 * i + 1];
-                wr -= cr * vr - ci * vi;
-                wi -= cr * vi + ci * vr;
-            }
-            I.P[2 * i] = wr;
-            I.P[2 * i + 1] = wi;
-            acc += wr * wr + wi * wi;
-        }
-    } else {
-        for (int64_t i = t.lo + threadIdx.x; i < t.hi; i += blockDim.x) {
-            double wr = I.P[i];
-            int j = 0;
-            for (; j + 4 <= it + 1; j += 4) {
-                double v[4];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) v[u] = I.VB[(size_t)(j + u) * cnt + i];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) wr -= I.coef[2 * (j + u)] * v[u];
-            }
-            for (; j <= it; ++j) wr -= I.coef[2 * j] * I.VB[(size_t)j * cnt + i];
-            I.P[i] = wr;
-            acc += wr * wr;
-        }
-    }
-    const double tb = block_sum(acc, lds);
+    if (I.pro[0] == 0.0 || (second && I.gate[0] == 0.0)) return;
+    const int it = *it_p + q;
+    const double tb = block_sum(t.cplx ? apply_of<true>(t, I, it) : apply_of<false>(t, I, it), lds);
     if (threadIdx.x == 0) part[blockIdx.x] = tb;
 }
 
 // Partial reorthogonalisation on the device (H. D. Simon, Math. Comp. 42 (1984)
-// 115-142), one wavefront per instance of the family: the estimates
+// 115-142), by one wavefront: the estimates
 // om_{j+1,k} of <phi_{j+1}, phi_k> follow the Lanczos recurrence,
 //   b[j+1] om_{j+1,k} = b[k+1] om_{j,k+1} + (a[k] - a[j]) om_{j,k} + b[k] om_{j,k-1} - b[j] om_{j-1,k},
 // plus a rounding term eps1 = eps sqrt(n); when one passes sqrt(eps), this
 // step and the next orthogonalise (pro[0] = 1) and the estimates restart at
 // eps1. Rows of omega rotate by step parity (j+1, j, j-1 mod 3).
-__global__ __launch_bounds__(64) void bk_pro(const BInst *__restrict__ insts, const int *__restrict__ active,
-                                             const int *__restrict__ it_p, int first_inst, int M) {
-    const int inst = first_inst + blockIdx.x;
-    if (!active[inst]) return;
-    const BInst I = insts[inst];
-    const int j = *it_p, lane = threadIdx.x;
+__device__ inline void estimate_loss(const BInst &I, int j, double bj1, int M) {
+    const int lane = threadIdx.x;
     const int64_t stride = M + 2;
     double *om_next = I.omega + (size_t)((j + 1) % 3) * stride;
     const double *om_cur = I.omega + (size_t)(j % 3) * stride;
     const double *om_prev = I.omega + (size_t)((j + 2) % 3) * stride;
     const double eps1 = 2.220446049250313e-16 * sqrt((double)I.n_rows);
-    const double bj1 = I.beta[j + 1];
     double worst = 0.0;
     for (int k = lane; k < j; k += 64) {
         double t = I.beta[k + 1] * om_cur[k + 1] + (I.alpha[k] - I.alpha[j]) * om_cur[k] - I.beta[j] * om_prev[k];
@@ -388,13 +435,31 @@ __global__ __launch_bounds__(64) void bk_pro(const BInst *__restrict__ insts, co
     }
 }
 
-__global__ void bk_advance(int *it_p) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) *it_p = *it_p + 1;
+// One block per instance: beta[it+1] = ||w|| and its inverse, then (partial) the
+// estimates that decide on this step's Gram-Schmidt passes.
+__global__ __launch_bounds__(kThreads) void bk_norm(const BInst *__restrict__ insts, const int *__restrict__ active,
+                                                    const int *__restrict__ it_p, int q,
+                                                    const double *__restrict__ part, int partial, int M) {
+    __shared__ double lds[kWaves], all;
+    const int inst = blockIdx.x;
+    if (!active[inst]) return;
+    const BInst I = insts[inst];
+    const int it = *it_p + q;
+    const double nb = sqrt(instance_sum(part, I.vec_first, I.vec_nblk, lds, &all));
+    if (threadIdx.x == 0) {
+        I.beta[it + 1] = nb;
+        I.invb[it + 1] = nb > 0.0 ? 1.0 / nb : 0.0;
+    }
+    if (partial && threadIdx.x < 64) estimate_loss(I, it, nb, M);
+}
+
+__global__ void bk_advance(int *it_p, int steps) {
+    if (threadIdx.x == 0 && blockIdx.x == 0) *it_p = *it_p + steps;
 }
 
 // start vectors and their norms (outside the graph)
 __global__ __launch_bounds__(kThreads) void bk_start(const BInst *__restrict__ insts, const BTask *__restrict__ tasks,
-                                                     double *__restrict__ part, uint64_t seed, int vs) {
+                                                     double *__restrict__ part, uint64_t seed) {
     __shared__ double lds[kWaves];
     const BTask t = tasks[blockIdx.x];
     const BInst I = insts[t.inst];
@@ -406,35 +471,22 @@ __global__ __launch_bounds__(kThreads) void bk_start(const BInst *__restrict__ i
     }
     const double tb = block_sum(acc, lds);
     if (threadIdx.x == 0) part[blockIdx.x] = tb;
-    (void)vs;
 }
 
-struct Family {
-    bool cplx = false;
-    std::vector<int> members;  // instance indices (global numbering)
-    int first_inst = 0;        // position of the family's first instance in the device BInst array
-    std::vector<BTask> spmv_tasks, vec_tasks;
-    DevBuf d_spmv_tasks, d_vec_tasks;
-    int spmv_first_block = 0, vec_first_block = 0;
-    int cpb = 4;      // chunks per block
-    int variant = 0;  // index into spmv_variants()
-};
+using SpmvKernel = void (*)(const BInst *, const BTask *, const int *, const int *, int, double *);
 
-using SpmvKernel = void (*)(const BInst *, const BTask *, const int *, const int *, double *);
-
-// The SpMV shapes the autotuner chooses among, per family: (stream policy,
-// slots per group). Entry 0 is the streamed 8-slot form.
+// The SpMV shapes the autotuner chooses among: (stream policy, slots per group). Entry 0 is the streamed 8-slot form.
 struct SpmvVariant {
     bool nt;
     int slots;
-    SpmvKernel real, cplx;
+    SpmvKernel kernel;
 };
 static const std::vector<SpmvVariant> &spmv_variants() {
     static const std::vector<SpmvVariant> v = {
-        {true, 8, bk_spmv<false, true, 8>, bk_spmv<true, true, 8>},
-        {true, 4, bk_spmv<false, true, 4>, bk_spmv<true, true, 4>},
-        {false, 4, bk_spmv<false, false, 4>, bk_spmv<true, false, 4>},
-        {false, 8, bk_spmv<false, false, 8>, bk_spmv<true, false, 8>},
+        {true, 8, bk_spmv<true, 8>},
+        {true, 4, bk_spmv<true, 4>},
+        {false, 4, bk_spmv<false, 4>},
+        {false, 8, bk_spmv<false, 8>},
     };
     return v;
 }
@@ -443,7 +495,7 @@ struct TileChoice {
     int cpb, variant;
 };
 
-// (complex, log2 rows, instances) -> tile choice; shared by every context of the
+// (complex instances, log2 rows, instances) -> tile choice; shared by every context of the
 // process, hence the lock
 static std::map<std::tuple<int, int, int>, TileChoice> g_tile_cache;
 static std::mutex g_tile_mutex;
@@ -473,6 +525,7 @@ __global__ __launch_bounds__(kThreads) void bk_combine(int64_t cnt, int m, const
                                                        const double *__restrict__ z, double *__restrict__ x) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < cnt; i += (int64_t)gridDim.x * blockDim.x) {
         double s = 0.0;
+#pragma unroll 8
         for (int j = 0; j < m; ++j) s = s + z[j] * V[(size_t)j * cnt + i];
         x[i] = s;
     }
@@ -502,23 +555,13 @@ static void run_batched(qmb_ctx *ctx, int n, const qmb_ell *const *ells, const q
         const bool partial = o.reorth == 2;  // device-side decisions (bk_pro)
         const int k_eigs = o.n_eigs;
 
-        // families: real first, then complex
-        Family fam[2];
-        fam[0].cplx = false;
-        fam[1].cplx = true;
-        for (int i = 0; i < n; ++i) fam[ells[i]->value_type == QMB_COMPLEX ? 1 : 0].members.push_back(i);
-        std::vector<int> order;  // device instance position -> global index
-        for (auto &f : fam) {
-            f.first_inst = (int)order.size();
-            for (int i : f.members) order.push_back(i);
-        }
         // per-instance device buffers
         std::vector<BInst> hin(n);
         std::vector<DevBuf> bufs;
         bufs.reserve((size_t)n * 6);
         DevBuf scal((size_t)n * (3 * M + 2) * sizeof(double));
         DevBuf coefs((size_t)n * M * 2 * sizeof(double));
-        DevBuf gates((size_t)n * sizeof(double));
+        DevBuf gates((size_t)n * 2 * sizeof(double));
         QMB_HIP(hipMemsetAsync(scal.p, 0, scal.bytes, ctx->stream));
         QMB_HIP(hipMemsetAsync(gates.p, 0, gates.bytes, ctx->stream));
         // orthogonality estimates: row 0 = om_0 = e_0, rows 1, 2 zero; flags:
@@ -536,7 +579,7 @@ static void run_batched(qmb_ctx *ctx, int n, const qmb_ell *const *ells, const q
             }
         }
         for (int pos = 0; pos < n; ++pos) {
-            const qmb_ell *e = ells[order[pos]];
+            const qmb_ell *e = ells[pos];
             const int vs = e->value_type == QMB_COMPLEX ? 2 : 1;
             const int64_t cnt = e->n_rows * vs;
             BInst &I = hin[pos];
@@ -547,6 +590,7 @@ static void run_batched(qmb_ctx *ctx, int n, const qmb_ell *const *ells, const q
             I.diag = e->diag.as<double>();
             I.vtab = e->vtab.as<double>();
             I.packed = e->packed;
+            I.cplx = vs == 2;
             I.re_bits = e->re_bits;
             I.col_bits = e->col_bits;
             I.n_rows = e->n_rows;
@@ -564,40 +608,31 @@ static void run_batched(qmb_ctx *ctx, int n, const qmb_ell *const *ells, const q
             I.beta = sc + M;
             I.invb = sc + 2 * M + 1;
             I.coef = coefs.as<double>() + (size_t)pos * M * 2;
-            I.gate = gates.as<double>() + pos;
+            I.gate = gates.as<double>() + 2 * (size_t)pos;
             I.pro = pros.as<double>() + 3 * (size_t)pos;
             I.omega = partial ? omegas.as<double>() + (size_t)pos * 3 * om_stride : nullptr;
         }
-        // vector task tables (ranges in doubles, both families in one table per family)
-        int total_vec_blocks = 0;
-        for (auto &f : fam) {
-            f.vec_first_block = total_vec_blocks;
-            for (size_t q = 0; q < f.members.size(); ++q) {
-                const int pos = f.first_inst + (int)q;
-                const qmb_ell *e = ells[order[pos]];
-                const int64_t cnt = e->n_rows * (f.cplx ? 2 : 1);
-                const int64_t per = f.cplx ? 2 * kVecPerBlock : kVecPerBlock;  // keep complex pairs together
-                hin[pos].vec_first = total_vec_blocks;
-                int nb = 0;
-                for (int64_t lo = 0; lo < cnt; lo += per, ++nb)
-                    f.vec_tasks.push_back(BTask{pos, 0, lo, std::min<int64_t>(cnt, lo + per)});
-                hin[pos].vec_nblk = nb;
-                total_vec_blocks += nb;
-            }
+        // task tables: vector ranges in doubles, SpMV ranges in chunks
+        std::vector<BTask> vec_tasks, spmv_tasks;
+        for (int pos = 0; pos < n; ++pos) {
+            BInst &I = hin[pos];
+            const int64_t cnt = I.n_rows * (I.cplx ? 2 : 1);
+            const int64_t per = I.cplx ? 2 * kVecPerBlock : kVecPerBlock;  // keep complex pairs together
+            I.vec_first = (int)vec_tasks.size();
+            for (int64_t lo = 0; lo < cnt; lo += per)
+                vec_tasks.push_back(BTask{pos, I.cplx, lo, std::min<int64_t>(cnt, lo + per)});
+            I.vec_nblk = (int)vec_tasks.size() - I.vec_first;
         }
-        const int nbv = total_vec_blocks;
-        auto build_spmv_tasks = [&](Family &f, int cpb, int &first_block_io) {
-            f.spmv_tasks.clear();
-            f.spmv_first_block = first_block_io;
-            for (size_t q = 0; q < f.members.size(); ++q) {
-                const int pos = f.first_inst + (int)q;
-                hin[pos].spmv_first = first_block_io + (int)f.spmv_tasks.size();
-                int nb = 0;
-                for (int64_t lo = 0; lo < hin[pos].n_chunks; lo += cpb, ++nb)
-                    f.spmv_tasks.push_back(BTask{pos, 0, lo, std::min<int64_t>(hin[pos].n_chunks, lo + cpb)});
-                hin[pos].spmv_nblk = nb;
+        const int nbv = (int)vec_tasks.size();
+        auto build_spmv_tasks = [&](int cpb) {
+            spmv_tasks.clear();
+            for (int pos = 0; pos < n; ++pos) {
+                BInst &I = hin[pos];
+                I.spmv_first = (int)spmv_tasks.size();
+                for (int64_t lo = 0; lo < I.n_chunks; lo += cpb)
+                    spmv_tasks.push_back(BTask{pos, I.cplx, lo, std::min<int64_t>(I.n_chunks, lo + cpb)});
+                I.spmv_nblk = (int)spmv_tasks.size() - I.spmv_first;
             }
-            first_block_io += (int)f.spmv_tasks.size();
         };
         // device tables
         DevBuf d_inst((size_t)n * sizeof(BInst)), d_active((size_t)n * sizeof(int)), d_it(sizeof(int));
@@ -605,47 +640,28 @@ static void run_batched(qmb_ctx *ctx, int n, const qmb_ell *const *ells, const q
         const int zero = 0;
         QMB_HIP(hipMemcpyAsync(d_it.p, &zero, sizeof(int), hipMemcpyHostToDevice, ctx->stream));
         QMB_HIP(hipMemcpyAsync(d_active.p, active.data(), n * sizeof(int), hipMemcpyHostToDevice, ctx->stream));
-        for (auto &f : fam) {
-            if (f.vec_tasks.empty()) continue;
-            f.d_vec_tasks.alloc(f.vec_tasks.size() * sizeof(BTask));
-            QMB_HIP(hipMemcpy(f.d_vec_tasks.p, f.vec_tasks.data(), f.vec_tasks.size() * sizeof(BTask),
-                              hipMemcpyHostToDevice));
-        }
-        // partial slots: block ids are offsets into one array per phase type
+        DevBuf d_vec_tasks(vec_tasks.size() * sizeof(BTask)), d_spmv_tasks;
+        QMB_HIP(hipMemcpy(d_vec_tasks.p, vec_tasks.data(), vec_tasks.size() * sizeof(BTask), hipMemcpyHostToDevice));
+        // partial sums by block of the SpMV and of the vector phases
         int64_t max_spmv_blocks = 0;
-        for (auto &f : fam)
-            for (int i : f.members) max_spmv_blocks += ells[i]->n_chunks;
-        DevBuf part((size_t)std::max<int64_t>(max_spmv_blocks, nbv) * sizeof(double) + 64);
+        for (int i = 0; i < n; ++i) max_spmv_blocks += ells[i]->n_chunks;
+        DevBuf spart((size_t)max_spmv_blocks * sizeof(double)), part((size_t)nbv * sizeof(double));
         DevBuf part2(reorth ? (size_t)M * nbv * 2 * sizeof(double) : 64);
 
         auto upload_inst = [&]() {
             QMB_HIP(hipMemcpy(d_inst.p, hin.data(), n * sizeof(BInst), hipMemcpyHostToDevice));
         };
-        // start vectors: per family, the vector task table; block ids must index `part`
+        // start vectors
         upload_inst();
-        for (auto &f : fam) {
-            if (f.vec_tasks.empty()) continue;
-            // bk_start uses blockIdx.x as the partial slot: launch with the family's table, slots offset
-            // by shifting the instance's vec_first to the family-local numbering
-            std::vector<BInst> local = hin;
-            for (size_t q = 0; q < f.members.size(); ++q) local[f.first_inst + q].vec_first -= f.vec_first_block;
-            DevBuf d_local((size_t)n * sizeof(BInst));
-            QMB_HIP(hipMemcpy(d_local.p, local.data(), n * sizeof(BInst), hipMemcpyHostToDevice));
-            hipLaunchKernelGGL(bk_start, dim3((unsigned)f.vec_tasks.size()), dim3(kThreads), 0, ctx->stream,
-                               d_local.as<BInst>(), f.d_vec_tasks.as<BTask>(), part.as<double>(), o.seed,
-                               f.cplx ? 2 : 1);
-            QMB_HIP(hipGetLastError());
-            hipLaunchKernelGGL(bk_finish, dim3((unsigned)f.members.size()), dim3(kThreads), 0, ctx->stream,
-                               d_local.as<BInst>(), nullptr, nullptr, part.as<double>(), f.first_inst, 2);
-            QMB_HIP(hipGetLastError());
-            QMB_HIP(hipStreamSynchronize(ctx->stream));
-        }
-        // The vector-phase kernels address `part` by family-local block id; make the
-        // instance descriptors family-local for the vector ranges.
-        for (auto &f : fam)
-            for (size_t q = 0; q < f.members.size(); ++q) hin[f.first_inst + q].vec_first -= f.vec_first_block;
+        hipLaunchKernelGGL(bk_start, dim3((unsigned)nbv), dim3(kThreads), 0, ctx->stream, d_inst.as<BInst>(),
+                           d_vec_tasks.as<BTask>(), part.as<double>(), o.seed);
+        QMB_HIP(hipGetLastError());
+        hipLaunchKernelGGL(bk_finish, dim3((unsigned)n), dim3(kThreads), 0, ctx->stream, d_inst.as<BInst>(), nullptr,
+                           nullptr, 0, part.as<double>(), 1);
+        QMB_HIP(hipGetLastError());
+        QMB_HIP(hipStreamSynchronize(ctx->stream));
 
-        // autotune the SpMV shape per family: the four kernel variants (stream
+        // autotune the SpMV shape: the four kernel variants (stream
         // policy x slots per group) at 4 chunks per block, then chunks per block
         // halved or doubled from there while that helps, under the best variant;
         // each candidate timed over 2 launches, every variant launched once
@@ -653,17 +669,15 @@ static void run_batched(qmb_ctx *ctx, int n, const qmb_ell *const *ells, const q
         // sectors, real and complex), this search found the fastest shape each
         // time with 6-8 candidates; timing all 24, with a warm launch and 3 timed
         // ones each, took as long as the 72-sector solve itself.
-        for (auto &f : fam) {
-            if (f.members.empty()) continue;
-            int64_t rows = 0;
-            for (int i : f.members) rows += ells[i]->n_rows;
-            const auto key = std::make_tuple((int)f.cplx, (int)std::log2((double)rows + 1.0), (int)f.members.size());
-            TileChoice tc{};
-            if (tile_cache_get(key, tc)) {
-                f.cpb = tc.cpb;
-                f.variant = tc.variant;
-                continue;
-            }
+        int n_cplx = 0;
+        int64_t rows = 0;
+        for (const BInst &I : hin) {
+            n_cplx += I.cplx;
+            rows += I.n_rows;
+        }
+        const auto key = std::make_tuple(n_cplx, (int)std::log2((double)rows + 1.0), n);
+        TileChoice tile{4, 0};
+        if (!tile_cache_get(key, tile)) {
             float best = 1e30f;
             TileChoice best_c{4, 0};
             hipEvent_t ea = nullptr, eb = nullptr;
@@ -685,25 +699,24 @@ static void run_batched(qmb_ctx *ctx, int n, const qmb_ell *const *ells, const q
                 const auto it = tried.find({cpb, vi});
                 if (it != tried.end()) return it->second;
                 if (cpb != cur_cpb) {
-                    int fb = 0;
-                    build_spmv_tasks(f, cpb, fb);
+                    build_spmv_tasks(cpb);
                     upload_inst();
-                    dt.alloc(f.spmv_tasks.size() * sizeof(BTask));
-                    QMB_HIP(hipMemcpy(dt.p, f.spmv_tasks.data(), f.spmv_tasks.size() * sizeof(BTask),
+                    dt.alloc(spmv_tasks.size() * sizeof(BTask));
+                    QMB_HIP(hipMemcpy(dt.p, spmv_tasks.data(), spmv_tasks.size() * sizeof(BTask),
                                       hipMemcpyHostToDevice));
                     cur_cpb = cpb;
                 }
-                const SpmvKernel k = f.cplx ? vars[vi].cplx : vars[vi].real;
-                const dim3 grid((unsigned)f.spmv_tasks.size());
+                const SpmvKernel k = vars[vi].kernel;
+                const dim3 grid((unsigned)spmv_tasks.size());
                 if (!warm[vi]) {
                     hipLaunchKernelGGL(k, grid, dim3(kThreads), 0, ctx->stream, d_inst.as<BInst>(), dt.as<BTask>(),
-                                       d_active.as<int>(), d_it.as<int>(), part.as<double>());
+                                       d_active.as<int>(), d_it.as<int>(), 0, spart.as<double>());
                     warm[vi] = 1;
                 }
                 QMB_HIP(hipEventRecord(ea, ctx->stream));
                 for (int rep = 0; rep < 2; ++rep)
                     hipLaunchKernelGGL(k, grid, dim3(kThreads), 0, ctx->stream, d_inst.as<BInst>(), dt.as<BTask>(),
-                                       d_active.as<int>(), d_it.as<int>(), part.as<double>());
+                                       d_active.as<int>(), d_it.as<int>(), 0, spart.as<double>());
                 QMB_HIP(hipEventRecord(eb, ctx->stream));
                 QMB_HIP(hipEventSynchronize(eb));
                 float t = 0.f;
@@ -725,68 +738,46 @@ static void run_batched(qmb_ctx *ctx, int n, const qmb_ell *const *ells, const q
                     c = nc;
                 }
             }
-            f.cpb = best_c.cpb;
-            f.variant = best_c.variant;
+            tile = best_c;
             tile_cache_put(key, best_c);
         }
-        // final SpMV task tables; spmv block ids are family-local too
-        for (auto &f : fam) {
-            if (f.members.empty()) continue;
-            int fb = 0;
-            build_spmv_tasks(f, f.cpb, fb);
-            f.d_spmv_tasks.alloc(f.spmv_tasks.size() * sizeof(BTask));
-            QMB_HIP(hipMemcpy(f.d_spmv_tasks.p, f.spmv_tasks.data(), f.spmv_tasks.size() * sizeof(BTask),
-                              hipMemcpyHostToDevice));
-        }
+        build_spmv_tasks(tile.cpb);
+        d_spmv_tasks.alloc(spmv_tasks.size() * sizeof(BTask));
+        QMB_HIP(hipMemcpy(d_spmv_tasks.p, spmv_tasks.data(), spmv_tasks.size() * sizeof(BTask), hipMemcpyHostToDevice));
         upload_inst();
         // tuning ran real SpMVs at it = 0: restore the state the first iteration expects
         QMB_HIP(hipMemcpyAsync(d_it.p, &zero, sizeof(int), hipMemcpyHostToDevice, ctx->stream));
 
-        // one iteration = every family's phases, then the counter advance
-        auto enqueue_iteration = [&](hipStream_t s) {
-            for (auto &f : fam) {
-                if (f.members.empty()) continue;
-                const unsigned nbs = (unsigned)f.spmv_tasks.size(), nvb = (unsigned)f.vec_tasks.size();
-                const int vs = f.cplx ? 2 : 1;
-                const unsigned nm = (unsigned)f.members.size();
-                const SpmvKernel ks = f.cplx ? spmv_variants()[f.variant].cplx : spmv_variants()[f.variant].real;
-                hipLaunchKernelGGL(ks, dim3(nbs), dim3(kThreads), 0, s, d_inst.as<BInst>(), f.d_spmv_tasks.as<BTask>(),
-                                   d_active.as<int>(), d_it.as<int>(), part.as<double>());
-                hipLaunchKernelGGL(bk_finish, dim3(nm), dim3(kThreads), 0, s, d_inst.as<BInst>(), d_active.as<int>(),
-                                   d_it.as<int>(), part.as<double>(), f.first_inst, 0);
-                hipLaunchKernelGGL(bk_update, dim3(nvb), dim3(kThreads), 0, s, d_inst.as<BInst>(),
-                                   f.d_vec_tasks.as<BTask>(), d_active.as<int>(), d_it.as<int>(), part.as<double>(),
-                                   vs);
-                hipLaunchKernelGGL(bk_finish, dim3(nm), dim3(kThreads), 0, s, d_inst.as<BInst>(), d_active.as<int>(),
-                                   d_it.as<int>(), part.as<double>(), f.first_inst, 1);
-                if (partial)
-                    hipLaunchKernelGGL(bk_pro, dim3(nm), dim3(64), 0, s, d_inst.as<BInst>(), d_active.as<int>(),
-                                       d_it.as<int>(), f.first_inst, M);
-                if (reorth) {
-                    for (int pass = 0; pass < 2; ++pass) {
-                        hipLaunchKernelGGL(f.cplx ? bk_rdots<true> : bk_rdots<false>, dim3(nvb, kJY), dim3(kThreads), 0,
-                                           s, d_inst.as<BInst>(), f.d_vec_tasks.as<BTask>(), d_active.as<int>(),
-                                           d_it.as<int>(), part2.as<double>(), (int)nvb, pass);
-                        hipLaunchKernelGGL(bk_rreduce, dim3((unsigned)f.members.size(), 4), dim3(kThreads), 0, s,
-                                           d_inst.as<BInst>(), d_active.as<int>(), d_it.as<int>(), part2.as<double>(),
-                                           (int)nvb, f.first_inst, pass);
-                        hipLaunchKernelGGL(f.cplx ? bk_rapply<true> : bk_rapply<false>, dim3(nvb), dim3(kThreads), 0,
-                                           s, d_inst.as<BInst>(), f.d_vec_tasks.as<BTask>(), d_active.as<int>(),
-                                           d_it.as<int>(), part.as<double>(), pass);
-                        // pass 0 decides whether pass 1 runs, per instance, on the device
-                        hipLaunchKernelGGL(bk_finish, dim3(nm), dim3(kThreads), 0, s, d_inst.as<BInst>(),
-                                           d_active.as<int>(), d_it.as<int>(), part.as<double>(), f.first_inst,
-                                           pass ? 4 : 3);
-                    }
-                }
+        // iteration *it_p + q. A launch of a phase costs some 4 us here whatever its
+        // instances do, so what one block per instance would sum is summed by the
+        // blocks that need it, and real and complex instances share the launches (72
+        // sectors of 24 sites 65.3 / 58.5 ms, 24 sectors of 16 sites 5.3 / 3.2).
+        const SpmvKernel ks = spmv_variants()[tile.variant].kernel;
+        const unsigned nbs = (unsigned)spmv_tasks.size(), nm = (unsigned)n;
+        const BInst *di = d_inst.as<BInst>();
+        const BTask *ds = d_spmv_tasks.as<BTask>(), *dv = d_vec_tasks.as<BTask>();
+        const int *da = d_active.as<int>(), *dit = d_it.as<int>();
+        double *sp = spart.as<double>(), *vp = part.as<double>(), *p2 = part2.as<double>();
+        auto enqueue_iteration = [&](hipStream_t s, int q) {
+            hipLaunchKernelGGL(ks, dim3(nbs), dim3(kThreads), 0, s, di, ds, da, dit, q, sp);
+            hipLaunchKernelGGL(bk_update, dim3((unsigned)nbv), dim3(kThreads), 0, s, di, dv, da, dit, q, sp, vp);
+            hipLaunchKernelGGL(bk_norm, dim3(nm), dim3(kThreads), 0, s, di, da, dit, q, vp, partial ? 1 : 0, M);
+            if (!reorth) return;
+            // pass 0 decides whether pass 1 runs, per instance, on the device
+            for (int pass = 0; pass < 2; ++pass) {
+                hipLaunchKernelGGL(bk_rdots, dim3((unsigned)nbv, kJY), dim3(kThreads), 0, s, di, dv, da, dit, q, vp, p2,
+                                   nbv, pass);
+                hipLaunchKernelGGL(bk_rreduce, dim3(nm, 4), dim3(kThreads), 0, s, di, da, dit, q, p2, nbv, pass);
+                hipLaunchKernelGGL(bk_rapply, dim3((unsigned)nbv), dim3(kThreads), 0, s, di, dv, da, dit, q, vp, pass);
             }
-            hipLaunchKernelGGL(bk_advance, dim3(1), dim3(64), 0, s, d_it.as<int>());
+            hipLaunchKernelGGL(bk_finish, dim3(nm), dim3(kThreads), 0, s, di, da, dit, q, vp, 0);
         };
         hipGraph_t graph = nullptr;
         hipGraphExec_t exec = nullptr;
         QMB_HIP(hipStreamSynchronize(ctx->stream));
         QMB_HIP(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-        for (int q = 0; q < chunk; ++q) enqueue_iteration(ctx->stream);
+        for (int q = 0; q < chunk; ++q) enqueue_iteration(ctx->stream, q);
+        hipLaunchKernelGGL(bk_advance, dim3(1), dim3(64), 0, ctx->stream, d_it.as<int>(), chunk);
         QMB_HIP(hipStreamEndCapture(ctx->stream, &graph));
         QMB_HIP(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
 
@@ -952,11 +943,10 @@ static void run_batched(qmb_ctx *ctx, int n, const qmb_ell *const *ells, const q
                                ctx->stream));
         QMB_HIP(hipStreamSynchronize(ctx->stream));
         for (int pos = 0; pos < n; ++pos) {
-            const int gi = order[pos];
-            for (int j = 0; j < k_eigs; ++j) evals[(size_t)gi * k_eigs + j] = ev[pos][j];
+            for (int j = 0; j < k_eigs; ++j) evals[(size_t)pos * k_eigs + j] = ev[pos][j];
             all_conv = all_conv && conv[pos];
             if (reports) {
-                qmb_lanczos_report &r = reports[gi];
+                qmb_lanczos_report &r = reports[pos];
                 std::memset(&r, 0, sizeof(r));
                 r.iters = iters[pos];
                 r.converged = conv[pos];
@@ -975,8 +965,7 @@ static void run_batched(qmb_ctx *ctx, int n, const qmb_ell *const *ells, const q
             // steps after convergence wrote only slots past their own m)
             DevBuf dz((size_t)M * sizeof(double));
             for (int pos = 0; pos < n; ++pos) {
-                const int gi = order[pos];
-                const qmb_ell *e = ells[gi];
+                const qmb_ell *e = ells[pos];
                 const int64_t cnt = e->n_rows * (e->value_type == QMB_COMPLEX ? 2 : 1);
                 const int m = (int)zvec[pos].size();
                 DevBuf X((size_t)cnt * sizeof(double));
@@ -990,7 +979,7 @@ static void run_batched(qmb_ctx *ctx, int n, const qmb_ell *const *ells, const q
                 } else {
                     QMB_HIP(hipMemsetAsync(X.p, 0, (size_t)cnt * sizeof(double), ctx->stream));
                 }
-                download(ctx, vecs[gi], X.p, (size_t)cnt * sizeof(double));  // waits: dz and X are reused or freed next
+                download(ctx, vecs[pos], X.p, (size_t)cnt * sizeof(double));  // waits: dz and X are reused or freed next
             }
         }
         if (!all_conv) throw Error{QMB_ERR_NOT_CONVERGED, "qmb_lanczos_batched: some instances did not converge"};
