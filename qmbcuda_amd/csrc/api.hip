@@ -355,38 +355,42 @@ __global__ __launch_bounds__(64) void chunk_stats_final(const int64_t *nnz_parti
     out[3] = err ? *err : 0;
 }
 
-// The whole of it for at most kScanOne chunks, by one block: widths (each wavefront
-// eight chunks at a time), offsets and statistics: one launch instead of three, which
-// are bound by their launches (a build with this and fewer other launches and waits:
-// 415 rows 168 -> 118 us, 56,450 rows 202 -> 181).
+// The whole of it for at most kScanOne chunks, by one block, a chunk a thread: widths,
+// offsets and statistics in one launch instead of three, which are bound by their
+// launches (a build with this and fewer other launches and waits: 415 rows 168 ->
+// 118 us, 56,450 rows 202 -> 149).
 constexpr int kScanOne = 1024;
 
 __global__ __launch_bounds__(kScanOne) void chunk_scan_one(const uint16_t *row_len, int64_t n_rows, int n_chunks,
                                                            int64_t *chunk_ptr, const int *err, int64_t *out) {
     constexpr int kWv = kScanOne / 64;
-    __shared__ int s_max[kScanOne];
     __shared__ int64_t s_sum[kWv], s_off[kWv];
     __shared__ int s_top[kWv];
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-    int64_t sum = 0;
-    for (int c0 = wv * 8; c0 < n_chunks; c0 += kWv * 8) {
-        int l[8];
+    int sum_c = 0, top = 0;
+    auto take = [&](int l) {
+        sum_c += l;
+        top = max(top, l);
+    };
+    const int64_t r0 = (int64_t)t * kChunk;
+    if (r0 + kChunk <= n_rows) {
+        const uint4 *p = reinterpret_cast<const uint4 *>(row_len + r0);
+        uint4 v[kChunk / 8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int64_t r = (int64_t)(c0 + u) * kChunk + lane;
-            l[u] = r < n_rows ? (int)row_len[r] : 0;
-        }
+        for (int i = 0; i < kChunk / 8; ++i) v[i] = p[i];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            sum += l[u];
-            for (int off = 32; off > 0; off >>= 1) l[u] = max(l[u], __shfl_xor(l[u], off, 64));
-            if (lane == 0 && c0 + u < n_chunks) s_max[c0 + u] = l[u];
-        }
+        for (int i = 0; i < kChunk / 8; ++i)
+            for (const uint32_t w : {v[i].x, v[i].y, v[i].z, v[i].w}) {
+                take((int)(w & 0xFFFFu));
+                take((int)(w >> 16));
+            }
+    } else {
+        for (int64_t r = r0; r < n_rows; ++r) take((int)row_len[r]);
     }
+    int64_t sum = sum_c;
     for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
     if (lane == 0) s_sum[wv] = sum;
     __syncthreads();
-    int top = t < n_chunks ? s_max[t] : 0;
     const int64_t width = (int64_t)kChunk * top;
     const int64_t incl = wave_inclusive(width);
     for (int off = 32; off > 0; off >>= 1) top = max(top, __shfl_xor(top, off, 64));
