@@ -607,14 +607,14 @@ __host__ __device__ __forceinline__ int64_t colex_rank_nib(S x, const T *tab, in
     return r;
 }
 
-// The nibble rank table in LDS, formed by the block from the binomial table (no
+// The nibble rank table in LDS, formed by the block from the staged binomial rows (no
 // entry for sites past n_sites is read).
 template <class S>
-__device__ inline void stage_rank_nib(typename RankOf<S>::T *tab, const uint64_t *bin, int n_sites, int n_nib,
-                                      int n_c) {
+__device__ inline void stage_rank_nib(typename RankOf<S>::T *tab, const typename RankOf<S>::T *bin, int n_sites,
+                                      int n_nib, int n_c) {
     for (int i = threadIdx.x; i < n_nib * n_c * 16; i += blockDim.x) {
         const int v = i & 15, c = (i >> 4) % n_c, k = (i >> 4) / n_c;
-        uint64_t r = 0;
+        typename RankOf<S>::T r = 0;
         int j = c;
 #pragma unroll
         for (int q = 0; q < 4; ++q)
@@ -622,7 +622,7 @@ __device__ inline void stage_rank_nib(typename RankOf<S>::T *tab, const uint64_t
                 ++j;
                 if (4 * k + q < n_sites && j < kBinJ) r += bin[(4 * k + q) * kBinJ + j];
             }
-        tab[i] = (typename RankOf<S>::T)r;
+        tab[i] = r;
     }
 }
 

@@ -37,12 +37,12 @@
 namespace qmb {
 
 constexpr int kExpThreads = 256;
-constexpr int kExpMaxBlocks = 2048;  // eight a CU
+constexpr int kExpMaxBlocks = 4096;  // 2048: 87 us for 82 (28 sites)
 constexpr size_t kExpRankBytes = 16 * 1024;  // the nibble rank table's LDS
 constexpr int kExpLdsTerms = 256;
 
 // A product of Sz alone: 24 B and not a whole TermC, so that the few hundred of a
-// structure factor stay in the scalar cache (378 terms, 717K rows: 188 / 108 us).
+// structure factor stay in the scalar cache (378 terms, 717K rows: 188 / 94 us).
 struct SzTerm {
     uint64_t sz;
     double2 coef;
@@ -53,6 +53,7 @@ struct SzTerm {
 struct ExpectTerms {
     int n_off, n_terms, n_sz;
     int imag;  // some coefficient has an imaginary part
+    int half;  // Hermitian, t[0, n_off) holds only the terms that raise the state
     const TermC *t;
     const SzTerm *z;
 };
@@ -75,9 +76,9 @@ __device__ __forceinline__ double signed_coef(double c, S down, S sz) {
 // passes 64 terms are tested at a time (uniform loads) and each lane then looks its
 // own candidates up, so that almost all lanes are busy, with the terms and the rank
 // table in LDS and the orbit search of the group's form (LUT). 28 sites, 717K rows,
-// 14 lookups a row: 147 us. AVG: every image of
-// the representative under the group; taken only when the operator's average has
-// too many terms to be formed on the host (ExpectTable).
+// seven lookups a row (half): 82 us; with all 14, 147. AVG: every image of the
+// representative under the group; taken only when the operator's average has too many
+// terms to be formed on the host (ExpectTable).
 template <class S, bool CPLX, bool AVG, int LUT>
 __global__ __launch_bounds__(kExpThreads, AVG ? 1 : 8) void expect_rows(
     GroupView gv, const uint64_t *binom, int n_nib, int n_c, int layout, int64_t n_rows, const uint64_t *reps,
@@ -102,10 +103,8 @@ __global__ __launch_bounds__(kExpThreads, AVG ? 1 : 8) void expect_rows(
         stage_images<S>(perm_lds, gv);
     }
     stage_orbit(gt, gv);
-    if (n_nib)
-        stage_rank_nib<S>(rank, binom, gv.n_sites, n_nib, n_c);
-    else
-        stage_binom_rows<S>(rank, binom, gv.n_sites);
+    R *bin = n_nib ? rank + n_nib * n_c * 16 : rank;
+    stage_binom_rows<S>(bin, binom, gv.n_sites);
     for (int i = threadIdx.x; i < n_lds; i += blockDim.x) {
         const TermC &tm = tv.t[i];
         off[i] = ExpectOff<S>{tm.coef, (S)tm.set, (S)tm.set_val, (S)tm.sz, 0};
@@ -113,6 +112,10 @@ __global__ __launch_bounds__(kExpThreads, AVG ? 1 : 8) void expect_rows(
     for (int i = threadIdx.x; i < gv.G; i += blockDim.x) s_chi[i] = chi[i];
     for (int i = threadIdx.x; i <= gv.G; i += blockDim.x) s_nrm[i] = nrm[i];
     __syncthreads();
+    if (n_nib) {
+        stage_rank_nib<S>(rank, bin, gv.n_sites, n_nib, n_c);
+        __syncthreads();
+    }
     const uint8_t *images = AVG && gv.lut >= 3 ? img_lds : perm_lds;
     double out_r = 0.0, out_i = 0.0;
     for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < n_rows;
@@ -165,6 +168,7 @@ __global__ __launch_bounds__(kExpThreads, AVG ? 1 : 8) void expect_rows(
                         n_nib ? colex_rank_nib<S>(rep2, rank, n_nib, n_c) : colex_rank<S>(rep2, rank), dict);
                     if (r2 < 0) continue;
                     if (layout == QMB_LAYOUT_REFERENCE && nullf[r2]) continue;
+                    if (tv.half && r2 < r) continue;
                     const double cr = signed_coef<S>(o.coef.x, down, o.sz), ci = signed_coef<S>(o.coef.y, down, o.sz);
                     // f = c * conj(chi(j)) * chi(gm) * n_t / n_r; mult = the target row's stabiliser size
                     double2 q = s_chi[gm];
@@ -172,7 +176,8 @@ __global__ __launch_bounds__(kExpThreads, AVG ? 1 : 8) void expect_rows(
                         const double2 cj = s_chi[j];
                         q = make_double2(cj.x * q.x + cj.y * q.y, cj.x * q.y - cj.y * q.x);
                     }
-                    const double ratio = mult == m_src ? 1.0 : s_nrm[mult] / s_nrm[m_src];
+                    double ratio = mult == m_src ? 1.0 : s_nrm[mult] / s_nrm[m_src];
+                    if (tv.half && r2 > r) ratio *= 2.0;
                     const double fr = (cr * q.x - ci * q.y) * ratio, fi = (cr * q.y + ci * q.x) * ratio;
                     if (CPLX) {
                         const double xr = x[2 * r2], xi = x[2 * r2 + 1];
@@ -198,7 +203,7 @@ __global__ __launch_bounds__(kExpThreads, AVG ? 1 : 8) void expect_rows(
     const double si = block_sum(out_i * scale, red);
     if (threadIdx.x == 0) {
         partials[2 * blockIdx.x] = sr;
-        partials[2 * blockIdx.x + 1] = si;
+        partials[2 * blockIdx.x + 1] = tv.half ? 0.0 : si;
     }
 }
 
@@ -262,6 +267,32 @@ private:
         }
     }
 };
+
+// T^dagger on the masks: the condition and the values set change places (a term sets
+// every site of its condition but those of projectors, which it sets to what they are).
+static TermC term_adjoint(const TermC &c) {
+    TermC d = c;
+    d.req_val = (c.req_val & ~c.set) | (c.set_val & c.set);
+    d.set_val = c.req_val & c.set;
+    d.coef = make_double2(c.coef.x, -c.coef.y);
+    return d;
+}
+
+// Whether distinct terms come with their adjoints' conjugate coefficients, exactly.
+static bool hermitian(const std::vector<TermC> &terms) {
+    TermSum sum;
+    for (const TermC &c : terms) sum.add(c);
+    const size_t n = sum.terms.size();
+    for (const TermC &c : terms) {
+        TermC d = term_adjoint(c);
+        d.coef = make_double2(-d.coef.x, -d.coef.y);
+        sum.add(d);
+        if (sum.terms.size() != n) return false;
+    }
+    for (const TermC &c : sum.terms)
+        if (c.coef.x != 0.0 || c.coef.y != 0.0) return false;
+    return true;
+}
 
 // g T g^-1 on the masks: the sites move; a spin flip turns the values round, and
 // the Sz factors then count the up spins: (-1)^(number of factors) over.
@@ -401,9 +432,15 @@ static unsigned char *scratch_ptr(int device) {
 // the group, so a row takes the image of its representative alone and not of all G
 // elements: equal terms of the average are looked up once (28 sites with the spin
 // flip: S+S- of two sites, half the lookups and no images to form; 717K rows, one
-// correlation 551 / 147 us). Formed on the host at about 20 ns an image, against 5 ps
+// correlation 551 us, 147 by the average, 82 with half as below). Formed on the host at about 20 ns an image, against 5 ps
 // an image and row on the GPU: for few images or at least 4096 rows, and as long as
 // the terms fit the scratch of qmb_expectation_noalloc, whose results are the same.
+//
+// half: the value of a Hermitian operator that commutes with the group is
+// sum_r M_rr |x_r|^2 + 2 Re sum_{t > r} x_r conj(M_rt x_t). A representative is the least
+// state of its orbit, so a term that lowers it ends in an orbit of a lower
+// representative, a lower row: entries M_rt with t >= r come from the terms that raise
+// the state alone, and only those are looked up.
 struct ExpectTable {
     std::vector<unsigned char> bytes;  // t[n_terms], z[n_sz]
     ExpectTerms view{};
@@ -428,6 +465,11 @@ struct ExpectTable {
                 for (TermC &c : terms) c.coef = make_double2(c.coef.x / g.G, c.coef.y / g.G);
             }
         }
+        view.half = !images && hermitian(terms);
+        if (view.half)
+            terms.erase(std::remove_if(terms.begin(), terms.end(),
+                                       [](const TermC &c) { return c.set_val < (c.req_val & c.set); }),
+                        terms.end());
         const auto mid = std::stable_partition(terms.begin(), terms.end(),
                                                [](const TermC &c) { return !is_diagonal(c); });
         const auto end = std::stable_partition(mid, terms.end(), [](const TermC &c) { return c.req != 0; });
@@ -459,11 +501,12 @@ static void launch_expectation(qmb_ctx *ctx, const qmb_basis *b, ExpectTable &ta
     const size_t rank_size = narrow ? 4 : 8;
     int n_nib = (b->n_sites + 3) / 4;
     const int n_c = b->n_up + 1;
-    size_t lds = (size_t)n_nib * n_c * 16 * rank_size;
-    if (lds > kExpRankBytes) {
+    const size_t nib_bytes = (size_t)n_nib * n_c * 16 * rank_size;
+    size_t lds = (size_t)b->n_sites * kBinJ * rank_size;
+    if (nib_bytes <= kExpRankBytes)
+        lds += nib_bytes;
+    else
         n_nib = 0;
-        lds = (size_t)b->n_sites * kBinJ * rank_size;
-    }
     lds += (size_t)std::min(tv.n_off, kExpLdsTerms) *
            (narrow ? sizeof(ExpectOff<uint32_t>) : sizeof(ExpectOff<uint64_t>));
     using K = decltype(&expect_rows<uint32_t, false, false, -1>);

@@ -114,3 +114,33 @@ def test_commutation(ctx, flip):
             print(f"[gpu-case] commutation flip={flip} {shape} {len(terms)} terms", flush=True)
             _, averaged = b.expectation(q.Terms(n, OM.conjugated_term_table(terms)), x)
             assert averaged != invariant(case, terms)
+
+
+def adjoint(t):
+    """The product of the adjoint factors in reverse order."""
+    return [(s, {SP: SM, SM: SP, SZ: SZ}[o], np.conj(c)) for s, o, c in reversed(t)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("label,mk,n_up,alphas,n_terms", CASES, ids=[c[0] for c in CASES])
+def test_hermitian_operators(ctx, label, mk, n_up, alphas, n_terms):
+    """A + A^dagger: only the terms that raise the state are looked up where the average is formed."""
+    case = mk()
+    n = case["n_sites"]
+    orb = oracle_orbits(case, n_up)
+    g = q.Group(case["group_el"], case["chars"], case["flip"])
+    half = operator(n, n_terms, 23)
+    table = OM.conjugated_term_table(half + [adjoint(t) for t in half])
+    for a in alphas:
+        keep = ~orb.null_mask(a)
+        rng = np.random.default_rng(a)
+        x = rng.normal(size=orb.n_orb) + 1j * rng.normal(size=orb.n_orb)
+        x[~keep] = 0.0
+        x /= np.linalg.norm(x)
+        print(f"[gpu-case] hermitian {label} irrep={a}", flush=True)
+        want = oracle.expectation(orb, table, a, x)
+        for layout in (q.LAYOUT_REFERENCE, q.LAYOUT_COMPACT):
+            b = q.Basis(ctx, g, n_up, a, layout)
+            got, _ = b.expectation(q.Terms(n, table), x if layout == q.LAYOUT_REFERENCE else x[keep])
+            # |A| < 20, sums of some 10^5 products of a unit vector
+            assert abs(got - want) < 1e-12 * max(1.0, abs(want))
