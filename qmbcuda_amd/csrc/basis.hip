@@ -71,7 +71,11 @@ constexpr int64_t kMaxMarkBlocks = 4096;
 // basis_compact's words per wavefront: up to 8 with this many wavefronts, more
 // with eight times as many (the words at low ranks hold most rows: 28-site ring,
 // 627K words, 39 us at 8 a wavefront, 111 us at 64; 25 sites, 81K words, 17 us
-// at 8, 29 us at 1, where most wavefronts find no row).
+// at 8, 29 us at 1, where most wavefronts find no row). Rows whose stabiliser costs
+// more want shorter tiles, since the tiles full of rows end last: twice the wavefronts
+// for a torus product (4x6 lattice, 42K words, 15.6 us at 2 a wavefront, 23 at 4; 5x6
+// 149 at 16, 194 at 32), four times for one with cosets (5x5 with quarter turns, 81K
+// words, 34 us at 2, 92 at 8).
 constexpr int64_t kMinCompactWaves = 8192;
 
 __device__ inline bool compatible(uint64_t slo, uint64_t shi, uint64_t tlo, uint64_t thi) {
@@ -578,8 +582,8 @@ qmb_status qmb_basis_build(qmb_ctx *ctx, const qmb_group *g, int n_up, int irrep
         b->nullf.alloc((size_t)std::max<int64_t>(rows, 1));
         if (rows > 0) {
             int tile_words = 64;
-            while (tile_words > 1 && b->n_words / tile_words < (tile_words > 8 ? 8 : 1) * kMinCompactWaves)
-                tile_words /= 2;
+            const int64_t waves = kMinCompactWaves * (g->lut == 4 ? 4 : g->lut == 1 ? 2 : 1);
+            while (tile_words > 1 && b->n_words / tile_words < (tile_words > 8 ? 8 : 1) * waves) tile_words /= 2;
             uint64_t periods = 0;
             for (int q = 2, m = g->n_sites; m > 1; ++q)
                 for (; m % q == 0; m /= q) periods |= 1ULL << (g->n_sites / q);

@@ -432,9 +432,10 @@ static unsigned char *scratch_ptr(int device) {
 // the group, so a row takes the image of its representative alone and not of all G
 // elements: equal terms of the average are looked up once (28 sites with the spin
 // flip: S+S- of two sites, half the lookups and no images to form; 717K rows, one
-// correlation 551 us, 147 by the average, 82 with half as below). Formed on the host at about 20 ns an image, against 5 ps
-// an image and row on the GPU: for few images or at least 4096 rows, and as long as
-// the terms fit the scratch of qmb_expectation_noalloc, whose results are the same.
+// correlation 551 us, 147 by the average, 82 with half as below). Formed on the host
+// at about 20 ns an image, against 5 ps an image and row on the GPU: for few images or
+// at least 4096 rows, and as long as the terms fit the scratch of
+// qmb_expectation_noalloc, whose results are the same.
 //
 // half: the value of a Hermitian operator that commutes with the group is
 // sum_r M_rr |x_r|^2 + 2 Re sum_{t > r} x_r conj(M_rt x_t). A representative is the least
