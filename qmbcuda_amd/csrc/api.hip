@@ -417,13 +417,9 @@ __global__ __launch_bounds__(kScanOne) void chunk_scan_one(const uint16_t *row_l
     out[3] = err ? *err : 0;
 }
 
-void scan_chunks_i64(qmb_ctx *ctx, const uint16_t *row_len, int64_t n_rows, int64_t *chunk_ptr, int64_t n_chunks,
-                     const int *d_err, int64_t *d_stats, int64_t (&h)[kScanStats]) {
-    DevBuf own, wid, np, mp, sums;
-    if (!d_stats) {
-        own.alloc(kScanStats * sizeof(int64_t));
-        d_stats = own.as<int64_t>();
-    }
+void launch_chunk_scan(qmb_ctx *ctx, const uint16_t *row_len, int64_t n_rows, int64_t *chunk_ptr, int64_t n_chunks,
+                       const int *d_err, int64_t *d_stats) {
+    DevBuf wid, np, mp, sums;
     if (n_chunks <= kScanOne) {
         hipLaunchKernelGGL(chunk_scan_one, dim3(1), dim3(kScanOne), 0, ctx->stream, row_len, n_rows, (int)n_chunks,
                            chunk_ptr, d_err, d_stats);
@@ -442,6 +438,11 @@ void scan_chunks_i64(qmb_ctx *ctx, const uint16_t *row_len, int64_t n_rows, int6
                            blocks, d_total, d_err, d_stats);
         QMB_HIP(hipGetLastError());
     }
+}
+
+void scan_chunks_i64(qmb_ctx *ctx, const uint16_t *row_len, int64_t n_rows, int64_t *chunk_ptr, int64_t n_chunks,
+                     const int *d_err, int64_t *d_stats, int64_t (&h)[kScanStats]) {
+    launch_chunk_scan(ctx, row_len, n_rows, chunk_ptr, n_chunks, d_err, d_stats);
     int64_t *st = ctx->host_stage<int64_t>(kScanStats * sizeof(int64_t));
     QMB_HIP(hipMemcpyAsync(st, d_stats, kScanStats * sizeof(int64_t), hipMemcpyDeviceToHost, ctx->stream));
     QMB_HIP(hipStreamSynchronize(ctx->stream));

@@ -65,6 +65,7 @@ __device__ inline bool set_insert(unsigned long long *set, int slots, unsigned l
 // are formed afterwards from the codes in use, with the same arithmetic, so
 // they are bit-identical to the FP64 form's.
 constexpr int kMaxCodes = 1 << 14;
+constexpr int64_t kOpenSlots = (int64_t)1 << 23;  // 32 MB of columns
 
 struct CodeView {
     const uint16_t *xcls = nullptr;  // [G] character class of each element
@@ -778,23 +779,17 @@ struct ValuePacking {
         return !(env && env[0] == '0');
     }
     // Whether the fill writes codes: the coefficient classes of the terms, the
-    // character classes of the irrep row and the stabiliser sizes present (hm, the mask
-    // of ell_stab_sizes) must give at most kMaxCodes codes. Sets up the code tables,
-    // the code array and the diagonal; used: kMaxCodes cleared bits.
+    // character classes of the irrep row and the stabiliser sizes m_of must give at most
+    // kMaxCodes codes. Sets up the code tables, the code array and the diagonal; used:
+    // kMaxCodes cleared bits.
     // QMB_VALUE_CODES=0 in the environment selects the FP64 fill and the value
     // collection pass instead (the route of tables with too many codes), so
     // tests can compare the two routes.
-    bool plan_codes(qmb_ctx *ctx, qmb_ell &e, const unsigned *hm, unsigned *used_bits, const DeviceTerms &dt,
+    bool plan_codes(qmb_ctx *ctx, qmb_ell &e, const std::vector<int> &m_of, unsigned *used_bits, const DeviceTerms &dt,
                     const double *ch, int G) {
         if (!on || dt.classes.size() > DeviceTerms::kMaxClasses || G > kMaxGroup) return false;
-        std::vector<int> m_of;
         std::vector<uint8_t> mcls(kMaxGroup + 1, 0xFF);
-        for (int m = 0; m <= kMaxGroup; ++m)
-            if ((hm[m >> 5] >> (m & 31)) & 1u) {
-                if (m < 1 || m > G) return false;  // not a stabiliser size of this group
-                mcls[m] = (uint8_t)m_of.size();
-                m_of.push_back(m);
-            }
+        for (size_t i = 0; i < m_of.size(); ++i) mcls[m_of[i]] = (uint8_t)i;
         std::vector<double2> xc;
         std::vector<uint16_t> xcls(G);
         for (int g = 0; g < G; ++g) {
@@ -861,7 +856,7 @@ struct ValuePacking {
                            e.chunk_ptr.as<int64_t>(), e.row_len.as<uint16_t>(), e.col.as<uint32_t>(),
                            codes.as<uint16_t>(), map.as<uint32_t>(), f, cplx ? 1 : 0, cb);
         QMB_HIP(hipGetLastError());
-        QMB_HIP(hipMemcpyAsync(ctx->host_stage<int>(8 * sizeof(int)), f, 8 * sizeof(int),
+        QMB_HIP(hipMemcpyAsync(ctx->host_stage<int>((8 + kScanStats) * sizeof(int64_t)), f, 8 * sizeof(int),
                                hipMemcpyDeviceToHost, ctx->stream));
     }
     void launch(qmb_ctx *ctx, qmb_ell &e) {
@@ -895,7 +890,7 @@ struct ValuePacking {
                                e.chunk_ptr.as<int64_t>(), e.row_len.as<uint16_t>(), e.col.as<uint32_t>(),
                                e.val.as<double>(), keys, f + 1, cb, e.diag.as<double>(), f + 3);
         QMB_HIP(hipGetLastError());
-        QMB_HIP(hipMemcpyAsync(ctx->host_stage<int>(8 * sizeof(int)), f, 8 * sizeof(int),
+        QMB_HIP(hipMemcpyAsync(ctx->host_stage<int>((8 + kScanStats) * sizeof(int64_t)), f, 8 * sizeof(int),
                                hipMemcpyDeviceToHost, ctx->stream));
     }
     // after the stream has drained (the flags were copied into the context's
@@ -1050,38 +1045,22 @@ qmb_status qmb_ell_build(qmb_ctx *ctx, const qmb_basis *b, const qmb_terms *t, i
                                nullptr, CodeView{}, cts);
             QMB_HIP(hipGetLastError());
         }
-        // the offsets are scanned and the stabiliser sizes collected before the overflow
-        // flag is read (one synchronisation)
         ValuePacking vp;
         if (n > 0 && !keep_fp64) vp.prepare(*e, reinterpret_cast<int *>(words.as<char>() + o_flags));
         const bool try_codes = vp.on && ValuePacking::codes_wanted();
-        if (try_codes) {
-            const unsigned blocks = (unsigned)std::min<int64_t>(1024, (n + kEllThreads - 1) / kEllThreads);
-            hipLaunchKernelGGL(ell_stab_sizes, dim3(blocks), dim3(kEllThreads), 0, ctx->stream, n,
-                               b->stab.as<uint8_t>(), reinterpret_cast<unsigned *>(d_stats + 4));
-            QMB_HIP(hipGetLastError());
-        }
-        int64_t stats[kScanStats] = {};
-        if (n > 0)
-            scan_chunks_i64(ctx, e->row_len.as<uint16_t>(), n, e->chunk_ptr.as<int64_t>(), e->n_chunks, d_err, d_stats,
-                            stats);
-        QMB_REQUIRE(stats[3] == 0, "qmb_ell_build: a row needs more than max_terms = " + std::to_string(W) + " slots");
-        e->stored = stats[0];
-        e->nnz = stats[1];
-        e->max_row_len = (int)stats[2];
-        e->col.alloc((size_t)std::max<int64_t>(e->stored, 1) * sizeof(int32_t));
-        // a packed build writes value codes (2 B per entry) instead of FP64 values
-        // when the factors of the values give few enough codes
-        unsigned mask[5];
-        std::memcpy(mask, stats + 4, sizeof mask);
-        const bool coded = try_codes && vp.plan_codes(ctx, *e, mask, reinterpret_cast<unsigned *>(words.as<char>() + o_used),
-                                                      dt, ch, g->G);
+        unsigned *used = reinterpret_cast<unsigned *>(words.as<char>() + o_used);
+        auto take_stats = [&](const int64_t *st) {
+            QMB_REQUIRE(st[3] == 0, "qmb_ell_build: a row needs more than max_terms = " + std::to_string(W) + " slots");
+            e->stored = st[0];
+            e->nnz = st[1];
+            e->max_row_len = (int)st[2];
+        };
         // the fill (coded, or with FP64 values), with the padding of the last chunk
         auto fill = [&](bool with_codes) {
             const EllRows kfill = ell_fill_kernel(narrow, cplx, with_codes, ts != 0, gv.lut);
             double *val = with_codes ? nullptr : e->val.as<double>();
-            hipLaunchKernelGGL(kfill, dim3(blocks_for(e->n_chunks * kChunk, ts)), dim3(kEllThreads), lds_bytes, ctx->stream, gv,
-                               ctx->binom.as<uint64_t>(), rank.tab(), rank.n_nib, rank.n_c, b->layout, n,
+            hipLaunchKernelGGL(kfill, dim3(blocks_for(e->n_chunks * kChunk, ts)), dim3(kEllThreads), lds_bytes,
+                               ctx->stream, gv, ctx->binom.as<uint64_t>(), rank.tab(), rank.n_nib, rank.n_c, b->layout, n,
                                b->reps.as<uint64_t>(),
                                b->stab.as<uint8_t>(), b->nullf.as<uint8_t>(), b->dict.as<uint64_t>(),
                                tv, n_lds, dt.chi, dt.nrm, W,
@@ -1089,15 +1068,67 @@ qmb_status qmb_ell_build(qmb_ctx *ctx, const qmb_basis *b, const qmb_terms *t, i
                                e->col.as<int32_t>(), val, with_codes ? vp.cv : CodeView{}, ts);
             QMB_HIP(hipGetLastError());
         };
-        if (!coded) e->val.alloc((size_t)std::max<int64_t>(e->stored, 1) * (cplx ? 16 : 8));
-        if (n > 0) {
-            fill(coded);
-            if (coded)
-                vp.launch_coded(ctx, *e);
-            else if (vp.on)
-                vp.launch(ctx, *e);
+        // a packed build writes value codes (2 B per entry) instead of FP64 values when
+        // the factors of the values give few enough codes
+        bool coded = false;
+        // A small matrix is built without a wait in between: its columns get the room
+        // of rows with every term (at most kOpenSlots slots), and its codes classes for
+        // every divisor of the group's order. Bound by launches and waits (415 rows:
+        // build 111 us waiting, 85 without; 56,450 rows 149 / 132).
+        const int64_t room = e->n_chunks * kChunk * ((int64_t)tv.n_off + 1);
+        if (try_codes && room <= kOpenSlots) {
+            std::vector<int> divisors;
+            for (int m = 1; m <= g->G; ++m)
+                if (g->G % m == 0) divisors.push_back(m);
+            e->stored = room;
+            coded = vp.plan_codes(ctx, *e, divisors, used, dt, ch, g->G);
         }
-        QMB_HIP(hipStreamSynchronize(ctx->stream));
+        if (coded) {
+            launch_chunk_scan(ctx, e->row_len.as<uint16_t>(), n, e->chunk_ptr.as<int64_t>(), e->n_chunks, d_err,
+                              d_stats);
+            e->col.alloc((size_t)room * sizeof(int32_t));
+            fill(true);
+            vp.launch_coded(ctx, *e);
+            int64_t *st = ctx->host_stage<int64_t>((8 + kScanStats) * sizeof(int64_t)) + 8;  // after the flags
+            QMB_HIP(hipMemcpyAsync(st, d_stats, kScanStats * sizeof(int64_t), hipMemcpyDeviceToHost, ctx->stream));
+            QMB_HIP(hipStreamSynchronize(ctx->stream));
+            take_stats(st);
+            e->col.bytes = (size_t)std::max<int64_t>(e->stored, 1) * sizeof(int32_t);
+        } else {
+            // the offsets are scanned and the stabiliser sizes collected before the
+            // overflow flag is read (one synchronisation)
+            int64_t stats[kScanStats] = {};
+            std::vector<int> sizes;
+            if (try_codes) {
+                const unsigned blocks = (unsigned)std::min<int64_t>(1024, (n + kEllThreads - 1) / kEllThreads);
+                hipLaunchKernelGGL(ell_stab_sizes, dim3(blocks), dim3(kEllThreads), 0, ctx->stream, n,
+                                   b->stab.as<uint8_t>(), reinterpret_cast<unsigned *>(d_stats + 4));
+                QMB_HIP(hipGetLastError());
+            }
+            if (n > 0)
+                scan_chunks_i64(ctx, e->row_len.as<uint16_t>(), n, e->chunk_ptr.as<int64_t>(), e->n_chunks, d_err,
+                                d_stats, stats);
+            take_stats(stats);
+            unsigned mask[5];
+            std::memcpy(mask, stats + 4, sizeof mask);
+            bool known = try_codes;
+            for (int m = 0; m <= kMaxGroup; ++m)
+                if ((mask[m >> 5] >> (m & 31)) & 1u) {
+                    known = known && m >= 1 && m <= g->G;  // else not a stabiliser size of this group
+                    sizes.push_back(m);
+                }
+            e->col.alloc((size_t)std::max<int64_t>(e->stored, 1) * sizeof(int32_t));
+            coded = known && vp.plan_codes(ctx, *e, sizes, used, dt, ch, g->G);
+            if (!coded) e->val.alloc((size_t)std::max<int64_t>(e->stored, 1) * (cplx ? 16 : 8));
+            if (n > 0) {
+                fill(coded);
+                if (coded)
+                    vp.launch_coded(ctx, *e);
+                else if (vp.on)
+                    vp.launch(ctx, *e);
+            }
+            QMB_HIP(hipStreamSynchronize(ctx->stream));
+        }
         if (vp.on && !vp.finish(ctx, *e) && coded) {
             // more distinct values than the index bits hold: the FP64 form
             e->val.alloc((size_t)std::max<int64_t>(e->stored, 1) * (cplx ? 16 : 8));

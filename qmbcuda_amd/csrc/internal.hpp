@@ -446,11 +446,12 @@ void upload(qmb_ctx *ctx, void *dst, const void *src, size_t bytes);
 
 // Exclusive scans on device (3-phase). Values come from a functor.
 int64_t scan_popcount_dict(qmb_ctx *ctx, uint64_t *dict, int64_t n_words);
-// Chunk offsets of a SELL-64 layout from its row lengths. h = {stored total (also
-// chunk_ptr[n_chunks]), entries, longest row, *d_err, then the words the caller has in
-// d_stats[4..8)}, read back in one synchronisation; d_stats: kScanStats words of device
-// memory, or NULL.
+// Chunk offsets of a SELL-64 layout from its row lengths, queued on the stream;
+// d_stats[0..4) (device) = stored total (also chunk_ptr[n_chunks]), entries, longest
+// row, *d_err. scan_chunks_i64 also reads d_stats[0..kScanStats) back.
 constexpr int kScanStats = 8;
+void launch_chunk_scan(qmb_ctx *ctx, const uint16_t *row_len, int64_t n_rows, int64_t *chunk_ptr, int64_t n_chunks,
+                       const int *d_err, int64_t *d_stats);
 void scan_chunks_i64(qmb_ctx *ctx, const uint16_t *row_len, int64_t n_rows, int64_t *chunk_ptr, int64_t n_chunks,
                      const int *d_err, int64_t *d_stats, int64_t (&h)[kScanStats]);
 

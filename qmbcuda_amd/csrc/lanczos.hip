@@ -1686,8 +1686,9 @@ qmb_ell *ell_from_reference_device(qmb_ctx *ctx, int64_t n, int W, const uint32_
                        err.as<int>());
     QMB_HIP(hipGetLastError());
     int64_t h[kScanStats];
+    DevBuf stats(kScanStats * sizeof(int64_t));
     scan_chunks_i64(ctx, e->row_len.as<uint16_t>(), n, e->chunk_ptr.as<int64_t>(), e->n_chunks, err.as<int>(),
-                    nullptr, h);
+                    stats.as<int64_t>(), h);
     int herr = (int)h[3];
     QMB_REQUIRE(herr == 0, "reference ELL: track out of range [0, max_terms]");
     e->stored = h[0];
