@@ -131,7 +131,7 @@ void download(qmb_ctx *ctx, void *dst, const void *src, size_t bytes) {
     int started = 1;
     try {
         for (; started < threads; ++started) helper[started] = std::thread(pieces, started);
-    } catch (const std::system_error &) {  // no thread to be had: the rest is done here
+    } catch (...) {  // no thread to be had: the rest is done here
     }
     pieces(0);
     for (int t = started; t < threads; ++t) pieces(t);
