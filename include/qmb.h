@@ -223,7 +223,8 @@ typedef struct {
                           * checkpoints; single-sector solves only); 1-3 keep max_iter vectors */
     int32_t fixed_iter;  /* 1: run exactly max_iter steps, no test (reference semantics) */
     int32_t start;       /* QMB_START_RANDOM, QMB_START_USER or QMB_START_DEVICE */
-    int32_t want_eigvec; /* 1: rebuild the ground-state vector (second pass) */
+    int32_t want_eigvec; /* 1: the ground-state vector too, from the Lanczos vectors (kept in
+                            up to a quarter of the free memory; else by a second pass) */
     int32_t profile;     /* k > 0: time every k-th SpMV (steps 0, k, 2k, ...) with HIP events */
     double tol;          /* eigenvalue tolerance, relative to max(1,|E|) (0 -> 1e-13) */
     uint64_t seed;       /* start-vector seed (reference default 2212456) */
@@ -314,8 +315,8 @@ double qmb_lanczos_eigvals_ref_device(double *E_tmp, int NStates, int NIter, int
  * eigenvector of the sector matrix, its eigenstate (no normalisation is applied).
  * A is any Sz-conserving operator as a conjugated term table, in the same form as
  * the Hamiltonian's. It need not commute with the group: the sector sees its group
- * average (1/G) sum_g g A g^-1, taken over every image of each row's representative;
- * when A commutes with the group (checked on the host) the average is skipped.
+ * average (1/G) sum_g g A g^-1, formed term by term on the host (with very many
+ * terms: taken over every image of each row's representative); when A commutes with the group (checked on the host) the average is skipped.
  * flags = QMB_EXPECT_GROUP_AVERAGE forces the average; *averaged (optional) = 1 when
  * it was taken. Differences from the reference kernel: every image of the source
  * contributes (it stops at the first image a term annihilates), and the pairing of
