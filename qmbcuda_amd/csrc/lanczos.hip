@@ -579,13 +579,33 @@ __global__ __launch_bounds__(kThreads) void vec_axpy(int64_t cnt, double c, cons
 // two block sums per vector; two or eight vectors a block 31 and 36 us).
 constexpr int kDotGroup = 4;
 
+// Partials of ||w||^2 after and before a first Gram-Schmidt pass.
+struct NormPair {
+    const double *now = nullptr, *old = nullptr;
+    int n_now = 0, n_old = 0;
+};
+
 template <bool CPLX>
 __global__ __launch_bounds__(kThreads) void reorth_dots(int64_t n, int64_t stride, int nv,
                                                         const double *__restrict__ V,
                                                         const double *__restrict__ w, double *__restrict__ part,
-                                                        int nb, const double *__restrict__ gate) {
+                                                        int nb, double *__restrict__ gate, NormPair norms) {
     __shared__ double lds[kWaves][2 * kDotGroup];
-    if (gated_off(gate)) return;
+    if (norms.now) {
+        // this pass's gate, from the norms before and after the first pass: every block
+        // sums them (as finish_sum would), the first one stores the gate
+        __shared__ double s_open;
+        const double now = sum_partials(norms.now, norms.n_now, lds[0]);
+        const double old = sum_partials(norms.old, norms.n_old, lds[0]);
+        if (threadIdx.x == 0) {
+            s_open = sqrt(now) < kDgks * sqrt(old) ? 1.0 : 0.0;
+            if (blockIdx.x == 0 && blockIdx.y == 0) *gate = s_open;
+        }
+        __syncthreads();
+        if (s_open == 0.0) return;
+    } else if (gated_off(gate)) {
+        return;
+    }
     const int j0 = blockIdx.y * kDotGroup;
     const int nj = min(kDotGroup, nv - j0);
     const double *vj[kDotGroup];  // past the last vector: the last one again, not used
@@ -740,7 +760,7 @@ static unsigned grid_for(int64_t work_items, int per_block) {
 }
 
 struct LzWork {
-    DevBuf partials, scal;  // scal: alpha[M], beta[M+1], invb[M+1], misc[8]
+    DevBuf partials, scal;  // partials: three arrays of kMaxBlocks; scal: alpha[M], beta[M+1], invb[M+1], misc[8]
     int M = 0;
     double *alpha() const { return scal.as<double>(); }
     double *beta() const { return scal.as<double>() + M; }
@@ -748,7 +768,7 @@ struct LzWork {
     double *misc() const { return scal.as<double>() + 3 * M + 2; }
     void init(qmb_ctx *ctx, int max_iter, bool clear) {
         M = max_iter;
-        partials.alloc(kMaxBlocks * sizeof(double) * 2);
+        partials.alloc(kMaxBlocks * sizeof(double) * 3);
         scal.alloc((size_t)(3 * M + 2 + 8) * sizeof(double));
         if (!clear) return;
         QMB_HIP(hipMemsetAsync(scal.p, 0, (size_t)(3 * M + 2 + 8) * sizeof(double), ctx->stream));
@@ -1043,7 +1063,10 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
     // were written by an explicit finish (start vector, last step before a
     // convergence check); otherwise K1(n) derives them from K2(n-1)'s partials.
     const bool fuse = rmode == 0;
-    double *part1 = wk.partials.as<double>(), *part2 = wk.partials.as<double>() + kMaxBlocks;
+    double *part1 = wk.partials.as<double>(), *part2 = part1 + kMaxBlocks, *part3 = part2 + kMaxBlocks;
+    const unsigned ablocks = grid_for(n, kThreads);  // reorth_apply
+    // up to what every block of the SpMV has loaded ahead (kPre): beyond, a launch costs less
+    const bool gs_fold = rmode == 1 && ablocks <= 4 * kThreads;
     const unsigned sblocks = spmv_blocks(e);
     std::vector<char> b_ready(M + 1, 0);
     b_ready[0] = 1;
@@ -1051,9 +1074,9 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
         // a[n] is left to K2, which sums K1's partials, in every scheme
         FusedBeta fb;
         fb.partials = part1;
-        if (fuse && !b_ready[it]) {
-            fb.bpart = part2;
-            fb.n_bpart = (int)ublocks;
+        if ((fuse || gs_fold) && !b_ready[it]) {
+            fb.bpart = fuse ? part2 : part3;
+            fb.n_bpart = (int)(fuse ? ublocks : ablocks);
             fb.beta_out = wk.beta() + it;
             fb.invb_out = wk.invb() + it;
         }
@@ -1112,25 +1135,29 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
     // w (in P) -= sum_j <V_j, w> V_j over nv vectors of stride cnt, classical
     // Gram-Schmidt; pass 1 only where pass 0 cancelled most of the norm (the flag
     // in misc[3] is set by pass 0's finish on the device); the new norm goes to
-    // b[bslot], 1/b[bslot] (before: the partials of the norm it had, or b[bslot] holds that norm)
-    const unsigned ablocks = grid_for(n, kThreads);
+    // b[bslot], 1/b[bslot] (before: the partials of the norm it had, or b[bslot] holds that norm).
+    // gs_fold (full reorthogonalisation): the blocks of the second pass's dots sum the
+    // norms and decide, and the next SpMV sums the last norm, two launches of ten fewer
+    // a step (4,654 rows 32.9 -> 29.9 us a step, 56,450 34.7 -> 32.0, 208,012 78.1 -> 76.9).
     auto gram_schmidt = [&](const double *V, int nv, int bslot, const double *before = nullptr) {
         double *gate = wk.misc() + 3;
         for (int pass = 0; pass < 2; ++pass) {
-            const double *g = pass ? gate : nullptr;
+            double *g = pass ? gate : nullptr;
+            const NormPair norms = pass && gs_fold ? NormPair{part3, before, (int)ablocks, (int)ublocks} : NormPair{};
             auto kd = cplx ? reorth_dots<true> : reorth_dots<false>;
             hipLaunchKernelGGL(kd, dim3(rblocks, (nv + kDotGroup - 1) / kDotGroup), dim3(kThreads), 0, ctx->stream,
-                               n, (int64_t)cnt, nv, V, P.as<double>(), rpart.as<double>(), (int)rblocks, g);
+                               n, (int64_t)cnt, nv, V, P.as<double>(), rpart.as<double>(), (int)rblocks, g, norms);
             QMB_HIP(hipGetLastError());
             hipLaunchKernelGGL(reorth_reduce, dim3(nv), dim3(kThreads), 0, ctx->stream, rpart.as<double>(),
                                (int)rblocks, rcoef.as<double>(), g);
             QMB_HIP(hipGetLastError());
             auto ka = cplx ? reorth_apply<true> : reorth_apply<false>;
             hipLaunchKernelGGL(ka, dim3(ablocks), dim3(kThreads), 0, ctx->stream, n, (int64_t)cnt, nv, V,
-                               rcoef.as<double>(), P.as<double>(), part1, g);
+                               rcoef.as<double>(), P.as<double>(), part3, g);
             QMB_HIP(hipGetLastError());
-            launch_finish(ctx, part1, ablocks, wk.beta() + bslot, wk.invb() + bslot, pass ? 1 : 2, gate,
-                          pass ? nullptr : before, ublocks);
+            if (!gs_fold)
+                launch_finish(ctx, part3, ablocks, wk.beta() + bslot, wk.invb() + bslot, pass ? 1 : 2, gate,
+                              pass ? nullptr : before, ublocks);
         }
     };
     // Selective orthogonalisation (B. N. Parlett and D. S. Scott, Math. Comp. 33
@@ -1160,6 +1187,10 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
         if (rmode == 1) {  // the norm before the orthogonalisation serves its gate only
             ++n_reorth;
             gram_schmidt(VB.as<double>(), it + 1, it + 1, part2);
+            if (gs_fold && finish) {
+                launch_finish(ctx, part3, ablocks, wk.beta() + it + 1, wk.invb() + it + 1, 1);
+                b_ready[it + 1] = 1;
+            }
             return;
         }
         launch_finish(ctx, part2, ublocks, wk.beta() + it + 1, wk.invb() + it + 1, 1);
