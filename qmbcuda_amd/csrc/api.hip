@@ -71,21 +71,21 @@ void upload(qmb_ctx *ctx, void *dst, const void *src, size_t bytes) {
 // each copy every kBulkThreads-th piece out of its two slots while the next ones
 // arrive: the runtime's own path does both with one thread, which also takes the
 // page faults of fresh memory (41 MB: 4450 us, 1500 by four threads; the transfer
-// alone is 740). Below 4 MB the threads cost what they save and one does it in pieces
-// of 256 KB; below 64 KB the runtime stages the copy itself.
+// alone is 740). Below 4 MB the threads cost what they save and one takes the pieces
+// (this / the runtime: 250 KB 76 / 171 us, 441 KB 76 / 69, 880 KB 110 / 103, 3.1 MB
+// 265 / 290; pieces of 256 KB 155 us at 880 KB); below 64 KB the runtime does it.
 constexpr size_t kStagedBytes = (size_t)64 << 10, kBulkBytes = (size_t)4 << 20, kBulkPiece = (size_t)2 << 20;
 constexpr int kBulkThreads = 4;
 
 // Pieces t, t + threads, ... through two slots.
-static hipError_t download_pieces(qmb_ctx *ctx, char *dst, const char *src, size_t bytes, int t, int threads,
-                                  size_t piece) {
+static hipError_t download_pieces(qmb_ctx *ctx, char *dst, const char *src, size_t bytes, int t, int threads) {
     hipError_t err = hipSetDevice(ctx->device);
     hipEvent_t done[2] = {};
     for (hipEvent_t &e : done)
         if (err == hipSuccess) err = hipEventCreateWithFlags(&e, hipEventDisableTiming);
     char *slot = ctx->bulk->as<char>() + (size_t)t * 2 * kBulkPiece;
-    const size_t step = threads * piece, first = (size_t)t * piece;
-    auto size = [&](size_t at) { return std::min(piece, bytes - at); };
+    const size_t step = threads * kBulkPiece, first = (size_t)t * kBulkPiece;
+    auto size = [&](size_t at) { return std::min(kBulkPiece, bytes - at); };
     auto issue = [&](size_t at, int k) {
         if (err != hipSuccess || at >= bytes) return;
         err = hipMemcpyAsync(slot + k * kBulkPiece, src + at, size(at), hipMemcpyDeviceToHost, ctx->stream);
@@ -121,12 +121,10 @@ void download(qmb_ctx *ctx, void *dst, const void *src, size_t bytes) {
     }
     if (!ctx->bulk) ctx->bulk = std::make_unique<PinnedBuf>(kBulkThreads * 2 * kBulkPiece);
     const int threads = bytes < kBulkBytes ? 1 : kBulkThreads;
-    const size_t piece = bytes < kBulkBytes ? kBulkPiece / 8 : kBulkPiece;
     hipError_t err[kBulkThreads] = {};
     std::thread helper[kBulkThreads];
     auto pieces = [&](int t) {
-        err[t] = download_pieces(ctx, static_cast<char *>(dst), static_cast<const char *>(src), bytes, t,
-                                 threads, piece);
+        err[t] = download_pieces(ctx, static_cast<char *>(dst), static_cast<const char *>(src), bytes, t, threads);
     };
     int started = 1;
     try {

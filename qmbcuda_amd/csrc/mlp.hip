@@ -422,7 +422,42 @@ __device__ inline void window_sums(const uint64_t (&st)[R], int ring, int n_win,
     }
 }
 
-// alpha_r, beta_r from the pattern table of this coupling; block max of alpha.
+// The largest alpha of some rows, the first of them that has it and its beta.
+struct Largest {
+    double a;
+    long long r;
+    double b;
+    __device__ void take(double a2, long long r2, double b2) {
+        if (a2 > a || (a2 == a && r2 < r)) {
+            a = a2;
+            r = r2;
+            b = b2;
+        }
+    }
+};
+
+__device__ inline Largest no_row() { return Largest{-1e300, LLONG_MAX, 0.0}; }
+
+// That of the block (256 threads), to every thread.
+__device__ inline Largest block_largest(Largest v, Largest *lds) {
+    for (int off = 32; off > 0; off >>= 1) {
+        const double a = __shfl_down(v.a, off, 64), b = __shfl_down(v.b, off, 64);
+        const long long r = __shfl_down(v.r, off, 64);
+        v.take(a, r, b);
+    }
+    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = v;
+    __syncthreads();
+    for (int i = 0; i < kWaves; ++i) v.take(lds[i].a, lds[i].r, lds[i].b);
+    // thread 0 has the block's; the others take it from there
+    __syncthreads();
+    if (threadIdx.x == 0) lds[0] = v;
+    __syncthreads();
+    return lds[0];
+}
+
+// alpha_r, beta_r from the pattern table of this coupling; the block's largest alpha
+// into part[block] (part[n_blocks + block] = its row, -1 for none, part[2 n_blocks +
+// block] = its beta).
 // beta_r also carries the Marshall sign prior pi * (up spins on sublattice A):
 // the network learns the phase relative to the bipartite sign rule, whose
 // state (and not the uniform one, which is the fully polarised multiplet and
@@ -433,7 +468,7 @@ __global__ __launch_bounds__(256) void mlp_state_logpsi(int64_t n, int n_win, co
                                                         double *__restrict__ beta, double *__restrict__ part) {
     __shared__ float2 t[256];
     __shared__ double2 t4[kGroupPat];
-    __shared__ double lds[kWaves];
+    __shared__ Largest lds[kWaves];
     __shared__ uint8_t wl[kMaxWin * kWin];
     constexpr int R = 4;
     for (int i = threadIdx.x; i < 256; i += blockDim.x) t[i] = reinterpret_cast<const float2 *>(tab)[i];
@@ -441,7 +476,7 @@ __global__ __launch_bounds__(256) void mlp_state_logpsi(int64_t n, int n_win, co
     __syncthreads();
     if (ring) group_table(t, t4);
     __syncthreads();
-    double mx = -1e300;
+    Largest best = no_row();
     const int64_t step = (int64_t)gridDim.x * blockDim.x;
     for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < n; r += R * step) {
         uint64_t st[R];
@@ -452,47 +487,39 @@ __global__ __launch_bounds__(256) void mlp_state_logpsi(int64_t n, int n_win, co
 #pragma unroll
         for (int i = 0; i < R; ++i) {
             if (r + i * step >= n) continue;
+            const double beta_r = b[i] + kMarshallPi * (double)__popcll(st[i] & sub_a);
             alpha[r + i * step] = a[i];
-            beta[r + i * step] = b[i] + kMarshallPi * (double)__popcll(st[i] & sub_a);
-            mx = fmax(mx, a[i]);
+            beta[r + i * step] = beta_r;
+            best.take(a[i], r + i * step, beta_r);
         }
     }
-    for (int off = 32; off > 0; off >>= 1) mx = fmax(mx, __shfl_down(mx, off, 64));
-    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = mx;
-    __syncthreads();
+    best = block_largest(best, lds);
     if (threadIdx.x == 0) {
-        double m = lds[0];
-        for (int i = 1; i < kWaves; ++i) m = fmax(m, lds[i]);
-        part[blockIdx.x] = m;
-    }
-}
-
-__global__ __launch_bounds__(256) void mlp_finish_max(const double *__restrict__ part, int n, double *__restrict__ out) {
-    __shared__ double lds[kWaves];
-    double mx = -1e300;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) mx = fmax(mx, part[i]);
-    for (int off = 32; off > 0; off >>= 1) mx = fmax(mx, __shfl_down(mx, off, 64));
-    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = mx;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double m = lds[0];
-        for (int i = 1; i < kWaves; ++i) m = fmax(m, lds[i]);
-        *out = m;
+        part[blockIdx.x] = best.a;
+        part[gridDim.x + blockIdx.x] = best.r == LLONG_MAX ? -1.0 : (double)best.r;
+        part[2 * gridDim.x + blockIdx.x] = best.b;
     }
 }
 
 // Real start vector x_r = |c_r| cos(beta_r - beta_ref) with beta_ref the phase
-// of the first representative of largest amplitude (alpha == amax). Block
+// of the first representative of largest amplitude, found by every block among the
+// n_best blocks' of mlp_state_logpsi (best; three launches fewer than by kernels of
+// their own: a start vector of 12 to 22 sites 98-105 us, 66-76 so). Block
 // partials: part[block] = sum of x_r^2, part[gridDim.x + block] = sum of xi_r^2
 // for the seeded noise xi_r = 2 u_r - 1 (u_r = element r of the SplitMix64
 // stream of `seed`) that the Lanczos start mixes in.
 __global__ __launch_bounds__(256) void mlp_state_start(int64_t n, int G, const uint8_t *__restrict__ stab,
                                                        const double *__restrict__ alpha,
-                                                       const double *__restrict__ beta, const double *__restrict__ amax,
-                                                       const double *__restrict__ beta_ref, uint64_t seed,
+                                                       const double *__restrict__ beta,
+                                                       const double *__restrict__ best, int n_best, uint64_t seed,
                                                        double *__restrict__ x, double *__restrict__ part) {
     __shared__ double lds[kWaves];
-    const double am = *amax, br = *beta_ref;
+    __shared__ Largest s_best[kWaves];
+    Largest top = no_row();
+    for (int i = threadIdx.x; i < n_best; i += blockDim.x)
+        if (best[n_best + i] >= 0.0) top.take(best[i], (long long)best[n_best + i], best[2 * n_best + i]);
+    top = block_largest(top, s_best);
+    const double am = top.a, br = top.b;
     double acc = 0.0, accn = 0.0;
     for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < n; r += (int64_t)gridDim.x * blockDim.x) {
         const double mag = exp(alpha[r] - am) * sqrt((double)G / (double)stab[r]);
@@ -518,45 +545,6 @@ __global__ __launch_bounds__(256) void mlp_mix_noise(int64_t n, uint64_t seed, d
         const double xi = 2.0 * splitmix_uniform(seed, (uint64_t)r) - 1.0;
         x[r] = x[r] * ix + xi * in;
     }
-}
-
-// Smallest index whose alpha equals amax: per-block minima (part[block] =
-// index as a double, exact below 2^53), then one block picks the minimum and
-// stores beta at that index.
-__device__ inline long long block_min_ll(long long v, long long *lds) {
-    for (int off = 32; off > 0; off >>= 1) {
-        const long long o = __shfl_down(v, off, 64);
-        v = o < v ? o : v;
-    }
-    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = v;
-    __syncthreads();
-    long long b = lds[0];
-    for (int i = 1; i < kWaves; ++i) b = lds[i] < b ? lds[i] : b;
-    __syncthreads();
-    return b;
-}
-
-__global__ __launch_bounds__(256) void mlp_argmax_part(int64_t n, const double *__restrict__ alpha,
-                                                       const double *__restrict__ amax, double *__restrict__ part) {
-    __shared__ long long lds[kWaves];
-    const double am = *amax;
-    long long best = LLONG_MAX;
-    for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < n; r += (int64_t)gridDim.x * blockDim.x)
-        if (alpha[r] == am && r < best) best = r;
-    const long long b = block_min_ll(best, lds);
-    if (threadIdx.x == 0) part[blockIdx.x] = b == LLONG_MAX ? -1.0 : (double)b;
-}
-
-__global__ __launch_bounds__(256) void mlp_beta_ref(int nb, const double *__restrict__ part,
-                                                    const double *__restrict__ beta, double *__restrict__ beta_ref) {
-    __shared__ long long lds[kWaves];
-    long long best = LLONG_MAX;
-    for (int i = threadIdx.x; i < nb; i += blockDim.x) {
-        const double v = part[i];
-        if (v >= 0.0 && (long long)v < best) best = (long long)v;
-    }
-    const long long b = block_min_ll(best, lds);
-    if (threadIdx.x == 0) *beta_ref = b == LLONG_MAX ? 0.0 : beta[b];
 }
 
 // out[0], out[1] = fixed-order sums of part[0..n) and part[n..2n).
@@ -925,16 +913,18 @@ void forward_rows(qmb_mlp *m, const std::vector<double> &coup, bool store) {
     qmb_ctx *ctx = m->ctx;
     const int rows = (int)(coup.size() / 2) * 256;
     m->ensure_rows(rows);
-    QMB_HIP(hipMemcpyAsync(m->coup.p, coup.data(), coup.size() * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
+    upload(ctx, m->coup.p, coup.data(), coup.size() * sizeof(double));
     hipLaunchKernelGGL(mlp_forward, dim3(rows / 32), dim3(kFwdThreads), 0, ctx->stream, m->theta.as<float>(),
                        m->w2bf.as<uint16_t>(), m->coup.as<double>(), m->out.as<float>(), m->H1.as<float>(),
                        m->H1q.as<uint16_t>(), m->H2.as<float>(), store ? 1 : 0);
     QMB_HIP(hipGetLastError());
 }
 
-// alpha/beta/amax of one state set for the coupling whose table starts at tab.
+// alpha/beta of one state set for the coupling whose table starts at tab.
+constexpr int64_t kStartWith = 16384;  // rows of a start vector read back with its norms
+
 struct StateWork {
-    DevBuf alpha, beta, part, amax, stats;
+    DevBuf alpha, beta, part, stats;  // part: mlp_state_logpsi's three, mlp_state_start's two a block
     int64_t cap = 0;
     int nb = 0;
     void ensure(int64_t n) {
@@ -942,8 +932,7 @@ struct StateWork {
         alpha.alloc(n * sizeof(double));
         beta.alloc(n * sizeof(double));
         nb = (int)std::min<int64_t>(1024, (n + 255) / 256);
-        part.alloc((size_t)nb * 4 * sizeof(double));
-        amax.alloc(sizeof(double));
+        part.alloc((size_t)nb * 5 * sizeof(double));
         stats.alloc(8 * sizeof(double));
         cap = n;
     }
@@ -954,9 +943,6 @@ void state_logpsi(qmb_ctx *ctx, const qmb_basis *b, const MlpGeom &gm, const flo
     hipLaunchKernelGGL(mlp_state_logpsi, dim3(w.nb), dim3(256), 0, ctx->stream, b->n_rows, gm.n_win,
                        gm.win.as<uint8_t>(), gm.ring, gm.sub_a, b->reps.as<uint64_t>(), tab, w.alpha.as<double>(),
                        w.beta.as<double>(), w.part.as<double>());
-    QMB_HIP(hipGetLastError());
-    hipLaunchKernelGGL(mlp_finish_max, dim3(1), dim3(256), 0, ctx->stream, w.part.as<double>(), w.nb,
-                       w.amax.as<double>());
     QMB_HIP(hipGetLastError());
 }
 
@@ -1035,32 +1021,33 @@ void batch_loss(qmb_mlp *m, bool want_grad) {
 // phase per representative, reference phase of the first largest amplitude,
 // x_r = |c_r| cos(beta_r - beta_ref); w.stats[0] = ||x||^2 and w.stats[1] =
 // ||xi||^2 of the seeded noise. Returns false when ||x||^2 is zero or not
-// finite (the caller then starts from the seeded random vector); only those
-// two numbers travel to the host.
+// finite (the caller then starts from the seeded random vector); those two numbers
+// travel to the host, and the vector into x when that is given.
 bool build_start(qmb_mlp *m, const qmb_basis *b, double delta, double j2, uint64_t seed, double *dx,
-                 StateWork &w) {
+                 StateWork &w, double *x = nullptr) {
     const int gi = geom_for(m, b);
     qmb_ctx *ctx = m->ctx;
     std::vector<double> coup = {delta, j2};
     forward_rows(m, coup, false);
     state_logpsi(ctx, b, m->geoms[gi], m->out.as<float>(), w);
-    DevBuf bref(sizeof(double));
-    hipLaunchKernelGGL(mlp_argmax_part, dim3(w.nb), dim3(256), 0, ctx->stream, b->n_rows, w.alpha.as<double>(),
-                       w.amax.as<double>(), w.part.as<double>());
-    QMB_HIP(hipGetLastError());
-    hipLaunchKernelGGL(mlp_beta_ref, dim3(1), dim3(256), 0, ctx->stream, w.nb, w.part.as<double>(),
-                       w.beta.as<double>(), bref.as<double>());
-    QMB_HIP(hipGetLastError());
     hipLaunchKernelGGL(mlp_state_start, dim3(w.nb), dim3(256), 0, ctx->stream, b->n_rows, b->group->G,
-                       b->stab.as<uint8_t>(), w.alpha.as<double>(), w.beta.as<double>(), w.amax.as<double>(),
-                       bref.as<double>(), seed, dx, w.part.as<double>());
+                       b->stab.as<uint8_t>(), w.alpha.as<double>(), w.beta.as<double>(), w.part.as<double>(), w.nb,
+                       seed, dx, w.part.as<double>() + 3 * w.nb);
     QMB_HIP(hipGetLastError());
-    hipLaunchKernelGGL(mlp_finish_sum2, dim3(1), dim3(256), 0, ctx->stream, w.part.as<double>(), w.nb,
+    hipLaunchKernelGGL(mlp_finish_sum2, dim3(1), dim3(256), 0, ctx->stream, w.part.as<double>() + 3 * w.nb, w.nb,
                        w.stats.as<double>());
     QMB_HIP(hipGetLastError());
-    double sums[2] = {0.0, 0.0};
-    QMB_HIP(hipMemcpyAsync(sums, w.stats.p, sizeof(sums), hipMemcpyDeviceToHost, ctx->stream));
+    // the norms, and a short vector with them, come back in one wait
+    const bool with = x && b->n_rows <= kStartWith;
+    double *sums = ctx->host_stage<double>((size_t)(2 + (with ? b->n_rows : 0)) * sizeof(double));
+    QMB_HIP(hipMemcpyAsync(sums, w.stats.p, 2 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+    if (with)
+        QMB_HIP(hipMemcpyAsync(sums + 2, dx, b->n_rows * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     QMB_HIP(hipStreamSynchronize(ctx->stream));
+    if (with)
+        std::copy(sums + 2, sums + 2 + b->n_rows, x);
+    else if (x)
+        download(ctx, x, dx, b->n_rows * sizeof(double));
     return std::isfinite(sums[0]) && sums[0] > 0.0 && sums[1] > 0.0;
 }
 
@@ -1272,8 +1259,7 @@ qmb_status qmb_mlp_start_vector(qmb_mlp *m, const qmb_basis *b, double delta, do
         QMB_REQUIRE(m && b && x, "qmb_mlp_start_vector: NULL argument");
         DevBuf dx((size_t)b->n_rows * sizeof(double));
         StateWork w;
-        const bool ok = build_start(m, b, delta, j2, 0, dx.as<double>(), w);
-        download(m->ctx, x, dx.p, b->n_rows * sizeof(double));
+        const bool ok = build_start(m, b, delta, j2, 0, dx.as<double>(), w, x);
         if (fallback) *fallback = ok ? 0 : 1;
     });
 }
