@@ -306,7 +306,7 @@ __global__ __launch_bounds__(kThreads) void lz_update(int64_t cnt, const double 
 
 // ---- small sectors: a window of steps in one workgroup -------------------------
 // The words of a small sector's matrix fit one CU's LDS beside the vector, so one
-// workgroup runs a whole window of the plain recurrence: the words, the value
+// workgroup runs a whole window of steps: the words, the value
 // tables and w stay in LDS (the values of an FP64 matrix are read from memory: it
 // takes the same route, so its results are the packed form's), phi_n, phi_{n-1} and y
 // in registers, and a step has two block sums instead of two launches. A step is a
@@ -320,8 +320,23 @@ __global__ __launch_bounds__(kThreads) void lz_update(int64_t cnt, const double 
 // phi_n into X and ||H x - e x|| into *res, from the kept vectors or (keep NULL) by
 // replaying the steps. host: pinned memory that takes a[n] at [n] and b[n] at [host_b +
 // n] too; it, X and res in pinned memory save a copy each.
+// FULL: every new w is orthogonalised against the kept phi (keep) as by
+// reorth_dots and reorth_apply, a second time where the first cancelled most of it: a
+// wavefront takes a kept vector at a time for its coefficient, a thread its own rows of
+// all of them, with 8 and 16 loads in flight (two eigenvalues and a vector, 415 rows:
+// 374 us, 418 with four vectors at a time and the remainders of the unrolled loops one
+// load each; 1299 in eight launches a step, which is what bounds a small sector there).
+// What is left is the latency of the L2 and, with more rows, one CU reading the basis
+// twice a step.
 constexpr int kSmallThreads = 1024, kSmallWaves = kSmallThreads / 64;
 constexpr size_t kSmallLds = 140 * 1024;  // vector and words; value tables of up to 16 KB beside them
+// Doubles of the kept basis up to which a step of full reorthogonalisation is done by
+// one workgroup: beyond, one CU's reading of it takes longer than the launches of the
+// general route (to convergence, 1,768 complex rows, two levels: 1597 us with 100,000,
+// 1643 with 150,000, 1779 with 250,000, 2270 without; 2,704 rows 1409, 1480, 1480,
+// 1456; 1,367 rows 652 and 1457 without). It counts steps, not windows, so results
+// do not depend on check_every.
+constexpr int64_t kSmallBasis = 100000;
 constexpr size_t kSmallKeep = (size_t)64 << 20;  // the kept vectors of a small sector
 
 // v plus its neighbour's by a DPP move (lanes without one add 0)
@@ -339,6 +354,9 @@ __device__ __forceinline__ double row_total(double v) {
     v = dpp_add<0x114>(v);
     return dpp_add<0x118>(v);
 }
+
+// Sum over the wavefront, valid in its last lane (row_bcast:15, 31).
+__device__ __forceinline__ double wave_total(double v) { return dpp_add<0x143, 0xc>(dpp_add<0x142, 0xa>(row_total(v))); }
 
 __device__ __forceinline__ double read_lane(double v, int lane) {
     return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
@@ -360,7 +378,9 @@ inline size_t small_lds_bytes(int64_t n, int64_t stored, int vs) {
 }
 inline size_t small_table_bytes(int n_values, int n_values_im) { return up16((size_t)(n_values + n_values_im) * 8); }
 
-template <bool CPLX, bool PACK, int KR>
+inline size_t small_coef_bytes(int64_t vectors, int vs) { return up16((size_t)vectors * vs * 8); }
+
+template <bool CPLX, bool PACK, int KR, bool FULL = false>
 __global__ __launch_bounds__(kSmallThreads) void lz_small(SmallMatrix m, int it0, int steps, int init, int random,
                                                           uint64_t seed, double *P, double *V0, double *V1,
                                                           double *alpha, double *beta, double *invb,
@@ -372,6 +392,7 @@ __global__ __launch_bounds__(kSmallThreads) void lz_small(SmallMatrix m, int it0
     double *x = small_lds;
     double *vt = x + (m.n * VS + 1) / 2 * 2;
     uint32_t *words = reinterpret_cast<uint32_t *>(vt + (m.n_values + m.n_values_im + 1) / 2 * 2);
+    double *coef = reinterpret_cast<double *>(words + (m.stored + 3) / 4 * 4);  // FULL only
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, n_waves = blockDim.x >> 6;
     for (int i = threadIdx.x; i < m.stored; i += blockDim.x) words[i] = m.words[i];
     for (int i = threadIdx.x; i < m.n_values; i += blockDim.x) vt[i] = m.vtab[i];
@@ -392,7 +413,8 @@ __global__ __launch_bounds__(kSmallThreads) void lz_small(SmallMatrix m, int it0
             const int i = r * VS + q;
             d[k][q] = PACK && r < m.n ? m.diag[i] : 0.0;
             w[k][q] = r < m.n ? (init && random ? splitmix_uniform(seed, (uint64_t)i) : P[i]) : 0.0;
-            prev[k][q] = r < m.n && it0 > 0 ? ((it0 - 1) & 1 ? V1 : V0)[i] : 0.0;
+            const double *last = FULL ? keep + (int64_t)(it0 - 1) * m.n * VS : (it0 - 1) & 1 ? V1 : V0;
+            prev[k][q] = r < m.n && it0 > 0 ? last[i] : 0.0;
             sum[k][q] = 0.0;
             if (r < m.n) x[i] = w[k][q];
         }
@@ -400,7 +422,7 @@ __global__ __launch_bounds__(kSmallThreads) void lz_small(SmallMatrix m, int it0
     // sum over the block, to every thread; alternate buffers leave one barrier between
     // a buffer's readers and its next writers
     auto block_total = [&](double v, int buf) {
-        v = dpp_add<0x143, 0xc>(dpp_add<0x142, 0xa>(row_total(v)));  // row_bcast:15, 31: lane 63 has all
+        v = wave_total(v);
         if (lane == 63) red[buf][wv] = v;
         __syncthreads();
         const int w = lane & (kSmallWaves - 1);
@@ -500,6 +522,75 @@ __global__ __launch_bounds__(kSmallThreads) void lz_small(SmallMatrix m, int it0
             }
         }
         b = sqrt(block_total(nn, 1));
+        if constexpr (FULL) {
+            // loads in flight: rows of a kept vector, kept vectors of a row
+            constexpr int R = CPLX ? 4 : 8, U = (CPLX ? 8 : 16) / (KR == 1 ? 1 : CPLX ? 4 : 2);
+            const int64_t stride = (int64_t)m.n * VS;
+            for (int pass = 0; pass < 2; ++pass) {
+                for (int j = wv; j <= it; j += n_waves) {
+                    const double *v = keep + j * stride;
+                    double re = 0.0, im = 0.0;
+                    for (int r0 = lane; r0 < m.n; r0 += 64 * R) {
+                        double p[R][VS];
+#pragma unroll
+                        for (int u = 0; u < R; ++u) {
+                            const int r = r0 + 64 * u;
+#pragma unroll
+                            for (int q = 0; q < VS; ++q) p[u][q] = r < m.n ? v[r * VS + q] : 0.0;
+                        }
+#pragma unroll
+                        for (int u = 0; u < R; ++u) {
+                            const int r = min(r0 + 64 * u, m.n - 1);
+                            if constexpr (CPLX) {
+                                re += p[u][0] * x[2 * r] + p[u][1] * x[2 * r + 1];
+                                im += p[u][0] * x[2 * r + 1] - p[u][1] * x[2 * r];
+                            } else {
+                                re += p[u][0] * x[r];
+                            }
+                        }
+                    }
+                    re = wave_total(re);
+                    if constexpr (CPLX) im = wave_total(im);
+                    if (lane == 63) {
+                        coef[j * VS] = re;
+                        if constexpr (CPLX) coef[j * VS + 1] = im;
+                    }
+                }
+                __syncthreads();
+                nn = 0.0;
+#pragma unroll
+                for (int k = 0; k < KR; ++k) {
+                    const int r = (wv + k * kSmallWaves) * 64 + lane;
+                    if (r >= m.n) continue;
+                    for (int j0 = 0; j0 <= it; j0 += U) {
+                        double p[U][VS];
+#pragma unroll
+                        for (int u = 0; u < U; ++u)
+#pragma unroll
+                            for (int q = 0; q < VS; ++q) p[u][q] = keep[min(j0 + u, it) * stride + r * VS + q];
+#pragma unroll
+                        for (int u = 0; u < U; ++u) {
+                            if (j0 + u > it) continue;
+                            const double *c = coef + (j0 + u) * VS;
+                            if constexpr (CPLX) {
+                                w[k][0] -= c[0] * p[u][0] - c[1] * p[u][1];
+                                w[k][1] -= c[0] * p[u][1] + c[1] * p[u][0];
+                            } else {
+                                w[k][0] -= c[0] * p[u][0];
+                            }
+                        }
+                    }
+#pragma unroll
+                    for (int q = 0; q < VS; ++q) {
+                        x[r * VS + q] = w[k][q];
+                        nn += w[k][q] * w[k][q];
+                    }
+                }
+                const double was = b;
+                b = sqrt(block_total(nn, 1));
+                if (!(b < kDgks * was)) break;
+            }
+        }
         s = b > 0.0 ? 1.0 / b : 0.0;
         if (threadIdx.x == 0) {
             alpha[it] = a;
@@ -524,7 +615,7 @@ __global__ __launch_bounds__(kSmallThreads) void lz_small(SmallMatrix m, int it0
                 x[i] = sum[k][q];  // every gather of w lies before the last barrier
             } else {
                 P[i] = w[k][q];
-                vlast[i] = prev[k][q];
+                if (!FULL) vlast[i] = prev[k][q];
             }
         }
     }
@@ -859,7 +950,7 @@ void launch_spmv(qmb_ctx *ctx, const qmb_ell *e, const double *x, double *y, boo
     if (lz && !fb) launch_finish(ctx, wk->partials.as<double>(), blocks, alpha_out, nullptr, 0);
 }
 
-// Whether a window of the plain recurrence runs in one workgroup (lz_small): the
+// Whether a window of steps runs in one workgroup (lz_small): the
 // words and a vector within kSmallLds, at most 4 rows a thread (2 complex).
 static bool fits_small(const qmb_ell *e) {
     const bool cplx = e->value_type == QMB_COMPLEX;
@@ -870,7 +961,7 @@ static bool fits_small(const qmb_ell *e) {
 static void launch_small(qmb_ctx *ctx, const qmb_ell *e, LzWork &wk, int it0, int steps, bool init, bool random,
                          uint64_t seed, double *P, double *V0, double *V1, const double *z = nullptr, double eig = 0.0,
                          double *X = nullptr, double *res = nullptr, double *keep = nullptr,
-                         double *host = nullptr) {
+                         double *host = nullptr, bool full = false) {
     const bool cplx = e->value_type == QMB_COMPLEX;
     SmallMatrix m{};
     m.n = (int)e->n_rows;
@@ -890,16 +981,20 @@ static void launch_small(qmb_ctx *ctx, const qmb_ell *e, LzWork &wk, int it0, in
         m.val = e->val.as<double>();
     }
     using K = decltype(&lz_small<false, false, 1>);
-    // [complex][packed][rows a thread: 1, 2, 4]
-    static const K table[2][2][3] = {{{lz_small<false, false, 1>, lz_small<false, false, 2>, lz_small<false, false, 4>},
-                                      {lz_small<false, true, 1>, lz_small<false, true, 2>, lz_small<false, true, 4>}},
-                                     {{lz_small<true, false, 1>, lz_small<true, false, 2>, nullptr},
-                                      {lz_small<true, true, 1>, lz_small<true, true, 2>, nullptr}}};
+    // [full reorthogonalisation][complex][packed][rows a thread: 1, 2, 4]
+#define QMB_SMALL(C, P, F) {lz_small<C, P, 1, F>, lz_small<C, P, 2, F>, C ? nullptr : lz_small<C, P, C ? 2 : 4, F>}
+    static const K table[2][2][2][3] = {
+        {{QMB_SMALL(false, false, false), QMB_SMALL(false, true, false)},
+         {QMB_SMALL(true, false, false), QMB_SMALL(true, true, false)}},
+        {{QMB_SMALL(false, false, true), QMB_SMALL(false, true, true)},
+         {QMB_SMALL(true, false, true), QMB_SMALL(true, true, true)}}};
+#undef QMB_SMALL
     const int kr = (int)((e->n_chunks + kSmallWaves - 1) / kSmallWaves);
-    const K k = table[cplx ? 1 : 0][e->packed ? 1 : 0][kr <= 1 ? 0 : kr <= 2 ? 1 : 2];
+    const K k = table[full ? 1 : 0][cplx ? 1 : 0][e->packed ? 1 : 0][kr <= 1 ? 0 : kr <= 2 ? 1 : 2];
     const size_t lds = small_lds_bytes(e->n_rows, e->stored, cplx ? 2 : 1) +
-                       small_table_bytes(m.n_values, m.n_values_im);
-    const int threads = 64 * (int)std::min<int64_t>(kSmallWaves, e->n_chunks);
+                       small_table_bytes(m.n_values, m.n_values_im) +
+                       (full ? small_coef_bytes(it0 + steps, cplx ? 2 : 1) : 0);
+    const int threads = full ? kSmallThreads : 64 * (int)std::min<int64_t>(kSmallWaves, e->n_chunks);
     hipLaunchKernelGGL(k, dim3(1), dim3(threads), lds, ctx->stream, m, it0, steps, init ? 1 : 0, random ? 1 : 0,
                        seed, P, V0, V1, wk.alpha(), wk.beta(), wk.invb(), z, eig, X, res,
                        keep, host, wk.M);
@@ -968,6 +1063,16 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
     const bool reorth = rmode != 0;
     const bool selective = rmode == 3;
     const bool small = rmode == 0 && !o.profile && fits_small(e);
+    // full reorthogonalisation: the steps n < small_steps run in one workgroup as well
+    const int64_t basis_steps = std::min<int64_t>(M, kSmallBasis / cnt);
+    const int vs = cplx ? 2 : 1;
+    const int small_steps =
+        rmode == 1 && !o.profile && fits_small(e) &&
+                small_lds_bytes(n, e->stored, vs) + small_coef_bytes(basis_steps, vs) <= kSmallLds
+            ? (int)basis_steps
+            : 0;
+    // lz_small draws the seeded vector and takes the norm itself
+    const bool own_start = small || small_steps > 0;
     // the selective scheme looks for converged Ritz pairs after every step
     const int check = o.fixed_iter ? M : selective ? 1 : (o.check_every > 0 ? o.check_every : 10);
     constexpr int kMaxGood = 8;  // Ritz vectors kept by the selective scheme (full reorthogonalisation beyond)
@@ -1047,13 +1152,12 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
         } else if (o.start == QMB_START_DEVICE) {
             QMB_REQUIRE(o.start_vec != nullptr, "qmb_lanczos: start == DEVICE needs start_vec");
             QMB_HIP(hipMemcpyAsync(P.p, o.start_vec, cnt * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
-        } else if (!small) {
+        } else if (!own_start) {
             hipLaunchKernelGGL(lz_random, dim3(grid_for(cnt, kThreads * 4)), dim3(kThreads), 0, ctx->stream, cnt,
                                o.seed, P.as<double>());
             QMB_HIP(hipGetLastError());
         }
-        // lz_small draws the seeded vector and takes the norm itself
-        if (!small) launch_norm(ctx, cnt, P.as<double>(), nullptr, 0.0, wk, wk.misc(), wk.invb());
+        if (!own_start) launch_norm(ctx, cnt, P.as<double>(), nullptr, 0.0, wk, wk.misc(), wk.invb());
     };
     const bool random_start = o.start == QMB_START_RANDOM;
     const unsigned ublocks = grid_for(cnt, kThreads * 4);
@@ -1362,12 +1466,15 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
     while (it < M) {
         const int win0 = it;
         const int win1 = std::min(M, it + next);
-        if (small) {
-            launch_small(ctx, e, wk, win0, win1 - win0, win0 == 0, random_start, o.seed, P.as<double>(),
+        const int small1 = small ? win1 : std::min(win1, small_steps);
+        if (small1 > win0) {
+            launch_small(ctx, e, wk, win0, small1 - win0, win0 == 0, random_start, o.seed, P.as<double>(),
                          V0.as<double>(), V1.as<double>(), nullptr, 0.0, nullptr, nullptr,
-                         small_keep.as<double>(), ctx->host_stage<double>((size_t)(2 * M + 1) * sizeof(double)));
-            it = it_q = win1;
+                         small ? small_keep.as<double>() : VB.as<double>(),
+                         ctx->host_stage<double>((size_t)(2 * M + 1) * sizeof(double)), !small);
+            it = it_q = small1;
             b_ready[it] = 1;
+            if (!small) n_reorth += small1 - win0;
         }
         for (; it < win1; ++it)
             if (it >= it_q) queue_step(it, it - win0, wpar, it + 1 == win1);
@@ -1376,7 +1483,7 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
         // into pinned memory
         const size_t span = (size_t)M + it + 1;
         double *st = ctx->host_stage<double>(span * sizeof(double));
-        const bool direct = small && !ck;  // the window's kernel has written its part there
+        const bool direct = small1 == win1 && !ck;  // the window's kernel has written its part there
         if (direct) {
             QMB_HIP(hipStreamSynchronize(ctx->stream));
         } else {
@@ -1522,28 +1629,30 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
     }
     double eig_res = 0.0;
     if (o.want_eigvec && !stopped) {
+        const bool small_vec = small_steps > 0;  // the kept basis and a small matrix
         // rebuild x = sum_j z0[j] phi_j (the reference's second pass, lanczos.cu:31-104)
         DevBuf X(cnt * sizeof(double));
-        if (reorth) {
+        if (reorth && !small_vec) {
             DevBuf dz(m * sizeof(double));
             QMB_HIP(hipMemcpyAsync(dz.p, z0.data(), m * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
             hipLaunchKernelGGL(basis_combine, dim3(grid_for(cnt, kThreads * 4)), dim3(kThreads), 0, ctx->stream, cnt,
                                (int64_t)cnt, m, VB.as<double>(), dz.as<double>(), X.as<double>(), 0);
             QMB_HIP(hipGetLastError());
-        } else if (small) {
+        } else if (small || small_vec) {
             // z, x and the residual in pinned memory; a replay reads z every step
             double *hz = ctx->host_stage<double>((size_t)(m + cnt + 1) * sizeof(double));
             std::copy(z0.begin(), z0.begin() + m, hz);
             const double *z = hz;
             DevBuf dz;
-            if (!small_keep.p) {
+            if (!small_keep.p && !small_vec) {
                 dz.alloc(m * sizeof(double));
                 QMB_HIP(hipMemcpyAsync(dz.p, hz, m * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
                 z = dz.as<double>();
                 init_start();
             }
             launch_small(ctx, e, wk, 0, m, true, random_start, o.seed, P.as<double>(), V0.as<double>(),
-                         V1.as<double>(), z, evals[0], hz + m, hz + m + cnt, small_keep.as<double>());
+                         V1.as<double>(), z, evals[0], hz + m, hz + m + cnt,
+                         small_vec ? VB.as<double>() : small_keep.as<double>());
             QMB_HIP(hipStreamSynchronize(ctx->stream));
             eig_res = hz[m + cnt];
             if (eigvec) std::copy(hz + m, hz + m + cnt, eigvec);
@@ -1572,11 +1681,9 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
                 k2(j, false);
             }
         }
-        if (!small) {
+        if (!small && !small_vec) {
             launch_spmv(ctx, e, X.as<double>(), Y.as<double>(), false, nullptr, nullptr, nullptr, nullptr);
             launch_norm(ctx, cnt, Y.as<double>(), X.as<double>(), evals[0], wk, wk.misc() + 1, wk.misc() + 2);
-        }
-        if (!small) {
             QMB_HIP(hipMemcpyAsync(&eig_res, wk.misc() + 1, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
             if (eigvec)
                 download(ctx, eigvec, X.p, cnt * sizeof(double));
