@@ -709,13 +709,17 @@ __global__ __launch_bounds__(1024) void ell_code_tables(const unsigned *used, in
     }
 }
 
-// In place, when the tables are complete and the indexes fit: every
-// off-diagonal slot k < len gets its value index(es) beside the column (slot 0
-// and the padding slots keep index 0, the value +0.0). Four slots at a time,
-// each slot's map read issued with its word load (6x6 sector: 12.2 ms; eight
-// slots, or the map staged in LDS and read after the loads, 14.4-16.8 ms).
-__global__ __launch_bounds__(kEllThreads) void ell_pack_codes(int64_t n_rows, const int64_t *chunk_ptr,
-                                                              const uint16_t *row_len, uint32_t *colw,
+// When the tables are complete and the indexes fit: every off-diagonal slot k <
+// len gets its value index(es) beside the column (slot 0 and the padding slots
+// keep index 0, the value +0.0). Four slots at a time, each slot's map read issued
+// with its word load (6x6 sector: 12.2 ms; eight slots, or the map staged in LDS
+// and read after the loads, 14.4-16.8 ms). In place (dst = colw), or with MOVE from
+// the room of a build without a wait into the matrix's own block, the slots that
+// stay as they are and those of the rows past n_rows (n_lanes) too.
+template <bool MOVE>
+__global__ __launch_bounds__(kEllThreads) void ell_pack_codes(int64_t n_rows, int64_t n_lanes,
+                                                              const int64_t *chunk_ptr, const uint16_t *row_len,
+                                                              const uint32_t *colw, uint32_t *dst,
                                                               const uint16_t *code, const uint32_t *map,
                                                               const int *f, int cplx, int cb) {
     if (!f[2] || (cplx && !f[5])) return;
@@ -724,24 +728,25 @@ __global__ __launch_bounds__(kEllThreads) void ell_pack_codes(int64_t n_rows, co
         sh2 = cb + index_bits(f[1]);
         if (sh2 + index_bits(f[4]) > 32) return;
     }
-    for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < n_rows;
+    for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < n_lanes;
          r += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t base = chunk_ptr[r / kChunk] + r % kChunk;
-        const int len = row_len[r];
-        for (int k = 1; k < len; k += 4) {
+        const int64_t chunk0 = chunk_ptr[r / kChunk], base = chunk0 + r % kChunk;
+        const int len = r < n_rows ? (int)row_len[r] : 0;
+        const int last = MOVE ? (int)((chunk_ptr[r / kChunk + 1] - chunk0) / kChunk) : len;
+        for (int k = MOVE ? 0 : 1; k < last; k += 4) {
             uint32_t m[4], w[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 const int64_t p = base + (int64_t)(k + u) * kChunk;
-                m[u] = k + u < len ? map[code[p]] : 0u;
-                w[u] = k + u < len ? colw[p] : 0u;
+                m[u] = k + u > 0 && k + u < len ? map[code[p]] : 0u;
+                w[u] = k + u < last ? colw[p] : 0u;
             }
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                if (k + u >= len) continue;
+                if (k + u >= last) continue;
                 const uint64_t ix = cplx ? (((uint64_t)(m[u] & 0xFFFFu) << cb) | ((uint64_t)(m[u] >> 16) << sh2))
                                          : (uint64_t)m[u] << cb;
-                colw[base + (int64_t)(k + u) * kChunk] = w[u] | (uint32_t)ix;
+                dst[base + (int64_t)(k + u) * kChunk] = w[u] | (uint32_t)ix;
             }
         }
     }
@@ -839,8 +844,8 @@ struct ValuePacking {
         return true;
     }
     // after a coded fill: codes in use -> their values -> sorted tables -> code
-    // to index map -> packed words
-    void launch_coded(qmb_ctx *ctx, qmb_ell &e) {
+    // to index map
+    void launch_tables(qmb_ctx *ctx, qmb_ell &e) {
         const int parts = cplx ? 2 : 1;
         e.vtab.alloc((size_t)parts * kMaxValues * 8);
         unsigned long long *keys = e.vtab.as<unsigned long long>();
@@ -852,9 +857,15 @@ struct ValuePacking {
         hipLaunchKernelGGL(ell_code_tables, dim3(1), dim3(1024), 0, ctx->stream, used, n_codes, ct, cplx ? 1 : 0, cap,
                            cval.as<double2>(), keys, f, map.as<uint32_t>());
         QMB_HIP(hipGetLastError());
-        hipLaunchKernelGGL(ell_pack_codes, dim3(blocks), dim3(kEllThreads), 0, ctx->stream, e.n_rows,
-                           e.chunk_ptr.as<int64_t>(), e.row_len.as<uint16_t>(), e.col.as<uint32_t>(),
-                           codes.as<uint16_t>(), map.as<uint32_t>(), f, cplx ? 1 : 0, cb);
+    }
+    // then the packed words, from the columns at colw (e.col itself: in place) into e.col
+    void launch_pack(qmb_ctx *ctx, qmb_ell &e, const uint32_t *colw) {
+        const bool move = colw != e.col.as<uint32_t>();
+        const int64_t lanes = move ? e.n_chunks * kChunk : e.n_rows;
+        const unsigned blocks = (unsigned)std::min<int64_t>(4096, (lanes + kEllThreads - 1) / kEllThreads);
+        hipLaunchKernelGGL(move ? ell_pack_codes<true> : ell_pack_codes<false>, dim3(blocks), dim3(kEllThreads), 0,
+                           ctx->stream, e.n_rows, lanes, e.chunk_ptr.as<int64_t>(), e.row_len.as<uint16_t>(), colw,
+                           e.col.as<uint32_t>(), codes.as<uint16_t>(), map.as<uint32_t>(), f, cplx ? 1 : 0, cb);
         QMB_HIP(hipGetLastError());
         QMB_HIP(hipMemcpyAsync(ctx->host_stage<int>((8 + kScanStats) * sizeof(int64_t)), f, 8 * sizeof(int),
                                hipMemcpyDeviceToHost, ctx->stream));
@@ -1056,7 +1067,7 @@ qmb_status qmb_ell_build(qmb_ctx *ctx, const qmb_basis *b, const qmb_terms *t, i
             e->max_row_len = (int)st[2];
         };
         // the fill (coded, or with FP64 values), with the padding of the last chunk
-        auto fill = [&](bool with_codes) {
+        auto fill = [&](bool with_codes, int32_t *col) {
             const EllRows kfill = ell_fill_kernel(narrow, cplx, with_codes, ts != 0, gv.lut);
             double *val = with_codes ? nullptr : e->val.as<double>();
             hipLaunchKernelGGL(kfill, dim3(blocks_for(e->n_chunks * kChunk, ts)), dim3(kEllThreads), lds_bytes,
@@ -1065,16 +1076,18 @@ qmb_status qmb_ell_build(qmb_ctx *ctx, const qmb_basis *b, const qmb_terms *t, i
                                b->stab.as<uint8_t>(), b->nullf.as<uint8_t>(), b->dict.as<uint64_t>(),
                                tv, n_lds, dt.chi, dt.nrm, W,
                                e->row_len.as<uint16_t>(), d_err, 0, e->chunk_ptr.as<int64_t>(),
-                               e->col.as<int32_t>(), val, with_codes ? vp.cv : CodeView{}, ts);
+                               col, val, with_codes ? vp.cv : CodeView{}, ts);
             QMB_HIP(hipGetLastError());
         };
         // a packed build writes value codes (2 B per entry) instead of FP64 values when
         // the factors of the values give few enough codes
         bool coded = false;
-        // A small matrix is built without a wait in between: its columns get the room
-        // of rows with every term (at most kOpenSlots slots), and its codes classes for
-        // every divisor of the group's order. Bound by launches and waits (415 rows:
-        // build 111 us waiting, 85 without; 56,450 rows 149 / 132).
+        // A small matrix is filled before its size is known: the columns get the room of
+        // rows with every term (at most kOpenSlots slots), and the codes classes for every
+        // divisor of the group's order. The size arrives while the fill runs, and the last
+        // pass writes the words into a block of that size: the room is given back. Bound by
+        // launches and waits (415 rows: build 111 us waiting, 85 without; 56,450 rows 149 /
+        // 132).
         const int64_t room = e->n_chunks * kChunk * ((int64_t)tv.n_off + 1);
         if (try_codes && room <= kOpenSlots) {
             std::vector<int> divisors;
@@ -1086,14 +1099,18 @@ qmb_status qmb_ell_build(qmb_ctx *ctx, const qmb_basis *b, const qmb_terms *t, i
         if (coded) {
             launch_chunk_scan(ctx, e->row_len.as<uint16_t>(), n, e->chunk_ptr.as<int64_t>(), e->n_chunks, d_err,
                               d_stats);
-            e->col.alloc((size_t)room * sizeof(int32_t));
-            fill(true);
-            vp.launch_coded(ctx, *e);
             int64_t *st = ctx->host_stage<int64_t>((8 + kScanStats) * sizeof(int64_t)) + 8;  // after the flags
+            if (!ctx->stats_read) QMB_HIP(hipEventCreateWithFlags(&ctx->stats_read, hipEventDisableTiming));
             QMB_HIP(hipMemcpyAsync(st, d_stats, kScanStats * sizeof(int64_t), hipMemcpyDeviceToHost, ctx->stream));
-            QMB_HIP(hipStreamSynchronize(ctx->stream));
+            QMB_HIP(hipEventRecord(ctx->stats_read, ctx->stream));
+            DevBuf wide((size_t)room * sizeof(int32_t));
+            fill(true, wide.as<int32_t>());
+            vp.launch_tables(ctx, *e);
+            QMB_HIP(hipEventSynchronize(ctx->stats_read));
             take_stats(st);
-            e->col.bytes = (size_t)std::max<int64_t>(e->stored, 1) * sizeof(int32_t);
+            e->col.alloc((size_t)std::max<int64_t>(e->stored, 1) * sizeof(int32_t), true);
+            vp.launch_pack(ctx, *e, wide.as<uint32_t>());
+            QMB_HIP(hipStreamSynchronize(ctx->stream));
         } else {
             // the offsets are scanned and the stabiliser sizes collected before the
             // overflow flag is read (one synchronisation)
@@ -1121,18 +1138,20 @@ qmb_status qmb_ell_build(qmb_ctx *ctx, const qmb_basis *b, const qmb_terms *t, i
             coded = known && vp.plan_codes(ctx, *e, sizes, used, dt, ch, g->G);
             if (!coded) e->val.alloc((size_t)std::max<int64_t>(e->stored, 1) * (cplx ? 16 : 8));
             if (n > 0) {
-                fill(coded);
-                if (coded)
-                    vp.launch_coded(ctx, *e);
-                else if (vp.on)
+                fill(coded, e->col.as<int32_t>());
+                if (coded) {
+                    vp.launch_tables(ctx, *e);
+                    vp.launch_pack(ctx, *e, e->col.as<uint32_t>());
+                } else if (vp.on) {
                     vp.launch(ctx, *e);
+                }
             }
             QMB_HIP(hipStreamSynchronize(ctx->stream));
         }
         if (vp.on && !vp.finish(ctx, *e) && coded) {
             // more distinct values than the index bits hold: the FP64 form
             e->val.alloc((size_t)std::max<int64_t>(e->stored, 1) * (cplx ? 16 : 8));
-            fill(false);
+            fill(false, e->col.as<int32_t>());
             QMB_HIP(hipStreamSynchronize(ctx->stream));
         }
         *out = e.release();

@@ -75,7 +75,8 @@ struct DevPool {
     size_t max_cached = (size_t)16 << 30;  // set from the device memory when the context is created
     static constexpr size_t kBig = (size_t)1 << 30;
 
-    void *get(size_t n, size_t &cap) {
+    // kept: a block that stays with its handle, handed out only within 1/8 of its size
+    void *get(size_t n, size_t &cap, bool kept = false) {
         {
             std::lock_guard<std::mutex> lock(m);
             if (!pending.empty() && hipStreamQuery(stream) == hipSuccess) {
@@ -83,7 +84,7 @@ struct DevPool {
                 pending.clear();
             }
             auto it = ready.lower_bound(n);
-            if (it != ready.end() && it->first <= (n >= kBig ? n + n / 8 : 2 * n)) {
+            if (it != ready.end() && it->first <= (kept || n >= kBig ? n + n / 8 : 2 * n)) {
                 void *p = it->second;
                 cap = it->first;
                 cached -= cap;
@@ -173,12 +174,12 @@ struct DevBuf {
         return *this;
     }
     ~DevBuf() { release(); }
-    void alloc(size_t n) {
+    void alloc(size_t n, bool kept = false) {
         release();
         if (n == 0) n = 8;
         pool = current_pool();
         if (pool) {
-            p = pool->get(n, cap);
+            p = pool->get(n, cap, kept);
         } else {
             QMB_HIP(hipMalloc(&p, n));
             cap = n;
@@ -320,6 +321,7 @@ struct qmb_ctx : qmb::Counted {
     std::unique_ptr<qmb::PinnedBuf> up;  // slots of upload(), used in turn
     size_t up_at = 0;
     hipEvent_t up_done = nullptr;  // after the last upload
+    hipEvent_t stats_read = nullptr;  // after the read-back of a build's statistics
     std::unique_ptr<qmb::PinnedBuf> bulk;  // slots of download_bulk (16 MB, made by the first large read-back)
     ~qmb_ctx() {
         if (stream) {
@@ -331,6 +333,7 @@ struct qmb_ctx : qmb::Counted {
         bulk.reset();
         up.reset();
         if (up_done) (void)hipEventDestroy(up_done);
+        if (stats_read) (void)hipEventDestroy(stats_read);
         pool.trim();
         pool.stream = nullptr;
         if (stream) (void)hipStreamDestroy(stream);
