@@ -749,6 +749,9 @@ static void check_closure_and_irreps(qmb_group &g) {
     };
     std::vector<int> first(G);
     for (int e = 0; e < G; ++e) first[e] = index.emplace(key(&g.perm[(size_t)e * n], g.flip[e]), e).first->second;
+    std::vector<int> times(G, 0);
+    for (int e = 0; e < G; ++e) ++times[first[e]];
+    for (int e = 0; e < G; ++e) g.uneven = g.uneven || times[first[e]] != times[0];
     g.irrep_ok.assign(g.n_irreps, 1);
     auto chi = [&](int a, int e) { return std::complex<double>(g.chars[((size_t)a * G + e) * 2], g.chars[((size_t)a * G + e) * 2 + 1]); };
     const double tol = 1e-9;

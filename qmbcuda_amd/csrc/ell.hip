@@ -1084,12 +1084,13 @@ qmb_status qmb_ell_build(qmb_ctx *ctx, const qmb_basis *b, const qmb_terms *t, i
         bool coded = false;
         // A small matrix is filled before its size is known: the columns get the room of
         // rows with every term (at most kOpenSlots slots), and the codes classes for every
-        // divisor of the group's order. The size arrives while the fill runs, and the last
+        // divisor of the group's order (other stabiliser sizes come from uneven lists only,
+        // whose sizes are collected). The size arrives while the fill runs, and the last
         // pass writes the words into a block of that size: the room is given back. Bound by
         // launches and waits (415 rows: build 111 us waiting, 85 without; 56,450 rows 149 /
         // 132).
         const int64_t room = e->n_chunks * kChunk * ((int64_t)tv.n_off + 1);
-        if (try_codes && room <= kOpenSlots) {
+        if (try_codes && room <= kOpenSlots && !g->uneven) {
             std::vector<int> divisors;
             for (int m = 1; m <= g->G; ++m)
                 if (g->G % m == 0) divisors.push_back(m);

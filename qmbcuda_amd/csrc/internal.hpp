@@ -350,6 +350,10 @@ struct qmb_group : qmb::Counted {
     std::vector<uint64_t> keep;
     std::vector<uint8_t> small, big;
     std::vector<uint8_t> irrep_ok;  // [n_irreps]: the row is a one-dimensional representation
+    // some elements are listed more often than others: stabiliser sizes count every
+    // appearance, so they need not divide G and a symmetric operator's sector matrix
+    // need not be symmetric
+    bool uneven = false;
     uint64_t hash = 0;              // FNV-1a of the element tables, flips and characters
     int lut = 0, lut_flip = 0;     // 1: full torus product with block width <= 8; 2: full ring;
                                    // 3: a full ring subgroup H times coset representatives
