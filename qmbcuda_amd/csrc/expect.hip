@@ -442,6 +442,9 @@ static unsigned char *scratch_ptr(int device) {
 // state of its orbit, so a term that lowers it ends in an orbit of a lower
 // representative, a lower row: entries M_rt with t >= r come from the terms that raise
 // the state alone, and only those are looked up.
+//
+// Both need every element listed equally often: of an uneven list the orbit weights of
+// M_rt and M_tr differ, and an image's weights are not those of its representative.
 struct ExpectTable {
     std::vector<unsigned char> bytes;  // t[n_terms], z[n_sz]
     ExpectTerms view{};
@@ -454,7 +457,7 @@ struct ExpectTable {
         std::vector<TermC> terms = std::move(own.terms);
         images = average;
         const size_t all = terms.size() * (size_t)g.G;
-        if (average && (all <= 4096 || n_rows >= 4096)) {
+        if (average && !g.uneven && (all <= 4096 || n_rows >= 4096)) {
             TermSum sum;
             for (const TermC &c : terms) {
                 for (int e = 0; e < g.G; ++e) sum.add(term_image(c, g, e));
@@ -466,7 +469,7 @@ struct ExpectTable {
                 for (TermC &c : terms) c.coef = make_double2(c.coef.x / g.G, c.coef.y / g.G);
             }
         }
-        view.half = !images && hermitian(terms);
+        view.half = !images && !g.uneven && hermitian(terms);
         if (view.half)
             terms.erase(std::remove_if(terms.begin(), terms.end(),
                                        [](const TermC &c) { return c.set_val < (c.req_val & c.set); }),

@@ -1,6 +1,7 @@
 """Element lists in which some elements appear more often than others. They are accepted;
-stabiliser sizes count every appearance, so a size need not divide the length of the list. The
-matrix against the plain formula over all listed elements."""
+stabiliser sizes count every appearance, so a size need not divide the length of the list
+and the sector matrix of a symmetric operator need not be symmetric. Matrix and
+expectation values against the plain formulas over all listed elements."""
 import numpy as np
 import pytest
 
@@ -54,6 +55,16 @@ def row(u, m_src, ge, table, reps):
     return out
 
 
+def value(x, ge, table, reps, average):
+    total = 0j
+    for r, rep in enumerate(reps):
+        m_src = sum(image(rep, p) == rep for p in ge)
+        us = [image(rep, p) for p in ge] if average else [rep]
+        mx = sum(v * x[r if t is None else t] for u in us for t, v in row(u, m_src, ge, table, reps)) / len(us)
+        total += x[r] * np.conj(mx)
+    return total
+
+
 @pytest.mark.gpu
 def test_matrix_with_a_size_that_does_not_divide(ctx, monkeypatch):
     print("[gpu-case] repeated elements: matrix", flush=True)
@@ -73,3 +84,28 @@ def test_matrix_with_a_size_that_does_not_divide(ctx, monkeypatch):
             want[r, r if t is None else t] += v.real
     assert np.array_equal(got[0], got[1])
     assert np.abs(got[0] - want).max() < 1e-15
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", [q.LAYOUT_COMPACT, q.LAYOUT_REFERENCE])
+@pytest.mark.parametrize("n,shifts", [(4, [0, 1, 2, 3, 2]), (8, [0, 1, 2, 3, 4, 5, 6, 7, 4]),
+                                      (8, list(range(8)) * 2)])  # the last: every element twice
+def test_expectation(ctx, n, shifts, layout):
+    print(f"[gpu-case] repeated elements: expectation n={n} G={len(shifts)} layout={layout}", flush=True)
+    ge, ch = ring_list(n, shifts)
+    b = q.Basis(ctx, q.Group(ge, ch), n // 2, 0, layout)
+    reps = [int(v) for v in b.export()[0]]
+    bonds = []
+    for i in range(n):
+        j = (i + 1) % n
+        bonds += [[(i, SP, 0.5 + 0j), (j, SM, 1 + 0j)], [(i, SM, 0.5 + 0j), (j, SP, 1 + 0j)],
+                  [(i, SZ, 1 + 0j), (j, SZ, 1 + 0j)]]
+    r = np.random.default_rng(n)
+    x = r.normal(size=len(reps)) + 1j * r.normal(size=len(reps))
+    x /= np.linalg.norm(x)
+    for terms, average in ((bonds, False), (bonds[:2], True)):
+        table = OM.conjugated_term_table(terms)
+        v, averaged = b.expectation(q.Terms(n, table), x)
+        assert averaged == average
+        # at most some 40 terms a row, each within 4 rounding units
+        assert abs(v - value(x, ge, table, reps, average)) < 1e-13
