@@ -181,7 +181,13 @@ struct DevBuf {
         if (pool) {
             p = pool->get(n, cap, kept);
         } else {
-            QMB_HIP(hipMalloc(&p, n));
+            const hipError_t e = hipMalloc(&p, n);
+            if (e != hipSuccess) {
+                p = nullptr;
+                (void)hipGetLastError();  // else the next launch's check would report it
+                throw Error{e == hipErrorOutOfMemory ? QMB_ERR_OOM : QMB_ERR_HIP,
+                            std::string("hipMalloc: ") + hipGetErrorString(e)};
+            }
             cap = n;
         }
         bytes = n;

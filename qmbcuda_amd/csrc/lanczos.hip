@@ -1134,7 +1134,8 @@ qmb_status run_lanczos(qmb_ctx *ctx, const qmb_ell *e, const qmb_lanczos_opts &o
             try {
                 kept.emplace_back((size_t)kKeepBlock * cnt * sizeof(double));
                 return kept.back().as<double>();
-            } catch (const Error &) {  // taken by another program meanwhile
+            } catch (const Error &err) {  // taken by another program meanwhile
+                if (err.code != QMB_ERR_OOM) throw;
                 keep_most = it;
             }
         }
