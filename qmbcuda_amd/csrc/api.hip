@@ -46,14 +46,12 @@ void ensure_binom(qmb_ctx *ctx) {
 constexpr size_t kUploadBytes = (size_t)64 << 10;
 
 void upload(qmb_ctx *ctx, void *dst, const void *src, size_t bytes) {
-    if (bytes > kUploadBytes) {
+    if (!ctx->up_done) QMB_HIP(hipEventCreateWithFlags(&ctx->up_done, hipEventDisableTiming));
+    if (!ctx->up && bytes <= kUploadBytes) ctx->up = PinnedBuf::or_none(kUploadBytes);
+    if (!ctx->up || bytes > kUploadBytes) {
         QMB_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream));
         QMB_HIP(hipStreamSynchronize(ctx->stream));
         return;
-    }
-    if (!ctx->up) {
-        ctx->up = std::make_unique<PinnedBuf>(kUploadBytes);
-        QMB_HIP(hipEventCreateWithFlags(&ctx->up_done, hipEventDisableTiming));
     }
     if (ctx->up_at + bytes > kUploadBytes) {  // round again, after the last of the previous round
         QMB_HIP(hipEventSynchronize(ctx->up_done));
@@ -114,12 +112,12 @@ void download(qmb_ctx *ctx, void *dst, const void *src, size_t bytes) {
         else
             plain = a.type != hipMemoryTypeUnregistered;
     }
-    if (plain) {
+    if (!plain && !ctx->bulk) ctx->bulk = PinnedBuf::or_none(kBulkThreads * 2 * kBulkPiece);
+    if (plain || !ctx->bulk) {
         QMB_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
         QMB_HIP(hipStreamSynchronize(ctx->stream));
         return;
     }
-    if (!ctx->bulk) ctx->bulk = std::make_unique<PinnedBuf>(kBulkThreads * 2 * kBulkPiece);
     const int threads = bytes < kBulkBytes ? 1 : kBulkThreads;
     hipError_t err[kBulkThreads] = {};
     std::thread helper[kBulkThreads];

@@ -210,7 +210,22 @@ struct DevBuf {
 // Page-locked host memory (hipHostMalloc) for copies that must not block the host.
 struct PinnedBuf {
     void *p = nullptr;
-    explicit PinnedBuf(size_t n) { QMB_HIP(hipHostMalloc(&p, n == 0 ? 8 : n, hipHostMallocDefault)); }
+    explicit PinnedBuf(size_t n) {
+        const hipError_t e = hipHostMalloc(&p, n == 0 ? 8 : n, hipHostMallocDefault);
+        if (e == hipSuccess) return;
+        p = nullptr;
+        (void)hipGetLastError();  // else the next launch's check would report it
+        throw Error{e == hipErrorOutOfMemory ? QMB_ERR_OOM : QMB_ERR_HIP,
+                    std::string("hipHostMalloc: ") + hipGetErrorString(e)};
+    }
+    // For callers that can do without: none when it cannot be had.
+    static std::unique_ptr<PinnedBuf> or_none(size_t n) {
+        try {
+            return std::make_unique<PinnedBuf>(n);
+        } catch (const Error &) {
+            return nullptr;
+        }
+    }
     PinnedBuf(const PinnedBuf &) = delete;
     PinnedBuf &operator=(const PinnedBuf &) = delete;
     ~PinnedBuf() {
@@ -318,9 +333,9 @@ struct qmb_ctx : qmb::Counted {
     template <class T>
     T *host_stage(size_t bytes) {
         if (bytes > stage_bytes) {
-            stage.reset();
-            stage_bytes = std::max<size_t>(bytes, 64 * 1024);
-            stage = std::make_unique<qmb::PinnedBuf>(stage_bytes);
+            const size_t grown = std::max<size_t>(bytes, 64 * 1024);
+            stage = std::make_unique<qmb::PinnedBuf>(grown);  // when it throws, the old one stays
+            stage_bytes = grown;
         }
         return stage->as<T>();
     }
@@ -449,12 +464,12 @@ inline void require_device_range(const qmb_ctx *ctx, const void *p, size_t bytes
 }
 
 // Device to host memory of the caller, after the work on the context's stream; the
-// data is there when it returns.
+// data is there when it returns. Without its pinned slots it is the runtime's copy.
 void download(qmb_ctx *ctx, void *dst, const void *src, size_t bytes);
 
 // A host table to the device on the context's stream, through pinned slots: the call
 // returns at once (a copy from ordinary memory waits for the stream: some 15 us each
-// in the build of a small matrix).
+// in the build of a small matrix; that one is taken where the slots cannot be had).
 void upload(qmb_ctx *ctx, void *dst, const void *src, size_t bytes);
 
 // Exclusive scans on device (3-phase). Values come from a functor.

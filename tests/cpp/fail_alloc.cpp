@@ -1,7 +1,7 @@
 // hipMalloc and hipHostMalloc in front of the HIP runtime's, for tests of a full device
 // and of missing page-locked memory: loaded with global symbols before libqmb, which then
 // calls these. A call whose size lies in the chosen range fails once `skip` such calls
-// have succeeded; every other call goes through.
+// have succeeded, `times` times; every other call goes through.
 #include <dlfcn.h>
 
 #include <cstddef>
@@ -9,9 +9,9 @@
 namespace {
 struct Rule {
     size_t lo = 1, hi = 0;  // no size
-    int skip = 0, error = 0, failed = 0;
+    int skip = 0, error = 0, times = 0, failed = 0;
     bool hit(size_t bytes) {
-        if (bytes < lo || bytes > hi) return false;
+        if (bytes < lo || bytes > hi || failed == times) return false;
         if (skip > 0) {
             --skip;
             return false;
@@ -45,8 +45,10 @@ int hipHostMalloc(void **p, size_t bytes, unsigned flags) {
     return host_rule.error;
 }
 
-void fail_device(size_t lo, size_t hi, int skip, int error) { device_rule = Rule{lo, hi, skip, error, 0}; }
-void fail_host(size_t lo, size_t hi, int skip, int error) { host_rule = Rule{lo, hi, skip, error, 0}; }
+void fail_device(size_t lo, size_t hi, int skip, int error, int times) {
+    device_rule = Rule{lo, hi, skip, error, times, 0};
+}
+void fail_host(size_t lo, size_t hi, int skip, int error, int times) { host_rule = Rule{lo, hi, skip, error, times, 0}; }
 int failed_device() { return device_rule.failed; }
 int failed_host() { return host_rule.failed; }
 }
