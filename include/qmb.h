@@ -224,7 +224,8 @@ typedef struct {
     int32_t fixed_iter;  /* 1: run exactly max_iter steps, no test (reference semantics) */
     int32_t start;       /* QMB_START_RANDOM, QMB_START_USER or QMB_START_DEVICE */
     int32_t want_eigvec; /* 1: the ground-state vector too, from the Lanczos vectors (kept in
-                            up to a quarter of the free memory; else by a second pass) */
+                            up to a quarter of the free memory while the call runs; 1 GiB of it
+                            stays with the context; else by a second pass) */
     int32_t profile;     /* k > 0: time every k-th SpMV (steps 0, k, 2k, ...) with HIP events */
     double tol;          /* eigenvalue tolerance, relative to max(1,|E|) (0 -> 1e-13) */
     uint64_t seed;       /* start-vector seed (reference default 2212456) */

@@ -92,6 +92,11 @@ struct DevPool {
                 return p;
             }
         }
+        cap = n;
+        return fresh(n);
+    }
+    // A block from the device; the cache is emptied when there is none.
+    void *fresh(size_t n) {
         void *p = nullptr;
         hipError_t e = hipMalloc(&p, n);
         if (e == hipErrorOutOfMemory) {
@@ -104,7 +109,6 @@ struct DevPool {
             throw Error{e == hipErrorOutOfMemory ? QMB_ERR_OOM : QMB_ERR_HIP,
                         std::string("hipMalloc: ") + hipGetErrorString(e)};
         }
-        cap = n;
         return p;
     }
     size_t cached_bytes() {
@@ -191,6 +195,16 @@ struct DevBuf {
             cap = n;
         }
         bytes = n;
+    }
+    // A block that goes back to the device, not to the pool.
+    void alloc_own(size_t n) {
+        release();
+        if (DevPool *from = current_pool()) {
+            p = from->fresh(n);
+            bytes = cap = n;
+        } else {
+            alloc(n);
+        }
     }
     void release() {
         if (p) {

@@ -1,6 +1,7 @@
 """Device memory that handles hold and that calls leave with the context, by the free
 memory of the device."""
 import ctypes as C
+import time
 
 import numpy as np
 import pytest
@@ -43,4 +44,30 @@ def test_kept_matrices_hold_what_they_report(n, n_up):
     print(f"held {held / 1e6:.1f} MB, limit {limit / 1e6:.1f} MB", flush=True)
     assert held <= limit
     del kept, b, t
+    c.close()
+
+
+@pytest.mark.gpu
+def test_kept_lanczos_vectors_are_given_back():
+    """A plain run for a vector keeps some 2.6 GB of Lanczos vectors while it runs; at most
+    1 GiB of them stays with the context."""
+    print("[gpu-case] kept Lanczos vectors given back", flush=True)
+    c = q.Context(0)
+    b, t = sector(c, 30, 15, 0)
+    e = q.Ell(c, b, t)
+    steps = 60
+    block = 16 * b.n_rows * 8
+    assert -(-steps // 16) * block > 2 * (1 << 30)
+    run = lambda vec: q.lanczos(e, max_iter=steps, fixed_iter=True, want_eigvec=vec, allow_unconverged=True)
+    run(False)
+    before = free_bytes()
+    run(True)
+    for _ in range(50):  # the device clears freed memory before it counts it as free
+        held = before - free_bytes()
+        if held <= (1 << 30) + (256 << 20):
+            break
+        time.sleep(0.1)
+    print(f"held {held / 1e6:.1f} MB", flush=True)
+    assert held <= (1 << 30) + (256 << 20)  # and the vector's own buffers
+    del e, b, t
     c.close()
