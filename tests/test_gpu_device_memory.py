@@ -8,7 +8,7 @@ import pytest
 
 import qmbcuda_amd as q
 import qmbcuda_amd.models as LM
-from helpers import DeviceBuffer
+from tests.helpers import DeviceBuffer
 
 
 def free_bytes():
