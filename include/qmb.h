@@ -334,7 +334,7 @@ qmb_status qmb_expectation(qmb_ctx *ctx, const qmb_basis *b, const qmb_terms *a,
  * re/im when is_complex); the result is the same as qmb_expectation's, bit for
  * bit. The per-block partial sums, the compiled terms and the group tables live
  * in a 1 MiB scratch array that the library keeps on each GPU until the process
- * ends: a table of more than 15292 terms is refused (QMB_ERR_INVALID; use
+ * ends: a table of more than 12233 terms is refused (QMB_ERR_INVALID; use
  * qmb_expectation). Every call on one GPU shares that scratch: calls that
  * overlap on one GPU (from several threads or contexts) race. */
 qmb_status qmb_expectation_noalloc(qmb_ctx *ctx, const qmb_basis *b, const qmb_terms *a, int is_complex,

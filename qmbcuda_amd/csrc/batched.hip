@@ -552,7 +552,7 @@ static void run_batched(qmb_ctx *ctx, int n, const qmb_ell *const *ells, const q
         const int M = ((o.max_iter + chunk - 1) / chunk) * chunk;
         const double tol = o.tol > 0 ? o.tol : 1e-13;
         const bool reorth = o.reorth != 0;
-        const bool partial = o.reorth == 2;  // device-side decisions (bk_pro)
+        const bool partial = o.reorth == 2;  // device-side decisions (estimate_loss)
         const int k_eigs = o.n_eigs;
 
         // per-instance device buffers

@@ -101,7 +101,6 @@ struct GroupLds {
     uint8_t small[kMaxGroup];
     uint8_t big[kMaxGroup];
     uint8_t flip[kMaxGroup];
-    uint8_t inv[kMaxGroup];
     uint8_t lut[kLutBytes];
     uint8_t cos[kCosBytes];
 };
@@ -112,7 +111,6 @@ __device__ inline void stage_group(GroupLds &t, const GroupView &g) {
         t.small[i] = g.small[i];
         t.big[i] = g.big[i];
         t.flip[i] = g.flip[i];
-        t.inv[i] = g.inv[i];
     }
     if (g.lut == 1 || g.lut == 2 || g.lut == 4)
         for (int i = threadIdx.x; i < kLutBytes; i += blockDim.x) t.lut[i] = g.lut_tab[i];
@@ -530,7 +528,7 @@ __host__ __device__ __forceinline__ unsigned ring_candidates(S y, int N, bool hf
     return tmin;
 }
 
-// ring_candidates with 64-bit masks.
+// ring_candidates with 64-bit masks for both widths: the form of the host check.
 template <class S>
 __host__ __device__ inline unsigned ring_windows(S y, int N, bool hf, uint64_t &c0, uint64_t &c1) {
     S a, b;

@@ -621,8 +621,6 @@ struct CodeTables {
     int n_chi = 0, n_m = 0;
 };
 
-__device__ inline uint32_t key_index(const unsigned long long *keys, int n, unsigned long long key, int *missing);
-
 // The value of a code, formed as the fill forms it (same operands, same operations,
 // no contraction).
 __device__ inline double2 code_value(int c, const CodeTables &ct, int cplx) {

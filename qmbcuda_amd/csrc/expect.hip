@@ -41,7 +41,7 @@ constexpr int kExpMaxBlocks = 4096;  // 2048: 87 us for 82 (28 sites)
 constexpr size_t kExpRankBytes = 16 * 1024;  // the nibble rank table's LDS
 constexpr int kExpLdsTerms = 256;
 
-// A product of Sz alone: 24 B and not a whole TermC, so that the few hundred of a
+// A product of Sz alone: 32 B and not a whole TermC (80), so that the few hundred of a
 // structure factor stay in the scalar cache (378 terms, 717K rows: 188 / 94 us).
 struct SzTerm {
     uint64_t sz;

@@ -357,7 +357,7 @@ struct qmb_ctx : qmb::Counted {
     size_t up_at = 0;
     hipEvent_t up_done = nullptr;  // after the last upload
     hipEvent_t stats_read = nullptr;  // after the read-back of a build's statistics
-    std::unique_ptr<qmb::PinnedBuf> bulk;  // slots of download_bulk (16 MB, made by the first large read-back)
+    std::unique_ptr<qmb::PinnedBuf> bulk;  // slots of download() (16 MB, made by the first read-back of 64 KB or more)
     ~qmb_ctx() {
         if (stream) {
             (void)hipSetDevice(device);

@@ -332,10 +332,9 @@ constexpr int kSmallThreads = 1024, kSmallWaves = kSmallThreads / 64;
 constexpr size_t kSmallLds = 140 * 1024;  // vector and words; value tables of up to 16 KB beside them
 // Doubles of the kept basis up to which a step of full reorthogonalisation is done by
 // one workgroup: beyond, one CU's reading of it takes longer than the launches of the
-// general route (to convergence, 1,768 complex rows, two levels: 1597 us with 100,000,
-// 1643 with 150,000, 1779 with 250,000, 2270 without; 2,704 rows 1409, 1480, 1480,
-// 1456; 1,367 rows 652 and 1457 without). It counts steps, not windows, so results
-// do not depend on check_every.
+// general route (to convergence, two levels, 1,768 complex rows: 1597 us with 100,000,
+// 1643 with 150,000, 1779 with 250,000, 2270 without; 1,367 rows 652 and 1457 without).
+// It counts steps, not windows, so results do not depend on check_every.
 constexpr int64_t kSmallBasis = 100000;
 constexpr size_t kSmallKeep = (size_t)64 << 20;  // the kept vectors of a small sector
 

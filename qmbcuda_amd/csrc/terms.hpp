@@ -1,6 +1,5 @@
 // Device form of a conjugated term table (the reference's BuildOperatorVecs
-// output, Q/exact_diagonalization/HeisenbergGenericXXZ_AbelianSymms_CUDA.cu:306-336)
-// and the application of one term to a basis state.
+// output, Q/exact_diagonalization/HeisenbergGenericXXZ_AbelianSymms_CUDA.cu:306-336).
 #pragma once
 
 #include <algorithm>
@@ -42,18 +41,6 @@ struct TermsView {
 // this does not depend on the state.
 inline bool is_diagonal(const TermC &c) { return c.set_val == (c.req_val & c.set); }
 inline bool never_acts(const TermC &c) { return (c.req_val & ~c.req) != 0; }
-
-// The term h on src. Returns false when the term annihilates src.
-template <class S>
-__device__ inline bool apply_term(const TermsView &tv, int h, S src, S &tgt, double &cr, double &ci) {
-    const TermC &t = tv.t[h];
-    if ((src & (S)t.req) != (S)t.req_val) return false;
-    tgt = (S)((src & (S)~(S)t.set) | (S)t.set_val);
-    const bool neg = (popc_s((S)(~src & (S)t.sz)) & 1) != 0;
-    cr = neg ? -t.coef.x : t.coef.x;
-    ci = neg ? -t.coef.y : t.coef.y;
-    return true;
-}
 
 // Host: the compiled form of term h of a table.
 inline TermC compile_term(const qmb_terms &tt, int h) {
